@@ -464,7 +464,7 @@ def attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
 
 # ---------------------------------------------------------------------------
 def gemm_tiled(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
-    """x [M, K] @ w [N, K]^T with float FMA chains (batch-invariant)."""
+    """x [M, K] @ w [N, K]^T in 32 bits, one chain of float fused multiply-adds an element (batch-invariant)."""
     _dev(x, w)
     _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1], f"gemm: x {tuple(x.shape)} vs w {tuple(w.shape)}")
     _need(x.dtype == w.dtype, "gemm: x and w must share a dtype")
@@ -935,7 +935,7 @@ def gemm_skinny_picked(x: torch.Tensor, w, ids: torch.Tensor, wts: Optional[torc
 
 
 def linear(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None, act: Optional[str] = None) -> torch.Tensor:
-    """y = x W^T, or f(x W^T) with ``act`` (an ungated activation: in the few-rows kernel's epilogue, else a kernel of its own).  float32 weights: the float FMA kernel (true 32-bit, whatever x was stored
+    """y = x W^T, or f(x W^T) with ``act`` (an ungated activation: in the few-rows kernel's epilogue, else a kernel of its own).  float32 weights: the float kernel (true 32-bit, whatever x was stored
     as).  bfloat16 weights stored tile by tile (a PackedWeight): the weight-streaming kernel for a
     few rows; beyond, the library's matrix product with float accumulation over the row-major
     copy, as the reference calls a library there (reference:

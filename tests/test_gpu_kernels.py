@@ -885,6 +885,37 @@ def test_gemm_tiled_is_a_true_float_product_and_batch_invariant(M, N, K):
         assert torch.equal(ops.gemm_tiled(x[M // 2:].contiguous(), w), got[M // 2:])
 
 
+@pytest.mark.parametrize("N,K", [(64, 32), (70, 36), (129, 35), (5200, 100), (3, 1)])
+def test_gemm_tiled_gives_the_same_rows_at_every_tile_height_and_in_groups(N, K):
+    """Tiles are 16, 32 or 64 rows high by the number of rows and columns; a row's bits are those of its product
+    alone, and in groups (empty ones, one row, edges of tiles) those of the plain product.  The bound
+    on the error is that of a chain of K fused multiply-adds."""
+    ops = _ops()
+    M = 300                                             # (at 5200 columns there are blocks enough for the tallest tile)
+    x, w = _rand(M, K, seed=3), _rand(N, K, seed=4)
+    full = ops.gemm_tiled(x, w)
+    exact = x.double() @ w.double().T
+    assert bool(((full.double() - exact).abs() <= K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all())
+    for rows in (1, 16, 17, 32, 33, 64, 65):
+        assert torch.equal(ops.gemm_tiled(x[7:7 + rows].contiguous(), w), full[7:7 + rows])
+    for counts in ([1, 0, 15, 16, 17], [0, 40, 24, 65, 0, 64, 3], [200]):
+        off = torch.tensor([0] + counts, device=DEV).cumsum(0).to(torch.int32)
+        n = sum(counts)
+        ws = _rand(len(counts), N, K, seed=5)
+        pick = torch.randperm(M, generator=torch.Generator().manual_seed(n))[:n].to(torch.int32).to(DEV)
+        got = ops.grouped_gemm(x, ws, off, pick, n)
+        for e, c in enumerate(counts):
+            if c:
+                a = int(off[e])
+                assert torch.equal(got[a:a + c], ops.gemm_tiled(x[pick[a:a + c].long()].contiguous(), ws[e].contiguous()))
+    # subnormal numbers stay, what is not finite passes on, and rows and columns keep to themselves
+    x[0], w[0] = 0.0, 0.0
+    x[0, 0], x[1, 0], x[2, 0], w[0, 0] = 2.0 ** -140, float("inf"), float("nan"), 1.0
+    got = ops.gemm_tiled(x, w)
+    assert float(got[0, 0]) == 2.0 ** -140 and float(got[1, 0]) == float("inf") and bool(got[2].isnan().all())
+    assert torch.equal(got[3:, 1:], full[3:, 1:])
+
+
 def test_the_library_says_which_head_sizes_its_attention_kernels_take():
     """The choice between the matrix-core kernels and the generic one asks the library: a head size is
     either compiled or goes to the generic kernel, which takes every size up to 256."""
