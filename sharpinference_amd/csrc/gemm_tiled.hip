@@ -1,10 +1,11 @@
 // C[M, N] = A[M, K] * W[N, K]^T in 32 bits, on the float matrix instruction (no reduced precision).
 //
 // The 32-bit path's matrix product, also the fallback for sizes the bfloat16 kernels refuse.
-// Every output element is one chain of float fused multiply-adds in an order of k that depends on
-// k alone (16 at a time; in each sixteen i, i + 4, i + 8, i + 12 for i = 0..3: a lane reads four
-// neighbouring k at once), so a row's result depends neither on how many other rows are in the batch
-// nor on where the row sits in it nor on the tile's height.  The grouped form runs E products at
+// Every output element is four chains of float fused multiply-adds, added at the end (their roundings are
+// half of one chain's), in an order of k that depends on k alone (of 32 k, chain 2 h + c takes places i, i + 4,
+// i + 8, i + 12 of sixteen number h, i = 2 c and 2 c + 1: a lane reads four neighbouring k at once), so a row's
+// result depends neither on how many other rows are in the batch nor on where the row sits in it nor on the
+// tile's height.  The grouped form runs E products at
 // once: rows [off[e], off[e+1]) of the (expert-sorted) row list use W[e]; A's rows may be gathered
 // through `a_rows`.
 //
@@ -19,6 +20,7 @@
 using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
 
 constexpr int BN = 64, BK = 32, LDK = BK + 4;
+constexpr int kChains = 4;
 constexpr int kTiledThreads = 256;
 
 // four consecutive elements at k; VEC: whole fours, aligned.  Places beyond the row are read inside it: `mask4` clears
@@ -130,11 +132,13 @@ __global__ __launch_bounds__(kTiledThreads) void gemm_tiled_kernel(const T* __re
 
   const int wr = (wid % WR) * RM * 16, wc = (wid / WR) * RN * 16;
   const int fr = lane & 15, fk = (lane >> 4) * 4;
-  f32x4 acc[RM][RN];
+  f32x4 acc[RM][RN][kChains];
 #pragma unroll
   for (int i = 0; i < RM; ++i)
 #pragma unroll
-    for (int j = 0; j < RN; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < RN; ++j)
+#pragma unroll
+      for (int c = 0; c < kChains; ++c) acc[i][j][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   auto products = [&](int buf) {
 #pragma unroll
@@ -149,8 +153,10 @@ __global__ __launch_bounds__(kTiledThreads) void gemm_tiled_kernel(const T* __re
 #pragma unroll
         for (int i = 0; i < RM; ++i)
 #pragma unroll
-          for (int j = 0; j < RN; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s], w[j][s], acc[i][j], 0, 0, 0);
+          for (int j = 0; j < RN; ++j) {
+            f32x4& c = acc[i][j][kk / 16 * 2 + s / 2];
+            c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s], w[j][s], c, 0, 0, 0);
+          }
     }
   };
   // Two pieces of k are on their way while one is multiplied; a buffer is written behind the barrier that ends its
@@ -181,7 +187,7 @@ __global__ __launch_bounds__(kTiledThreads) void gemm_tiled_kernel(const T* __re
 #pragma unroll
       for (int j = 0; j < RN; ++j) {
         const int n = n0 + wc + 16 * j + fr;
-        if (n < N) C[(size_t)m * N + n] = from_f32<TO>(acc[i][j][v]);
+        if (n < N) C[(size_t)m * N + n] = from_f32<TO>((acc[i][j][0][v] + acc[i][j][1][v]) + (acc[i][j][2][v] + acc[i][j][3][v]));
       }
     }
 }
