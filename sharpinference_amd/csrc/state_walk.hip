@@ -37,27 +37,17 @@
 // start states one after the other (for the gates, with m' = max(F + m, m_L):
 // S' = exp(F + m - m') S + exp(m_L - m') L); WALK_FINAL walks every segment from its start state,
 // writes the outputs, and the entry's last segment leaves the new state in the slot.
-#include "common.h"
+#include "state_walk.h"
 
-enum : int { WALK_EXP_GATES = 0, WALK_STATE_SPACE = 1, WALK_FIXED_DECAY = 2 };
 enum : int { WALK_WHOLE = 0, WALK_LOCAL = 1, WALK_FINAL = 2 };
-constexpr int kWalkCols = 8;       // value columns of a block
 constexpr int kWalkChunk = 8;      // tokens staged at a time
-constexpr float kWalkFloor = 1e-6f;
 
 SHARPI_EXPORT int sharpi_state_walk_cols() { return kWalkCols; }
 
-// floats of a slice: S, then (exponential gates) n and 8 floats that begin with m
-static inline __host__ __device__ int walk_slice_floats(int dkp, int mode) {
-  return (dkp / 8) * 64 + (mode == WALK_EXP_GATES ? dkp + 8 : 0);
-}
 SHARPI_EXPORT int sharpi_state_walk_slice_floats(int dk, int mode) {
   const int dkp = dk <= 32 ? 32 : dk <= 64 ? 64 : dk <= 128 ? 128 : 256;
   return walk_slice_floats(dkp, mode);
 }
-
-__device__ __forceinline__ float softplus_f32(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
-__device__ __forceinline__ float log_sigmoid_f32(float x) { return fminf(x, 0.f) - log1pf(expf(-fabsf(x))); }
 
 // 16 bytes of a row as floats
 __device__ __forceinline__ void load16(const float* p, float* v) {
@@ -82,7 +72,7 @@ __global__ __launch_bounds__(kWave) void state_walk_kernel(
     const int* __restrict__ state_slots, const int* __restrict__ cu_tokens, float* __restrict__ out, int nh, int dk,
     int dv, int ncb, int vec, const int* __restrict__ segs, float* __restrict__ seg_local,
     const float* __restrict__ seg_start, float* __restrict__ seg_decay, const int* __restrict__ positions,
-    const float* __restrict__ inv_freq, int rot_dim, float k_scale) {
+    const float* __restrict__ inv_freq, int rot_dim, float k_scale, int below) {
   constexpr int DKP = RPL * 8;
   constexpr int V = 16 / (int)sizeof(T);            // elements of a 16-byte load
   __shared__ __attribute__((aligned(16))) float q_s[PHASE == WALK_LOCAL ? 1 : kWalkChunk][DKP];     // (no outputs, no queries)
@@ -98,6 +88,7 @@ __global__ __launch_bounds__(kWave) void state_walk_kernel(
     e = blockIdx.z;
     t_first = cu_tokens[e];
     t_end = cu_tokens[e + 1];
+    if (t_end - t_first >= below) return;           // (the chunk form has the others)
   } else {
     const int* sg = segs + 4 * blockIdx.z;
     e = sg[0];
@@ -109,7 +100,7 @@ __global__ __launch_bounds__(kWave) void state_walk_kernel(
   if (t_end <= t_first) return;
   const size_t seg_at = (((size_t)blockIdx.z * nh + h) * ncb + cb) * slice;
   float* st = state + (((size_t)state_slots[e] * nh + h) * ncb + cb) * slice;      // the request's slot
-  const float* from = PHASE == WALK_FINAL ? seg_start + seg_at : st;
+  const float* from = PHASE == WALK_FINAL && !(last && t_first == cu_tokens[e]) ? seg_start + seg_at : st;   // (an entry's only segment starts from the slot)
   const int c = cb * kWalkCols + j;
   const int qk_head = h / heads_per_group;
 
@@ -329,7 +320,7 @@ __global__ __launch_bounds__(kCombineThreads) void state_walk_combine_kernel(
     int ncb, int dkp) {
   const int h = blockIdx.y, e = blockIdx.z;
   const int first = ent_segs[2 * e], count = ent_segs[2 * e + 1];
-  if (count <= 0) return;
+  if (count <= 1) return;                       // nothing (one segment starts from the slot)
   const int slice = walk_slice_floats(dkp, MODE);
   const int moved = (dkp / 8) * 64 + (MODE == WALK_EXP_GATES ? dkp : 0);     // S and n; the maximum lies behind them
   const int idx = blockIdx.x * kCombineThreads + threadIdx.x;              // over the head's slices
@@ -373,22 +364,13 @@ __global__ __launch_bounds__(kCombineThreads) void state_walk_combine_kernel(
   }
 }
 
-struct WalkArgs {
-  const void* proj; int stride, q_off, k_off, v_off, heads_per_group;
-  const float* gates; int gate_stride; const float *p0, *p1, *p2;
-  float cap, q_scale; float* state; const int *state_slots, *cu_tokens; float* out;
-  int n_entries, nh, dk, dv;
-  const int *segs, *ent_segs; int n_segs; float *seg_local, *seg_start, *seg_decay;
-  const int* positions; const float* inv_freq; int rot_dim; float k_scale;      // WALK_FIXED_DECAY
-};
-
 template <typename T, int RPL, int MODE, int PHASE>
-static void launch_walk_phase(const WalkArgs& a, int ncb, int vec, hipStream_t stream) {
+static void launch_walk_phase(const WalkArgs& a, int ncb, int vec, hipStream_t stream, int below = 0x7fffffff) {
   dim3 grid(ncb, a.nh, PHASE == WALK_WHOLE ? a.n_entries : a.n_segs);
   state_walk_kernel<T, RPL, MODE, PHASE><<<grid, kWave, 0, stream>>>(
       (const T*)a.proj, a.stride, a.q_off, a.k_off, a.v_off, a.heads_per_group, a.gates, a.gate_stride, a.p0, a.p1, a.p2,
       a.cap, a.q_scale, a.state, a.state_slots, a.cu_tokens, a.out, a.nh, a.dk, a.dv, ncb, vec, a.segs, a.seg_local,
-      a.seg_start, a.seg_decay, a.positions, a.inv_freq, a.rot_dim, a.k_scale);
+      a.seg_start, a.seg_decay, a.positions, a.inv_freq, a.rot_dim, a.k_scale, below);
 }
 
 template <typename T, int RPL, int MODE>
@@ -398,12 +380,24 @@ static int launch_walk_rpl(const WalkArgs& a, int ncb, int vec, hipStream_t stre
     SHARPI_CHECK_LAUNCH();
     return SHARPI_OK;
   }
-  launch_walk_phase<T, RPL, MODE, WALK_LOCAL>(a, ncb, vec, stream);
-  SHARPI_CHECK_LAUNCH();
+  constexpr int dtype = sizeof(T) == 4 ? DT_F32 : DT_BF16;
+  const bool chunks = state_chunk_takes(a, dtype);
+  if (chunks) {
+    const int rc = state_chunk_local(a, dtype, MODE, stream);
+    if (rc != SHARPI_OK) return rc;
+    if (a.n_entries > 1 || a.n_segs < 2) {          // (one entry of several segments: nothing short)
+      launch_walk_phase<T, RPL, MODE, WALK_WHOLE>(a, ncb, vec, stream, state_chunk_from());
+      SHARPI_CHECK_LAUNCH();
+    }
+  } else {
+    launch_walk_phase<T, RPL, MODE, WALK_LOCAL>(a, ncb, vec, stream);
+    SHARPI_CHECK_LAUNCH();
+  }
   const int moved = RPL * 64 + (MODE == WALK_EXP_GATES ? RPL * 8 : 0);
   state_walk_combine_kernel<MODE><<<dim3(ceil_div(ncb * moved, kCombineThreads), a.nh, a.n_entries), kCombineThreads, 0, stream>>>(
       a.state, a.state_slots, a.ent_segs, a.seg_local, a.seg_start, a.seg_decay, a.nh, ncb, RPL * 8);
   SHARPI_CHECK_LAUNCH();
+  if (chunks) return state_chunk_final(a, dtype, MODE, stream);
   launch_walk_phase<T, RPL, MODE, WALK_FINAL>(a, ncb, vec, stream);
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;

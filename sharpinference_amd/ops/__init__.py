@@ -464,7 +464,7 @@ def attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
 
 # ---------------------------------------------------------------------------
 def gemm_tiled(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
-    """x [M, K] @ w [N, K]^T in 32 bits, one chain of float fused multiply-adds an element (batch-invariant)."""
+    """x [M, K] @ w [N, K]^T in 32 bits, chains of float fused multiply-adds (batch-invariant)."""
     _dev(x, w)
     _need(x.dim() == 2 and w.dim() == 2 and x.shape[1] == w.shape[1], f"gemm: x {tuple(x.shape)} vs w {tuple(w.shape)}")
     _need(x.dtype == w.dtype, "gemm: x and w must share a dtype")
@@ -1681,6 +1681,11 @@ def _walk_rows(dk: int) -> int:
     return 32 if dk <= 32 else 64 if dk <= 64 else 128 if dk <= 128 else 256
 
 
+def walk_takes_chunks(dk: int, dv: int) -> bool:
+    """Whether :func:`state_walk` runs its segments as matrix products at these sizes (csrc/state_chunk.hip)."""
+    return _lib.state_chunk_takes(dk, dv)
+
+
 def walk_state_shape(nh: int, dk: int, dv: int, mode: int) -> tuple:
     """A request's recurrent state as the walk keeps it: [heads, ceil(dv / 8), slice].  A slice holds 8
     value columns: DKP x 8 floats of the matrix (DKP = dk rounded up to 32 / 64 / 128 / 256; row
@@ -1731,7 +1736,8 @@ def state_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, heads_per
     segment by segment side by side.  A stretch of tokens acts on the state as S -> D S + L (D the product of
     its decays, one number a head; L what it makes of a zero state), so every segment is first walked from
     nothing, the true start states follow one from the other, and a second walk from those writes the
-    outputs (results equal to rounding).  Returns float32 [T, nh * dv]."""
+    outputs (results equal to rounding); at the sizes of :func:`walk_takes_chunks` both passes are matrix
+    products over the segment instead of walks.  Returns float32 [T, nh * dv]."""
     _dev(proj, gates, state, inv_freq, *params)
     T, N = proj.shape
     groups = nh // heads_per_group if heads_per_group > 0 else 0

@@ -172,6 +172,16 @@ def latent_attention_takes(rank: int, dr: int) -> bool:
     return _takes[key]
 
 
+def state_chunk_takes(dk: int, dv: int) -> bool:
+    """Whether a recurrent state with one decay a head, dk x dv, takes long entries in chunk form."""
+    key = ("state chunk", int(dk), int(dv))
+    if key not in _takes:
+        fn = load().sharpi_state_chunk_takes
+        fn.argtypes, fn.restype = [c_int, c_int], c_int
+        _takes[key] = bool(fn(int(dk), int(dv)))
+    return _takes[key]
+
+
 def delta_chunk_floats(n_chunks: int, nh: int, dk: int, dv: int) -> int:
     """Scratch floats of the gated delta rule's chunked form."""
     fn = load().sharpi_delta_chunk_floats

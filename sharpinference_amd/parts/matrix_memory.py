@@ -11,7 +11,7 @@ from .. import ops
 from ..cache.spec import MixedSpec, StateSpec
 from ..ops.profile import section
 from .base import INIT_NORM_WEIGHT, LayerCache, ParamSpec, Part, StepContext, TensorSource
-from .linear_attention import SEGMENT_UP_TO_BLOCKS, WALK_SEGMENTS
+from .linear_attention import WALK_SEGMENTS, segments_for
 
 
 def _fuse(parts, hidden: int) -> torch.Tensor:
@@ -24,11 +24,18 @@ def _fuse(parts, hidden: int) -> torch.Tensor:
     return fused
 
 
-def _segments_for(ctx: StepContext, nh: int, dv: int):
-    """The step's segment lists where a walk of whole entries would leave the chip idle (a long entry alone
-    in its step), else None."""
-    whole_blocks = ctx.n_entries * nh * ((dv + ops.WALK_STATE_COLS - 1) // ops.WALK_STATE_COLS)
-    return ctx.extras.get(WALK_SEGMENTS.key) if whole_blocks < SEGMENT_UP_TO_BLOCKS else None
+def _segments_for(ctx: StepContext, nh: int, dk: int, dv: int, turned: bool = False):
+    """The step's segment lists where this layer takes them.  Segments that run as matrix products pay by the
+    microseconds measured of both forms (16 to 64 heads, steps of 16 to 8,192 tokens): a walk takes 0.6 for every token
+    of the longest entry, more where the entries' blocks exceed what the chip holds at once (2,500); the products take
+    35 and 0.0017 for every token and 128 value columns, 1.4 times that where q and k are turned first (``turned``).
+    Other sizes: the rule of the walks."""
+    if not ops.walk_takes_chunks(dk, dv):
+        return segments_for(ctx, nh, dv, ops.WALK_STATE_COLS)
+    blocks = ctx.n_entries * nh * (dv // ops.WALK_STATE_COLS)
+    walk = 0.6 * ctx.max_entry_len * max(1.0, blocks / 2500)
+    products = 35.0 + 0.0017 * ctx.n_tokens * nh * dv / 128 * (1.4 if turned else 1.0)
+    return ctx.extras.get(WALK_SEGMENTS.key) if walk > products else None
 
 
 class MatrixMemory(Part):
@@ -113,7 +120,7 @@ class MatrixMemory(Part):
                      flops=4.0 * T * qk * self.dv):
             o = ops.state_walk(proj, 0, qk, 2 * qk, 1, gates, (self.b_i, self.b_f), self.cap, self.dk ** -0.5,
                                ops.WALK_EXP_GATES, state, ctx, self.nh, self.dk, self.dv,
-                               segments=_segments_for(ctx, self.nh, self.dv))
+                               segments=_segments_for(ctx, self.nh, self.dk, self.dv))
         with section("head norm + gate", nbytes=T * vv * (4 + 2 * width)):
             y = ops.group_norm_gate(o, self.w_norm, self.eps, self.nh, ctx.act_dtype, proj, 2 * qk + vv, ops.GATE_SIGMOID_ACT)
         with section("o", nbytes=width * self.hidden * (vv + T) + width * T * vv, flops=2.0 * T * self.hidden * vv):
@@ -216,7 +223,7 @@ class StateSpaceMixer(Part):
                      flops=4.0 * T * self.nh * self.N * self.dv):
             y = ops.state_walk(xbc, self.inner + self.G * self.N, self.inner, 0, self.nh // self.G, dt,
                                (self.dt_bias, self.a_log, self.d_skip), 0.0, 1.0, ops.WALK_STATE_SPACE, states[0], ctx,
-                               self.nh, self.N, self.dv, segments=_segments_for(ctx, self.nh, self.dv))
+                               self.nh, self.N, self.dv, segments=_segments_for(ctx, self.nh, self.N, self.dv))
         with section("head norm + gate", nbytes=T * self.inner * (4 + 2 * width)):
             y = ops.group_norm_gate(y, self.w_norm, self.eps, self.norm_groups, ctx.act_dtype, proj, 0, ops.GATE_SILU, gate_first=True)
         with section("o", nbytes=width * self.hidden * (self.inner + T) + width * T * self.inner, flops=2.0 * T * self.hidden * self.inner):
@@ -292,7 +299,7 @@ class Retention(Part):
         with section("recurrence", nbytes=lambda: 8 * ctx.n_entries * qk * self.dv + T * (width * (2 * qk + vv) + 4 * vv),
                      flops=4.0 * T * qk * self.dv):
             o = ops.state_walk(proj, 0, qk, 2 * qk, 1, None, (self._decay_t,), 0.0, 1.0, ops.WALK_FIXED_DECAY, state, ctx,
-                               self.nh, self.dk, self.dv, segments=_segments_for(ctx, self.nh, self.dv),
+                               self.nh, self.dk, self.dv, segments=_segments_for(ctx, self.nh, self.dk, self.dv, turned=True),
                                inv_freq=self.rotary.table(x.device) if self.rotary is not None else None,
                                k_scale=self.dk ** -0.5)
         with section("head norm + gate", nbytes=T * vv * (4 + 2 * width)):
