@@ -34,7 +34,8 @@ __host__ __device__ inline int plan_parts(int n_sib) { return n_sib <= 2 ? 2 : n
 // what a unit weighs when units are dealt to the XCDs: its share of the group's (siblings x column blocks)
 __host__ __device__ inline int plan_weight(int n_sib) { return n_sib * (kPlanMaxParts / plan_parts(n_sib)); }
 // column blocks [first, first + count) of part `part` of `parts`, of nb column blocks in all
-__host__ __device__ inline int plan_part_first(int part, int parts, int nb) { return (int)((long long)part * nb / parts); }
+// (parts is a power of two)
+__host__ __device__ inline int plan_part_first(int part, int parts, int nb) { return (int)((unsigned)part * (unsigned)nb / (unsigned)parts); }
 __host__ __device__ inline int plan_units_per_xcd_max(int n_groups) { return (kPlanMaxParts * n_groups + kPlanXcds - 1) / kPlanXcds + 1; }
 __host__ __device__ inline int plan_stride(int n_groups) { return 1 + 4 * plan_units_per_xcd_max(n_groups); }
 // behind the XCDs' unit lists: one ticket counter per XCD (the next slot of that XCD's walk to hand
