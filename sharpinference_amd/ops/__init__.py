@@ -672,6 +672,53 @@ def attention_latent(q: torch.Tensor, rows: torch.Tensor, group, ctx, scale: flo
     return out
 
 
+LATENT_PAGE_KEYS = _lib.LATENT_PAGE_KEYS      # keys of a page of expanded latents
+
+
+def latent_expand_ok(dtype: torch.dtype, dn: int, dr: int, dv: int, rank: int) -> bool:
+    """Whether a step's latents can be expanded into keys and values of these widths, and the flash kernel takes those."""
+    return _lib.latent_expand_takes(dn, dr, dv, rank) and prefill_attention_ok(dtype, dn + dr, dv)
+
+
+def latent_expand(rows: torch.Tensor, group, pages: torch.Tensor, w_ukv: torch.Tensor, dn: int, dr: int, dv: int,
+                  rank: int) -> Tuple[torch.Tensor, torch.Tensor]:
+    """The cached rows (rows [pages, 1, page_size, rank + dr] behind group.block_table) of the listed pages of 128 keys
+    (int32 [n, 4] = (entry, page of its sequence, first key that is there, end of the keys that are there)) as keys and
+    values of every head: K [n, heads, 128, dn + dr] with the shared rotated part behind each head's own, V [n, heads,
+    dv, 128].  w_ukv [heads, dn + dv, rank]: a head's key rows, then its value rows.  Keys that are not there hold
+    the nearest one's values."""
+    _dev(rows, pages, w_ukv, group.block_table)
+    _i32(pages, "pages")
+    _i32(group.block_table, "block_table")
+    _need(latent_expand_ok(rows.dtype, dn, dr, dv, rank), "latent_expand: these widths are not taken")
+    _need(rows.dim() == 4 and rows.shape[1] == 1 and rows.shape[3] == rank + dr, "latent_expand: rows [pages, 1, page_size, rank + dr]")
+    _need(w_ukv.dtype == rows.dtype and w_ukv.dim() == 3 and tuple(w_ukv.shape[1:]) == (dn + dv, rank), "latent_expand: w_ukv [heads, dn + dv, rank]")
+    _need(pages.dim() == 2 and pages.shape[1] == 4, "latent_expand: pages [n, 4]")
+    n, nh = pages.shape[0], w_ukv.shape[0]
+    k = torch.empty(n, nh, LATENT_PAGE_KEYS, dn + dr, dtype=rows.dtype, device=rows.device)
+    v = torch.empty(n, nh, dv, LATENT_PAGE_KEYS, dtype=rows.dtype, device=rows.device)
+    _run("sharpi_latent_expand", _ptr(rows), _ptr(group.block_table), _ptr(pages), _ptr(w_ukv), _ptr(k), _ptr(v), n, nh, dn, dr, dv,
+         rank, rows.shape[2], group.block_table.shape[1], rows.shape[0], _stream())
+    return k, v
+
+
+def latent_queries(q: torch.Tensor, positions: torch.Tensor, inv_freq: Optional[torch.Tensor], magnitude: float, nh: int, dn: int,
+                   dr: int) -> torch.Tensor:
+    """The leading nh * (dn + dr) columns of q [T, N] as [T, nh * (dn + dr)], every head's last dr elements turned (as in
+    :func:`latent_prep`)."""
+    _dev(q, positions, inv_freq)
+    _i32(positions, "positions")
+    T = q.shape[0]
+    _need(q.dim() == 2 and q.dtype == torch.bfloat16 and q.shape[1] >= nh * (dn + dr) and q.shape[1] % 8 == 0 and positions.shape == (T,),
+          "latent_queries: q bfloat16 [T, a multiple of 8 columns], positions [T]")
+    _need(inv_freq is None or (inv_freq.dtype == torch.float32 and inv_freq.dim() == 1 and 2 * inv_freq.shape[0] <= dr),
+          "latent_queries: inv_freq float32 [pairs], 2 * pairs <= dr")
+    out = torch.empty(T, nh * (dn + dr), dtype=q.dtype, device=q.device)
+    _run("sharpi_latent_queries", _ptr(q), q.shape[1], _ptr(positions), _ptr(inv_freq), inv_freq.shape[0] if inv_freq is not None else 0,
+         float(magnitude), _ptr(out), T, nh, dn, dr, _stream())
+    return out
+
+
 # ---------------------------------------------------------------------------
 # weights stored for streaming
 # ---------------------------------------------------------------------------

@@ -75,6 +75,8 @@ _SIGNATURES = {
     "sharpi_lowrank": [P, I, I, I, I, I, P, I, P, P, I, P, I, I, P, I, P, P],
     "sharpi_delta_step": [P, I, I, I, P, I, P, P, P, I, I, P, P, P, P, I, I, I, I, I, F, P, F, P, P, P],
     "sharpi_delta_chunks": [P, I, I, I, P, I, P, P, P, I, I, P, P, P, P, I, I, I, I, I, F, P, P, I, P, P, P],
+    "sharpi_latent_expand": [P, P, P, P, P, P, I, I, I, I, I, I, I, I, I, P],
+    "sharpi_latent_queries": [P, I, P, P, I, F, P, I, I, I, I, P],
     "sharpi_map_difference": [P, I, F, F, F, P, I, I, P, I, I, I, P],
 }
 
@@ -91,6 +93,7 @@ ROUTER_MAX_EXPERTS = 1024   # experts the routing kernels hold scores for
 GLA_STATE_COLS = 8          # value columns of a linear-attention state that lie together in memory
 WALK_STATE_COLS = 8         # value columns of a slice of a scalar-decay recurrent state (csrc/state_walk.hip)
 DELTA_CHUNK_TOKENS = 16     # tokens of a chunk of the gated delta rule (csrc/delta_rule.hip)
+LATENT_PAGE_KEYS = 128      # keys of a page of expanded latents (csrc/latent_expand.hip)
 _BUILT_WITH = {
     "sharpi_attention_decode_split_keys": DECODE_RUN_KEYS,
     "sharpi_attention_prefill_tile_tokens": PREFILL_TILE_TOKENS,
@@ -100,6 +103,7 @@ _BUILT_WITH = {
     "sharpi_gla_state_cols": GLA_STATE_COLS,
     "sharpi_state_walk_cols": WALK_STATE_COLS,
     "sharpi_delta_chunk_tokens": DELTA_CHUNK_TOKENS,
+    "sharpi_latent_page_keys": LATENT_PAGE_KEYS,
 }
 
 
@@ -169,6 +173,16 @@ def latent_attention_takes(rank: int, dr: int) -> bool:
         fn = load().sharpi_attention_latent_mfma_takes
         fn.argtypes, fn.restype = [c_int, c_int], c_int
         _takes[key] = bool(fn(int(rank), int(dr)))
+    return _takes[key]
+
+
+def latent_expand_takes(dn: int, dr: int, dv: int, rank: int) -> bool:
+    """Whether keys of dn + dr and values of dv elements a head are expanded from latents of `rank` elements."""
+    key = ("expand", int(dn), int(dr), int(dv), int(rank))
+    if key not in _takes:
+        fn = load().sharpi_latent_expand_takes
+        fn.argtypes, fn.restype = [c_int] * 4, c_int
+        _takes[key] = bool(fn(*key[1:]))
     return _takes[key]
 
 

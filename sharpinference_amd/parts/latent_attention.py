@@ -1,15 +1,59 @@
 """The latent attention mixer: keys and values of all heads kept as one low-rank row per token."""
 from __future__ import annotations
 
-from typing import Dict, Optional, Tuple
+from types import SimpleNamespace
+from typing import Dict, List, Optional, Tuple
 
+import numpy as np
 import torch
 
 from .. import ops
-from ..cache.spec import KVSpec, WINDOW_NONE
+from ..cache.spec import KVSpec, WINDOW_NONE, WINDOW_SLIDING
 from ..ops.profile import section
 from .attention import _WORK_LISTS
-from .base import LayerCache, ParamSpec, Part, StepContext, TensorSource
+from .base import HostStep, LayerCache, ParamSpec, Part, StepContext, StepPlanner, TensorSource
+
+
+# A step's prompt portions attend over expanded keys and values where the (query, key) pairs they hold are at least
+# EXPAND_FROM_TOKENS times the keys to expand (a key's expansion costs about what 28 pairs save), and, times the heads, at
+# least EXPAND_FROM_PAIRS (the two launches more).  Microseconds of a step through four such layers over the shared rows
+# and over expanded keys: 64 heads behind 2,000 keys, 32 tokens 1,338 / 1,268, 128: 2,210 / 1,488, 512: 4,655 / 1,844;
+# behind none, 64 tokens 695 / 698, 128: 853 / 757, 512: 1,691 / 1,054; 16 heads behind 2,000, 32 tokens 1,118 / 777;
+# behind none, 128 tokens 661 / 713, 512: 872 / 705.
+EXPAND_FROM_TOKENS = 32
+EXPAND_FROM_PAIRS = 1 << 19
+EXPAND_MAX_BYTES = 2 << 30         # ... and the expanded keys and values take at most this much for the layer's time
+
+
+class LatentPages(StepPlanner):
+    """The pages of 128 keys that a step's prompt portions see through a window: the list of them (entry, page of its
+    sequence, first key that is there, end of the keys) and the block table of a cache that holds just them."""
+
+    def __init__(self, window_kind: int, window: int):
+        self.spec = KVSpec(1, 1, window_kind, window)
+        self.key = f"latent pages {window_kind} {window}"
+
+    def plan(self, host: HostStep) -> Tuple[List[np.ndarray], dict]:
+        long = [e for e, n in enumerate(host.lens) if n > 1]
+        pages, spans, pairs = [], [], 0
+        for e in long:
+            lo, hi = self.spec.first_visible(host.starts[e]), host.starts[e] + host.lens[e]
+            first, end = lo // ops.LATENT_PAGE_KEYS, (hi - 1) // ops.LATENT_PAGE_KEYS + 1
+            spans.append((e, first, len(pages), end - first))
+            pages += [(e, b, lo, hi) for b in range(first, end)]
+            pairs += host.lens[e] * (hi - lo)
+        table = np.full((host.n_entries, max((f + n for _, f, _, n in spans), default=0)), -1, dtype=np.int32)
+        for e, first, at, n in spans:
+            table[e, first:first + n] = np.arange(at, at + n, dtype=np.int32)
+        single = [int(host.cu_tokens[e]) for e, n in enumerate(host.lens) if n == 1]
+        rows = (single[0], single[-1] + 1) if single and single[-1] - single[0] + 1 == len(single) else None
+        return [np.asarray(pages, dtype=np.int32).reshape(-1), table.reshape(-1)], dict(
+            pages=len(pages), entries=host.n_entries, pairs=pairs, keys=sum(n for *_, n in spans) * ops.LATENT_PAGE_KEYS,
+            decode_rows=rows, scattered=bool(single) and rows is None)
+
+    def attach(self, ctx: StepContext, views: List[torch.Tensor], facts: dict) -> None:
+        n = facts["pages"]
+        ctx.extras[self.key] = (views[0].view(n, 4), views[1].view(facts["entries"], -1), facts) if n else None
 
 
 class LatentAttention(Part):
@@ -19,12 +63,15 @@ class LatentAttention(Part):
     With h the input: q = W_q h, per head [dn unrotated | dr rotated]; W_dkv h gives rank + dr
     elements, the first rank RMS-normed (weight ``dkv.norm``) into c, the last dr rotated into the
     shared key part.  A head's unrotated key is W_uk c and its value W_uv c; its score against a
-    key is (q_n . W_uk c + q_r . k_r) * scale.  Neither keys nor values are ever formed: the
+    key is (q_n . W_uk c + q_r . k_r) * scale.  Neither keys nor values are kept: the
     unrotated query is taken through W_uk first (q_n^T W_uk) c, so that all heads attend over the
     cached rows [c | k_r] themselves (the score is one dot product over rank + dr elements, the
     weighted sum of the rows' first rank elements is taken through W_uv afterwards).  Softmax in
     float, with ``sink``: one learned term exp(sink_h) more in the denominator, without key or
     value.  With ``gate`` the heads' outputs are multiplied by sigmoid(W_g h) before W_o.
+    Prompt portions of some length are the exception: for them the keys and values of the rows they see are
+    expanded, used in the flash kernel and dropped (csrc/latent_expand.hip), which costs a third of the
+    products; the cache is the same.
 
     ``q_rank``: queries come through a latent of their own, q = W_uq rms_norm(W_dq h) (weight
     ``dq.norm``), instead of W_q h.
@@ -66,13 +113,15 @@ class LatentAttention(Part):
         self.w_in = None                                   # [q (or dq) | g | dkv] rows: one product of the input
         self.w_uk_t: Optional[torch.Tensor] = None         # [heads, rank, dn]: W_uk per head, transposed
         self.w_uv: Optional[torch.Tensor] = None           # [heads, dv, rank]
+        self.w_ukv: Optional[torch.Tensor] = None          # [heads, dn + dv, rank]: both row by row, where prompts expand keys
+        self.pages = LatentPages(self.window_kind, self.window)
         self.w_o = None
         self.w_norm: Optional[torch.Tensor] = None         # float32 [rank]
         self.w_sink: Optional[torch.Tensor] = None         # float32 [heads]
 
     # -- what it needs --------------------------------------------------------
     def step_planners(self):
-        return (_WORK_LISTS,)
+        return (_WORK_LISTS, self.pages)
 
     def cache_spec(self) -> KVSpec:
         return KVSpec(1, self.rank + self.dr, *self.kept, self.rank, values_in_keys=True)
@@ -149,6 +198,9 @@ class LatentAttention(Part):
         uk = source.get(prefix + n["uk"]).to(dt)
         self.w_uk_t = uk.view(self.nh, self.dn, self.rank).transpose(1, 2).contiguous()
         self.w_uv = source.get(prefix + n["uv"]).to(dt).view(self.nh, self.dv, self.rank).contiguous()
+        # (with a gate per output element the shared form rounds once, behind the gate; the flash kernel would round before it too)
+        if dt == torch.bfloat16 and uk.is_cuda and not self.has_gate and ops.latent_expand_ok(dt, self.dn, self.dr, self.dv, self.rank):
+            self.w_ukv = torch.cat([uk.view(self.nh, self.dn, self.rank), self.w_uv], dim=1).contiguous()
         self.w_o = ops.pack_weight(source.get(prefix + n["o"]))
         if self.has_sink:
             self.w_sink = source.get(prefix + n["sink"]).float().contiguous()
@@ -167,36 +219,88 @@ class LatentAttention(Part):
         store = self.own_latent and cache.write
         if self.own_latent and not cache.write:
             raise ValueError("a latent layer with a down projection of its own must own its cache")
-        q_full = torch.empty(T, self.nh * D, dtype=ctx.act_dtype, device=x.device)
         inv_freq = self.rotary.table(x.device) if self.rotary is not None else None
         rows = (cache.k, g.slot_mapping) if store else (None, None)
         common = (ctx.positions, inv_freq, self.w_norm, self.eps, self.nh, self.dn, self.dr, self.rank)
         magnitude = getattr(self.rotary, "magnitude", 1.0)
+        pages = self._pages_to_expand(ctx, proj)
+        q_full = None if pages is not None else torch.empty(T, self.nh * D, dtype=ctx.act_dtype, device=x.device)
         if self.q_rank:
             with section("latents + cache write", nbytes=width * T * (2 * self.q_rank + 2 * D)):
                 cq = ops.latent_prep(None, 0, kv_off if store else None, None, *rows, *common, magnitude=magnitude, kv=proj,
                                      q_latent=(proj, 0, self.w_q_norm))
             with section("uq", nbytes=width * (self.q_dim * self.q_rank + T * (self.q_rank + self.q_dim)), flops=2.0 * T * self.q_dim * self.q_rank):
                 q = ops.linear(cq, self.w_uq, ctx.act_dtype)
-            with section("rotary", nbytes=width * T * 2 * self.nh * self.dr):
-                ops.latent_prep(q, 0, None, q_full, None, None, *common, magnitude=magnitude)
+            if q_full is not None:
+                with section("rotary", nbytes=width * T * 2 * self.nh * self.dr):
+                    ops.latent_prep(q, 0, None, q_full, None, None, *common, magnitude=magnitude)
         else:
             q = proj
-            with section("latent + rotary + cache write", nbytes=width * T * (2 * self.nh * self.dr + 2 * D)):
-                ops.latent_prep(q, 0, kv_off if store else None, q_full, *rows, *common, magnitude=magnitude)
+            if q_full is not None or store:
+                with section("latent + rotary + cache write", nbytes=width * T * (2 * self.nh * self.dr + 2 * D)):
+                    ops.latent_prep(q, 0, kv_off if store else None, q_full, *rows, *common, magnitude=magnitude)
+        gate = proj if self.has_gate else None
+        if pages is not None:
+            o = self._attend_expanded(q, pages, ctx, cache, inv_freq, magnitude)
+        else:
+            o = torch.empty(T, self.o_dim, dtype=ctx.act_dtype, device=x.device)
+            self._attend_shared(q, q_full, gate, g_off, o, ctx, cache)
+        with section("o", nbytes=width * self.hidden * (self.o_dim + T) + width * T * self.o_dim, flops=2.0 * T * self.hidden * self.o_dim):
+            return ops.linear(o, self.w_o, ctx.act_dtype)
+
+    def _attend_shared(self, q: torch.Tensor, q_full: torch.Tensor, gate: Optional[torch.Tensor], g_off: int, o: torch.Tensor, ctx,
+                       cache: LayerCache) -> None:
+        """Attention over the shared rows into o [T, o_dim]: queries through W_uk (q_full holds their rotated parts), the
+        weighted latents through W_uv."""
+        T, D, width = q.shape[0], self.rank + self.dr, q.element_size()
         with section("q through uk", nbytes=width * (self.nh * self.dn * self.rank + T * self.nh * (self.dn + self.rank)),
                      flops=2.0 * T * self.nh * self.dn * self.rank):
             ops.head_gemm(q, 0, self.dn + self.dr, self.w_uk_t, q_full, 0, D)
         with section("attention", nbytes=lambda: self._keys_held(ctx) * D * width + T * self.nh * (D + self.rank) * width,
                      flops=lambda: 2.0 * self._keys_read(ctx) * self.nh * (D + self.rank)):
-            o_lat = ops.attention_latent(q_full, cache.k, g, ctx, self.scale, self.nh, self.rank, self.dr, sink=self.w_sink,
+            o_lat = ops.attention_latent(q_full, cache.k, cache.group, ctx, self.scale, self.nh, self.rank, self.dr, sink=self.w_sink,
                                          window_kind=self.window_kind, window=self.window)
-        o = torch.empty(T, self.o_dim, dtype=ctx.act_dtype, device=x.device)
         with section("uv + gate", nbytes=width * (self.o_dim * self.rank + T * (self.nh * self.rank + 2 * self.o_dim)),
                      flops=2.0 * T * self.o_dim * self.rank):
-            ops.head_gemm(o_lat, 0, self.rank, self.w_uv, o, 0, self.dv, gate=proj if self.has_gate else None, gate_off=g_off)
-        with section("o", nbytes=width * self.hidden * (self.o_dim + T) + width * T * self.o_dim, flops=2.0 * T * self.hidden * self.o_dim):
-            return ops.linear(o, self.w_o, ctx.act_dtype)
+            ops.head_gemm(o_lat, 0, self.rank, self.w_uv, o, 0, self.dv, gate=gate, gate_off=g_off)
+
+    def _pages_to_expand(self, ctx: StepContext, proj: torch.Tensor):
+        """The step's pages where its prompt portions attend over expanded keys and values, else None: bfloat16 layers of
+        widths the kernels take, portions long enough to pay for the expansion, the single tokens (which keep to the
+        shared rows) side by side in the batch."""
+        if self.w_ukv is None or ctx.act_dtype != torch.bfloat16 or proj.shape[1] % 8 or self.window_kind not in (WINDOW_NONE, WINDOW_SLIDING):
+            return None
+        pages = ctx.extras.get(self.pages.key)
+        if pages is None or pages[2]["scattered"]:
+            return None
+        facts = pages[2]
+        size = 2 * facts["keys"] * self.nh * (self.dn + self.dr + self.dv)
+        pays = facts["pairs"] >= EXPAND_FROM_TOKENS * facts["keys"] and facts["pairs"] * self.nh >= EXPAND_FROM_PAIRS
+        return pages if pays and size <= EXPAND_MAX_BYTES else None
+
+    def _attend_expanded(self, q: torch.Tensor, pages, ctx: StepContext, cache: LayerCache, inv_freq: Optional[torch.Tensor],
+                         magnitude: float) -> torch.Tensor:
+        listed, table, facts = pages
+        T, hd = q.shape[0], self.dn + self.dr
+        with section("expand uk, uv", nbytes=2 * facts["keys"] * (self.rank + self.dr + self.nh * (hd + self.dv)),
+                     flops=2.0 * facts["keys"] * self.nh * (self.dn + self.dv) * self.rank):
+            k, v = ops.latent_expand(cache.k, cache.group, listed, self.w_ukv, self.dn, self.dr, self.dv, self.rank)
+        with section("rotary", nbytes=2 * T * 2 * self.nh * hd):
+            qr = ops.latent_queries(q, ctx.positions, inv_freq, magnitude, self.nh, self.dn, self.dr)
+        with section("attention", nbytes=2 * (facts["keys"] + T) * self.nh * (hd + self.dv),
+                     flops=lambda: 2.0 * self._keys_read(ctx) * self.nh * (hd + self.dv)):
+            o = ops.attention_prefill(qr, k, v, table, ctx.positions, ctx.prefill_tiles, self.window_kind, self.window, self.scale, self.nh,
+                                      self.nh, hd, tile_tokens=ctx.prefill_tile_tokens, sink=self.w_sink, vd=self.dv)
+        if facts["decode_rows"] is not None:
+            a, b = facts["decode_rows"]
+            alone = SimpleNamespace(entry_of_token=ctx.entry_of_token[a:b], positions=ctx.positions[a:b], n_decode=b - a, decode_tokens=None,
+                                    n_prefill_tiles=0, entry_lens=[1] * (b - a),
+                                    entry_starts=[s for s, n in zip(ctx.entry_starts, ctx.entry_lens) if n == 1])
+            q_full = torch.empty(b - a, self.nh * (self.rank + self.dr), dtype=q.dtype, device=q.device)
+            ops.latent_prep(q[a:b], 0, None, q_full, None, None, alone.positions, inv_freq, self.w_norm, self.eps, self.nh, self.dn, self.dr,
+                            self.rank, magnitude=magnitude)
+            self._attend_shared(q[a:b], q_full, None, 0, o[a:b], alone, cache)
+        return o
 
     def _keys_read(self, ctx: StepContext) -> int:
         spec = KVSpec(1, 1, self.window_kind, self.window)
