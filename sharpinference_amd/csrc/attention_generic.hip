@@ -1,7 +1,7 @@
 // Attention over the paged cache, one block per (token, head), float arithmetic throughout.
 //
-// This is the reference-grade kernel: it serves the 32-bit path for every size and stands in
-// for the tiled kernels on sizes they refuse.  The keys of a query at position p are
+// This is the reference-grade kernel: it serves the 32-bit path for the sizes attention_float.hip is not compiled
+// for and stands in for the tiled kernels on sizes they refuse.  The keys of a query at position p are
 // [start, p] with start = 0 (all keys), floor(p / W) * W (chunk-local) or max(0, p - W + 1)
 // (sliding).  Keys are visited in blocks of 64 dealt round-robin to the block's four waves, so
 // the order of every sum depends on (start, p) alone: not on how the tokens were batched.
@@ -133,6 +133,13 @@ __global__ __launch_bounds__(kAttnWaves* kWave) void attn_generic_kernel(
   }
 }
 
+// the float matrix instruction's form (attention_float.hip)
+bool attention_float_takes(const void* q, const void* k, const void* v, const void* out, int hd, int vd, int page_size);
+int attention_float(const float* q, const float* k, const float* v, const int* block_table, const int* entry_of_token,
+                    const int* positions, float* out, int window_kind, int window, float scale, int n_tokens, int nh, int nkv, int hd,
+                    int vd, int page_size, int max_blocks, int num_pages, float softcap, int sink, const float* sink_vals, int keep,
+                    const float* gate, int gate_stride, hipStream_t stream);
+
 SHARPI_EXPORT int sharpi_attention_generic(const void* q, const void* k_cache, const void* v_cache, int dtype,
                                            const int* block_table, const int* entry_of_token,
                                            const int* positions, void* out, int window_kind, int window,
@@ -144,6 +151,10 @@ SHARPI_EXPORT int sharpi_attention_generic(const void* q, const void* k_cache, c
   if (page_size <= 0 || max_blocks <= 0 || num_pages <= 0) return SHARPI_ERR_ARG;
   if (window_kind < 0 || window_kind > 2 || (window_kind != 0 && window <= 0) || !(softcap >= 0.f)) return SHARPI_ERR_ARG;
   if (keep < 0 || (gate && gate_stride < nh)) return SHARPI_ERR_ARG;
+  if (dtype == DT_F32 && attention_float_takes(q, k_cache, v_cache, out, hd, vd, page_size))
+    return attention_float((const float*)q, (const float*)k_cache, (const float*)v_cache, block_table, entry_of_token, positions,
+                           (float*)out, window_kind, window, scale, n_tokens, nh, nkv, hd, vd, page_size, max_blocks, num_pages,
+                           softcap, sink, sink_vals, window_kind == 0 ? 0 : keep, (const float*)gate, gate_stride, stream);
   dim3 grid(n_tokens, nh), block(kAttnWaves * kWave);
   if (dtype == DT_F32)
     attn_generic_kernel<float><<<grid, block, 0, stream>>>(
