@@ -291,7 +291,94 @@ __device__ __forceinline__ void wave_dot_rows(const T* const (&xr)[TT], const TW
   for (int i = 0; i < TT; ++i) out[i] = wave_sum(s[i]);
 }
 
-template <typename T, typename TW, int TT>
+// Eight neighbouring elements as they lie in memory.
+template <typename T> struct Run8;
+template <> struct Run8<float> {
+  float4 a, b;
+  __device__ __forceinline__ void load(const float* p) {
+    a = *reinterpret_cast<const float4*>(p);
+    b = *reinterpret_cast<const float4*>(p + 4);
+  }
+  __device__ __forceinline__ void floats(float (&v)[8]) const {
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  }
+};
+template <> struct Run8<bf16_t> {
+  uint4 a;
+  __device__ __forceinline__ void load(const bf16_t* p) { a = *reinterpret_cast<const uint4*>(p); }
+  __device__ __forceinline__ void floats(float (&v)[8]) const { load8(reinterpret_cast<const bf16_t*>(&a), v); }
+};
+
+// One wave: the EE x TT products of EE router rows and TT token rows, bit for bit those of wave_dot_rows (the same chain
+// a lane, the lanes added in the same pairs); hidden % 8 == 0.  What bounds it: a row read for one product
+// costs the cache's 64 bytes a cycle more than its eight multiply-adds a lane, so a row is read for EE or TT of them,
+// the next run's loads are sent before this run is added (not at 16 products, where they cost the registers that let
+// the block's other waves cover them), and the lanes' sums go up the tree together: half of them by half of the lanes.  Lane v * 64 / (EE * TT) returns product v = ee * TT + i.
+template <typename T, typename TW, int EE, int TT>
+__device__ __forceinline__ float wave_dots(const T* const (&xr)[TT], const TW* const (&wrow)[EE], int hidden, int lane) {
+  constexpr int N = EE * TT;
+  float s[N];
+#pragma unroll
+  for (int v = 0; v < N; ++v) s[v] = 0.f;
+  const auto add = [&](const Run8<TW> (&wc)[EE], const Run8<T> (&xc)[TT]) {
+    float a[TT][8];
+#pragma unroll
+    for (int i = 0; i < TT; ++i) xc[i].floats(a[i]);
+#pragma unroll
+    for (int e = 0; e < EE; ++e) {
+      float b[8];
+      wc[e].floats(b);
+#pragma unroll
+      for (int i = 0; i < TT; ++i)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) s[e * TT + i] = fmaf(a[i][j], b[j], s[e * TT + i]);
+    }
+  };
+  const auto load = [&](int c, Run8<TW> (&wc)[EE], Run8<T> (&xc)[TT]) {
+#pragma unroll
+    for (int e = 0; e < EE; ++e) wc[e].load(wrow[e] + c);
+#pragma unroll
+    for (int i = 0; i < TT; ++i) xc[i].load(xr[i] + c);
+  };
+  int c = lane * 8;
+  if constexpr (N == 16) {
+    for (; c < hidden; c += kWave * 8) {
+      Run8<TW> wc[EE];
+      Run8<T> xc[TT];
+      load(c, wc, xc);
+      add(wc, xc);
+    }
+  } else {
+    Run8<TW> w0[EE], w1[EE];
+    Run8<T> x0[TT], x1[TT];
+    if (c < hidden) load(c, w0, x0);
+    while (c < hidden) {
+      const int c1 = c + kWave * 8, c2 = c1 + kWave * 8;
+      if (c1 < hidden) load(c1, w1, x1);
+      __builtin_amdgcn_sched_barrier(0);
+      add(w0, x0);
+      if (c1 >= hidden) break;
+      if (c2 < hidden) load(c2, w0, x0);
+      __builtin_amdgcn_sched_barrier(0);
+      add(w1, x1);
+      c = c2;
+    }
+  }
+  int off = kWave / 2;
+#pragma unroll
+  for (int m = N / 2; m > 0; m >>= 1, off >>= 1) {
+    const bool high = lane & off;
+#pragma unroll
+    for (int v = 0; v < m; ++v) {
+      const float other = __shfl_xor(high ? s[v] : s[v + m], off, kWave);
+      s[v] = (high ? s[v + m] : s[v]) + other;
+    }
+  }
+  for (; off > 0; off >>= 1) s[0] += __shfl_xor(s[0], off, kWave);
+  return s[0];
+}
+
+template <typename T, typename TW, int EE, int TT>
 __global__ __launch_bounds__(1024) void router_topk_kernel(const T* __restrict__ x, const TW* __restrict__ wr,
                                                            int* __restrict__ topk_ids,
                                                            float* __restrict__ topk_w,
@@ -309,7 +396,17 @@ __global__ __launch_bounds__(1024) void router_topk_kernel(const T* __restrict__
   const T* xr[TT];
 #pragma unroll
   for (int i = 0; i < TT; ++i) xr[i] = x + (size_t)min(t0 + i, n_tokens - 1) * hidden;   // beyond the last: computed, not kept
-  for (int e = w; e < n_experts; e += nw) {
+  if constexpr (EE > 0) {
+    constexpr int N = EE * TT, W = kWave / N;
+    for (int e0 = w * EE; e0 < n_experts; e0 += nw * EE) {
+      const TW* wrow[EE];
+#pragma unroll
+      for (int x = 0; x < EE; ++x) wrow[x] = wr + (size_t)min(e0 + x, n_experts - 1) * hidden;
+      const float v = wave_dots<T, TW, EE, TT>(xr, wrow, hidden, lane);
+      const int e = e0 + lane / W / TT;
+      if (lane % W == 0 && e < n_experts) g[lane / W % TT][e] = bias ? v + bias[e] : v;
+    }
+  } else for (int e = w; e < n_experts; e += nw) {
     float v[TT];
     wave_dot_rows<T, TW, TT>(xr, wr + (size_t)e * hidden, hidden, lane, v);
     if (lane == 0) {
@@ -442,21 +539,29 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
   if (n_groups < 1 || keep < 1 || keep > n_groups || n_experts % n_groups != 0 || k > keep * (n_experts / n_groups)) return SHARPI_ERR_ARG;
   if (group_top < 1 || group_top > kMaxGroupTop) return SHARPI_ERR_ARG;
   const int split_choice = corr != nullptr || keep < n_groups;
-  // one wave per expert at a time: enough waves for the experts, at most 16; with many tokens four
-  // share a block (and each fetch of a router row)
-  const int tt = n_tokens >= 64 ? 4 : 1;
+  // What it measured (one expert a wave, four tokens a block from 64 tokens before): 3000 rows 2048 wide of 128 experts
+  // 90 -> 56 us, 64 rows 4096 wide 47 -> 19, 1660 rows 2048 wide of 64 experts with float weights 36 -> 32; 16 experts the same (latency).
+  // Few tokens, or rows that cannot be read in runs of 8: a block a token, a wave an expert at a time (enough waves for the
+  // experts, at most 16).  From 64 tokens: four experts a wave (one where there are fewer than 64 experts: each wave has
+  // one then), for four tokens a block where a token a block would be more than one block a compute unit.
+  const bool runs = (hidden & 7) == 0 && n_tokens >= 64;
+  const int tt = runs ? (n_tokens > 256 ? 4 : 1) : n_tokens >= 64 ? 4 : 1;
+  const int ee = !runs ? 0 : n_experts >= 64 ? 4 : 1;
   dim3 grid(ceil_div(n_tokens, tt)), block(kWave * (n_experts >= 16 ? 16 : n_experts >= 8 ? 8 : 4));
   const size_t lds = split_choice ? (size_t)tt * (n_experts + n_groups) * sizeof(float) : 0;
+#define ROUTER_LAUNCH_AT(TX, TWT, EEV, TTV)                                                                      \
+  router_topk_kernel<TX, TWT, EEV, TTV><<<grid, block, lds, stream>>>((const TX*)x, (const TWT*)wr, topk_ids, topk_w, \
+                                                                      gate_out, n_tokens, hidden, n_experts, k, gate, \
+                                                                      renorm, corr, n_groups, keep, split_choice, bias, w_scale, group_top)
 #define ROUTER_LAUNCH(TX, TWT)                                                                                   \
   do {                                                                                                           \
-    if (tt == 4)                                                                                                 \
-      router_topk_kernel<TX, TWT, 4><<<grid, block, lds, stream>>>((const TX*)x, (const TWT*)wr, topk_ids, topk_w, \
-                                                                 gate_out, n_tokens, hidden, n_experts, k, gate, \
-                                                                 renorm, corr, n_groups, keep, split_choice, bias, w_scale, group_top); \
-    else                                                                                                         \
-      router_topk_kernel<TX, TWT, 1><<<grid, block, lds, stream>>>((const TX*)x, (const TWT*)wr, topk_ids, topk_w, \
-                                                                 gate_out, n_tokens, hidden, n_experts, k, gate, \
-                                                                 renorm, corr, n_groups, keep, split_choice, bias, w_scale, group_top); \
+    if (ee == 4) {                                                                                               \
+      if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, 4, 4); else ROUTER_LAUNCH_AT(TX, TWT, 4, 1);                        \
+    } else if (ee == 1) {                                                                                        \
+      if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, 1, 4); else ROUTER_LAUNCH_AT(TX, TWT, 1, 1);                        \
+    } else {                                                                                                     \
+      if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, 0, 4); else ROUTER_LAUNCH_AT(TX, TWT, 0, 1);                        \
+    }                                                                                                            \
   } while (0)
   if (x_dtype == DT_F32 && w_dtype == DT_F32) ROUTER_LAUNCH(float, float);
   else if (x_dtype == DT_BF16 && w_dtype == DT_BF16) ROUTER_LAUNCH(bf16_t, bf16_t);
@@ -464,32 +569,61 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
   else if (x_dtype == DT_F32 && w_dtype == DT_BF16) ROUTER_LAUNCH(float, bf16_t);
   else return SHARPI_ERR_ARG;
 #undef ROUTER_LAUNCH
+#undef ROUTER_LAUNCH_AT
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
 }
 
-// One block: the expert-sorted list of the (token, pick) pairs; count and cursor are LDS of
-// n_experts ints.  Every thread of the block calls it; the pairs must be visible to the block.
+// One block: the expert-sorted list of the (token, pick) pairs; cursor is LDS of n_experts ints, count and
+// plan_scratch of one more.  Every thread of the block calls it; the pairs must be visible to the block.
+//
+// Bound: latency, one block's chain of loads, counters and sums.  So a thread has eight pairs in flight, one wave
+// makes the prefix sum, and every group counts the units before its own from one number a group (one thread's
+// walks over the groups and a pair a round trip: 18000 pairs of 128 experts 48 -> 32, 512 pairs 26 -> 13 us).
+constexpr unsigned kPlanRankParts = 32;        // (above kPlanMaxParts)
 __device__ void permute_block(const int* __restrict__ topk_ids, const float* __restrict__ topk_w,
                               int* __restrict__ offsets, int* __restrict__ sorted_token,
                               float* __restrict__ sorted_w, int* __restrict__ inv_pos, int* __restrict__ plan,
                               int n_pairs, int k, int n_experts, int shared_group, int* count, int* cursor,
                               int* plan_scratch) {
-  for (int e = threadIdx.x; e < n_experts; e += blockDim.x) count[e] = 0;
+  constexpr int kAhead = 8;                  // pairs a thread has in flight: one block is alone with its loads' latency
+  const int step = blockDim.x;
+  for (int e = threadIdx.x; e < n_experts; e += step) count[e] = 0;
   __syncthreads();
-  for (int i = threadIdx.x; i < n_pairs; i += blockDim.x)
-    if (topk_ids[i] < n_experts) atomicAdd(&count[topk_ids[i]], 1);
+  for (int i0 = threadIdx.x; i0 < n_pairs; i0 += kAhead * step) {
+    int id[kAhead];
+#pragma unroll
+    for (int x = 0; x < kAhead; ++x) id[x] = topk_ids[min(i0 + x * step, n_pairs - 1)];
+#pragma unroll
+    for (int x = 0; x < kAhead; ++x)
+      if (i0 + x * step < n_pairs && id[x] < n_experts) atomicAdd(&count[id[x]], 1);
+  }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    int run = 0;
-    for (int e = 0; e < n_experts; ++e) {
+  if (threadIdx.x < kWave) {                 // one wave's prefix sum: a lane a run of neighbouring experts
+    const int per = (n_experts + kWave - 1) / kWave, e0 = min((int)threadIdx.x * per, n_experts), e1 = min(e0 + per, n_experts);
+    int mine = 0;
+    for (int e = e0; e < e1; ++e) mine += count[e];
+    int run = mine;                          // inclusive over the lanes, then what lies before the lane's own
+#pragma unroll
+    for (int off = 1; off < kWave; off <<= 1) {
+      const int o = __shfl_up(run, off, kWave);
+      if ((int)threadIdx.x >= off) run += o;
+    }
+    const int all = __shfl(run, kWave - 1, kWave);
+    run -= mine;
+    for (int e = e0; e < e1; ++e) {
       offsets[e] = run;
       cursor[e] = run;
       run += count[e];
     }
-    offsets[n_experts] = run;
-    // an always-on expert as one more group: every token once, in token order, with weight 1
-    if (shared_group) offsets[n_experts + 1] = run + n_pairs / k;
+    if (threadIdx.x == 0) {
+      offsets[n_experts] = all;
+      // an always-on expert as one more group: every token once, in token order, with weight 1
+      if (shared_group) {
+        offsets[n_experts + 1] = all + n_pairs / k;
+        count[n_experts] = n_pairs / k;
+      }
+    }
   }
   if (shared_group) {
     for (int t = threadIdx.x; t < n_pairs / k; t += blockDim.x) {
@@ -504,31 +638,24 @@ __device__ void permute_block(const int* __restrict__ topk_ids, const float* __r
     // row, rows alternating in direction so that the XCDs' loads stay level.
     const int n_groups = n_experts + (shared_group ? 1 : 0);
     const int stride = plan_stride(n_groups);
-    if (shared_group && threadIdx.x == 0) count[n_experts] = n_pairs / k;
     __syncthreads();
-    // unit_base[g]: units of the groups before g (in cursor's place it would clash: a second array)
-    int* unit_base = plan_scratch;
-    if (threadIdx.x == 0) {
-      int run = 0;
-      for (int g = 0; g < n_groups; ++g) {
-        unit_base[g] = run;
-        if (count[g] > 0) run += plan_parts(plan_siblings(count[g]));
-      }
-      unit_base[n_groups] = run;
+    // a group's weight and units as one number that orders groups as the deal does and tells their units; 0: no rows
+    int* rank = plan_scratch;
+    for (int g = threadIdx.x; g < n_groups; g += step) {
+      const int sg = plan_siblings(count[g]);
+      rank[g] = count[g] == 0 ? 0 : plan_weight(sg) * (int)kPlanRankParts + plan_parts(sg);
     }
     __syncthreads();
-    const int units = unit_base[n_groups];
-    for (int g = threadIdx.x; g < n_groups; g += blockDim.x) {
+    for (int g = threadIdx.x; g < n_groups; g += step) {
       if (count[g] == 0) continue;
       const int sg = plan_siblings(count[g]);
       const int wg = plan_weight(sg), pg = plan_parts(sg);
       // units that come before this group's: of heavier groups all, of equally heavy ones those of lower index
       int before = 0;
+#pragma unroll 8
       for (int j = 0; j < n_groups; ++j) {
-        if (count[j] == 0 || j == g) continue;
-        const int sj = plan_siblings(count[j]);
-        const int wj = plan_weight(sj);
-        if (wj > wg || (wj == wg && j < g)) before += plan_parts(sj);
+        const int wj = (unsigned)rank[j] / kPlanRankParts;
+        before += wj > wg || (wj == wg && j < g) ? (unsigned)rank[j] % kPlanRankParts : 0;
       }
       for (int part = 0; part < pg; ++part) {
         const int u = before + part;
@@ -541,29 +668,43 @@ __device__ void permute_block(const int* __restrict__ topk_ids, const float* __r
         pu[3] = sg;
       }
     }
-    if (threadIdx.x < kPlanXcds) {
-      // XCD x holds one unit of every full row of 8, and of the last row the units that exist
-      const int x = threadIdx.x;
-      int n = 0;
-      for (int pos = 0; pos * kPlanXcds < units; ++pos) {
-        const int u = pos * kPlanXcds + ((pos & 1) ? kPlanXcds - 1 - x : x);
-        if (u < units) ++n;
+    if (threadIdx.x >= kWave && threadIdx.x < 2 * kWave) {       // (the second wave: the first has groups to place)
+      int units = 0;
+      for (int g = threadIdx.x - kWave; g < n_groups; g += kWave) units += (unsigned)rank[g] % kPlanRankParts;
+#pragma unroll
+      for (int off = kWave / 2; off > 0; off >>= 1) units += __shfl_xor(units, off, kWave);
+      const int x = threadIdx.x - kWave;
+      if (x < kPlanXcds) {
+        // XCD x holds one unit of every full row of 8, and of the last row its own if it exists
+        const int rows = units / kPlanXcds, left = units % kPlanXcds;
+        plan[x * stride] = rows + (((rows & 1) ? kPlanXcds - 1 - x : x) < left ? 1 : 0);
       }
-      plan[x * stride] = n;
     }
     if (threadIdx.x < kPlanCounters) plan[plan_counters_at(n_groups) + threadIdx.x] = 0;
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < n_pairs; i += blockDim.x) {
-    const int e = topk_ids[i];
-    if (e >= n_experts) {                // an identity expert: no product, no row (whoever sums the pairs asks the id)
-      inv_pos[i] = 0;
-      continue;
+  for (int i0 = threadIdx.x; i0 < n_pairs; i0 += kAhead * step) {
+    int id[kAhead], row[kAhead];
+    float wt[kAhead];
+#pragma unroll
+    for (int x = 0; x < kAhead; ++x) {
+      const int i = min(i0 + x * step, n_pairs - 1);
+      id[x] = topk_ids[i];
+      wt[x] = topk_w[i];
     }
-    const int r = atomicAdd(&cursor[e], 1);
-    sorted_token[r] = i / k;
-    sorted_w[r] = topk_w[i];
-    inv_pos[i] = r;
+#pragma unroll
+    for (int x = 0; x < kAhead; ++x)
+      row[x] = i0 + x * step < n_pairs && id[x] < n_experts ? atomicAdd(&cursor[id[x]], 1) : -1;
+#pragma unroll
+    for (int x = 0; x < kAhead; ++x) {
+      const int i = i0 + x * step;
+      if (i >= n_pairs) break;
+      if (row[x] >= 0) {
+        sorted_token[row[x]] = (unsigned)i / (unsigned)k;
+        sorted_w[row[x]] = wt[x];
+      }
+      inv_pos[i] = max(row[x], 0);       // (an identity expert: no product, no row; whoever sums the pairs asks the id)
+    }
   }
 }
 
@@ -576,7 +717,7 @@ __global__ __launch_bounds__(1024) void moe_permute_kernel(const int* __restrict
                                                            int n_pairs, int k, int n_experts, int shared_group) {
   __shared__ int count[kMaxExperts + 1];
   __shared__ int cursor[kMaxExperts];
-  __shared__ int plan_scratch[kMaxExperts + 2];
+  __shared__ int plan_scratch[kMaxExperts + 1];
   permute_block(topk_ids, topk_w, offsets, sorted_token, sorted_w, inv_pos, plan, n_pairs, k, n_experts,
                 shared_group, count, cursor, plan_scratch);
 }
