@@ -3,15 +3,18 @@
 // first R elements.
 //
 // A block of eight waves works on up to 64 (token, head) rows of one request against one run of
-// keys [run * RUN, (run + 1) * RUN): 16 rows (16 heads of a token, or all heads of several
-// consecutive tokens where a layer has fewer than 16) belong to a pair of waves, each of which
-// forms the scores and the softmax state of the rows (the same bits in both) and one half of their
-// output elements, so that a wave's accumulators take 64 registers for a latent of 512 and two
-// waves fit a SIMD.
-// Keys come in chunks of 32, staged in LDS once for the block: the rows as they lie in the cache
-// (the A operand of S^T = K Q^T, contraction over elements), and their first R elements once more,
-// transposed [element][key] (the A operand of O^T = V^T P^T, contraction over keys), made from the
-// staged rows by the block itself, so the cache holds every latent once.  Probabilities enter the
+// keys [run * RUN, (run + 1) * RUN).  16 rows (16 heads of a token, or all heads of several
+// consecutive tokens where a layer has fewer than 16) are a row group; a prompt's block has four of them, a
+// single token's as many as its heads fill, and the eight waves are dealt evenly: each of a group's 2, 4 or 8 waves
+// has its softmax state (the same bits in all) and a slice of its output elements.
+// Keys come in chunks of 32, staged in LDS once for the block, as they lie in the cache: the A operand of S^T = K Q^T
+// (contraction over elements) as rows, and, through the transposing LDS read, the A operand of O^T = V^T P^T
+// (contraction over keys).  The group's first two waves form 16 keys' scores each and leave them for the others.
+// Bound: with four row groups the LDS reads of keys and values; for single tokens of 16 heads the chain of a chunk
+// (fetch, scores, softmax, values), so the slices are small, two blocks fit a compute unit and a chunk is fetched
+// ahead.  (With two waves a group whatever the rows, scores formed twice and a transposed copy of every chunk, 64
+// single tokens of 16 heads over 1500 keys of 576 took 88 us, now 46; 110 MB, 16 us at the memory's rate.)
+// Probabilities enter the
 // second product as a bfloat16 pair hi + lo; the softmax state is float.  A row whose keys lie in
 // one run is finished here (with the sink term, if any); a row with more runs leaves (max, sum,
 // unnormalised output) per run, and the merge kernel adds the runs in ascending order and applies
@@ -23,15 +26,16 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-constexpr int kLmWaves = 4;           // row groups of 16 rows a block
-constexpr int kLmHalves = 2;          // waves a row group: each takes half of the output elements
+typedef __attribute__((__vector_size__(4 * sizeof(short)))) short s16x4;
+
+constexpr int kLmWaves = 8;           // waves a block
+constexpr int kLmGroups = 4;          // row groups of 16 rows a block, at most
 constexpr int kLmChunk = 32;          // keys a chunk
-constexpr int kLmVtLd = kLmChunk + 8; // elements a row of the transposed tile (rows 16 bytes apart in banks)
 
 struct LmGeom {
   int H, R, D, d32, r16;   // heads, latent width, row width, 32-element steps of a row, 16-element tiles of the output
   int hpw, tb;             // heads and tokens of a wave's 16 rows
-  int htb, tgb;            // head tiles and token groups of a block's four waves
+  int htb, tgb;            // head tiles and token groups of a block's row groups
   int ldk;                 // elements a staged row takes in LDS
 };
 
@@ -42,25 +46,36 @@ __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
 // the first key a query at position p sees (window 0: all earlier ones)
 __device__ __forceinline__ int first_seen(int p, int window) { return window > 0 && p >= window ? p - window + 1 : 0; }
 
-template <int MAXD32, int MAXR16>
-__global__ __launch_bounds__(kLmWaves* kLmHalves* kWave) void attn_latent_mfma_kernel(
+// four keys' (rows ld elements apart) values of one of 16 neighbouring elements a lane: lane l of 16 gives the address of
+// row l / 4, elements 4 (l % 4) on, and receives element l of the four rows
+__device__ __forceinline__ s16x4 read_transposed(const bf16_t* p) {
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)p);
+}
+
+// S waves a row group, 8 / S groups a block.
+template <int MAXD32, int MAXR16, int S>
+__global__ __launch_bounds__(kLmWaves* kWave, S == 8 ? 4 : 2) void attn_latent_mfma_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ rows, const int* __restrict__ block_table,
     const int* __restrict__ entry_of_token, const int* __restrict__ positions, const int* __restrict__ tiles,
     const int* __restrict__ token_list, int tile_subs, const float* __restrict__ sink, bf16_t* __restrict__ out,
     float* __restrict__ part_o, float* __restrict__ part_ml, float scale, LmGeom gm, int run_keys, int max_runs,
     int page_size, int max_blocks, int num_pages, int window) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-  bf16_t* kt = reinterpret_cast<bf16_t*>(smem);                    // [32][ldk]
-  bf16_t* vt = kt + kLmChunk * gm.ldk;                             // [R][kLmVtLd], keys in the order the second product wants
+  constexpr int GR = kLmWaves / S;
+  constexpr bool kQueriesInLds = S == 8;                           // (the registers of two blocks a compute unit)
+  f32x4* ex = reinterpret_cast<f32x4*>(smem);                      // [GR][2][64]: scores on their way to a group's waves
+  bf16_t* kt = reinterpret_cast<bf16_t*>(ex + GR * 2 * kWave);     // [32][ldk]
+  bf16_t* qs = kt + kLmChunk * gm.ldk;                             // [16][ldk], where the queries are in LDS
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  const int w = (tid >> 6) & (kLmWaves - 1), half = tid >> 8;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), w = wv % GR, slice = wv / GR;
   const int g = lane >> 4, m16 = lane & 15;
   const int tpb = gm.tgb * gm.tb;
-  // this wave's 16-element tiles of the output: the first or the second half of them
-  constexpr int MAXH = (MAXR16 + 1) / 2;
-  const int r_lo = half ? (gm.r16 + 1) / 2 : 0;
-  const int r_n = half ? gm.r16 - r_lo : (gm.r16 + 1) / 2;
+  // this wave's 16-element tiles of the output
+  constexpr int MAXH = (MAXR16 + S - 1) / S;
+  const int r_lo = min(slice * ((gm.r16 + S - 1) / S), gm.r16);
+  const int r_n = min((gm.r16 + S - 1) / S, gm.r16 - r_lo);
 
   // the block's tokens: a piece of a prompt tile, or one listed token
   int tok0, cnt, e;
@@ -95,15 +110,21 @@ __global__ __launch_bounds__(kLmWaves* kLmHalves* kWave) void attn_latent_mfma_k
   const int k_row = first_seen(p_row, window);      // the first key this row sees
   const bool wave_ok = __any(row_ok);
 
-  bf16x8 qf[MAXD32];
-  {
-    const bf16_t* qrow = q + ((size_t)token * gm.H + (row_ok ? head : 0)) * gm.D;
+  bf16x8 qf[kQueriesInLds ? 1 : MAXD32];
+  const bf16_t* qrow = q + ((size_t)token * gm.H + (row_ok ? head : 0)) * gm.D;
+  const auto query = [&](int j) {
+    uint4 v = make_uint4(0, 0, 0, 0);
+    const int d = 32 * j + 8 * g;
+    if (j < gm.d32 && row_ok && d < gm.D) v = *reinterpret_cast<const uint4*>(qrow + d);
+    return v;
+  };
+  if constexpr (kQueriesInLds) {           // (one group: the block's waves share its steps)
+    for (int j = wv; j < gm.d32; j += kLmWaves) *reinterpret_cast<uint4*>(qs + m16 * gm.ldk + 32 * j + 8 * g) = query(j);
+  } else {
 #pragma unroll
     for (int j = 0; j < MAXD32; ++j) {
-      uint4 v = make_uint4(0, 0, 0, 0);
-      const int d = 32 * j + 8 * g;
-      if (j < gm.d32 && row_ok && d < gm.D) v = *reinterpret_cast<const uint4*>(qrow + d);
-      qf[j] = *reinterpret_cast<bf16x8*>(&v);
+      const uint4 v = query(j);
+      qf[j] = *reinterpret_cast<const bf16x8*>(&v);
     }
   }
   // the columns of the staged rows beyond D stay zero
@@ -136,7 +157,7 @@ __global__ __launch_bounds__(kLmWaves* kLmHalves* kWave) void attn_latent_mfma_k
   };
   // (with the widest rows the registers do not reach for rows held across the products: they are
   // then requested where they are stored, and the SIMD's other wave covers the wait)
-  constexpr bool kAhead = MAXD32 <= 10;
+  constexpr bool kAhead = MAXD32 <= 10 || S > 2;
   const bf16_t* cur_row = row_of(k_begin);
   if (kAhead) fetch(cur_row);
   const bf16_t* next_row = row_of(k_begin + kLmChunk);
@@ -149,37 +170,37 @@ __global__ __launch_bounds__(kLmWaves* kLmHalves* kWave) void attn_latent_mfma_k
       const int c8 = st_c + 16 * j;
       if (c8 < d8) *reinterpret_cast<uint4*>(kt + st_r * gm.ldk + 8 * c8) = stage[j];
     }
-    if (kAhead) fetch(next_row);           // the next chunk's rows are on their way while this one is transposed and multiplied
+    if (kAhead) fetch(next_row);           // the next chunk's rows are on their way while this one is multiplied
     cur_row = next_row;
     next_row = row_of(c0 + 2 * kLmChunk);
     __syncthreads();
-    // element d of keys {4 gq + i, 16 + 4 gq + i} -> vt[d][8 gq ..]: the order in which a lane of the
-    // first product holds its probabilities
-    for (int gq = 0; gq < 4; ++gq)
-      for (int d = tid; d < gm.R; d += blockDim.x) {
-        const uint16_t* col = reinterpret_cast<const uint16_t*>(kt) + d;
-        uint32_t x[4];
+    if (wave_ok && slice < 2) {            // the scores of keys 16 slice .. 16 slice + 15, to the group's waves
+      f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
+      const bf16_t* krow = kt + (16 * slice + m16) * gm.ldk + 8 * g;
+      if constexpr (kQueriesInLds) {
+        for (int j0 = 0; j0 < gm.d32; j0 += 4) {
+          bf16x8 kf[4], qv[4];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          x[i] = (uint32_t)col[(4 * gq + 2 * i) * gm.ldk] | ((uint32_t)col[(4 * gq + 2 * i + 1) * gm.ldk] << 16);
-          x[2 + i] = (uint32_t)col[(16 + 4 * gq + 2 * i) * gm.ldk] | ((uint32_t)col[(16 + 4 * gq + 2 * i + 1) * gm.ldk] << 16);
+          for (int x = 0; x < 4; ++x) {
+            const int j = min(j0 + x, gm.d32 - 1);
+            kf[x] = *reinterpret_cast<const bf16x8*>(krow + 32 * j);
+            qv[x] = *reinterpret_cast<const bf16x8*>(qs + m16 * gm.ldk + 8 * g + 32 * j);
+          }
+#pragma unroll
+          for (int x = 0; x < 4; ++x)
+            if (j0 + x < gm.d32) sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[x], qv[x], sc, 0, 0, 0);
         }
-        *reinterpret_cast<uint4*>(vt + d * kLmVtLd + 8 * gq) = make_uint4(x[0], x[1], x[2], x[3]);
+      } else {
+#pragma unroll
+        for (int j = 0; j < MAXD32; ++j)
+          if (j < gm.d32)
+            sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(krow + 32 * j), qf[j], sc, 0, 0, 0);
       }
+      ex[(w * 2 + slice) * kWave + lane] = sc;
+    }
     __syncthreads();
     if (!wave_ok) continue;
-
-    f32x4 s[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
-#pragma unroll
-    for (int j = 0; j < MAXD32; ++j) {
-      if (j < gm.d32) {
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kt + (16 * u + m16) * gm.ldk + 32 * j + 8 * g);
-          s[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[j], s[u], 0, 0, 0);
-        }
-      }
-    }
+    const f32x4 s[2] = {ex[w * 2 * kWave + lane], ex[(w * 2 + 1) * kWave + lane]};
     float sv[8];
     float mx = -INFINITY;
 #pragma unroll
@@ -223,7 +244,11 @@ __global__ __launch_bounds__(kLmWaves* kLmHalves* kWave) void attn_latent_mfma_k
 #pragma unroll
     for (int d = 0; d < MAXH; ++d) {
       if (d < r_n) {
-        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(vt + (16 * (r_lo + d) + m16) * kLmVtLd + 8 * g);
+        // the values of element 16 (r_lo + d) + m16 of keys 4 g .. 4 g + 3 and 16 + 4 g ..: the order in which the lane
+        // holds its probabilities
+        const bf16_t* vp = kt + (4 * g + (m16 >> 2)) * gm.ldk + 16 * (r_lo + d) + 4 * (m16 & 3);
+        const s16x4 v0 = read_transposed(vp), v1 = read_transposed(vp + 16 * gm.ldk);
+        const bf16x8 vf = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
         const f32x4 a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf_hi, acc[d], 0, 0, 0);
         acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, pf_lo, a, 0, 0, 0);
       }
@@ -259,7 +284,7 @@ __global__ __launch_bounds__(kLmWaves* kLmHalves* kWave) void attn_latent_mfma_k
   for (int d = 0; d < MAXH; ++d) {
     if (d < r_n) *reinterpret_cast<float4*>(po + 16 * d + 4 * g) = make_float4(acc[d][0], acc[d][1], acc[d][2], acc[d][3]);
   }
-  if (g == 0 && half == 0) {
+  if (g == 0 && slice == 0) {
     part_ml[(rh * max_runs + run - run0) * 2] = m_run;
     part_ml[(rh * max_runs + run - run0) * 2 + 1] = l_run;
   }
@@ -323,7 +348,8 @@ static int pow2_ceil(int v) {
   return p;
 }
 
-static LmGeom lm_geom(int H, int R, int dr) {
+// `single`: one token a block, and no more row groups than its heads fill
+static LmGeom lm_geom(int H, int R, int dr, bool single) {
   LmGeom g;
   g.H = H; g.R = R; g.D = R + dr;
   g.d32 = (g.D + 31) / 32;
@@ -331,8 +357,8 @@ static LmGeom lm_geom(int H, int R, int dr) {
   g.hpw = H >= 16 ? 16 : pow2_ceil(H);
   g.tb = 16 / g.hpw;
   const int ht = ceil_div(H, g.hpw);
-  g.htb = ht >= 4 ? 4 : pow2_ceil(ht);
-  g.tgb = kLmWaves / g.htb;
+  g.htb = ht >= kLmGroups ? kLmGroups : pow2_ceil(ht);
+  g.tgb = single ? 1 : kLmGroups / g.htb;
   g.ldk = g.d32 * 32 + 8;
   return g;
 }
@@ -344,7 +370,7 @@ SHARPI_EXPORT int sharpi_attention_latent_mfma_takes(int R, int dr) {
 
 // Tokens of one request that a block of the kernel works on (the prompt tiles are cut into pieces of this many).
 SHARPI_EXPORT int sharpi_attention_latent_mfma_block_tokens(int H) {
-  const LmGeom g = lm_geom(H, 16, 0);
+  const LmGeom g = lm_geom(H, 16, 0, false);
   return g.tgb * g.tb;
 }
 
@@ -367,16 +393,17 @@ SHARPI_EXPORT int sharpi_attention_latent_mfma(const void* q, const void* rows, 
   if (run_keys <= 0 || run_keys % kLmChunk || max_runs <= 0 || max_runs > 65535) return SHARPI_ERR_ARG;
   if (page_size <= 0 || max_blocks <= 0 || num_pages <= 0 || (tiles && tile_tokens <= 0)) return SHARPI_ERR_ARG;
   if (window < 0 || grid_runs < max_runs || grid_runs > 65535) return SHARPI_ERR_ARG;
-  const LmGeom g = lm_geom(H, R, dr);
+  const LmGeom g = lm_geom(H, R, dr, tiles == nullptr);
   const int tpb = g.tgb * g.tb;
   const int subs = tiles ? ceil_div(tile_tokens, tpb) : 1;
   const int head_blocks = ceil_div(ceil_div(H, g.hpw), g.htb);
   if (head_blocks > 65535) return SHARPI_ERR_ARG;
-  dim3 grid(n_items * subs, grid_runs, head_blocks), block(kLmWaves * kLmHalves * kWave);
-  const size_t lds = ((size_t)kLmChunk * g.ldk + (size_t)R * kLmVtLd) * sizeof(bf16_t);
-#define LM_LAUNCH(MD, MR)                                                                                         \
+  dim3 grid(n_items * subs, grid_runs, head_blocks), block(kLmWaves * kWave);
+  const int groups = g.htb * g.tgb, waves = kLmWaves / groups;     // waves a row group: 2, 4 or 8
+  const size_t lds = (size_t)(kLmChunk + (waves == 8 ? 16 : 0)) * g.ldk * sizeof(bf16_t) + (size_t)groups * 2 * kWave * sizeof(f32x4);
+#define LM_LAUNCH(MD, MR, SV)                                                                                         \
   do {                                                                                                            \
-    auto kern = attn_latent_mfma_kernel<MD, MR>;                                                                  \
+    auto kern = attn_latent_mfma_kernel<MD, MR, SV>;                                                                  \
     static size_t allowed = 48 * 1024;       /* dynamic LDS this instantiation may take (raised once per size) */  \
     if (lds > allowed) {                                                                                          \
       hipError_t e_ = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds); \
@@ -387,10 +414,17 @@ SHARPI_EXPORT int sharpi_attention_latent_mfma(const void* q, const void* rows, 
                                        positions, tiles, token_list, subs, sink, (bf16_t*)out, part_o, part_ml,   \
                                        scale, g, run_keys, max_runs, page_size, max_blocks, num_pages, window);   \
   } while (0)
-  if (g.d32 <= 5 && g.r16 <= 8) LM_LAUNCH(5, 8);
-  else if (g.d32 <= 10 && g.r16 <= 16) LM_LAUNCH(10, 16);
-  else if (g.d32 <= 18) LM_LAUNCH(18, 32);      // rows of up to 576: eight registers fewer than the widest form, which spills
-  else LM_LAUNCH(20, 32);
+#define LM_SIZES(SV)                                                                                              \
+  do {                                                                                                            \
+    if (g.d32 <= 5 && g.r16 <= 8) LM_LAUNCH(5, 8, SV);                                                            \
+    else if (g.d32 <= 10 && g.r16 <= 16) LM_LAUNCH(10, 16, SV);                                                   \
+    else if (g.d32 <= 18) LM_LAUNCH(18, 32, SV);   /* rows of up to 576: eight registers fewer than the widest form */ \
+    else LM_LAUNCH(20, 32, SV);                                                                                   \
+  } while (0)
+  if (waves == 8) LM_SIZES(8);
+  else if (waves == 4) LM_SIZES(4);
+  else LM_SIZES(2);
+#undef LM_SIZES
 #undef LM_LAUNCH
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;

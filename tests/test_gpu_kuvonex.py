@@ -284,6 +284,21 @@ def test_the_matrix_core_kernel_over_latent_rows(H, R, dr, S, how):
     assert _rel_rms(none.cpu().reshape(S, -1), want0.reshape(S, -1)) < 8e-3
 
 
+@pytest.mark.parametrize("H, R, dr", [(16, 512, 64), (2, 80, 24), (17, 512, 128), (31, 208, 8), (33, 16, 0), (65, 256, 32)])
+def test_a_rows_bits_are_the_same_however_many_waves_share_it(H, R, dr):
+    """Single tokens of up to 16, 32 and more heads (8, 4, 2 waves a row) against the prompt tiles' 2; 128 keys are one run of both."""
+    from sharpinference_amd import ops
+
+    S = 128
+    q, keys, rows, bt = _latent_case(H, R, dr, S, "bfloat16", seed=H)
+    outs = []
+    for tiles in (True, False):
+        ctx = _Ctx(torch.zeros(S, dtype=torch.int32, device=DEV), torch.arange(S, dtype=torch.int32, device=DEV), tiles=tiles, singles=not tiles)
+        outs.append(ops.attention_latent(q.reshape(S, -1).to(DEV), rows.to(DEV), _Group(bt.to(DEV), S), ctx, (R + dr) ** -0.5, H, R, dr,
+                                         sink=torch.linspace(-4.0, 4.0, H, device=DEV), kernel="mfma"))
+    assert torch.equal(*outs)
+
+
 def test_sizes_the_matrix_core_kernel_refuses_go_to_the_float_kernel():
     from sharpinference_amd import ops
 
