@@ -13,7 +13,8 @@
 // Bound: with four row groups the LDS reads of keys and values; for single tokens of 16 heads the chain of a chunk
 // (fetch, scores, softmax, values), so the slices are small, two blocks fit a compute unit and a chunk is fetched
 // ahead.  (With two waves a group whatever the rows, scores formed twice and a transposed copy of every chunk, 64
-// single tokens of 16 heads over 1500 keys of 576 took 88 us, now 46; 110 MB, 16 us at the memory's rate.)
+// single tokens of 16 heads over 1500 keys of 576 took 88 us, now 46 (110 MB, 16 us at the memory's rate), of 64 heads 107,
+// now 87; a prompt of 2048 tokens at 16 heads 531, now 403, at 64 heads 1634, now 1265.)
 // Probabilities enter the
 // second product as a bfloat16 pair hi + lo; the softmax state is float.  A row whose keys lie in
 // one run is finished here (with the sink term, if any); a row with more runs leaves (max, sum,
@@ -155,8 +156,8 @@ __global__ __launch_bounds__(kLmWaves* kWave, S == 8 ? 4 : 2) void attn_latent_m
       stage[j] = (src && c8 < d8) ? *reinterpret_cast<const uint4*>(src + 8 * c8) : make_uint4(0, 0, 0, 0);
     }
   };
-  // (with the widest rows the registers do not reach for rows held across the products: they are
-  // then requested where they are stored, and the SIMD's other wave covers the wait)
+  // (with the widest rows and two waves a group, rows held across the products were no faster, 406 against 403 us: they
+  // are then requested where they are stored, and the SIMD's other wave covers the wait)
   constexpr bool kAhead = MAXD32 <= 10 || S > 2;
   const bf16_t* cur_row = row_of(k_begin);
   if (kAhead) fetch(cur_row);
