@@ -24,6 +24,8 @@
 // its rows sees a key, and a row's runs are counted from the first in which it sees one itself.
 #include "common.h"
 
+#include <type_traits>
+
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
@@ -327,13 +329,30 @@ __global__ __launch_bounds__(kLmMergeWaves* kWave) void attn_latent_merge_kernel
     const int d = d0 + 4 * lane;
     const bool on = d < R;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int r = 0; r < n_runs; ++r) {
-      const float wr = r < kWave ? __shfl(w_lane, r, kWave) : expf(ml[2 * r] - M);
-      if (on) {
-        const float4 v = *reinterpret_cast<const float4*>(po + (size_t)r * R + d);
-        o.x += v.x * wr; o.y += v.y * wr; o.z += v.z * wr; o.w += v.w * wr;
+    // Eight runs' pieces are requested before the first is added (one at a time the chain of reads of what other dies have
+    // just written was the kernel's time: 64 rows of 16 heads, 12 runs of 512 elements 12.3 -> 7.6 us), two where a row
+    // has no more (prompts: 2048 tokens 18.8 us, with eight 21.5, now 17.0).
+    const auto add_runs = [&](auto batch) {
+      constexpr int B = decltype(batch)::value;
+      for (int r0 = 0; r0 < n_runs; r0 += B) {
+        float4 v[B];
+        float wr[B];
+#pragma unroll
+        for (int i = 0; i < B; ++i) v[i] = *reinterpret_cast<const float4*>(po + (size_t)min(r0 + i, n_runs - 1) * R + (on ? d : 0));
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+          const int r = min(r0 + i, n_runs - 1);
+          wr[i] = r < kWave ? __shfl(w_lane, r, kWave) : expf(ml[2 * r] - M);
+        }
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+          if (r0 + i >= n_runs) break;
+          o.x += v[i].x * wr[i]; o.y += v[i].y * wr[i]; o.z += v[i].z * wr[i]; o.w += v[i].w * wr[i];
+        }
       }
-    }
+    };
+    if (n_runs > 2) add_runs(std::integral_constant<int, 8>{});
+    else add_runs(std::integral_constant<int, 2>{});
     if (on) {
       uint2 pk;
       pk.x = pack_bf16(o.x * inv, o.y * inv);
