@@ -284,6 +284,24 @@ def test_the_matrix_core_kernel_over_latent_rows(H, R, dr, S, how):
     assert _rel_rms(none.cpu().reshape(S, -1), want0.reshape(S, -1)) < 8e-3
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T, N, k, weighted", [(1, 8, 1, True), (5, 255, 2, False), (3, 2049, 3, True), (64, 2304, 6, True), (2, 12288, 9, False)])
+def test_an_expert_sum_formed_in_the_norm_is_the_combine_kernels(T, N, k, weighted, dtype):
+    """Rows around eight columns a thread (2,048), odd and even numbers of picks: the same bits as with the sum formed first."""
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(N + k)
+    y = torch.randn(T * k, N, generator=g).to(DT[dtype]).to(DEV)
+    pos = torch.randperm(T * k, generator=g).to(torch.int32).to(DEV)
+    weights = torch.rand(T, k, generator=g).to(DEV) if weighted else None
+    h, w = torch.randn(T, N, generator=g).to(DEV), torch.rand(N, generator=g).to(DEV)
+    lazy = ops.ExpertSum(y, pos, None, T, k, weights)
+    got, first = h.clone(), h.clone()
+    ops.norm_add(got, lazy, w, 1e-6, None)
+    ops.norm_add(first, lazy.tensor(), w, 1e-6, None)
+    assert torch.equal(got, first)
+
+
 @pytest.mark.parametrize("H, R, dr", [(16, 512, 64), (2, 80, 24), (17, 512, 128), (31, 208, 8), (33, 16, 0), (65, 256, 32)])
 def test_a_rows_bits_are_the_same_however_many_waves_share_it(H, R, dr):
     """Single tokens of up to 16, 32 and more heads (8, 4, 2 waves a row) against the prompt tiles' 2; 128 keys are one run of both."""
