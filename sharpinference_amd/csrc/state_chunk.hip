@@ -41,6 +41,7 @@ __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __
 struct SegWeights {
   float uh[kSeg], ul[kSeg], b[kSeg], rh[kSeg], rl[kSeg], inter[kSeg], e[kSeg], end[kSeg];
   float inter_end, log_decay, m_end;
+  int odd[kChunkWaves];              // whether a wave staged a value that is no number
 };
 
 __device__ __forceinline__ void split(double x, float& hi, float& lo) {
@@ -74,16 +75,26 @@ __device__ void segment_weights(SegWeights& w, const WalkArgs& a, int h, int t0,
       }
     }
   }
+  // a logarithm that is no number stays out of the sums (a lane's first token has the pair's less the second) and is put back
+  // into those from its token on
+  const uint64_t odd0 = __ballot(!(fabs(f[0]) < INFINITY)), odd1 = __ballot(!(fabs(f[1]) < INFINITY));
+  if (odd0 >> lane & 1) f[0] = 0.0;
+  if (odd1 >> lane & 1) f[1] = 0.0;
   double upto = f[0] + f[1];                         // inclusive sums over the lanes
 #pragma unroll
   for (int o = 1; o < kWave; o <<= 1) {
     const double x = __shfl_up(upto, o, kWave);
     if (lane >= o) upto += x;
   }
-  const double G1 = upto, G0 = upto - f[1];
+  double G1 = upto, G0 = upto - f[1];
+  if (odd0 | odd1) {
+    const uint64_t from = 1ull << lane, odd = (odd0 | odd1) & (from - 1);     // of earlier lanes, then of the lane's own tokens
+    if (odd || (odd0 & from)) G0 = NAN;
+    if (odd || ((odd0 | odd1) & from)) G1 = NAN;
+  }
   const double u0 = i[0] - G0, u1 = i[1] - G1;
   double r0 = -G0, r1 = -G1, r_end, inter0 = G0, inter1 = G1;
-  const double G_end = __shfl(upto, kWave - 1, kWave);        // (tokens beyond the segment add nothing)
+  const double G_end = __shfl(G1, kWave - 1, kWave);          // (tokens beyond the segment add nothing)
   if (MODE == WALK_EXP_GATES) {
     double top = fmax(u0, u1);
 #pragma unroll
@@ -123,30 +134,48 @@ template <typename KT> __device__ __forceinline__ KT zero_of();
 template <> __device__ __forceinline__ float zero_of<float>() { return 0.f; }
 template <> __device__ __forceinline__ bf16_t zero_of<bf16_t>() { return bf16_t{0}; }
 
-// `rows` (a multiple of 16) rows of W elements from column `off` of proj into LDS rows of W + kPad, zeros beyond nt; 16-byte loads
+// The largest magnitudes of 16 bytes' elements so far, as their bits (of bfloat16 two by two), and whether one of them is infinite
+// or no number.
+template <typename T> struct Magnitudes;
+template <> struct Magnitudes<float> {
+  uint32_t most = 0;
+  __device__ __forceinline__ void add(uint32_t x) { most = max(most, x & 0x7fffffffu); }
+  __device__ __forceinline__ bool odd() const { return most >= 0x7f800000u; }
+};
+template <> struct Magnitudes<bf16_t> {
+  using u16x2 = __attribute__((__vector_size__(4))) unsigned short;
+  u16x2 most = {0, 0};
+  __device__ __forceinline__ void add(uint32_t x) { most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, x & 0x7fff7fffu)); }
+  __device__ __forceinline__ bool odd() const { return most[0] >= 0x7f80 || most[1] >= 0x7f80; }
+};
+
+// `rows` (a multiple of 16) rows of W elements from column `off` of proj into LDS rows of W + kPad, zeros beyond nt; 16-byte loads.
+// Returns whether the thread's elements hold one that is no number.
 template <typename T, typename KT, int W, int LD>
-__device__ __forceinline__ void stage_rows(KT* dst, const T* __restrict__ proj, int stride, int off, int t0, int nt, int rows) {
+__device__ __forceinline__ bool stage_rows(KT* dst, const T* __restrict__ proj, int stride, int off, int t0, int nt, int rows) {
   constexpr int V = 16 / (int)sizeof(T);
+  Magnitudes<T> seen;
   for (int idx = threadIdx.x; idx < rows * (W / V); idx += kChunkThreads) {
     const int t = idx / (W / V), c = (idx % (W / V)) * V;
     const T* src = proj + (size_t)(t0 + min(t, nt - 1)) * stride + off + c;
     KT* to = dst + t * LD + c;
-    if constexpr (sizeof(KT) == 2) {
-      uint4 x = *reinterpret_cast<const uint4*>(src);
-      if (t >= nt) x = make_uint4(0, 0, 0, 0);
-      *reinterpret_cast<uint4*>(to) = x;
+    uint4 raw = *reinterpret_cast<const uint4*>(src);
+    if (t >= nt) raw = make_uint4(0, 0, 0, 0);
+    seen.add(raw.x);
+    seen.add(raw.y);
+    seen.add(raw.z);
+    seen.add(raw.w);
+    if constexpr (sizeof(KT) == sizeof(T)) {
+      *reinterpret_cast<uint4*>(to) = raw;
     } else {
       float x[V];
-      if constexpr (sizeof(T) == 2) load8(src, x);
-      else {
-        const float4 y = *reinterpret_cast<const float4*>(src);
-        x[0] = y.x; x[1] = y.y; x[2] = y.z; x[3] = y.w;
-      }
+      load8(reinterpret_cast<const T*>(&raw), x);
 #pragma unroll
       for (int i = 0; i < V; i += 4)
-        *reinterpret_cast<float4*>(to + i) = t < nt ? make_float4(x[i], x[i + 1], x[i + 2], x[i + 3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+        *reinterpret_cast<float4*>(to + i) = make_float4(x[i], x[i + 1], x[i + 2], x[i + 3]);
     }
   }
+  return seen.odd();
 }
 
 // rotary positions on staged floats: element i of a row with element i + half
@@ -297,7 +326,8 @@ __device__ __forceinline__ void state_chunk_final_block(const WalkArgs& a) {
   }
   if constexpr (TURN) __syncthreads();
   stage_rows<T, KT, DK, DK + kPadK>(k_s, proj, a.stride, k_col, t0, nt, rows);
-  stage_rows<T, T, DV, DV + kPadV>(v_s, proj, a.stride, a.v_off + h * DV, t0, nt, rows);
+  const bool odd_v = __any(stage_rows<T, T, DV, DV + kPadV>(v_s, proj, a.stride, a.v_off + h * DV, t0, nt, rows));
+  if (lane == 0) w.odd[wid] = odd_v;
   if (wid == kChunkWaves - 1) segment_weights<MODE, false>(w, a, h, t0, nt, MODE == WALK_EXP_GATES ? from[NOFF + DK] : 0.f, lane);
 
   // the part of the start state, S_0^T q (its weight comes afterwards: nothing here waits for the staged rows)
@@ -349,7 +379,7 @@ __device__ __forceinline__ void state_chunk_final_block(const WalkArgs& a) {
 #pragma unroll
       for (int v = 0; v < 4; ++v) acc[ct][v] *= inter;
     // the segment's own keys, 16 at a time
-    for (int kb = 0; kb <= qt; ++kb) {
+    const auto keys = [&](int kb, auto apart) {
       f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
       const KT* krow = k_s + (kb * 16 + i) * (DK + kPadK);
       if constexpr (HALF) {
@@ -374,10 +404,36 @@ __device__ __forceinline__ void state_chunk_final_block(const WalkArgs& a) {
         const int s = kb * 16 + 4 * g + v;
         const float p = s <= t ? sc[v] * a.q_scale * (expf((w.uh[s] - rh) + (w.ul[s] - rl)) * w.b[s]) : 0.f;
         if (MODE == WALK_EXP_GATES) den += p;
+        if constexpr (decltype(apart)::value) {
+          for (int kg = 0; kg < 4; ++kg) {
+            const float ps = __shfl(p, i + 16 * kg, kWave);
+            const T* row = v_s + (kb * 16 + 4 * kg + v) * (DV + kPadV) + 4 * g;
+            const bool sees = kb * 16 + 4 * kg + v <= t;
 #pragma unroll
-        for (int ct = 0; ct < NCT; ++ct) acc[ct] = mfma_f32(to_f32<T>(v_s[s * (DV + kPadV) + ct * 16 + i]), p, acc[ct]);
+            for (int ct = 0; ct < NCT; ++ct)
+#pragma unroll
+              for (int y = 0; y < 4; ++y) {
+                const float x = to_f32<T>(row[ct * 16 + y]);
+                if (sees && !(fabsf(x) < INFINITY)) acc[ct][y] = fmaf(ps, x, acc[ct][y]);
+              }
+          }
+        }
+#pragma unroll
+        for (int ct = 0; ct < NCT; ++ct) {
+          float x = to_f32<T>(v_s[s * (DV + kPadV) + ct * 16 + i]);
+          if constexpr (decltype(apart)::value) x = fabsf(x) < INFINITY ? x : 0.f;
+          acc[ct] = mfma_f32(x, p, acc[ct]);
+        }
       }
-    }
+    };
+    // Among the queries' own 16 tokens a later one's weight is 0, and 0 times a value that is no number is none: where the
+    // segment holds such values, they are taken out of that product and added to the queries that see them.
+    int odd = 0;
+#pragma unroll
+    for (int x = 0; x < kChunkWaves; ++x) odd |= w.odd[x];
+    const int plain = __builtin_amdgcn_readfirstlane(odd ? qt - 1 : qt);
+    for (int kb = 0; kb <= plain; ++kb) keys(kb, std::false_type{});
+    if (plain < qt) keys(qt, std::true_type{});
     float inv = 1.f;
     if (MODE == WALK_EXP_GATES) {
       den += __shfl_xor(den, 16, kWave);

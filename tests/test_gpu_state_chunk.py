@@ -116,3 +116,63 @@ def test_segments_as_matrix_products_are_as_exact_as_the_walk(dtype, mode, H, G,
         tail = chunk_state[slots][:, :, :, dk * 8:dk * 8 + dk + 1]
         assert torch.equal(tail, tail[:, :, :1].expand_as(tail))
     assert float(chunk_state[[4, 8]].abs().max()) == 0.0           # slots no entry names
+
+
+def _modes(mode, H, dk, g):
+    """(code, parameters, frequencies, keys' scale) of a mode, as the layers that walk such states have them."""
+    from sharpinference_amd import ops
+
+    code = {"gates": ops.WALK_EXP_GATES, "space": ops.WALK_STATE_SPACE, "fixed": ops.WALK_FIXED_DECAY}[mode]
+    par = {"gates": (torch.randn(H, generator=g), torch.randn(H, generator=g)),
+           "space": (torch.randn(H, generator=g) * 0.5, torch.randn(H, generator=g) * 0.5 - 1.0, torch.randn(H, generator=g)),
+           "fixed": (1.0 - 2.0 ** (-3.0 - torch.arange(H) * 4.0),)}[mode]
+    freqs = 10000.0 ** (-torch.arange(dk // 4, dtype=torch.float32) / (dk // 4)) if mode == "fixed" else None
+    return code, tuple(p.to(DEV) for p in par), freqs.to(DEV) if freqs is not None else None, dk ** -0.5 if mode == "fixed" else 1.0
+
+
+def _walk(mode, lens, rows, gates, modes, H, dk, dv, segmented=True, state=None):
+    from sharpinference_amd import ops
+
+    code, par, freqs, k_scale = modes
+    ctx = _Step(lens, [0] * len(lens), range(len(lens)))
+    segments = tuple(torch.from_numpy(x).to(DEV) for x in ops.gla_segments(ctx.lens, ctx.cu)) if segmented else None
+    state = torch.zeros(len(lens), *ops.walk_state_shape(H, dk, dv, code), device=DEV) if state is None else state
+    out = ops.state_walk(rows, 0, H * dk, 2 * H * dk, 1, gates, par, 8.0, dk ** -0.5, code, state, ctx, H, dk, dv,
+                         segments=segments, inv_freq=freqs, k_scale=k_scale)
+    return out.view(-1, H, dv), state
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("mode, dk, dv", [("gates", 128, 128), ("space", 128, 64), ("fixed", 64, 128)])
+def test_what_is_no_number_stays_with_its_token_and_later_ones(dtype, mode, dk, dv):
+    """A token's value, key, query or gate that is infinite or no number: tokens before it have the same bits as without it,
+    whichever tile and segment they share with it; a value spoils one output column alone, from its token on."""
+    g = torch.Generator().manual_seed(dk + dv)
+    H, lens = 2, [300, 40]
+    n = sum(lens)
+    modes = _modes(mode, H, dk, g)
+    rows = torch.randn(n, 2 * H * dk + H * dv, generator=g).to(DT[dtype]).to(DEV)
+    gates = torch.randn(n, 2 * H, generator=g).to(DEV) if mode != "fixed" else None
+    clean = _walk(mode, lens, rows, gates, modes, H, dk, dv)[0]
+    v_col = lambda h, c: 2 * H * dk + h * dv + c
+    for bad in (float("inf"), float("nan")):
+        for t, h, c in ((5, 0, 17), (141, 1, dv - 1), (287, 0, 0), (299, 1, 33), (333, 0, 1)):
+            x = rows.clone()
+            x[t, v_col(h, c)] = bad
+            got = _walk(mode, lens, x, gates, modes, H, dk, dv)[0]
+            spoilt = torch.zeros_like(clean, dtype=torch.bool)
+            spoilt[t:300 if t < 300 else n, h, c] = True
+            assert torch.equal(got[~spoilt], clean[~spoilt])
+            assert not bool(got[spoilt].isfinite().any())
+        for t in (6, 141, 287, 333):
+            for what in ("key", "query", "gate"):
+                x, z = rows.clone(), gates
+                if what == "gate":
+                    if gates is None:
+                        continue
+                    z = gates.clone()
+                    z[t, 0] = bad
+                else:
+                    x[t, 3 if what == "query" else H * dk + 3] = bad
+                got = _walk(mode, lens, x, z, modes, H, dk, dv)[0]
+                assert torch.equal(got[:t], clean[:t]) and torch.equal(got[:, 1], clean[:, 1])
