@@ -49,6 +49,12 @@ __device__ __forceinline__ void split(double x, float& hi, float& lo) {
   lo = isinf(hi) ? 0.f : (float)(x - (double)hi);
 }
 
+// Logarithms of decays below this count as it: such a decay is 0 in float, and so are the products it is in, while sums
+// of 128 of them still carry the others' logarithms (a decay of 0 itself would make them infinite, and differences of
+// infinite sums are no numbers).
+constexpr double kLeastLog = -1e4;
+__device__ __forceinline__ double log_of_decay(double x) { return x < kLeastLog ? kLeastLog : x; }
+
 // By one wave: two neighbouring tokens a lane.  LOCAL: from nothing (the maximum starts at minus infinity).
 template <int MODE, bool LOCAL>
 __device__ void segment_weights(SegWeights& w, const WalkArgs& a, int h, int t0, int nt, float m_start, int lane) {
@@ -61,7 +67,7 @@ __device__ void segment_weights(SegWeights& w, const WalkArgs& a, int h, int t0,
     i[x] = MODE == WALK_EXP_GATES ? -INFINITY : 0.0;
     b[x] = 0.0;
     if (MODE == WALK_FIXED_DECAY) {
-      if (live) f[x] = log((double)a.p0[h]), b[x] = a.k_scale;
+      if (live) f[x] = log_of_decay(log((double)a.p0[h])), b[x] = a.k_scale;
     } else if (live) {
       const float* row = a.gates + (size_t)(t0 + t) * a.gate_stride;
       if (MODE == WALK_EXP_GATES) {
@@ -70,7 +76,7 @@ __device__ void segment_weights(SegWeights& w, const WalkArgs& a, int h, int t0,
         b[x] = 1.0;
       } else {
         const float dt = softplus_f32(row[h] + a.p0[h]);
-        f[x] = -expf(a.p1[h]) * dt;
+        f[x] = log_of_decay(-expf(a.p1[h]) * dt);
         b[x] = dt;
       }
     }

@@ -176,3 +176,25 @@ def test_what_is_no_number_stays_with_its_token_and_later_ones(dtype, mode, dk, 
                     x[t, 3 if what == "query" else H * dk + 3] = bad
                 got = _walk(mode, lens, x, z, modes, H, dk, dv)[0]
                 assert torch.equal(got[:t], clean[:t]) and torch.equal(got[:, 1], clean[:, 1])
+
+
+
+@pytest.mark.parametrize("mode", ["space", "fixed"])
+def test_decays_of_zero_forget_what_was_before(mode):
+    """A step size so large, or a stored decay, that a token's decay is 0: its logarithm is minus infinity, what follows is what
+    the walk of the whole entry makes of it, here and in the state that is left."""
+    g = torch.Generator().manual_seed(11)
+    H, dk, dv, lens = 2, 128, 64, [300, 90]
+    modes = list(_modes(mode, H, dk, g))
+    rows = torch.randn(sum(lens), 2 * H * dk + H * dv, generator=g).to(DEV)
+    gates = None
+    if mode == "space":
+        gates = torch.randn(sum(lens), 2 * H, generator=g).to(DEV)
+        modes[1][1][0] = 100.0                                     # exp(100) is beyond float: every decay of the head is 0
+        modes[1][1][1] = 60.0                                      # 1e26: finite logarithms, decays of 0 where the step is not tiny
+    else:
+        modes[1][0][0] = 0.0
+    (got, state), (want, walked) = (_walk(mode, lens, rows, gates, modes, H, dk, dv, s) for s in (True, False))
+    # an output is one product of 128 and two of a head's own sums: a few roundings of the largest
+    assert float((got - want).abs().max()) <= 2e-6 * float(want.abs().max())
+    assert float((state - walked).abs().max()) <= 2e-6 * float(walked.abs().max())
