@@ -293,7 +293,7 @@ __device__ __forceinline__ void state_chunk_final_block(const WalkArgs& a) {
   const int e = sg[0], t0 = sg[1], nt = sg[2];
   const bool last = sg[3] != 0;
   const bool only = last && t0 == a.cu_tokens[e];    // an entry's only segment starts from the slot
-  if (nt <= 0 || (only && nt < kChunkFrom)) return;
+  if (nt <= 0 || (only ? nt < kChunkFrom : (int)blockIdx.y >= a.n_scratch)) return;
   const int rows = min(kSeg, (nt + 15) / 16 * 16), tiles = rows / 16;
   const T* proj = static_cast<const T*>(a.proj);
   const int ncb = DV / kWalkCols, slice = walk_slice_floats(DK, MODE);
@@ -493,7 +493,7 @@ static int launch_chunk(const WalkArgs& a, bool final, hipStream_t stream) {
   constexpr size_t kt = MODE == WALK_FIXED_DECAY ? sizeof(float) : sizeof(T);
   constexpr size_t lds = kSeg * (DK + kPadK) * kt + kSeg * (NCT * 16 + kPadV) * sizeof(T) + sizeof(SegWeights);
   static_assert(lds <= 160 * 1024, "a block's LDS");
-  const dim3 grid(a.nh, a.n_segs);
+  const dim3 grid(a.nh, final ? a.n_segs : a.n_scratch);
   void (*kern)(const WalkArgs) = state_chunk_local_kernel<T, DK, NCT, MODE>;
   if (final) {
     if constexpr (MODE == WALK_FIXED_DECAY) kern = state_chunk_final_turned_kernel<T, DK, NCT>;

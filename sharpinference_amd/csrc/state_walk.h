@@ -21,7 +21,7 @@ struct WalkArgs {
   const float* gates; int gate_stride; const float *p0, *p1, *p2;
   float cap, q_scale; float* state; const int *state_slots, *cu_tokens; float* out;
   int n_entries, nh, dk, dv;
-  const int *segs, *ent_segs; int n_segs; float *seg_local, *seg_start, *seg_decay;
+  const int *segs, *ent_segs; int n_segs, n_scratch; float *seg_local, *seg_start, *seg_decay;
   const int* positions; const float* inv_freq; int rot_dim; float k_scale;      // WALK_FIXED_DECAY
 };
 

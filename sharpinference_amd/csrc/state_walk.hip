@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kWave) void state_walk_kernel(
     const int* __restrict__ state_slots, const int* __restrict__ cu_tokens, float* __restrict__ out, int nh, int dk,
     int dv, int ncb, int vec, const int* __restrict__ segs, float* __restrict__ seg_local,
     const float* __restrict__ seg_start, float* __restrict__ seg_decay, const int* __restrict__ positions,
-    const float* __restrict__ inv_freq, int rot_dim, float k_scale, int below) {
+    const float* __restrict__ inv_freq, int rot_dim, float k_scale, int below, int n_scratch) {
   constexpr int DKP = RPL * 8;
   constexpr int V = 16 / (int)sizeof(T);            // elements of a 16-byte load
   __shared__ __attribute__((aligned(16))) float q_s[PHASE == WALK_LOCAL ? 1 : kWalkChunk][DKP];     // (no outputs, no queries)
@@ -100,7 +100,9 @@ __global__ __launch_bounds__(kWave) void state_walk_kernel(
   if (t_end <= t_first) return;
   const size_t seg_at = (((size_t)blockIdx.z * nh + h) * ncb + cb) * slice;
   float* st = state + (((size_t)state_slots[e] * nh + h) * ncb + cb) * slice;      // the request's slot
-  const float* from = PHASE == WALK_FINAL && !(last && t_first == cu_tokens[e]) ? seg_start + seg_at : st;   // (an entry's only segment starts from the slot)
+  const bool from_slot = PHASE != WALK_FINAL || (last && t_first == cu_tokens[e]);     // (an entry's only segment)
+  if (!from_slot && (int)blockIdx.z >= n_scratch) return;
+  const float* from = from_slot ? st : seg_start + seg_at;
   const int c = cb * kWalkCols + j;
   const int qk_head = h / heads_per_group;
 
@@ -317,10 +319,10 @@ template <int MODE>
 __global__ __launch_bounds__(kCombineThreads) void state_walk_combine_kernel(
     const float* __restrict__ state, const int* __restrict__ state_slots, const int* __restrict__ ent_segs,
     const float* __restrict__ seg_local, float* __restrict__ seg_start, const float* __restrict__ seg_decay, int nh,
-    int ncb, int dkp) {
+    int ncb, int dkp, int n_scratch) {
   const int h = blockIdx.y, e = blockIdx.z;
   const int first = ent_segs[2 * e], count = ent_segs[2 * e + 1];
-  if (count <= 1) return;                       // nothing (one segment starts from the slot)
+  if (count <= 1 || first + count > n_scratch) return;      // nothing (one segment starts from the slot)
   const int slice = walk_slice_floats(dkp, MODE);
   const int moved = (dkp / 8) * 64 + (MODE == WALK_EXP_GATES ? dkp : 0);     // S and n; the maximum lies behind them
   const int idx = blockIdx.x * kCombineThreads + threadIdx.x;              // over the head's slices
@@ -366,11 +368,11 @@ __global__ __launch_bounds__(kCombineThreads) void state_walk_combine_kernel(
 
 template <typename T, int RPL, int MODE, int PHASE>
 static void launch_walk_phase(const WalkArgs& a, int ncb, int vec, hipStream_t stream, int below = 0x7fffffff) {
-  dim3 grid(ncb, a.nh, PHASE == WALK_WHOLE ? a.n_entries : a.n_segs);
+  dim3 grid(ncb, a.nh, PHASE == WALK_WHOLE ? a.n_entries : PHASE == WALK_LOCAL ? a.n_scratch : a.n_segs);
   state_walk_kernel<T, RPL, MODE, PHASE><<<grid, kWave, 0, stream>>>(
       (const T*)a.proj, a.stride, a.q_off, a.k_off, a.v_off, a.heads_per_group, a.gates, a.gate_stride, a.p0, a.p1, a.p2,
       a.cap, a.q_scale, a.state, a.state_slots, a.cu_tokens, a.out, a.nh, a.dk, a.dv, ncb, vec, a.segs, a.seg_local,
-      a.seg_start, a.seg_decay, a.positions, a.inv_freq, a.rot_dim, a.k_scale, below);
+      a.seg_start, a.seg_decay, a.positions, a.inv_freq, a.rot_dim, a.k_scale, below, a.n_scratch);
 }
 
 template <typename T, int RPL, int MODE>
@@ -382,21 +384,23 @@ static int launch_walk_rpl(const WalkArgs& a, int ncb, int vec, hipStream_t stre
   }
   constexpr int dtype = sizeof(T) == 4 ? DT_F32 : DT_BF16;
   const bool chunks = state_chunk_takes(a, dtype);
-  if (chunks) {
-    const int rc = state_chunk_local(a, dtype, MODE, stream);
-    if (rc != SHARPI_OK) return rc;
-    if (a.n_entries > 1 || a.n_segs < 2) {          // (one entry of several segments: nothing short)
-      launch_walk_phase<T, RPL, MODE, WALK_WHOLE>(a, ncb, vec, stream, state_chunk_from());
+  if (a.n_scratch > 0) {
+    if (chunks) {
+      const int rc = state_chunk_local(a, dtype, MODE, stream);
+      if (rc != SHARPI_OK) return rc;
+    } else {
+      launch_walk_phase<T, RPL, MODE, WALK_LOCAL>(a, ncb, vec, stream);
       SHARPI_CHECK_LAUNCH();
     }
-  } else {
-    launch_walk_phase<T, RPL, MODE, WALK_LOCAL>(a, ncb, vec, stream);
+    const int moved = RPL * 64 + (MODE == WALK_EXP_GATES ? RPL * 8 : 0);
+    state_walk_combine_kernel<MODE><<<dim3(ceil_div(ncb * moved, kCombineThreads), a.nh, a.n_entries), kCombineThreads, 0, stream>>>(
+        a.state, a.state_slots, a.ent_segs, a.seg_local, a.seg_start, a.seg_decay, a.nh, ncb, RPL * 8, a.n_scratch);
     SHARPI_CHECK_LAUNCH();
   }
-  const int moved = RPL * 64 + (MODE == WALK_EXP_GATES ? RPL * 8 : 0);
-  state_walk_combine_kernel<MODE><<<dim3(ceil_div(ncb * moved, kCombineThreads), a.nh, a.n_entries), kCombineThreads, 0, stream>>>(
-      a.state, a.state_slots, a.ent_segs, a.seg_local, a.seg_start, a.seg_decay, a.nh, ncb, RPL * 8);
-  SHARPI_CHECK_LAUNCH();
+  if (chunks && (a.n_entries > 1 || a.n_segs < 2)) {          // (one entry of several segments: nothing short)
+    launch_walk_phase<T, RPL, MODE, WALK_WHOLE>(a, ncb, vec, stream, state_chunk_from());
+    SHARPI_CHECK_LAUNCH();
+  }
   if (chunks) return state_chunk_final(a, dtype, MODE, stream);
   launch_walk_phase<T, RPL, MODE, WALK_FINAL>(a, ncb, vec, stream);
   SHARPI_CHECK_LAUNCH();
@@ -426,7 +430,7 @@ static int state_walk_any(const WalkArgs& a, int dtype, int mode, hipStream_t st
     return SHARPI_ERR_ARG;
   }
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
-  if (a.segs && (!a.ent_segs || !a.seg_local || !a.seg_start || !a.seg_decay || a.n_segs < a.n_entries || a.n_segs > 65535)) return SHARPI_ERR_ARG;
+  if (a.segs && (!a.ent_segs || !a.seg_local || !a.seg_start || !a.seg_decay || a.n_segs < a.n_entries || a.n_segs > 65535 || a.n_scratch < 0 || a.n_scratch > a.n_segs)) return SHARPI_ERR_ARG;
   if (mode == WALK_EXP_GATES) {
     if (dtype == DT_F32) return launch_state_walk<float, WALK_EXP_GATES>(a, stream);
     return launch_state_walk<bf16_t, WALK_EXP_GATES>(a, stream);
@@ -453,26 +457,27 @@ SHARPI_EXPORT int sharpi_state_walk(const void* proj, int dtype, int stride, int
                                     int dk, int dv, const int* positions, const float* inv_freq, int rot_dim, float k_scale,
                                     hipStream_t stream) {
   const WalkArgs a{proj, stride, q_off, k_off, v_off, heads_per_group, gates, gate_stride, p0, p1, p2, cap, q_scale, state,
-                   state_slots, cu_tokens, out, n_entries, nh, dk, dv, nullptr, nullptr, 0, nullptr, nullptr, nullptr,
+                   state_slots, cu_tokens, out, n_entries, nh, dk, dv, nullptr, nullptr, 0, 0, nullptr, nullptr, nullptr,
                    positions, inv_freq, rot_dim, k_scale};
   return state_walk_any(a, dtype, mode, stream);
 }
 
 // The same walk with long entries cut into segments that are walked side by side (results equal to
-// rounding).  segs int [n_segs, 4] = (entry, first row, tokens, 1 if the entry's last), in the entries'
-// order; ent_segs int [n_entries, 2] = (first segment, segments); seg_local and seg_start float [n_segs, nh,
-// ceil(dv / 8), slice]; seg_decay float [n_segs, nh].
+// rounding).  segs int [n_segs, 4] = (entry, first row, tokens, 1 if the entry's last), an entry's one after the
+// other, those of entries with several first; ent_segs int [n_entries, 2] = (first segment, segments).  An entry's only
+// segment starts from its slot and leaves into it; the first n_scratch segments, which hold all others, have their place in
+// seg_local and seg_start float [n_scratch, nh, ceil(dv / 8), slice] and seg_decay float [n_scratch, nh].
 SHARPI_EXPORT int sharpi_state_walk_segmented(const void* proj, int dtype, int stride, int q_off, int k_off, int v_off,
                                               int heads_per_group, const float* gates, int gate_stride, const float* p0,
                                               const float* p1, const float* p2, float cap, float q_scale, int mode,
                                               float* state, const int* state_slots, const int* cu_tokens, float* out,
                                               int n_entries, int nh, int dk, int dv, const int* segs, const int* ent_segs,
-                                              int n_segs, float* seg_local, float* seg_start, float* seg_decay,
+                                              int n_segs, int n_scratch, float* seg_local, float* seg_start, float* seg_decay,
                                               const int* positions, const float* inv_freq, int rot_dim, float k_scale,
                                               hipStream_t stream) {
   if (!segs) return SHARPI_ERR_ARG;
   const WalkArgs a{proj, stride, q_off, k_off, v_off, heads_per_group, gates, gate_stride, p0, p1, p2, cap, q_scale, state,
-                   state_slots, cu_tokens, out, n_entries, nh, dk, dv, segs, ent_segs, n_segs, seg_local, seg_start, seg_decay,
+                   state_slots, cu_tokens, out, n_entries, nh, dk, dv, segs, ent_segs, n_segs, n_scratch, seg_local, seg_start, seg_decay,
                    positions, inv_freq, rot_dim, k_scale};
   return state_walk_any(a, dtype, mode, stream);
 }

@@ -1465,17 +1465,25 @@ GLA_SEGMENT_TOKENS = 128       # tokens of a segment of the segmented walk
 def gla_segments(lens, cu_tokens):
     """The work lists of the segmented walk for entries of `lens` tokens whose rows start at
     `cu_tokens`: (segs int32 [n, 4] = (entry, first row, tokens, 1 if the entry's last), ent_segs int32
-    [entries, 2] = (first segment, segments)), as numpy arrays."""
+    [entries, 2] = (first segment, segments)), as numpy arrays.  The segments of entries with several come first
+    (see :func:`segments_with_scratch`)."""
     import numpy as np
 
-    segs, ents = [], []
-    for e, n in enumerate(lens):
-        first = len(segs)
+    segs, ents = [], [(0, 0)] * len(lens)
+    several = [e for e, n in enumerate(lens) if n > GLA_SEGMENT_TOKENS]
+    for e in several + [e for e, n in enumerate(lens) if n <= GLA_SEGMENT_TOKENS]:
+        n, first = lens[e], len(segs)
         for o in range(0, n, GLA_SEGMENT_TOKENS):
             m = min(GLA_SEGMENT_TOKENS, n - o)
             segs.append((e, int(cu_tokens[e]) + o, m, 1 if o + m == n else 0))
-        ents.append((first, len(segs) - first))
+        ents[e] = (first, len(segs) - first)
     return np.asarray(segs, dtype=np.int32).reshape(-1, 4), np.asarray(ents, dtype=np.int32).reshape(-1, 2)
+
+
+def segments_with_scratch(ent_segs) -> int:
+    """How many of the leading segments of :func:`gla_segments` belong to entries with several: those need a place for
+    what they make of nothing and for their start state in :func:`state_walk`, an entry's only segment does not."""
+    return int(ent_segs[ent_segs[:, 1] > 1, 1].sum())
 
 
 def gla_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, alpha: torch.Tensor, q_scale: float,
@@ -1498,7 +1506,7 @@ def gla_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, alpha: torc
           "gla_walk: the step's per-entry arrays do not fit")
     out = torch.empty(T, nh * dv, dtype=torch.float32, device=proj.device)
     if segments is not None:
-        segs, ent_segs = segments
+        segs, ent_segs = segments[:2]
         _dev(segs, ent_segs)
         _i32(segs, "segs")
         _i32(ent_segs, "ent_segs")
@@ -1779,7 +1787,8 @@ def state_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, heads_per
       are first turned by rotary positions, element i with element i + r/2 by the angle position x
       inv_freq[i], in float; the result is o.
 
-    ``segments`` = (segs, ent_segs) on the device (see :func:`gla_segments`): long entries are then walked
+    ``segments`` = (segs, ent_segs) on the device (see :func:`gla_segments`), and, if given, how many leading segments need
+    scratch (:func:`segments_with_scratch`; else all have some): long entries are then walked
     segment by segment side by side.  A stretch of tokens acts on the state as S -> D S + L (D the product of
     its decays, one number a head; L what it makes of a zero state), so every segment is first walked from
     nothing, the true start states follow one from the other, and a second walk from those writes the
@@ -1817,21 +1826,23 @@ def state_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, heads_per
     g_stride = gates.shape[1] if gates is not None else 0
     rot = (_ptr(ctx.positions) if rot_dim else None, _ptr(inv_freq) if rot_dim else None, rot_dim, float(k_scale))
     if segments is not None:
-        segs, ent_segs = segments
+        segs, ent_segs = segments[:2]
         _dev(segs, ent_segs)
         _i32(segs, "segs")
         _i32(ent_segs, "ent_segs")
         n_segs = segs.numel() // 4
         _need(segs.numel() == 4 * n_segs and ent_segs.numel() == 2 * ctx.n_entries and n_segs >= ctx.n_entries,
               "state_walk: segs [n, 4] and ent_segs [entries, 2] wanted")
-        shape = (n_segs,) + walk_state_shape(nh, dk, dv, mode)
+        n_scratch = int(segments[2]) if len(segments) > 2 else n_segs
+        _need(0 <= n_scratch <= n_segs, "state_walk: at most all segments need scratch")
+        shape = (max(1, n_scratch),) + walk_state_shape(nh, dk, dv, mode)
         seg_local = torch.empty(shape, dtype=torch.float32, device=proj.device)
         seg_start = torch.empty(shape, dtype=torch.float32, device=proj.device)
-        seg_decay = torch.empty(n_segs, nh, dtype=torch.float32, device=proj.device)
+        seg_decay = torch.empty(max(1, n_scratch), nh, dtype=torch.float32, device=proj.device)
         _run("sharpi_state_walk_segmented", _ptr(proj), _code(proj.dtype), N, int(q_off), int(k_off), int(v_off),
              int(heads_per_group), _ptr(gates), g_stride, _ptr(p[0]), _ptr(p[1]), _ptr(p[2]), float(cap), float(q_scale),
              int(mode), _ptr(state), _ptr(ctx.state_slots), _ptr(ctx.cu_tokens), _ptr(out), ctx.n_entries, nh, dk, dv,
-             _ptr(segs), _ptr(ent_segs), n_segs, _ptr(seg_local), _ptr(seg_start), _ptr(seg_decay), *rot, _stream())
+             _ptr(segs), _ptr(ent_segs), n_segs, n_scratch, _ptr(seg_local), _ptr(seg_start), _ptr(seg_decay), *rot, _stream())
         return out
     _run("sharpi_state_walk", _ptr(proj), _code(proj.dtype), N, int(q_off), int(k_off), int(v_off), int(heads_per_group),
          _ptr(gates), g_stride, _ptr(p[0]), _ptr(p[1]), _ptr(p[2]), float(cap), float(q_scale), int(mode), _ptr(state),

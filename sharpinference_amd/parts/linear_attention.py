@@ -28,10 +28,10 @@ class WalkSegments(StepPlanner):
             empty = np.zeros(0, dtype=np.int32)
             return [empty, empty], dict(n_segs=0)
         segs, ents = ops.gla_segments(host.lens, host.cu_tokens)
-        return [segs.reshape(-1), ents.reshape(-1)], dict(n_segs=segs.shape[0])
+        return [segs.reshape(-1), ents.reshape(-1)], dict(n_segs=segs.shape[0], n_scratch=ops.segments_with_scratch(ents))
 
     def attach(self, ctx: StepContext, views: List[torch.Tensor], facts: dict) -> None:
-        ctx.extras[self.key] = (views[0], views[1]) if facts["n_segs"] else None
+        ctx.extras[self.key] = (views[0], views[1], facts["n_scratch"]) if facts["n_segs"] else None
 
 
 _SEGMENTS = WalkSegments()

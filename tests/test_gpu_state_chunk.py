@@ -198,3 +198,30 @@ def test_decays_of_zero_forget_what_was_before(mode):
     # an output is one product of 128 and two of a head's own sums: a few roundings of the largest
     assert float((got - want).abs().max()) <= 2e-6 * float(want.abs().max())
     assert float((state - walked).abs().max()) <= 2e-6 * float(walked.abs().max())
+
+
+
+def test_scratch_is_for_entries_of_several_segments_alone():
+    """200 decoding requests beside one prompt of three segments: what is allocated beside the outputs are two states a
+    segment of the prompt."""
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(3)
+    H, dk, dv, lens = 4, 128, 128, [1] * 100 + [300] + [1] * 100
+    modes = _modes("fixed", H, dk, g)
+    rows = torch.randn(sum(lens), 3 * H * dk, generator=g).to(DEV)
+    state = torch.zeros(len(lens), *ops.walk_state_shape(H, dk, dv, ops.WALK_FIXED_DECAY), device=DEV)
+    code, par, freqs, k_scale = modes
+    ctx = _Step(lens, [0] * len(lens), range(len(lens)))
+    segs, ents = ops.gla_segments(ctx.lens, ctx.cu)
+    segments = (torch.from_numpy(segs).to(DEV), torch.from_numpy(ents).to(DEV), ops.segments_with_scratch(ents))
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    torch.cuda.reset_peak_memory_stats()
+    out = ops.state_walk(rows, 0, H * dk, 2 * H * dk, 1, None, par, 8.0, dk ** -0.5, code, state, ctx, H, dk, dv, segments=segments,
+                         inv_freq=freqs, k_scale=k_scale)
+    one = state[0].numel() * 4
+    assert torch.cuda.max_memory_allocated() - before <= out.numel() * 4 + 2 * 3 * one + 65536
+    want, walked = _walk("fixed", lens, rows, None, modes, H, dk, dv, False)
+    assert float((out.view_as(want) - want).abs().max()) <= 2e-6 * float(want.abs().max())
+    assert float((state - walked).abs().max()) <= 2e-6 * float(walked.abs().max())
