@@ -33,7 +33,6 @@ constexpr int kSeg = 128;              // tokens of a segment at most
 constexpr int kChunkWaves = 8;
 constexpr int kChunkThreads = kChunkWaves * kWave;
 constexpr int kPadK = 8, kPadV = 16;   // elements behind an LDS row of k and of v (bfloat16: banks 4 and 8 apart from row to row)
-constexpr int kChunkFrom = 32;         // entries of fewer tokens are walked (state_walk.hip)
 
 __device__ __forceinline__ f32x4 mfma_f32(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
@@ -480,7 +479,7 @@ __global__ __launch_bounds__(kChunkThreads) __attribute__((amdgpu_waves_per_eu(2
 // 1 where long entries of heads of dk key and dv value channels take the chunk form
 SHARPI_EXPORT int sharpi_state_chunk_takes(int dk, int dv) { return (dk == 64 || dk == 128) && (dv == 64 || dv == 128); }
 
-int state_chunk_from() { return kChunkFrom; }
+SHARPI_EXPORT int sharpi_state_chunk_from() { return kChunkFrom; }
 
 bool state_chunk_takes(const WalkArgs& a, int dtype) {
   const int V = dtype == DT_BF16 ? 8 : 4;            // 16-byte loads of every head's rows, 16-byte stores of the outputs
@@ -493,7 +492,7 @@ static int launch_chunk(const WalkArgs& a, bool final, hipStream_t stream) {
   constexpr size_t kt = MODE == WALK_FIXED_DECAY ? sizeof(float) : sizeof(T);
   constexpr size_t lds = kSeg * (DK + kPadK) * kt + kSeg * (NCT * 16 + kPadV) * sizeof(T) + sizeof(SegWeights);
   static_assert(lds <= 160 * 1024, "a block's LDS");
-  const dim3 grid(a.nh, final ? a.n_segs : a.n_scratch);
+  const dim3 grid(a.nh, !final ? a.n_scratch : a.n_long < 0 ? a.n_segs : a.n_long);
   void (*kern)(const WalkArgs) = state_chunk_local_kernel<T, DK, NCT, MODE>;
   if (final) {
     if constexpr (MODE == WALK_FIXED_DECAY) kern = state_chunk_final_turned_kernel<T, DK, NCT>;

@@ -21,13 +21,13 @@ struct WalkArgs {
   const float* gates; int gate_stride; const float *p0, *p1, *p2;
   float cap, q_scale; float* state; const int *state_slots, *cu_tokens; float* out;
   int n_entries, nh, dk, dv;
-  const int *segs, *ent_segs; int n_segs, n_scratch; float *seg_local, *seg_start, *seg_decay;
+  const int *segs, *ent_segs; int n_segs, n_scratch, n_long; float *seg_local, *seg_start, *seg_decay;
   const int* positions; const float* inv_freq; int rot_dim; float k_scale;      // WALK_FIXED_DECAY
 };
 
 // The segments' first and last pass in chunk form (state_chunk.hip), for the sizes state_chunk_takes names; entries
-// of fewer than state_chunk_from() tokens are left out and walked.
-int state_chunk_from();
+// of fewer than kChunkFrom tokens are left out and walked (a.n_long: the leading segments of all others).
+constexpr int kChunkFrom = 32;
 bool state_chunk_takes(const WalkArgs& a, int dtype);
 int state_chunk_local(const WalkArgs& a, int dtype, int mode, hipStream_t stream);
 int state_chunk_final(const WalkArgs& a, int dtype, int mode, hipStream_t stream);

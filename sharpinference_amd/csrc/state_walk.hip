@@ -317,10 +317,12 @@ constexpr int kCombineAhead = 8;
 
 template <int MODE>
 __global__ __launch_bounds__(kCombineThreads) void state_walk_combine_kernel(
-    const float* __restrict__ state, const int* __restrict__ state_slots, const int* __restrict__ ent_segs,
+    const float* __restrict__ state, const int* __restrict__ state_slots, const int* __restrict__ cu_tokens,
+    const int* __restrict__ segs, const int* __restrict__ ent_segs,
     const float* __restrict__ seg_local, float* __restrict__ seg_start, const float* __restrict__ seg_decay, int nh,
     int ncb, int dkp, int n_scratch) {
-  const int h = blockIdx.y, e = blockIdx.z;
+  const int h = blockIdx.y, e = segs ? segs[4 * blockIdx.z] : blockIdx.z;
+  if (segs && segs[4 * blockIdx.z + 1] != cu_tokens[e]) return;     // (an entry's first segment has the entry's blocks)
   const int first = ent_segs[2 * e], count = ent_segs[2 * e + 1];
   if (count <= 1 || first + count > n_scratch) return;      // nothing (one segment starts from the slot)
   const int slice = walk_slice_floats(dkp, MODE);
@@ -384,6 +386,10 @@ static int launch_walk_rpl(const WalkArgs& a, int ncb, int vec, hipStream_t stre
   }
   constexpr int dtype = sizeof(T) == 4 ? DT_F32 : DT_BF16;
   const bool chunks = state_chunk_takes(a, dtype);
+  if (chunks && a.n_long < a.n_segs) {                        // (first: what the passes leave each other stays in the caches)
+    launch_walk_phase<T, RPL, MODE, WALK_WHOLE>(a, ncb, vec, stream, kChunkFrom);
+    SHARPI_CHECK_LAUNCH();
+  }
   if (a.n_scratch > 0) {
     if (chunks) {
       const int rc = state_chunk_local(a, dtype, MODE, stream);
@@ -392,16 +398,15 @@ static int launch_walk_rpl(const WalkArgs& a, int ncb, int vec, hipStream_t stre
       launch_walk_phase<T, RPL, MODE, WALK_LOCAL>(a, ncb, vec, stream);
       SHARPI_CHECK_LAUNCH();
     }
+    // blocks of every entry, or of every segment that may be the first of one, whichever are fewer
     const int moved = RPL * 64 + (MODE == WALK_EXP_GATES ? RPL * 8 : 0);
-    state_walk_combine_kernel<MODE><<<dim3(ceil_div(ncb * moved, kCombineThreads), a.nh, a.n_entries), kCombineThreads, 0, stream>>>(
-        a.state, a.state_slots, a.ent_segs, a.seg_local, a.seg_start, a.seg_decay, a.nh, ncb, RPL * 8, a.n_scratch);
+    const dim3 grid(ceil_div(ncb * moved, kCombineThreads), a.nh, min(a.n_entries, a.n_scratch));
+    state_walk_combine_kernel<MODE><<<grid, kCombineThreads, 0, stream>>>(
+        a.state, a.state_slots, a.cu_tokens, a.n_scratch < a.n_entries ? a.segs : nullptr, a.ent_segs, a.seg_local, a.seg_start,
+        a.seg_decay, a.nh, ncb, RPL * 8, a.n_scratch);
     SHARPI_CHECK_LAUNCH();
   }
-  if (chunks && (a.n_entries > 1 || a.n_segs < 2)) {          // (one entry of several segments: nothing short)
-    launch_walk_phase<T, RPL, MODE, WALK_WHOLE>(a, ncb, vec, stream, state_chunk_from());
-    SHARPI_CHECK_LAUNCH();
-  }
-  if (chunks) return state_chunk_final(a, dtype, MODE, stream);
+  if (chunks) return a.n_long != 0 ? state_chunk_final(a, dtype, MODE, stream) : SHARPI_OK;
   launch_walk_phase<T, RPL, MODE, WALK_FINAL>(a, ncb, vec, stream);
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
@@ -430,7 +435,8 @@ static int state_walk_any(const WalkArgs& a, int dtype, int mode, hipStream_t st
     return SHARPI_ERR_ARG;
   }
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
-  if (a.segs && (!a.ent_segs || !a.seg_local || !a.seg_start || !a.seg_decay || a.n_segs < a.n_entries || a.n_segs > 65535 || a.n_scratch < 0 || a.n_scratch > a.n_segs)) return SHARPI_ERR_ARG;
+  if (a.segs && (!a.ent_segs || !a.seg_local || !a.seg_start || !a.seg_decay || a.n_segs < a.n_entries || a.n_segs > 65535 || a.n_scratch < 0 || a.n_scratch > a.n_segs || a.n_long > a.n_segs ||
+                 (a.n_long >= 0 && a.n_long < a.n_scratch))) return SHARPI_ERR_ARG;
   if (mode == WALK_EXP_GATES) {
     if (dtype == DT_F32) return launch_state_walk<float, WALK_EXP_GATES>(a, stream);
     return launch_state_walk<bf16_t, WALK_EXP_GATES>(a, stream);
@@ -457,27 +463,28 @@ SHARPI_EXPORT int sharpi_state_walk(const void* proj, int dtype, int stride, int
                                     int dk, int dv, const int* positions, const float* inv_freq, int rot_dim, float k_scale,
                                     hipStream_t stream) {
   const WalkArgs a{proj, stride, q_off, k_off, v_off, heads_per_group, gates, gate_stride, p0, p1, p2, cap, q_scale, state,
-                   state_slots, cu_tokens, out, n_entries, nh, dk, dv, nullptr, nullptr, 0, 0, nullptr, nullptr, nullptr,
+                   state_slots, cu_tokens, out, n_entries, nh, dk, dv, nullptr, nullptr, 0, 0, 0, nullptr, nullptr, nullptr,
                    positions, inv_freq, rot_dim, k_scale};
   return state_walk_any(a, dtype, mode, stream);
 }
 
 // The same walk with long entries cut into segments that are walked side by side (results equal to
 // rounding).  segs int [n_segs, 4] = (entry, first row, tokens, 1 if the entry's last), an entry's one after the
-// other, those of entries with several first; ent_segs int [n_entries, 2] = (first segment, segments).  An entry's only
-// segment starts from its slot and leaves into it; the first n_scratch segments, which hold all others, have their place in
-// seg_local and seg_start float [n_scratch, nh, ceil(dv / 8), slice] and seg_decay float [n_scratch, nh].
+// other, those of entries with several first, then those of at least kChunkFrom tokens (n_long up to there; -1: not known); ent_segs int
+// [n_entries, 2] = (first segment, segments).  An entry's only segment starts from its slot and leaves into it; the first
+// n_scratch segments, which hold all others, have their place in seg_local and seg_start float [n_scratch, nh,
+// ceil(dv / 8), slice] and seg_decay float [n_scratch, nh].
 SHARPI_EXPORT int sharpi_state_walk_segmented(const void* proj, int dtype, int stride, int q_off, int k_off, int v_off,
                                               int heads_per_group, const float* gates, int gate_stride, const float* p0,
                                               const float* p1, const float* p2, float cap, float q_scale, int mode,
                                               float* state, const int* state_slots, const int* cu_tokens, float* out,
                                               int n_entries, int nh, int dk, int dv, const int* segs, const int* ent_segs,
-                                              int n_segs, int n_scratch, float* seg_local, float* seg_start, float* seg_decay,
+                                              int n_segs, int n_scratch, int n_long, float* seg_local, float* seg_start, float* seg_decay,
                                               const int* positions, const float* inv_freq, int rot_dim, float k_scale,
                                               hipStream_t stream) {
   if (!segs) return SHARPI_ERR_ARG;
   const WalkArgs a{proj, stride, q_off, k_off, v_off, heads_per_group, gates, gate_stride, p0, p1, p2, cap, q_scale, state,
-                   state_slots, cu_tokens, out, n_entries, nh, dk, dv, segs, ent_segs, n_segs, n_scratch, seg_local, seg_start, seg_decay,
+                   state_slots, cu_tokens, out, n_entries, nh, dk, dv, segs, ent_segs, n_segs, n_scratch, n_long, seg_local, seg_start, seg_decay,
                    positions, inv_freq, rot_dim, k_scale};
   return state_walk_any(a, dtype, mode, stream);
 }

@@ -1460,18 +1460,19 @@ def gla_decays_from_middle(proj: torch.Tensor, a_off: int, rank: int, w: torch.T
 
 
 GLA_SEGMENT_TOKENS = 128       # tokens of a segment of the segmented walk
+WALK_CHUNK_FROM = _lib.WALK_CHUNK_FROM       # entries of fewer tokens are walked token by token in every form
 
 
 def gla_segments(lens, cu_tokens):
     """The work lists of the segmented walk for entries of `lens` tokens whose rows start at
     `cu_tokens`: (segs int32 [n, 4] = (entry, first row, tokens, 1 if the entry's last), ent_segs int32
-    [entries, 2] = (first segment, segments)), as numpy arrays.  The segments of entries with several come first
-    (see :func:`segments_with_scratch`)."""
+    [entries, 2] = (first segment, segments)), as numpy arrays.  The segments of entries with several come first, then
+    those of at least WALK_CHUNK_FROM tokens (see :func:`segment_counts`)."""
     import numpy as np
 
     segs, ents = [], [(0, 0)] * len(lens)
-    several = [e for e, n in enumerate(lens) if n > GLA_SEGMENT_TOKENS]
-    for e in several + [e for e, n in enumerate(lens) if n <= GLA_SEGMENT_TOKENS]:
+    rank = [0 if n > GLA_SEGMENT_TOKENS else 1 if n >= WALK_CHUNK_FROM else 2 for n in lens]
+    for e in sorted(range(len(lens)), key=rank.__getitem__):
         n, first = lens[e], len(segs)
         for o in range(0, n, GLA_SEGMENT_TOKENS):
             m = min(GLA_SEGMENT_TOKENS, n - o)
@@ -1480,10 +1481,12 @@ def gla_segments(lens, cu_tokens):
     return np.asarray(segs, dtype=np.int32).reshape(-1, 4), np.asarray(ents, dtype=np.int32).reshape(-1, 2)
 
 
-def segments_with_scratch(ent_segs) -> int:
-    """How many of the leading segments of :func:`gla_segments` belong to entries with several: those need a place for
-    what they make of nothing and for their start state in :func:`state_walk`, an entry's only segment does not."""
-    return int(ent_segs[ent_segs[:, 1] > 1, 1].sum())
+def segment_counts(lens) -> Tuple[int, int]:
+    """Of the segments of :func:`gla_segments`: (how many leading ones belong to entries with several, which need a place
+    for what they make of nothing and for their start state in :func:`state_walk`; how many belong to those or have
+    at least WALK_CHUNK_FROM tokens, which are run as products where the sizes take it)."""
+    several = sum((n + GLA_SEGMENT_TOKENS - 1) // GLA_SEGMENT_TOKENS for n in lens if n > GLA_SEGMENT_TOKENS)
+    return several, several + sum(WALK_CHUNK_FROM <= n <= GLA_SEGMENT_TOKENS for n in lens)
 
 
 def gla_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, alpha: torch.Tensor, q_scale: float,
@@ -1787,8 +1790,7 @@ def state_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, heads_per
       are first turned by rotary positions, element i with element i + r/2 by the angle position x
       inv_freq[i], in float; the result is o.
 
-    ``segments`` = (segs, ent_segs) on the device (see :func:`gla_segments`), and, if given, how many leading segments need
-    scratch (:func:`segments_with_scratch`; else all have some): long entries are then walked
+    ``segments`` = (segs, ent_segs) on the device (see :func:`gla_segments`) and, if at hand, their :func:`segment_counts`: long entries are then walked
     segment by segment side by side.  A stretch of tokens acts on the state as S -> D S + L (D the product of
     its decays, one number a head; L what it makes of a zero state), so every segment is first walked from
     nothing, the true start states follow one from the other, and a second walk from those writes the
@@ -1833,8 +1835,9 @@ def state_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, heads_per
         n_segs = segs.numel() // 4
         _need(segs.numel() == 4 * n_segs and ent_segs.numel() == 2 * ctx.n_entries and n_segs >= ctx.n_entries,
               "state_walk: segs [n, 4] and ent_segs [entries, 2] wanted")
-        n_scratch = int(segments[2]) if len(segments) > 2 else n_segs
-        _need(0 <= n_scratch <= n_segs, "state_walk: at most all segments need scratch")
+        n_scratch, n_long = segments[2] if len(segments) > 2 else (n_segs, -1)         # (-1: not known)
+        _need(0 <= n_scratch <= n_segs and n_long <= n_segs and (n_long == -1 or n_long >= n_scratch),
+              "state_walk: (segments of several, long segments) of all segments wanted")
         shape = (max(1, n_scratch),) + walk_state_shape(nh, dk, dv, mode)
         seg_local = torch.empty(shape, dtype=torch.float32, device=proj.device)
         seg_start = torch.empty(shape, dtype=torch.float32, device=proj.device)
@@ -1842,7 +1845,7 @@ def state_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, heads_per
         _run("sharpi_state_walk_segmented", _ptr(proj), _code(proj.dtype), N, int(q_off), int(k_off), int(v_off),
              int(heads_per_group), _ptr(gates), g_stride, _ptr(p[0]), _ptr(p[1]), _ptr(p[2]), float(cap), float(q_scale),
              int(mode), _ptr(state), _ptr(ctx.state_slots), _ptr(ctx.cu_tokens), _ptr(out), ctx.n_entries, nh, dk, dv,
-             _ptr(segs), _ptr(ent_segs), n_segs, n_scratch, _ptr(seg_local), _ptr(seg_start), _ptr(seg_decay), *rot, _stream())
+             _ptr(segs), _ptr(ent_segs), n_segs, int(n_scratch), int(n_long), _ptr(seg_local), _ptr(seg_start), _ptr(seg_decay), *rot, _stream())
         return out
     _run("sharpi_state_walk", _ptr(proj), _code(proj.dtype), N, int(q_off), int(k_off), int(v_off), int(heads_per_group),
          _ptr(gates), g_stride, _ptr(p[0]), _ptr(p[1]), _ptr(p[2]), float(cap), float(q_scale), int(mode), _ptr(state),

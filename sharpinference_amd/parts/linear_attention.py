@@ -1,7 +1,7 @@
 """The gated linear attention mixer: a matrix-valued state per head instead of a cache of keys."""
 from __future__ import annotations
 
-from typing import Dict, List, Optional, Tuple
+from typing import Dict, List, NamedTuple, Optional, Tuple
 
 import numpy as np
 import torch
@@ -17,6 +17,24 @@ SEGMENT_FROM_TOKENS = 512     # ... layers that walk segments token by token tak
 SEGMENT_UP_TO_BLOCKS = 2048   # ... while whole entries would give fewer blocks than this
 
 
+class EntrySpans(NamedTuple):
+    """What a step's entries are to a recurrent state: how many, their tokens, the longest; and of those too short to go
+    through it in products."""
+
+    entries: int
+    tokens: int
+    longest: int
+    short: int
+    short_tokens: int
+    longest_short: int
+    several: bool          # some entry has several segments
+
+    @classmethod
+    def of(cls, lens) -> "EntrySpans":
+        short = [n for n in lens if n < ops.WALK_CHUNK_FROM]
+        return cls(len(lens), sum(lens), max(lens), len(short), sum(short), max(short, default=0), max(lens) > ops.GLA_SEGMENT_TOKENS)
+
+
 class WalkSegments(StepPlanner):
     """The work lists of the segmented walk, made once a step for all layers that walk a state: none
     unless some entry is long (decode steps and short portions are walked whole)."""
@@ -28,10 +46,10 @@ class WalkSegments(StepPlanner):
             empty = np.zeros(0, dtype=np.int32)
             return [empty, empty], dict(n_segs=0)
         segs, ents = ops.gla_segments(host.lens, host.cu_tokens)
-        return [segs.reshape(-1), ents.reshape(-1)], dict(n_segs=segs.shape[0], n_scratch=ops.segments_with_scratch(ents))
+        return [segs.reshape(-1), ents.reshape(-1)], dict(n_segs=segs.shape[0], counts=ops.segment_counts(host.lens), spans=EntrySpans.of(host.lens))
 
     def attach(self, ctx: StepContext, views: List[torch.Tensor], facts: dict) -> None:
-        ctx.extras[self.key] = (views[0], views[1], facts["n_scratch"]) if facts["n_segs"] else None
+        ctx.extras[self.key] = (views[0], views[1], facts["counts"], facts["spans"]) if facts["n_segs"] else None
 
 
 _SEGMENTS = WalkSegments()

@@ -24,18 +24,31 @@ def _fuse(parts, hidden: int) -> torch.Tensor:
     return fused
 
 
+def _walk_us(entries: int, tokens: int, longest: int, dk: int, cells: int) -> float:
+    """About how long whole entries walk a state of `cells` = heads * dk * dv numbers: as long as the longest entry's chain of
+    tokens, all tokens' products, or the states' way from and to memory."""
+    return 4.0 + max(0.33 * longest * (1.0 + dk / 128), 0.25e-6 * tokens * cells, 1.6e-6 * entries * cells)
+
+
 def _segments_for(ctx: StepContext, nh: int, dk: int, dv: int, turned: bool = False):
-    """The step's segment lists where this layer takes them.  Segments that run as matrix products pay by the
-    microseconds measured of both forms (16 to 64 heads, steps of 16 to 8,192 tokens): a walk takes 0.6 for every token
-    of the longest entry, more where the entries' blocks exceed what the chip holds at once (2,500); the products take
-    35 and 0.0017 for every token and 128 value columns, 1.4 times that where q and k are turned first (``turned``).
-    Other sizes: the rule of the walks."""
+    """The step's segment lists where this layer takes them.  Sizes whose segments run as matrix products take the form that
+    should be the faster: the walk of all entries, or that of the short ones and then the products of the others, which
+    take a block's 20 us (32 where q and k are turned first, ``turned``) once, or twice for segments that follow each other,
+    and grow with the long entries' tokens.  The numbers are those of both forms at ten sizes (4 to 128 heads) and 43 steps (32
+    to 2,000 tokens beside 0 to 256 single ones): the choice is within 6 % of the faster form in all but four of
+    them.  Other sizes: the rule of the walks."""
     if not ops.walk_takes_chunks(dk, dv):
         return segments_for(ctx, nh, dv, ops.WALK_STATE_COLS)
-    blocks = ctx.n_entries * nh * (dv // ops.WALK_STATE_COLS)
-    walk = 0.6 * ctx.max_entry_len * max(1.0, blocks / 2500)
-    products = 35.0 + 0.0017 * ctx.n_tokens * nh * dv / 128 * (1.4 if turned else 1.0)
-    return ctx.extras.get(WALK_SEGMENTS.key) if walk > products else None
+    segments = ctx.extras.get(WALK_SEGMENTS.key)
+    if segments is None:
+        return None
+    s, cells = segments[3], nh * dk * dv
+    walk = _walk_us(s.entries, s.tokens, s.longest, dk, cells)
+    products = (32.0 if turned else 20.0) * (0.5 + dk / 256) * (2 if s.several else 1) \
+        + (0.16e-6 if turned else 0.09e-6) * (s.tokens - s.short_tokens) * cells
+    if s.short:
+        products += _walk_us(s.short, s.short_tokens, s.longest_short, dk, cells)
+    return segments if walk > products else None
 
 
 class MatrixMemory(Part):

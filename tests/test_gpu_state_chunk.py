@@ -214,7 +214,7 @@ def test_scratch_is_for_entries_of_several_segments_alone():
     code, par, freqs, k_scale = modes
     ctx = _Step(lens, [0] * len(lens), range(len(lens)))
     segs, ents = ops.gla_segments(ctx.lens, ctx.cu)
-    segments = (torch.from_numpy(segs).to(DEV), torch.from_numpy(ents).to(DEV), ops.segments_with_scratch(ents))
+    segments = (torch.from_numpy(segs).to(DEV), torch.from_numpy(ents).to(DEV), ops.segment_counts(lens))
     torch.cuda.synchronize()
     before = torch.cuda.memory_allocated()
     torch.cuda.reset_peak_memory_stats()

@@ -110,3 +110,35 @@ def test_attention_work_lists_cut_a_step_into_decode_tokens_and_tiles():
     arrays, _ = AttentionWorkLists().plan(host)
     null = AttentionWorkLists().null(host, arrays)
     assert [a.size for a in null] == [a.size for a in arrays] and null[0].tolist() == [0, 1, 2]
+
+
+def test_recurrent_states_take_products_only_where_they_are_the_faster_form():
+    """A layer's choice between walking all entries and running the long ones as matrix products, at steps where both were timed
+    (microseconds of the walk, and of the products behind the walk of the short entries)."""
+    from types import SimpleNamespace
+
+    import numpy as np
+
+    from sharpinference_amd import ops
+    from sharpinference_amd.parts.base import HostStep
+    from sharpinference_amd.parts.linear_attention import WALK_SEGMENTS
+    from sharpinference_amd.parts.matrix_memory import _segments_for
+
+    def takes(lens, nh, dk, dv, turned=False):
+        cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        arrays, facts = WALK_SEGMENTS.plan(HostStep(len(lens), int(cu[-1]), list(lens), [0] * len(lens), cu))
+        ctx = SimpleNamespace(extras={}, n_entries=len(lens), n_tokens=int(cu[-1]), max_entry_len=max(lens))
+        WALK_SEGMENTS.attach(ctx, arrays, facts)
+        chosen = _segments_for(ctx, nh, dk, dv, turned)
+        assert chosen is None or tuple(chosen[2]) == ops.segment_counts(lens)
+        return chosen is not None
+
+    for lens, nh, dk, dv, turned, walk, products in (
+            ([64] + [1] * 256, 64, 128, 64, False, 188, 345), ([200] + [1] * 256, 64, 128, 64, False, 193, 352),
+            ([300] + [1] * 256, 128, 128, 64, False, 384, 639), ([64] + [1] * 256, 16, 128, 128, True, 97, 154),
+            ([200] + [1] * 256, 32, 128, 128, False, 247, 427), ([64] + [1] * 64, 32, 128, 128, True, 65, 100),
+            ([1000, 900] + [1] * 16, 16, 128, 128, False, 725, 89), ([2000], 16, 128, 128, False, 1436, 76),
+            ([2000], 64, 128, 64, False, 1072, 140), ([500] * 4, 16, 128, 128, True, 413, 130), ([1500] + [1] * 64, 4, 64, 64, True, 606, 46),
+            ([64], 64, 128, 64, False, 40, 25), ([64] * 6, 16, 128, 128, False, 60, 25), ([64] * 30, 16, 128, 128, True, 136, 109)):
+        assert takes(lens, nh, dk, dv, turned) == (products < walk), (lens[0], len(lens), nh)
+    assert not takes([63] * 3, 16, 128, 128) and not takes([1] * 64, 16, 128, 128)        # steps without a list
