@@ -33,10 +33,11 @@ def _walk_us(entries: int, tokens: int, longest: int, dk: int, cells: int) -> fl
 def _segments_for(ctx: StepContext, nh: int, dk: int, dv: int, turned: bool = False):
     """The step's segment lists where this layer takes them.  Sizes whose segments run as matrix products take the form that
     should be the faster: the walk of all entries, or that of the short ones and then the products of the others, which
-    take a block's 20 us (32 where q and k are turned first, ``turned``) once, or twice for segments that follow each other,
-    and grow with the long entries' tokens.  The numbers are those of both forms at ten sizes (4 to 128 heads) and 43 steps (32
-    to 2,000 tokens beside 0 to 256 single ones): the choice is within 6 % of the faster form in all but four of
-    them.  Other sizes: the rule of the walks."""
+    take a block's 20 us (28 where q and k are turned first, ``turned``; 48 in one pass behind short entries, whose
+    states push the rows out of the caches) once, or twice for segments that follow each other, and grow with the long
+    entries' tokens.  The numbers are those of both forms at ten sizes (4 to 128 heads) and 33 steps (64 to 2,000 tokens
+    beside 0 to 256 single ones): the choice is within 6 % of the faster form in all but 10 of the 330, and in those it is the
+    walk.  Other sizes: the rule of the walks."""
     if not ops.walk_takes_chunks(dk, dv):
         return segments_for(ctx, nh, dv, ops.WALK_STATE_COLS)
     segments = ctx.extras.get(WALK_SEGMENTS.key)
@@ -44,7 +45,8 @@ def _segments_for(ctx: StepContext, nh: int, dk: int, dv: int, turned: bool = Fa
         return None
     s, cells = segments[3], nh * dk * dv
     walk = _walk_us(s.entries, s.tokens, s.longest, dk, cells)
-    products = (32.0 if turned else 20.0) * (0.5 + dk / 256) * (2 if s.several else 1) \
+    block = (28.0 if s.several or not s.short else 48.0) if turned else 20.0
+    products = block * (0.5 + dk / 256) * (2 if s.several else 1) \
         + (0.16e-6 if turned else 0.09e-6) * (s.tokens - s.short_tokens) * cells
     if s.short:
         products += _walk_us(s.short, s.short_tokens, s.longest_short, dk, cells)

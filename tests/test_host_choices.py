@@ -134,11 +134,11 @@ def test_recurrent_states_take_products_only_where_they_are_the_faster_form():
         return chosen is not None
 
     for lens, nh, dk, dv, turned, walk, products in (
-            ([64] + [1] * 256, 64, 128, 64, False, 188, 345), ([200] + [1] * 256, 64, 128, 64, False, 193, 352),
+            ([64] + [1] * 256, 64, 128, 64, False, 185, 219), ([200] + [1] * 256, 64, 128, 64, False, 193, 352),
             ([300] + [1] * 256, 128, 128, 64, False, 384, 639), ([64] + [1] * 256, 16, 128, 128, True, 97, 154),
-            ([200] + [1] * 256, 32, 128, 128, False, 247, 427), ([64] + [1] * 64, 32, 128, 128, True, 65, 100),
-            ([1000, 900] + [1] * 16, 16, 128, 128, False, 725, 89), ([2000], 16, 128, 128, False, 1436, 76),
-            ([2000], 64, 128, 64, False, 1072, 140), ([500] * 4, 16, 128, 128, True, 413, 130), ([1500] + [1] * 64, 4, 64, 64, True, 606, 46),
-            ([64], 64, 128, 64, False, 40, 25), ([64] * 6, 16, 128, 128, False, 60, 25), ([64] * 30, 16, 128, 128, True, 136, 109)):
+            ([200] + [1] * 256, 32, 128, 128, False, 247, 427), ([64] + [1] * 64, 32, 128, 128, True, 65, 100), ([96] + [1] * 64, 16, 128, 128, True, 77, 97),
+            ([1000, 900] + [1] * 16, 16, 128, 128, False, 736, 97), ([2000], 16, 128, 128, False, 1436, 76),
+            ([2000], 64, 128, 64, False, 1072, 140), ([500] * 4, 16, 128, 128, True, 353, 119), ([1500] + [1] * 64, 4, 64, 64, True, 606, 46),
+            ([64], 64, 128, 64, False, 34, 20), ([64] * 6, 16, 128, 128, False, 60, 25), ([64] * 30, 16, 128, 128, True, 136, 109)):
         assert takes(lens, nh, dk, dv, turned) == (products < walk), (lens[0], len(lens), nh)
     assert not takes([63] * 3, 16, 128, 128) and not takes([1] * 64, 16, 128, 128)        # steps without a list
