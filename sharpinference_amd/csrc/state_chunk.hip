@@ -29,7 +29,6 @@
 using f32x4 = __attribute__((__vector_size__(4 * sizeof(float)))) float;
 using bf16x8 = __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16;
 
-constexpr int kSeg = 128;              // tokens of a segment at most
 constexpr int kChunkWaves = 8;
 constexpr int kChunkThreads = kChunkWaves * kWave;
 constexpr int kPadK = 8, kPadV = 16;   // elements behind an LDS row of k and of v (bfloat16: banks 4 and 8 apart from row to row)
@@ -256,9 +255,9 @@ __global__ __launch_bounds__(kChunkThreads) void state_chunk_local_kernel(const 
   SegWeights& w = *reinterpret_cast<SegWeights*>(v_s + kSeg * (DV + kPadV));
   const int h = blockIdx.x;
   const int* sg = a.segs + 4 * blockIdx.y;
-  const int t0 = sg[1], nt = sg[2];
+  const int t0 = sg[1], nt = min(sg[2], kSeg);
   if (sg[3] != 0 || nt <= 0) return;                 // nobody starts from what an entry's last segment makes
-  const int rows = min(kSeg, (nt + 15) / 16 * 16);
+  const int rows = (nt + 15) / 16 * 16;
   const T* proj = static_cast<const T*>(a.proj);
   stage_rows<T, KT, DK, DK + kPadK>(k_s, proj, a.stride, a.k_off + (h / a.heads_per_group) * DK, t0, nt, rows);
   stage_rows<T, T, DV, DV + kPadV>(v_s, proj, a.stride, a.v_off + h * DV, t0, nt, rows);
@@ -289,11 +288,11 @@ __device__ __forceinline__ void state_chunk_final_block(const WalkArgs& a) {
   SegWeights& w = *reinterpret_cast<SegWeights*>(v_s + kSeg * (DV + kPadV));
   const int h = blockIdx.x, lane = threadIdx.x & (kWave - 1), wid = threadIdx.x >> 6, g = lane >> 4, i = lane & 15;
   const int* sg = a.segs + 4 * blockIdx.y;
-  const int e = sg[0], t0 = sg[1], nt = sg[2];
+  const int e = sg[0], t0 = sg[1], nt = min(sg[2], kSeg);
   const bool last = sg[3] != 0;
   const bool only = last && t0 == a.cu_tokens[e];    // an entry's only segment starts from the slot
   if (nt <= 0 || (only ? nt < kChunkFrom : (int)blockIdx.y >= a.n_scratch)) return;
-  const int rows = min(kSeg, (nt + 15) / 16 * 16), tiles = rows / 16;
+  const int rows = (nt + 15) / 16 * 16, tiles = rows / 16;
   const T* proj = static_cast<const T*>(a.proj);
   const int ncb = DV / kWalkCols, slice = walk_slice_floats(DK, MODE);
   const size_t per_head = (size_t)ncb * slice;
@@ -480,6 +479,7 @@ __global__ __launch_bounds__(kChunkThreads) __attribute__((amdgpu_waves_per_eu(2
 SHARPI_EXPORT int sharpi_state_chunk_takes(int dk, int dv) { return (dk == 64 || dk == 128) && (dv == 64 || dv == 128); }
 
 SHARPI_EXPORT int sharpi_state_chunk_from() { return kChunkFrom; }
+SHARPI_EXPORT int sharpi_state_segment_tokens() { return kSeg; }
 
 bool state_chunk_takes(const WalkArgs& a, int dtype) {
   const int V = dtype == DT_BF16 ? 8 : 4;            // 16-byte loads of every head's rows, 16-byte stores of the outputs

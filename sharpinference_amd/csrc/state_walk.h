@@ -28,6 +28,7 @@ struct WalkArgs {
 // The segments' first and last pass in chunk form (state_chunk.hip), for the sizes state_chunk_takes names; entries
 // of fewer than kChunkFrom tokens are left out and walked (a.n_long: the leading segments of all others).
 constexpr int kChunkFrom = 32;
+constexpr int kSeg = 128;          // tokens of a segment at most (the lists are cut to it: a chunk's LDS holds no more)
 bool state_chunk_takes(const WalkArgs& a, int dtype);
 int state_chunk_local(const WalkArgs& a, int dtype, int mode, hipStream_t stream);
 int state_chunk_final(const WalkArgs& a, int dtype, int mode, hipStream_t stream);

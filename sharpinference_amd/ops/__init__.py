@@ -1459,7 +1459,7 @@ def gla_decays_from_middle(proj: torch.Tensor, a_off: int, rank: int, w: torch.T
     return alpha
 
 
-GLA_SEGMENT_TOKENS = 128       # tokens of a segment of the segmented walk
+GLA_SEGMENT_TOKENS = _lib.SEGMENT_TOKENS     # tokens of a segment of the segmented walk, at most
 WALK_CHUNK_FROM = _lib.WALK_CHUNK_FROM       # entries of fewer tokens are walked token by token in every form
 
 

@@ -92,6 +92,7 @@ FUSED_NORM_ROUTER_MAX_HIDDEN = 8192   # widest row of the norm + router kernel
 ROUTER_MAX_EXPERTS = 1024   # experts the routing kernels hold scores for
 GLA_STATE_COLS = 8          # value columns of a linear-attention state that lie together in memory
 WALK_STATE_COLS = 8         # value columns of a slice of a scalar-decay recurrent state (csrc/state_walk.hip)
+SEGMENT_TOKENS = 128        # tokens of a segment of a recurrent state, at most (csrc/state_walk.h holds so many in LDS)
 WALK_CHUNK_FROM = 32        # tokens from which an entry goes through a scalar-decay state in products (csrc/state_walk.h)
 DELTA_CHUNK_TOKENS = 16     # tokens of a chunk of the gated delta rule (csrc/delta_rule.hip)
 LATENT_PAGE_KEYS = 128      # keys of a page of expanded latents (csrc/latent_expand.hip)
@@ -103,6 +104,7 @@ _BUILT_WITH = {
     "sharpi_add_rmsnorm_router_max_hidden": FUSED_NORM_ROUTER_MAX_HIDDEN,
     "sharpi_gla_state_cols": GLA_STATE_COLS,
     "sharpi_state_walk_cols": WALK_STATE_COLS,
+    "sharpi_state_segment_tokens": SEGMENT_TOKENS,
     "sharpi_state_chunk_from": WALK_CHUNK_FROM,
     "sharpi_delta_chunk_tokens": DELTA_CHUNK_TOKENS,
     "sharpi_latent_page_keys": LATENT_PAGE_KEYS,

@@ -225,3 +225,17 @@ def test_scratch_is_for_entries_of_several_segments_alone():
     want, walked = _walk("fixed", lens, rows, None, modes, H, dk, dv, False)
     assert float((out.view_as(want) - want).abs().max()) <= 2e-6 * float(want.abs().max())
     assert float((state - walked).abs().max()) <= 2e-6 * float(walked.abs().max())
+
+
+
+@pytest.mark.parametrize("pad, lens", [(0, [20]), (0, [100]), (0, [300]), (0, [128, 31]), (3, [300, 20, 1])])
+def test_one_entry_alone_and_rows_that_cannot_be_read_in_sixteen_bytes(pad, lens):
+    """One entry below the chunk form's tokens, of one segment, of several; rows of odd strides take the walk in segments."""
+    g = torch.Generator().manual_seed(sum(lens))
+    H, dk, dv = 2, 128, 128
+    modes = _modes("gates", H, dk, g)
+    rows = torch.randn(sum(lens), 3 * H * dk + pad, generator=g).to(torch.bfloat16).to(DEV)
+    gates = torch.randn(sum(lens), 2 * H, generator=g).to(DEV)
+    (got, state), (want, walked) = (_walk("gates", lens, rows, gates, modes, H, dk, dv, s) for s in (True, False))
+    assert float((got - want).norm() / want.norm()) < 1e-5
+    assert float((state - walked).abs().max()) <= 1e-5 * float(walked.abs().max() + 1)

@@ -142,3 +142,27 @@ def test_recurrent_states_take_products_only_where_they_are_the_faster_form():
             ([64], 64, 128, 64, False, 34, 20), ([64] * 6, 16, 128, 128, False, 60, 25), ([64] * 30, 16, 128, 128, True, 136, 109)):
         assert takes(lens, nh, dk, dv, turned) == (products < walk), (lens[0], len(lens), nh)
     assert not takes([63] * 3, 16, 128, 128) and not takes([1] * 64, 16, 128, 128)        # steps without a list
+
+
+def test_segments_are_cut_to_what_the_kernels_hold():
+    """The tokens of a segment and those from which an entry is run in products are the library's own numbers, checked when it is
+    loaded; every list keeps to them, its entries of several segments first and the short ones last."""
+    import numpy as np
+
+    from sharpinference_amd import ops
+    from sharpinference_amd.ops import lib
+
+    assert lib._BUILT_WITH["sharpi_state_segment_tokens"] == ops.GLA_SEGMENT_TOKENS
+    assert lib._BUILT_WITH["sharpi_state_chunk_from"] == ops.WALK_CHUNK_FROM
+    lens = [1, 300, 31, 32, 128, 129, 7, 1000]
+    cu = np.concatenate([[0], np.cumsum(lens)])
+    segs, ents = ops.gla_segments(lens, cu)
+    assert int(segs[:, 2].max()) == ops.GLA_SEGMENT_TOKENS
+    for e, (first, count) in enumerate(ents):
+        mine = segs[first:first + count]
+        assert (mine[:, 0] == e).all() and mine[:, 3].tolist() == [0] * (count - 1) + [1]
+        assert mine[:, 1].tolist() == [cu[e] + 128 * i for i in range(count)] and mine[:, 2].sum() == lens[e]
+    several, long = ops.segment_counts(lens)
+    single = ents[segs[:, 0], 1] == 1
+    assert (several, long) == (3 + 2 + 8, 3 + 2 + 8 + 2) and not single[:several].any() and single[several:].all()
+    assert (segs[several:long, 2] >= ops.WALK_CHUNK_FROM).all() and (segs[long:, 2] < ops.WALK_CHUNK_FROM).all()
