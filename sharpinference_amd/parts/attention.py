@@ -17,6 +17,16 @@ SHORT_PROMPT_TOKENS = 1536   # up to so many prompt tokens in a step, tiles of h
                              # 20-25 % less attention time from 512 to 1,536 tokens, 6 % more at 2,048)
 
 
+def prompt_tile_tokens(lens) -> int:
+    """The rows of a step's prompt tiles."""
+    return PREFILL_TILE_TOKENS if sum(n for n in lens if n > 1) > SHORT_PROMPT_TOKENS else PREFILL_TILE_TOKENS // 2
+
+
+def prompt_tiles(host: HostStep, entries, tile: int, base: int = 0) -> List[Tuple[int, int, int]]:
+    """(entry, first token counted from row `base`, rows) of the given entries' tiles."""
+    return [(e, int(host.cu_tokens[e]) - base + o, min(tile, host.lens[e] - o)) for e in entries for o in range(0, host.lens[e], tile)]
+
+
 class AttentionWorkLists(StepPlanner):
     """How the attention kernels split a batch: the tokens of entries of one token (the split-K
     decode kernel's list; none when every token is one, the kernel then takes them all) and the
@@ -29,9 +39,8 @@ class AttentionWorkLists(StepPlanner):
     def plan(self, host: HostStep) -> Tuple[List[np.ndarray], dict]:
         lens, cu = host.lens, host.cu_tokens
         dec = [int(cu[i]) for i in range(host.n_entries) if lens[i] == 1]
-        tile = PREFILL_TILE_TOKENS if sum(n for n in lens if n > 1) > SHORT_PROMPT_TOKENS else PREFILL_TILE_TOKENS // 2
-        tiles = [(i, int(cu[i]) + o, min(tile, lens[i] - o)) for i in range(host.n_entries) if lens[i] > 1
-                 for o in range(0, lens[i], tile)]
+        tile = prompt_tile_tokens(lens)
+        tiles = prompt_tiles(host, [i for i in range(host.n_entries) if lens[i] > 1], tile)
         arrays = [np.asarray(dec, dtype=np.int32), np.asarray(tiles, dtype=np.int32).reshape(-1)]
         return arrays, dict(n_dec=len(dec), n_tiles=len(tiles), tile=tile, all_decode=len(dec) == host.n_tokens)
 

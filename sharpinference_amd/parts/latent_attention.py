@@ -9,51 +9,93 @@ import torch
 
 from .. import ops
 from ..cache.spec import KVSpec, WINDOW_NONE, WINDOW_SLIDING
+from ..ops.lib import PREFILL_TILE_TOKENS
 from ..ops.profile import section
-from .attention import _WORK_LISTS
+from .attention import _WORK_LISTS, prompt_tile_tokens, prompt_tiles
 from .base import HostStep, LayerCache, ParamSpec, Part, StepContext, StepPlanner, TensorSource
 
 
-# A step's prompt portions attend over expanded keys and values where the (query, key) pairs they hold are at least
+# A step's prompt portions attend over expanded keys and values where their queries times the keys of their spans are at least
 # EXPAND_FROM_TOKENS times the keys to expand (a key's expansion costs about what 28 pairs save), and, times the heads, at
 # least EXPAND_FROM_PAIRS (the two launches more).  Microseconds of a step through four such layers over the shared rows
 # and over expanded keys: 64 heads behind 2,000 keys, 32 tokens 1,338 / 1,268, 128: 2,210 / 1,488, 512: 4,655 / 1,844;
 # behind none, 64 tokens 695 / 698, 128: 853 / 757, 512: 1,691 / 1,054; 16 heads behind 2,000, 32 tokens 1,118 / 777;
-# behind none, 128 tokens 661 / 713, 512: 872 / 705.
+# behind none, 128 tokens 661 / 713, 512: 872 / 705.  A window makes the queries see fewer pairs than that, and the shared
+# rows' kernel no faster: 2,000 tokens of 64 heads, window 64: 2,486 / 1,292, window 16: 2,345 / 1,273.
 EXPAND_FROM_TOKENS = 32
 EXPAND_FROM_PAIRS = 1 << 19
-EXPAND_MAX_BYTES = 2 << 30         # ... and the expanded keys and values take at most this much for the layer's time
+EXPAND_MAX_BYTES = 2 << 30         # ... and the expanded keys and values take at most this much for the layer's time: the
+                                   # portions with the most keys give way
+
+
+def _few_queries_lose(n: int, span: int, keys: int, heads: int, context: int, tile: int) -> bool:
+    """Whether a portion of few queries (fewer than make up for their keys) is the slower for an expansion of its keys beside
+    portions that pay.  Either way one block a head walks the keys, in microseconds: the expansion 0.8 for 1,024 keys and head,
+    the flash kernel 0.05 a key (0.075 in tiles of the full height), the shared rows 0.13 a key of a run and 150 of
+    launches.  A step through four layers, expanded / left out: 2,000 tokens and 2 behind 32,000 keys, 64 heads 17,470 /
+    11,060, 16 heads 12,430 / 9,970; 1,000 tokens and 4 behind 24,000, 64 heads 10,330 / 10,070, 16 heads 6,940 / 9,360; behind
+    6,000, 64 heads 3,130 / 3,340."""
+    expanded = 0.8 * keys * heads / 1024 + (0.05 if tile < PREFILL_TILE_TOKENS else 0.075) * span
+    return n < EXPAND_FROM_TOKENS and expanded > 0.13 * min(ops.latent_run_keys(context, True), span) + 150.0
 
 
 class LatentPages(StepPlanner):
-    """The pages of 128 keys that a step's prompt portions see through a window: the list of them (entry, page of its
-    sequence, first key that is there, end of the keys) and the block table of a cache that holds just them."""
+    """Which of a step's prompt portions attend over expanded keys and values, seen through a window by `heads` heads of
+    `width` elements of key and value.  For them the list of pages of 128 keys (entry, page of its sequence, first key that
+    is there, end of the keys), the block table of a cache that holds just those, and their tiles; for the other portions
+    the stretches of neighbouring rows and their tiles, counted from the stretch's first row."""
 
-    def __init__(self, window_kind: int, window: int):
+    def __init__(self, window_kind: int, window: int, heads: int, width: int):
         self.spec = KVSpec(1, 1, window_kind, window)
-        self.key = f"latent pages {window_kind} {window}"
+        self.heads, self.key_bytes = int(heads), 2 * int(heads) * int(width)
+        self.key = f"latent pages {window_kind} {window} {heads} {width}"
 
     def plan(self, host: HostStep) -> Tuple[List[np.ndarray], dict]:
+        nothing = [np.zeros(0, dtype=np.int32)] * 4, dict(pages=0)
         long = [e for e, n in enumerate(host.lens) if n > 1]
-        pages, spans, pairs = [], [], 0
+        if not long:
+            return nothing
+        tile = prompt_tile_tokens(host.lens)
+        context = max(host.starts[e] + host.lens[e] for e in range(host.n_entries))
+        spans = {}                                                # the entries' (first key, end, first page, end)
         for e in long:
             lo, hi = self.spec.first_visible(host.starts[e]), host.starts[e] + host.lens[e]
-            first, end = lo // ops.LATENT_PAGE_KEYS, (hi - 1) // ops.LATENT_PAGE_KEYS + 1
-            spans.append((e, first, len(pages), end - first))
+            spans[e] = (lo, hi, lo // ops.LATENT_PAGE_KEYS, (hi - 1) // ops.LATENT_PAGE_KEYS + 1)
+        keys = {e: (end - first) * ops.LATENT_PAGE_KEYS for e, (_, _, first, end) in spans.items()}
+        chosen = [e for e, (lo, hi, _, _) in spans.items()
+                  if not _few_queries_lose(host.lens[e], hi - lo, keys[e], self.heads, context, tile)]
+        while chosen and sum(keys[e] for e in chosen) * self.key_bytes > EXPAND_MAX_BYTES:
+            chosen.remove(max(chosen, key=keys.__getitem__))
+        pairs = sum(host.lens[e] * (spans[e][1] - spans[e][0]) for e in chosen)
+        if not chosen or pairs < EXPAND_FROM_TOKENS * sum(keys[e] for e in chosen) or pairs * self.heads < EXPAND_FROM_PAIRS:
+            return nothing
+        pages = []
+        table = np.full((host.n_entries, max(spans[e][3] for e in chosen)), -1, dtype=np.int32)
+        for e in chosen:
+            lo, hi, first, end = spans[e]
+            table[e, first:end] = np.arange(len(pages), len(pages) + end - first, dtype=np.int32)
             pages += [(e, b, lo, hi) for b in range(first, end)]
-            pairs += host.lens[e] * (hi - lo)
-        table = np.full((host.n_entries, max((f + n for _, f, _, n in spans), default=0)), -1, dtype=np.int32)
-        for e, first, at, n in spans:
-            table[e, first:first + n] = np.arange(at, at + n, dtype=np.int32)
-        single = [int(host.cu_tokens[e]) for e, n in enumerate(host.lens) if n == 1]
-        rows = (single[0], single[-1] + 1) if single and single[-1] - single[0] + 1 == len(single) else None
-        return [np.asarray(pages, dtype=np.int32).reshape(-1), table.reshape(-1)], dict(
-            pages=len(pages), entries=host.n_entries, pairs=pairs, keys=sum(n for *_, n in spans) * ops.LATENT_PAGE_KEYS,
-            decode_rows=rows, scattered=bool(single) and rows is None)
+        tiles = prompt_tiles(host, chosen, tile)
+        rest, other = [], []                                      # (first row, end, first tile, end, entries) of what is left out
+        for e in (e for e in long if e not in chosen):
+            a, b = int(host.cu_tokens[e]), int(host.cu_tokens[e + 1])
+            if not rest or rest[-1][1] != a:
+                rest.append([a, b, len(other), 0, []])
+            other += prompt_tiles(host, [e], tile, rest[-1][0])
+            rest[-1][1], rest[-1][3] = b, len(other)
+            rest[-1][4].append(e)
+        single = [e for e, n in enumerate(host.lens) if n == 1]
+        if single:
+            a, b = int(host.cu_tokens[single[0]]), int(host.cu_tokens[single[-1] + 1])
+            rest.append([a, b, 0, 0, single])
+        arrays = [np.asarray(x, dtype=np.int32).reshape(-1) for x in (pages, table, tiles, other)]
+        return arrays, dict(pages=len(pages), entries=host.n_entries, keys=len(pages) * ops.LATENT_PAGE_KEYS, tile=tile, rest=rest,
+                            scattered=bool(single) and b - a != len(single))
 
     def attach(self, ctx: StepContext, views: List[torch.Tensor], facts: dict) -> None:
         n = facts["pages"]
-        ctx.extras[self.key] = (views[0].view(n, 4), views[1].view(facts["entries"], -1), facts) if n else None
+        ctx.extras[self.key] = (views[0].view(n, 4), views[1].view(facts["entries"], -1), views[2].view(-1, 3), views[3].view(-1, 3),
+                                facts) if n else None
 
 
 class LatentAttention(Part):
@@ -114,7 +156,7 @@ class LatentAttention(Part):
         self.w_uk_t: Optional[torch.Tensor] = None         # [heads, rank, dn]: W_uk per head, transposed
         self.w_uv: Optional[torch.Tensor] = None           # [heads, dv, rank]
         self.w_ukv: Optional[torch.Tensor] = None          # [heads, dn + dv, rank]: both row by row, where prompts expand keys
-        self.pages = LatentPages(self.window_kind, self.window)
+        self.pages = LatentPages(self.window_kind, self.window, self.nh, self.dn + self.dr + self.dv)
         self.w_o = None
         self.w_norm: Optional[torch.Tensor] = None         # float32 [rank]
         self.w_sink: Optional[torch.Tensor] = None         # float32 [heads]
@@ -265,22 +307,17 @@ class LatentAttention(Part):
             ops.head_gemm(o_lat, 0, self.rank, self.w_uv, o, 0, self.dv, gate=gate, gate_off=g_off)
 
     def _pages_to_expand(self, ctx: StepContext, proj: torch.Tensor):
-        """The step's pages where its prompt portions attend over expanded keys and values, else None: bfloat16 layers of
+        """The step's pages where prompt portions of it attend over expanded keys and values, else None: bfloat16 layers of
         widths the kernels take, portions long enough to pay for the expansion, the single tokens (which keep to the
         shared rows) side by side in the batch."""
         if self.w_ukv is None or ctx.act_dtype != torch.bfloat16 or proj.shape[1] % 8 or self.window_kind not in (WINDOW_NONE, WINDOW_SLIDING):
             return None
         pages = ctx.extras.get(self.pages.key)
-        if pages is None or pages[2]["scattered"]:
-            return None
-        facts = pages[2]
-        size = 2 * facts["keys"] * self.nh * (self.dn + self.dr + self.dv)
-        pays = facts["pairs"] >= EXPAND_FROM_TOKENS * facts["keys"] and facts["pairs"] * self.nh >= EXPAND_FROM_PAIRS
-        return pages if pays and size <= EXPAND_MAX_BYTES else None
+        return None if pages is None or pages[4]["scattered"] else pages
 
     def _attend_expanded(self, q: torch.Tensor, pages, ctx: StepContext, cache: LayerCache, inv_freq: Optional[torch.Tensor],
                          magnitude: float) -> torch.Tensor:
-        listed, table, facts = pages
+        listed, table, tiles, other, facts = pages
         T, hd = q.shape[0], self.dn + self.dr
         with section("expand uk, uv", nbytes=2 * facts["keys"] * (self.rank + self.dr + self.nh * (hd + self.dv)),
                      flops=2.0 * facts["keys"] * self.nh * (self.dn + self.dv) * self.rank):
@@ -289,13 +326,15 @@ class LatentAttention(Part):
             qr = ops.latent_queries(q, ctx.positions, inv_freq, magnitude, self.nh, self.dn, self.dr)
         with section("attention", nbytes=2 * (facts["keys"] + T) * self.nh * (hd + self.dv),
                      flops=lambda: 2.0 * self._keys_read(ctx) * self.nh * (hd + self.dv)):
-            o = ops.attention_prefill(qr, k, v, table, ctx.positions, ctx.prefill_tiles, self.window_kind, self.window, self.scale, self.nh,
-                                      self.nh, hd, tile_tokens=ctx.prefill_tile_tokens, sink=self.w_sink, vd=self.dv)
-        if facts["decode_rows"] is not None:
-            a, b = facts["decode_rows"]
-            alone = SimpleNamespace(entry_of_token=ctx.entry_of_token[a:b], positions=ctx.positions[a:b], n_decode=b - a, decode_tokens=None,
-                                    n_prefill_tiles=0, entry_lens=[1] * (b - a),
-                                    entry_starts=[s for s, n in zip(ctx.entry_starts, ctx.entry_lens) if n == 1])
+            o = ops.attention_prefill(qr, k, v, table, ctx.positions, tiles, self.window_kind, self.window, self.scale, self.nh,
+                                      self.nh, hd, tile_tokens=facts["tile"], sink=self.w_sink, vd=self.dv)
+        # the step's other rows, over the shared rows: its single tokens, and the stretches of portions that do not pay
+        for a, b, t0, t1, entries in facts["rest"]:
+            single = t0 == t1
+            alone = SimpleNamespace(entry_of_token=ctx.entry_of_token[a:b], positions=ctx.positions[a:b], n_decode=b - a if single else 0,
+                                    decode_tokens=None, n_prefill_tiles=t1 - t0, prefill_tiles=None if single else other[t0:t1],
+                                    prefill_tile_tokens=facts["tile"], entry_lens=[ctx.entry_lens[e] for e in entries],
+                                    entry_starts=[ctx.entry_starts[e] for e in entries])
             q_full = torch.empty(b - a, self.nh * (self.rank + self.dr), dtype=q.dtype, device=q.device)
             ops.latent_prep(q[a:b], 0, None, q_full, None, None, alone.positions, inv_freq, self.w_norm, self.eps, self.nh, self.dn, self.dr,
                             self.rank, magnitude=magnitude)

@@ -111,3 +111,54 @@ def test_prompts_over_expanded_keys_are_as_exact_as_over_the_shared_rows(name, p
     e_new, e_shared = torch.cat(errs, dim=1).pow(2).mean(dim=1).sqrt().tolist()
     print(f"{name}: expanded {e_new:.3e} shared {e_shared:.3e}")
     assert e_new <= 1.2 * e_shared and float(torch.cat(errs, dim=1)[0].max()) < 0.1
+
+
+@pytest.mark.parametrize("name, plain", [("rigodra", plain_rigodra), ("pagonex", plain_pagonex)])
+def test_portions_left_out_of_the_expansion_keep_to_the_shared_rows(name, plain, tmp_path, monkeypatch):
+    """Portions of few tokens, as those that would lose by an expansion of a long context, before, between and behind
+    portions that are expanded, beside each other, and beside decoding requests: every row of logits against the plain model
+    in 64 bits, held to what the shared rows alone give (1.2 times over all rows: the two round in different places)."""
+    from sharpinference_amd import load_config
+    from sharpinference_amd.engine import Engine, StepEntry
+    from sharpinference_amd.parts import latent_attention as L
+    from sharpinference_amd.weights.loader import write_random_model
+
+    cfg, d = _latent_only(name), str(tmp_path / name)
+    write_random_model(load_config(cfg), d, 7, std=0.1, std_by_suffix={"embed": 1.0})
+    reqs = {r: _tokens(300, 128, i) for i, r in enumerate("abcdef")}
+    steps = [[("a", 9), ("b", 130), ("c", 5), ("d", 20)], [("e", 1), ("f", 1), ("a", 70), ("c", 100), ("b", 17), ("d", 140)],
+             [("b", 150), ("e", 2), ("c", 120), ("a", 30), ("f", 40)], [("a", 1), ("b", 1), ("c", 1), ("d", 60), ("e", 19)]]
+    left_out = []
+    real = L.LatentAttention._attend_shared
+    monkeypatch.setattr(L.LatentAttention, "_attend_shared", lambda self, q, *a: left_out.append(q.shape[0]) or real(self, q, *a))
+    monkeypatch.setattr(L, "_few_queries_lose", lambda n, *a: n < 40)
+    monkeypatch.setattr(L, "EXPAND_FROM_PAIRS", 0)
+
+    def run(least):
+        monkeypatch.setattr(L, "EXPAND_FROM_TOKENS", least)
+        eng = Engine(d, dtype="bfloat16", max_num_seqs=6, kv_tokens=2000, max_model_len=512, max_tokens_per_step=512, decode_graphs=False)
+        got, at = {r: [] for r in reqs}, {r: 0 for r in reqs}
+        for r in reqs:
+            eng.add_request(r)
+        for step in steps:
+            o = eng.step([StepEntry(r, reqs[r][at[r]:at[r] + n], tuple(range(n))) for r, n in step]).cpu()
+            i = 0
+            for r, n in step:
+                got[r].append(o[i:i + n])
+                i += n
+                at[r] += n
+        return {r: torch.cat(v).double() for r, v in got.items()}
+
+    new = run(1)
+    # three layers a step; what each step leaves over the shared rows, a stretch a call
+    assert left_out == [9, 25] * 3 + [17, 2] * 3 + [2, 30] * 3 + [19, 3] * 3
+    shared = run(1 << 30)
+    raw, w = plain.read_config(d), plain.load_weights(d, torch.float64)
+    errs = []
+    for r, toks in reqs.items():
+        n = new[r].shape[0]
+        want = plain.forward(raw, w, toks[:n]).double()
+        errs.append(torch.stack([(x[r] - want).norm(dim=-1) / want.norm(dim=-1) for x in (new, shared)]))
+    e_new, e_shared = torch.cat(errs, dim=1).pow(2).mean(dim=1).sqrt().tolist()
+    print(f"{name}: some left out {e_new:.3e} shared {e_shared:.3e}")
+    assert e_new <= 1.2 * e_shared and float(torch.cat(errs, dim=1)[0].max()) < 0.1

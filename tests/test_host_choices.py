@@ -166,3 +166,44 @@ def test_segments_are_cut_to_what_the_kernels_hold():
     single = ents[segs[:, 0], 1] == 1
     assert (several, long) == (3 + 2 + 8, 3 + 2 + 8 + 2) and not single[:several].any() and single[several:].all()
     assert (segs[several:long, 2] >= ops.WALK_CHUNK_FROM).all() and (segs[long:, 2] < ops.WALK_CHUNK_FROM).all()
+
+
+def _latent_pages(lens, starts, kind=0, window=0, heads=64, width=320):
+    """The step's plan of a latent layer -> (entries whose keys are expanded, pages, block table, tiles, the other tiles, facts)"""
+    import numpy as np
+
+    from sharpinference_amd.parts.base import HostStep
+    from sharpinference_amd.parts.latent_attention import LatentPages
+
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    (pages, table, tiles, other), facts = LatentPages(kind, window, heads, width).plan(HostStep(len(lens), int(cu[-1]), lens, starts, cu))
+    pages = pages.reshape(-1, 4).tolist()
+    return sorted({p[0] for p in pages}), pages, table.reshape(len(lens), -1), tiles.reshape(-1, 3).tolist(), other.reshape(-1, 3).tolist(), facts
+
+
+def test_prompt_portions_expand_their_keys_where_it_is_the_faster_form():
+    from sharpinference_amd.cache.spec import WINDOW_SLIDING
+
+    # a long prompt beside a few tokens behind a long context: the context's keys stay as they are
+    chosen, pages, table, tiles, other, facts = _latent_pages([2000, 2], [0, 30000])
+    assert chosen == [0] and len(pages) == 16 and table[0, :16].tolist() == list(range(16)) and int(table[1].max()) == -1
+    assert sum(t[2] for t in tiles) == 2000 and other == [[1, 0, 2]] and facts["rest"] == [[2000, 2002, 0, 1, [1]]]
+    assert _latent_pages([2000, 2], [0, 30000], heads=16)[0] == [0]
+    # ... unless the flash kernel walks them faster than the shared rows are walked
+    assert _latent_pages([1000, 4], [0, 24000], heads=16)[0] == [0, 1] and _latent_pages([1000, 4], [0, 3000])[0] == [0, 1]
+    assert _latent_pages([2000, 2], [0, 30000], WINDOW_SLIDING, 1024)[0] == [0, 1]
+    assert _latent_pages([2000, 300], [0, 20000])[0] == [0, 1]                    # (queries enough for their keys)
+    # a context whose expanded keys would not fit leaves the other prompts theirs
+    assert _latent_pages([2000, 4000], [0, 60000])[0] == [0] and _latent_pages([2000, 4000], [0, 60000], heads=16)[0] == [0, 1]
+    # too little work in all, portions that are too short
+    assert _latent_pages([80], [0], heads=16)[0] == [] and _latent_pages([80] * 6, [0] * 6, heads=16)[0] == list(range(6))
+    assert _latent_pages([31, 1, 1], [2000, 5, 6])[0] == [] and _latent_pages([40, 1, 1], [2000, 5, 6])[0] == [0]
+    assert _latent_pages([1] * 8, [2000] * 8)[0] == []
+    # what is left out: neighbouring portions together, the single tokens apart
+    far = 30000
+    chosen, _, _, tiles, other, facts = _latent_pages([1, 1, 5, 9, 700, 3, 600, 2, 4], [9, 9, far, far, 0, far, 64, far, far])
+    assert chosen == [4, 6]
+    assert facts["rest"] == [[2, 16, 0, 2, [2, 3]], [716, 719, 2, 3, [5]], [1319, 1325, 3, 5, [7, 8]], [0, 2, 0, 0, [0, 1]]]
+    assert other == [[2, 0, 5], [3, 5, 9], [5, 0, 3], [7, 0, 2], [8, 2, 4]] and not facts["scattered"]
+    assert [t for t in tiles if t[0] == 6][0] == [6, 719, 64] and sum(t[2] for t in tiles) == 1300
+    assert _latent_pages([1, 700, 1], [9, 0, 9])[5]["scattered"]
