@@ -163,7 +163,7 @@ class LatentAttention(Part):
 
     # -- what it needs --------------------------------------------------------
     def step_planners(self):
-        return (_WORK_LISTS, self.pages)
+        return (_WORK_LISTS, self.pages) if self.w_ukv is not None else (_WORK_LISTS,)     # (known once the weights are there)
 
     def cache_spec(self) -> KVSpec:
         return KVSpec(1, self.rank + self.dr, *self.kept, self.rank, values_in_keys=True)

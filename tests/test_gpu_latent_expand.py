@@ -162,3 +162,22 @@ def test_portions_left_out_of_the_expansion_keep_to_the_shared_rows(name, plain,
     e_new, e_shared = torch.cat(errs, dim=1).pow(2).mean(dim=1).sqrt().tolist()
     print(f"{name}: some left out {e_new:.3e} shared {e_shared:.3e}")
     assert e_new <= 1.2 * e_shared and float(torch.cat(errs, dim=1)[0].max()) < 0.1
+
+
+def test_only_layers_that_can_expand_have_the_pages_planned(tmp_path):
+    """Layers with a gate for every output element, and layers in 32 bits, keep to the shared rows: their steps list no pages."""
+    import tiny_kuvonex
+    from sharpinference_amd import load_config
+    from sharpinference_amd.engine import Engine
+    from sharpinference_amd.parts.latent_attention import LatentPages
+    from sharpinference_amd.weights.loader import write_random_model
+
+    def planned(cfg, dtype):
+        d = str(tmp_path / cfg["architecture"])
+        write_random_model(load_config(cfg), d, 7, std=0.1)
+        eng = Engine(d, dtype=dtype, max_num_seqs=1, kv_tokens=64, max_model_len=64, max_tokens_per_step=64, decode_graphs=False)
+        return sum(isinstance(p, LatentPages) for p in eng.runner.planners)
+
+    gated = _latent_only("rigodra")
+    assert planned(gated, "bfloat16") == 1 and planned(gated, "float32") == 0
+    assert planned(next(iter(tiny_kuvonex.CONFIGS.values())), "bfloat16") == 0
