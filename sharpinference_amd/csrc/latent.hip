@@ -18,7 +18,7 @@
 constexpr int kMaxPairs = 128;   // rotated pairs of a head's rotated part
 
 // ---------------------------------------------------------------------------
-template <typename TD, typename TO>
+template <typename TD, typename TO, int kCols>
 __global__ __launch_bounds__(256) void norm_add_kernel(float* __restrict__ h, const TD* __restrict__ delta,
                                                        const float* __restrict__ w, TO* __restrict__ out, int hidden,
                                                        float eps, const int* __restrict__ sum_pos,
@@ -26,9 +26,8 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* __restrict__ h, co
   extern __shared__ float rowbuf[];
   __shared__ float red[16];
   const int t = blockIdx.x;
-  // Bound: latency (a few rows), so eight of a thread's columns are read at a time, and two picks of each (a load at a time
-  // 64 rows 2048 wide of six picks took 20.6 us, now 6.3).  The sums keep their order: a thread's columns ascending.
-  constexpr int kCols = 8;
+  // Bound: latency (a few rows), so up to eight of a thread's columns are read at a time, and two picks of each (a load at a
+  // time 64 rows 2048 wide of six picks took 20.6 us, now 6.3).  The sums keep their order: a thread's columns ascending.
   float ss = 0.f;
   for (int c0 = threadIdx.x; c0 < hidden; c0 += kCols * blockDim.x) {
     float d[kCols];
@@ -99,9 +98,18 @@ SHARPI_EXPORT int sharpi_norm_add(float* h, const void* delta, int d_dtype, cons
   if (hidden <= 0 || hidden > 12288 || !(eps > 0.f) || !delta || !w || (sum_pos && sum_k <= 0)) return SHARPI_ERR_ARG;
   dim3 grid(n_tokens), block(256);
   const size_t lds = (size_t)hidden * sizeof(float);
+  // kCols: a thread's columns, up to eight (eight where there are two read the row's last four times: 8192 rows 512 wide
+  // 12.3 -> 15.7 us, with two 12.3 again)
+#define NORM_ADD_AT(TDV, TOV, COLS)                                                                               \
+  norm_add_kernel<TDV, TOV, COLS><<<grid, block, lds, stream>>>(h, (const TDV*)delta, w, (TOV*)out, hidden, eps,  \
+                                                                sum_pos, sum_w, sum_k)
 #define NORM_ADD(TDV, TOV)                                                                                       \
-  norm_add_kernel<TDV, TOV><<<grid, block, lds, stream>>>(h, (const TDV*)delta, w, (TOV*)out, hidden, eps,       \
-                                                          sum_pos, sum_w, sum_k)
+  do {                                                                                                           \
+    if (hidden <= 256) NORM_ADD_AT(TDV, TOV, 1);                                                                 \
+    else if (hidden <= 512) NORM_ADD_AT(TDV, TOV, 2);                                                            \
+    else if (hidden <= 1024) NORM_ADD_AT(TDV, TOV, 4);                                                           \
+    else NORM_ADD_AT(TDV, TOV, 8);                                                                               \
+  } while (0)
   const int od = out ? out_dtype : d_dtype;
   if (d_dtype == DT_F32 && od == DT_F32) NORM_ADD(float, float);
   else if (d_dtype == DT_BF16 && od == DT_BF16) NORM_ADD(bf16_t, bf16_t);
@@ -109,6 +117,7 @@ SHARPI_EXPORT int sharpi_norm_add(float* h, const void* delta, int d_dtype, cons
   else if (d_dtype == DT_BF16 && od == DT_F32) NORM_ADD(bf16_t, float);
   else return SHARPI_ERR_ARG;
 #undef NORM_ADD
+#undef NORM_ADD_AT
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
 }

@@ -302,6 +302,27 @@ def test_an_expert_sum_formed_in_the_norm_is_the_combine_kernels(T, N, k, weight
     assert torch.equal(got, first)
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T, N", [(7, 1), (3, 256), (5, 257), (2, 512), (4, 513), (3, 1024), (2, 1025), (9, 2049)])
+def test_the_norm_into_the_stream_at_the_edges_of_a_threads_columns(T, N, dtype):
+    """One, two, four or eight columns of a thread at a time, by the width: as the norm in 64 bits, and the same bits with an
+    expert sum formed on the way.  Bound: a sum of N squares in any order, and a handful of roundings of each term."""
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(N)
+    y = torch.randn(T * 3, N, generator=g).to(DT[dtype]).to(DEV)
+    pos = torch.randperm(T * 3, generator=g).to(torch.int32).to(DEV)
+    h, w = torch.randn(T, N, generator=g).to(DEV), torch.rand(N, generator=g).to(DEV)
+    lazy = ops.ExpertSum(y, pos, None, T, 3, torch.rand(T, 3, generator=g).to(DEV))
+    delta, got, first = lazy.tensor(), h.clone(), h.clone()
+    ops.norm_add(got, lazy, w, 1e-6, None)
+    ops.norm_add(first, delta, w, 1e-6, None)
+    assert torch.equal(got, first)
+    d = delta.double()
+    term = d / (d.pow(2).mean(-1, keepdim=True) + 1e-6).sqrt() * w.double()
+    assert bool(((first.double() - h.double() - term).abs() <= 2.0 ** -24 * ((N / 256 + 16) * term.abs() + 2 * h.double().abs())).all())
+
+
 @pytest.mark.parametrize("H, R, dr", [(16, 512, 64), (2, 80, 24), (17, 512, 128), (31, 208, 8), (33, 16, 0), (65, 256, 32)])
 def test_a_rows_bits_are_the_same_however_many_waves_share_it(H, R, dr):
     """Single tokens of up to 16, 32 and more heads (8, 4, 2 waves a row) against the prompt tiles' 2; 128 keys are one run of both."""
