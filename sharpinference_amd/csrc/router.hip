@@ -542,11 +542,15 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
   // What it measured (one expert a wave, four tokens a block from 64 tokens before): 3000 rows 2048 wide of 128 experts
   // 90 -> 56 us, 64 rows 4096 wide 47 -> 19, 1660 rows 2048 wide of 64 experts with float weights 36 -> 32; 16 experts the same (latency).
   // Few tokens, or rows that cannot be read in runs of 8: a block a token, a wave an expert at a time (enough waves for the
-  // experts, at most 16).  From 64 tokens: four experts a wave (one where there are fewer than 64 experts: each wave has
-  // one then), for four tokens a block where a token a block would be more than one block a compute unit.
+  // experts, at most 16).  From 64 tokens: four experts a wave (one where there are fewer than 64 experts: a wave has
+  // few then), for four tokens a block where a token a block would be more than one block a compute unit.  Four tokens of few
+  // experts are bound by the loads of the tokens' rows: two runs on their way at a time (wave_dot_rows) are faster than one
+  // (wave_dots) where those rows are floats (12,000 rows 1024 wide of 16 experts 45 / 65 us, of 63 130 / 148; 3,000 rows
+  // 2048 wide of 32 34 / 37) or the experts at most 16 (3,000 bfloat16 rows 5120 wide of 8: 15.6 / 16.7), else not
+  // (12,000 bfloat16 rows 1024 wide of 32: 77 / 68).
   const bool runs = (hidden & 7) == 0 && n_tokens >= 64;
   const int tt = runs ? (n_tokens > 256 ? 4 : 1) : n_tokens >= 64 ? 4 : 1;
-  const int ee = !runs ? 0 : n_experts >= 64 ? 4 : 1;
+  const int ee = !runs ? 0 : n_experts >= 64 ? 4 : tt == 4 && (x_dtype == DT_F32 || n_experts <= 16) ? 0 : 1;
   dim3 grid(ceil_div(n_tokens, tt)), block(kWave * (n_experts >= 16 ? 16 : n_experts >= 8 ? 8 : 4));
   const size_t lds = split_choice ? (size_t)tt * (n_experts + n_groups) * sizeof(float) : 0;
 #define ROUTER_LAUNCH_AT(TX, TWT, EEV, TTV)                                                                      \
@@ -558,7 +562,8 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
     if (ee == 4) {                                                                                               \
       if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, 4, 4); else ROUTER_LAUNCH_AT(TX, TWT, 4, 1);                        \
     } else if (ee == 1) {                                                                                        \
-      if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, 1, 4); else ROUTER_LAUNCH_AT(TX, TWT, 1, 1);                        \
+      if (tt == 1) ROUTER_LAUNCH_AT(TX, TWT, 1, 1);                                                              \
+      else if constexpr (sizeof(TX) == 2) ROUTER_LAUNCH_AT(TX, TWT, 1, 4);                                       \
     } else {                                                                                                     \
       if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, 0, 4); else ROUTER_LAUNCH_AT(TX, TWT, 0, 1);                        \
     }                                                                                                            \
