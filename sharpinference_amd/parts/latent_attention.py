@@ -17,10 +17,10 @@ from .base import HostStep, LayerCache, ParamSpec, Part, StepContext, StepPlanne
 
 # A step's prompt portions attend over expanded keys and values where their queries times the keys of their spans are at least
 # EXPAND_FROM_TOKENS times the keys to expand (a key's expansion costs about what 28 pairs save), and, times the heads, at
-# least EXPAND_FROM_PAIRS (the two launches more).  Microseconds of a step through four such layers over the shared rows
-# and over expanded keys: 64 heads behind 2,000 keys, 32 tokens 1,338 / 1,268, 128: 2,210 / 1,488, 512: 4,655 / 1,844;
-# behind none, 64 tokens 695 / 698, 128: 853 / 757, 512: 1,691 / 1,054; 16 heads behind 2,000, 32 tokens 1,118 / 777;
-# behind none, 128 tokens 661 / 713, 512: 872 / 705.  A window makes the queries see fewer pairs than that, and the shared
+# least EXPAND_FROM_PAIRS (the two launches more), and where the whole of it saves time (_saved).  Microseconds of a step through
+# four such layers over the shared rows and over expanded keys: 64 heads behind 2,000 keys, 40 tokens 1,177 / 1,354, 64: 1,757 /
+# 1,347, 400: 3,213 / 1,595; behind none, 100 tokens 961 / 928, 400: 1,262 / 979; 16 heads behind 2,000, 40 tokens 1,140 / 1,031;
+# behind none, 200 tokens 977 / 947, 700: 1,054 / 1,001.  A window makes the queries see fewer pairs than that, and the shared
 # rows' kernel no faster: 2,000 tokens of 64 heads, window 64: 2,486 / 1,292, window 16: 2,345 / 1,273.
 EXPAND_FROM_TOKENS = 32
 EXPAND_FROM_PAIRS = 1 << 19
@@ -37,6 +37,25 @@ def _few_queries_lose(n: int, span: int, keys: int, heads: int, context: int, ti
     6,000, 64 heads 3,130 / 3,340."""
     expanded = 0.8 * keys * heads / 1024 + (0.05 if tile < PREFILL_TILE_TOKENS else 0.075) * span
     return n < EXPAND_FROM_TOKENS and expanded > 0.13 * min(ops.latent_run_keys(context, True), span) + 150.0
+
+
+# What a step leaves over the shared rows goes in stretches of neighbouring rows, five launches more each: a layer's time with the
+# host that makes them, in microseconds (the first: as FIRST_STRETCH times the pairs of the expansion's two launches).
+STRETCH_US = 75.0
+FIRST_STRETCH = 20
+PAIR_US = 5.0 / (1 << 20)          # (a layer's time for a query, a key and a head: 6.5 over the shared rows, 1.5 in the flash kernel)
+
+
+def _saved(pairs: int, keys: int, span: int, heads: int, context: int, tile: int) -> float:
+    """What an expansion saves a layer, in microseconds: `pairs` of query and key, `keys` to expand, `span` keys of the longest
+    portion, which one block walks in either form.  Measured, a layer of four with experts behind them, and this: 64 heads, 200
+    tokens 26 / 15, 400 107 / 55, 1,500 692 / 668, 40 behind 2,000 -37 / -46, 64 behind 2,000 106 / 95; 16 heads, 400 tokens 33 / 38,
+    1,500 160 / 211, 100 behind 2,000 141 / 150.  A stretch took 30 to 60 of it (up to 90 where nothing else kept the GPU busy).
+    Steps of 8 single tokens beside a portion, expanded / shared, microseconds: 64 heads, 200 tokens 1,940 / 1,860, 400 2,071 / 2,377,
+    64 behind 2,000 2,407 / 2,705; 16 heads, 400 tokens 1,991 / 1,917, 700 2,081 / 2,215, 64 behind 2,000 2,050 / 2,634; two single
+    tokens around 700 tokens of 64 heads 2,407 / 2,957."""
+    walk = 0.13 * min(ops.latent_run_keys(context, True), span) - (0.05 if tile < PREFILL_TILE_TOKENS else 0.075) * span
+    return walk + PAIR_US * pairs * heads - 0.8 * keys * heads / 1024
 
 
 class LatentPages(StepPlanner):
@@ -66,8 +85,22 @@ class LatentPages(StepPlanner):
                   if not _few_queries_lose(host.lens[e], hi - lo, keys[e], self.heads, context, tile)]
         while chosen and sum(keys[e] for e in chosen) * self.key_bytes > EXPAND_MAX_BYTES:
             chosen.remove(max(chosen, key=keys.__getitem__))
-        pairs = sum(host.lens[e] * (spans[e][1] - spans[e][0]) for e in chosen)
-        if not chosen or pairs < EXPAND_FROM_TOKENS * sum(keys[e] for e in chosen) or pairs * self.heads < EXPAND_FROM_PAIRS:
+        pairs, all_keys = sum(host.lens[e] * (spans[e][1] - spans[e][0]) for e in chosen), sum(keys[e] for e in chosen)
+        if not chosen or pairs < EXPAND_FROM_TOKENS * all_keys or pairs * self.heads < EXPAND_FROM_PAIRS:
+            return nothing
+        rest, other, single = [], [], []                          # (first row, end, first tile, end, entries) of what is left out
+        for e in (e for e in range(host.n_entries) if e not in chosen):
+            a, b = int(host.cu_tokens[e]), int(host.cu_tokens[e + 1])
+            of = single if host.lens[e] == 1 else rest
+            if not of or of[-1][1] != a:
+                of.append([a, a, len(other), 0, []])
+            if of is rest:
+                other += prompt_tiles(host, [e], tile, rest[-1][0])
+            of[-1][1], of[-1][3] = b, len(other)
+            of[-1][4].append(e)
+        rest += [[a, b, 0, 0, entries] for a, b, _, _, entries in single]
+        price = FIRST_STRETCH * EXPAND_FROM_PAIRS * PAIR_US + STRETCH_US * (len(rest) - 1) if rest else 0.0
+        if _saved(pairs, all_keys, max(spans[e][1] - spans[e][0] for e in chosen), self.heads, context, tile) < price:
             return nothing
         pages = []
         table = np.full((host.n_entries, max(spans[e][3] for e in chosen)), -1, dtype=np.int32)
@@ -76,21 +109,8 @@ class LatentPages(StepPlanner):
             table[e, first:end] = np.arange(len(pages), len(pages) + end - first, dtype=np.int32)
             pages += [(e, b, lo, hi) for b in range(first, end)]
         tiles = prompt_tiles(host, chosen, tile)
-        rest, other = [], []                                      # (first row, end, first tile, end, entries) of what is left out
-        for e in (e for e in long if e not in chosen):
-            a, b = int(host.cu_tokens[e]), int(host.cu_tokens[e + 1])
-            if not rest or rest[-1][1] != a:
-                rest.append([a, b, len(other), 0, []])
-            other += prompt_tiles(host, [e], tile, rest[-1][0])
-            rest[-1][1], rest[-1][3] = b, len(other)
-            rest[-1][4].append(e)
-        single = [e for e, n in enumerate(host.lens) if n == 1]
-        if single:
-            a, b = int(host.cu_tokens[single[0]]), int(host.cu_tokens[single[-1] + 1])
-            rest.append([a, b, 0, 0, single])
         arrays = [np.asarray(x, dtype=np.int32).reshape(-1) for x in (pages, table, tiles, other)]
-        return arrays, dict(pages=len(pages), entries=host.n_entries, keys=len(pages) * ops.LATENT_PAGE_KEYS, tile=tile, rest=rest,
-                            scattered=bool(single) and b - a != len(single))
+        return arrays, dict(pages=len(pages), entries=host.n_entries, keys=len(pages) * ops.LATENT_PAGE_KEYS, tile=tile, rest=rest)
 
     def attach(self, ctx: StepContext, views: List[torch.Tensor], facts: dict) -> None:
         n = facts["pages"]
@@ -308,12 +328,11 @@ class LatentAttention(Part):
 
     def _pages_to_expand(self, ctx: StepContext, proj: torch.Tensor):
         """The step's pages where prompt portions of it attend over expanded keys and values, else None: bfloat16 layers of
-        widths the kernels take, portions long enough to pay for the expansion, the single tokens (which keep to the
-        shared rows) side by side in the batch."""
+        widths the kernels take, portions long enough to pay for the expansion (single tokens and the
+        rest keep to the shared rows)."""
         if self.w_ukv is None or ctx.act_dtype != torch.bfloat16 or proj.shape[1] % 8 or self.window_kind not in (WINDOW_NONE, WINDOW_SLIDING):
             return None
-        pages = ctx.extras.get(self.pages.key)
-        return None if pages is None or pages[4]["scattered"] else pages
+        return ctx.extras.get(self.pages.key)
 
     def _attend_expanded(self, q: torch.Tensor, pages, ctx: StepContext, cache: LayerCache, inv_freq: Optional[torch.Tensor],
                          magnitude: float) -> torch.Tensor:

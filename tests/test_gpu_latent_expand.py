@@ -127,12 +127,13 @@ def test_portions_left_out_of_the_expansion_keep_to_the_shared_rows(name, plain,
     write_random_model(load_config(cfg), d, 7, std=0.1, std_by_suffix={"embed": 1.0})
     reqs = {r: _tokens(300, 128, i) for i, r in enumerate("abcdef")}
     steps = [[("a", 9), ("b", 130), ("c", 5), ("d", 20)], [("e", 1), ("f", 1), ("a", 70), ("c", 100), ("b", 17), ("d", 140)],
-             [("b", 150), ("e", 2), ("c", 120), ("a", 30), ("f", 40)], [("a", 1), ("b", 1), ("c", 1), ("d", 60), ("e", 19)]]
+             [("b", 150), ("e", 2), ("c", 120), ("a", 30), ("f", 40)], [("a", 1), ("d", 60), ("b", 1), ("c", 1), ("e", 19)]]
     left_out = []
     real = L.LatentAttention._attend_shared
     monkeypatch.setattr(L.LatentAttention, "_attend_shared", lambda self, q, *a: left_out.append(q.shape[0]) or real(self, q, *a))
     monkeypatch.setattr(L, "_few_queries_lose", lambda n, *a: n < 40)
     monkeypatch.setattr(L, "EXPAND_FROM_PAIRS", 0)
+    monkeypatch.setattr(L, "STRETCH_US", 0.0)
 
     def run(least):
         monkeypatch.setattr(L, "EXPAND_FROM_TOKENS", least)
@@ -151,7 +152,7 @@ def test_portions_left_out_of_the_expansion_keep_to_the_shared_rows(name, plain,
 
     new = run(1)
     # three layers a step; what each step leaves over the shared rows, a stretch a call
-    assert left_out == [9, 25] * 3 + [17, 2] * 3 + [2, 30] * 3 + [19, 3] * 3
+    assert left_out == [9, 25] * 3 + [17, 2] * 3 + [2, 30] * 3 + [19, 1, 2] * 3
     shared = run(1 << 30)
     raw, w = plain.read_config(d), plain.load_weights(d, torch.float64)
     errs = []

@@ -196,14 +196,19 @@ def test_prompt_portions_expand_their_keys_where_it_is_the_faster_form():
     # a context whose expanded keys would not fit leaves the other prompts theirs
     assert _latent_pages([2000, 4000], [0, 60000])[0] == [0] and _latent_pages([2000, 4000], [0, 60000], heads=16)[0] == [0, 1]
     # too little work in all, portions that are too short
-    assert _latent_pages([80], [0], heads=16)[0] == [] and _latent_pages([80] * 6, [0] * 6, heads=16)[0] == list(range(6))
-    assert _latent_pages([31, 1, 1], [2000, 5, 6])[0] == [] and _latent_pages([40, 1, 1], [2000, 5, 6])[0] == [0]
+    assert _latent_pages([80], [0], heads=16)[0] == [] and _latent_pages([100] * 6, [0] * 6, heads=16)[0] == list(range(6))
+    assert _latent_pages([31, 1, 1], [2000, 5, 6])[0] == [] and _latent_pages([64, 1, 1], [2000, 5, 6])[0] == [0]
+    assert _latent_pages([40], [2000])[0] == [] and _latent_pages([40], [2000], heads=16)[0] == [0]
     assert _latent_pages([1] * 8, [2000] * 8)[0] == []
     # what is left out: neighbouring portions together, the single tokens apart
     far = 30000
-    chosen, _, _, tiles, other, facts = _latent_pages([1, 1, 5, 9, 700, 3, 600, 2, 4], [9, 9, far, far, 0, far, 64, far, far])
+    chosen, _, _, tiles, other, facts = _latent_pages([1, 1, 5, 9, 1000, 3, 900, 2, 4], [9, 9, far, far, 0, far, 64, far, far])
     assert chosen == [4, 6]
-    assert facts["rest"] == [[2, 16, 0, 2, [2, 3]], [716, 719, 2, 3, [5]], [1319, 1325, 3, 5, [7, 8]], [0, 2, 0, 0, [0, 1]]]
-    assert other == [[2, 0, 5], [3, 5, 9], [5, 0, 3], [7, 0, 2], [8, 2, 4]] and not facts["scattered"]
-    assert [t for t in tiles if t[0] == 6][0] == [6, 719, 64] and sum(t[2] for t in tiles) == 1300
-    assert _latent_pages([1, 700, 1], [9, 0, 9])[5]["scattered"]
+    assert facts["rest"] == [[2, 16, 0, 2, [2, 3]], [1016, 1019, 2, 3, [5]], [1919, 1925, 3, 5, [7, 8]], [0, 2, 0, 0, [0, 1]]]
+    assert other == [[2, 0, 5], [3, 5, 9], [5, 0, 3], [7, 0, 2], [8, 2, 4]]
+    assert [t for t in tiles if t[0] == 6][0][:2] == [6, 1019] and sum(t[2] for t in tiles) == 1900
+    # rows left to the shared form, a stretch each for neighbours: only where the prompts' work is enough for the launches
+    assert _latent_pages([1, 700, 1, 1], [9, 0, 9, 9])[5]["rest"] == [[0, 1, 0, 0, [0]], [701, 703, 0, 0, [2, 3]]]
+    for n, heads, behind, alone, beside, around in ((200, 64, 0, 1, 0, 0), (1000, 16, 0, 1, 1, 1), (400, 64, 0, 1, 1, 0), (100, 16, 2000, 1, 1, 1), (1500, 16, 0, 1, 1, 1)):
+        chosen = [_latent_pages(lens, [behind if n > 1 else 50 for n in lens], heads=heads)[0] for lens in ([n], [1] * 8 + [n], [1, n, 1])]
+        assert [len(c) for c in chosen] == [alone, beside, around], (n, heads, behind, chosen)
