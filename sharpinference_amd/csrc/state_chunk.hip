@@ -394,14 +394,16 @@ __device__ __forceinline__ void state_chunk_final_block(const WalkArgs& a) {
           sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, *reinterpret_cast<const bf16x8*>(&q[st * 8]), sc, 0, 0, 0);
         }
       } else {
+        f32x4 sums[4] = {sc, sc, sc, sc};              // four chains: half the rounding of one
 #pragma unroll
         for (int st = 0; st < EL / 4; ++st) {
           const int gh = st * 4 / RPL, r = st * 4 % RPL;
           const float4 kf = *reinterpret_cast<const float4*>(krow + (g + 4 * gh) * RPL + r);
           const float kv[4] = {kf.x, kf.y, kf.z, kf.w};
 #pragma unroll
-          for (int j = 0; j < 4; ++j) sc = mfma_f32(kv[j], q[st * 4 + j], sc);
+          for (int j = 0; j < 4; ++j) sums[j] = mfma_f32(kv[j], q[st * 4 + j], sums[j]);
         }
+        sc = (sums[0] + sums[1]) + (sums[2] + sums[3]);
       }
 #pragma unroll
       for (int v = 0; v < 4; ++v) {

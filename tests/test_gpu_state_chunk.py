@@ -57,7 +57,7 @@ def _recurrence(mode, q, k, v, gates, par, cap, freqs, k_scale):
                                                ("space", 2, 1, 64, 128), ("fixed", 2, 2, 128, 128), ("fixed", 2, 2, 64, 64)])
 def test_segments_as_matrix_products_are_as_exact_as_the_walk(dtype, mode, H, G, dk, dv):
     """Entries at the edges of segments (128 tokens) and of tiles (16), single tokens among them, from states that earlier
-    steps left: outputs and states against the recurrence in 64 bits, over all entries together no further off than 1.5
+    steps left: outputs and states against the recurrence in 64 bits, over all entries together no further off than 1.1
     times what the token-by-token walk of the same rows is.  (One entry's few rows say little by themselves: where n . q
     cancels, a row's error is that of its sums over a small remainder, whichever way they are ordered; an entry alone is
     held to 1e-5, a hundred roundings of its largest term.)"""
@@ -111,7 +111,7 @@ def test_segments_as_matrix_products_are_as_exact_as_the_walk(dtype, mode, H, G,
     for what, pairs in errors.items():
         e_chunk, e_walk = (float(np.sqrt(np.mean([p[j] ** 2 for p in pairs]))) for j in (0, 1))
         print(mode, dtype, what, f"chunks {e_chunk:.2e} walk {e_walk:.2e}")
-        assert e_chunk <= 1.5 * e_walk + 2.0 ** -24 and max(p[0] for p in pairs) < 1e-5, (what, pairs)
+        assert e_chunk <= 1.1 * e_walk and max(p[0] for p in pairs) < 1e-5, (what, pairs)
     if mode == "gates":                                            # every slice keeps a copy of the normaliser and the maximum
         tail = chunk_state[slots][:, :, :, dk * 8:dk * 8 + dk + 1]
         assert torch.equal(tail, tail[:, :, :1].expand_as(tail))
