@@ -64,7 +64,7 @@ def test_prompts_over_expanded_keys_are_as_exact_as_over_the_shared_rows(name, p
     """Portions of 33 to 200 tokens, alone, beside each other and beside decoding requests (side by side, and scattered, which
     keeps to the shared rows), first portions and later ones: every row of logits against the plain model in 64 bits, both
     ways.  The two round in different places, so a row may be further off one way; over all rows the expanded
-    form's error is held to 1.2 times the other's."""
+    form's error is held to 1.05 times the other's."""
     from sharpinference_amd import load_config
     from sharpinference_amd.engine import Engine, StepEntry
     from sharpinference_amd.parts import latent_attention as L
@@ -110,14 +110,14 @@ def test_prompts_over_expanded_keys_are_as_exact_as_over_the_shared_rows(name, p
         errs.append(torch.stack([(x[r] - want).norm(dim=-1) / want.norm(dim=-1) for x in (new, shared)]))
     e_new, e_shared = torch.cat(errs, dim=1).pow(2).mean(dim=1).sqrt().tolist()
     print(f"{name}: expanded {e_new:.3e} shared {e_shared:.3e}")
-    assert e_new <= 1.2 * e_shared and float(torch.cat(errs, dim=1)[0].max()) < 0.1
+    assert e_new <= 1.05 * e_shared and float(torch.cat(errs, dim=1)[0].max()) < 0.1
 
 
 @pytest.mark.parametrize("name, plain", [("rigodra", plain_rigodra), ("pagonex", plain_pagonex)])
 def test_portions_left_out_of_the_expansion_keep_to_the_shared_rows(name, plain, tmp_path, monkeypatch):
     """Portions of few tokens, as those that would lose by an expansion of a long context, before, between and behind
     portions that are expanded, beside each other, and beside decoding requests: every row of logits against the plain model
-    in 64 bits, held to what the shared rows alone give (1.2 times over all rows: the two round in different places)."""
+    in 64 bits, held to what the shared rows alone give (1.05 times over all rows: the two round in different places)."""
     from sharpinference_amd import load_config
     from sharpinference_amd.engine import Engine, StepEntry
     from sharpinference_amd.parts import latent_attention as L
@@ -162,7 +162,7 @@ def test_portions_left_out_of_the_expansion_keep_to_the_shared_rows(name, plain,
         errs.append(torch.stack([(x[r] - want).norm(dim=-1) / want.norm(dim=-1) for x in (new, shared)]))
     e_new, e_shared = torch.cat(errs, dim=1).pow(2).mean(dim=1).sqrt().tolist()
     print(f"{name}: some left out {e_new:.3e} shared {e_shared:.3e}")
-    assert e_new <= 1.2 * e_shared and float(torch.cat(errs, dim=1)[0].max()) < 0.1
+    assert e_new <= 1.05 * e_shared and float(torch.cat(errs, dim=1)[0].max()) < 0.1
 
 
 def test_only_layers_that_can_expand_have_the_pages_planned(tmp_path):
