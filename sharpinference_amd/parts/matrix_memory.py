@@ -65,7 +65,8 @@ class MatrixMemory(Part):
     What is kept per request is S, n and m in its state slot (``ops.walk_state_shape``): no pages.
     The gates' pre-activations are a product of their own with a float result; the gates, the
     maximum, the state, the normaliser and the norm are float whatever the activations are stored
-    as.  A step walks each entry's tokens in order from the slot's state (csrc/state_walk.hip)."""
+    as.  A step walks each entry's tokens in order from the slot's state (csrc/state_walk.hip); long entries go in
+    segments side by side where that is faster, as matrix products at 64 or 128 channels (csrc/state_chunk.hip)."""
 
     NAMES = {"q": "q", "k": "k", "v": "v", "g": "g", "o": "o", "norm": "norm", "i": "i", "i_bias": "i.b", "f": "f", "f_bias": "f.b"}
 
@@ -253,9 +254,10 @@ class Retention(Part):
     its root mean square (no weight), the heads side by side are multiplied by silu(W_g h) and projected by W_o.
 
     What is kept per request is S alone, in its state slot (``ops.walk_state_shape``): no pages.  The
-    rotation (on the staged floats, inside the walk), the state, its sums and the norm are float whatever
+    rotation (on the staged floats, inside the recurrence's kernels), the state, its sums and the norm are float whatever
     the activations are stored as.  A step walks each entry's tokens in order from the slot's state
-    (csrc/state_walk.hip), long entries in segments side by side."""
+    (csrc/state_walk.hip); long entries go in segments side by side where that is faster, as matrix products at 64 or
+    128 channels (csrc/state_chunk.hip)."""
 
     NAMES = {"q": "q", "k": "k", "v": "v", "g": "g", "o": "o"}
 
