@@ -1470,15 +1470,25 @@ def gla_segments(lens, cu_tokens):
     those of at least WALK_CHUNK_FROM tokens (see :func:`segment_counts`)."""
     import numpy as np
 
-    segs, ents = [], [(0, 0)] * len(lens)
-    rank = [0 if n > GLA_SEGMENT_TOKENS else 1 if n >= WALK_CHUNK_FROM else 2 for n in lens]
-    for e in sorted(range(len(lens)), key=rank.__getitem__):
+    segs, ents = [], np.zeros((len(lens), 2), dtype=np.int32)
+    long = [e for e, n in enumerate(lens) if n >= WALK_CHUNK_FROM]
+    for e in sorted(long, key=lambda e: lens[e] <= GLA_SEGMENT_TOKENS):
         n, first = lens[e], len(segs)
         for o in range(0, n, GLA_SEGMENT_TOKENS):
             m = min(GLA_SEGMENT_TOKENS, n - o)
             segs.append((e, int(cu_tokens[e]) + o, m, 1 if o + m == n else 0))
-        ents[e] = (first, len(segs) - first)
-    return np.asarray(segs, dtype=np.int32).reshape(-1, 4), np.asarray(ents, dtype=np.int32).reshape(-1, 2)
+        ents[e] = first, len(segs) - first
+    segs = np.asarray(segs, dtype=np.int32).reshape(-1, 4)
+    short = [e for e, n in enumerate(lens) if 0 < n < WALK_CHUNK_FROM]
+    if short:                                              # (256 single tokens one by one took 250 us of the step's start)
+        tail = np.ones((len(short), 4), dtype=np.int32)
+        tail[:, 0] = at = np.asarray(short)
+        tail[:, 1] = np.asarray(cu_tokens)[at]
+        tail[:, 2] = np.asarray(lens)[at]
+        ents[at, 0] = np.arange(segs.shape[0], segs.shape[0] + len(short))
+        ents[at, 1] = 1
+        segs = np.concatenate([segs, tail])
+    return segs, ents
 
 
 def segment_counts(lens) -> Tuple[int, int]:

@@ -11,8 +11,8 @@ from ..cache.spec import StateSpec
 from ..ops.profile import section
 from .base import INIT_NORM_WEIGHT, HostStep, LayerCache, ParamSpec, Part, StepContext, StepPlanner, TensorSource
 
-CHUNK_FROM_TOKENS = 64        # a step whose longest entry has this many tokens gets the segments' work lists; layers that run
-                              # segments as matrix products take them
+CHUNK_FROM_TOKENS = 64        # a step whose longest entry has this many tokens gets the segments' work lists of layers that
+                              # may run segments as matrix products
 SEGMENT_FROM_TOKENS = 512     # ... layers that walk segments token by token take them from this many tokens on,
 SEGMENT_UP_TO_BLOCKS = 2048   # ... while whole entries would give fewer blocks than this
 
@@ -36,13 +36,14 @@ class EntrySpans(NamedTuple):
 
 
 class WalkSegments(StepPlanner):
-    """The work lists of the segmented walk, made once a step for all layers that walk a state: none
-    unless some entry is long (decode steps and short portions are walked whole)."""
+    """The work lists of the segmented walk, made once a step for all layers that walk a state this way: none
+    unless some entry has ``from_tokens`` tokens (decode steps and short portions are walked whole)."""
 
-    key = "linear attention"
+    def __init__(self, key: str, from_tokens: int):
+        self.key, self.from_tokens = key, int(from_tokens)
 
     def plan(self, host: HostStep) -> Tuple[List[np.ndarray], dict]:
-        if not host.lens or max(host.lens) < CHUNK_FROM_TOKENS:
+        if not host.lens or max(host.lens) < self.from_tokens:
             empty = np.zeros(0, dtype=np.int32)
             return [empty, empty], dict(n_segs=0)
         segs, ents = ops.gla_segments(host.lens, host.cu_tokens)
@@ -52,16 +53,16 @@ class WalkSegments(StepPlanner):
         ctx.extras[self.key] = (views[0], views[1], facts["counts"], facts["spans"]) if facts["n_segs"] else None
 
 
-_SEGMENTS = WalkSegments()
-WALK_SEGMENTS = _SEGMENTS         # every mixer that walks a state token by token shares the step's one list
+_SEGMENTS = WalkSegments("linear attention", SEGMENT_FROM_TOKENS)
+WALK_SEGMENTS = WalkSegments("state walk", CHUNK_FROM_TOKENS)     # the mixers with one decay a head share the step's one list
 
 
-def segments_for(ctx: StepContext, nh: int, dv: int, cols: int):
+def segments_for(ctx: StepContext, planner: WalkSegments, nh: int, dv: int, cols: int):
     """The step's segment lists for a layer that walks token by token (blocks of `cols` value columns), where whole
     entries would leave the chip idle: a long entry nearly alone in its step.  Else None."""
     whole_blocks = ctx.n_entries * nh * ((dv + cols - 1) // cols)
     wanted = ctx.max_entry_len >= SEGMENT_FROM_TOKENS and whole_blocks < SEGMENT_UP_TO_BLOCKS
-    return ctx.extras.get(WALK_SEGMENTS.key) if wanted else None
+    return ctx.extras.get(planner.key) if wanted else None
 
 
 class GatedLinearAttention(Part):
@@ -161,7 +162,7 @@ class GatedLinearAttention(Part):
         with section("recurrence", nbytes=lambda: 8 * ctx.n_entries * qk * self.dv + T * (width * (2 * qk + vv) + 4 * (qk + vv)),
                      flops=4.0 * T * qk * self.dv):
             # a long entry alone in its step: walked in segments side by side (twice the sums on many times the blocks)
-            segments = segments_for(ctx, self.nh, self.dv, ops.GLA_STATE_COLS)
+            segments = segments_for(ctx, _SEGMENTS, self.nh, self.dv, ops.GLA_STATE_COLS)
             o = ops.gla_walk(proj, 0, qk, 2 * qk, alpha, self.dk ** -0.5, state, ctx, self.nh, self.dk, self.dv, segments=segments)
         with section("head norm + gate", nbytes=T * vv * (4 + 2 * width)):
             y = ops.head_norm_gate(o, self.w_norm, self.eps, self.nh, self.dv, ctx.act_dtype,

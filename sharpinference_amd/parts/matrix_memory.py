@@ -39,7 +39,7 @@ def _segments_for(ctx: StepContext, nh: int, dk: int, dv: int, turned: bool = Fa
     beside 0 to 256 single ones): the choice is within 6 % of the faster form in all but 10 of the 330, and in those it is the
     walk.  Other sizes: the rule of the walks."""
     if not ops.walk_takes_chunks(dk, dv):
-        return segments_for(ctx, nh, dv, ops.WALK_STATE_COLS)
+        return segments_for(ctx, WALK_SEGMENTS, nh, dv, ops.WALK_STATE_COLS)
     segments = ctx.extras.get(WALK_SEGMENTS.key)
     if segments is None:
         return None

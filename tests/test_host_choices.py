@@ -162,10 +162,29 @@ def test_segments_are_cut_to_what_the_kernels_hold():
         mine = segs[first:first + count]
         assert (mine[:, 0] == e).all() and mine[:, 3].tolist() == [0] * (count - 1) + [1]
         assert mine[:, 1].tolist() == [cu[e] + 128 * i for i in range(count)] and mine[:, 2].sum() == lens[e]
+    assert [segs[first, 0] for first, _ in ents] == list(range(len(lens)))                # (every entry's own, whatever the order)
     several, long = ops.segment_counts(lens)
     single = ents[segs[:, 0], 1] == 1
     assert (several, long) == (3 + 2 + 8, 3 + 2 + 8 + 2) and not single[:several].any() and single[several:].all()
     assert (segs[several:long, 2] >= ops.WALK_CHUNK_FROM).all() and (segs[long:, 2] < ops.WALK_CHUNK_FROM).all()
+
+
+def test_segments_are_listed_for_the_layers_that_may_take_them():
+    """Layers with a decay per key channel, which walk their segments, have lists from 512 tokens on; layers with one decay a head,
+    whose segments are products, from 64."""
+    import numpy as np
+
+    from sharpinference_amd.parts.base import HostStep
+    from sharpinference_amd.parts.linear_attention import GatedLinearAttention
+    from sharpinference_amd.parts.matrix_memory import MatrixMemory
+
+    parts = GatedLinearAttention.__new__(GatedLinearAttention), MatrixMemory.__new__(MatrixMemory)
+    for n, made in ((63, [0, 0]), (64, [0, 1]), (511, [0, 1]), (512, [1, 1])):
+        lens = [1, n, 5]
+        cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+        host = HostStep(3, int(cu[-1]), lens, [0] * 3, cu)
+        assert [int(p.step_planners()[0].plan(host)[1]["n_segs"] > 0) for p in parts] == made
+    assert parts[0].step_planners()[0].key != parts[1].step_planners()[0].key
 
 
 def _latent_pages(lens, starts, kind=0, window=0, heads=64, width=320):
