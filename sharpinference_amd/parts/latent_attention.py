@@ -89,8 +89,9 @@ class LatentPages(StepPlanner):
         if not chosen or pairs < EXPAND_FROM_TOKENS * all_keys or pairs * self.heads < EXPAND_FROM_PAIRS:
             return nothing
         rest, other, single = [], [], []                          # (first row, end, first tile, end, entries) of what is left out
-        for e in (e for e in range(host.n_entries) if e not in chosen):
-            a, b = int(host.cu_tokens[e]), int(host.cu_tokens[e + 1])
+        rows, expanded = host.cu_tokens.tolist(), set(chosen)
+        for e in (e for e in range(host.n_entries) if e not in expanded):
+            a, b = rows[e], rows[e + 1]
             of = single if host.lens[e] == 1 else rest
             if not of or of[-1][1] != a:
                 of.append([a, a, len(other), 0, []])
