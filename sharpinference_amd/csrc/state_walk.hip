@@ -435,7 +435,7 @@ static int state_walk_any(const WalkArgs& a, int dtype, int mode, hipStream_t st
     return SHARPI_ERR_ARG;
   }
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
-  if (a.segs && (!a.ent_segs || !a.seg_local || !a.seg_start || !a.seg_decay || a.n_segs < a.n_entries || a.n_segs > 65535 || a.n_scratch < 0 || a.n_scratch > a.n_segs || a.n_long > a.n_segs ||
+  if (a.segs && (!a.ent_segs || (a.n_scratch > 0 && (!a.seg_local || !a.seg_start || !a.seg_decay)) || a.n_segs < a.n_entries || a.n_segs > 65535 || a.n_scratch < 0 || a.n_scratch > a.n_segs || a.n_long > a.n_segs ||
                  (a.n_long >= 0 && a.n_long < a.n_scratch))) return SHARPI_ERR_ARG;
   if (mode == WALK_EXP_GATES) {
     if (dtype == DT_F32) return launch_state_walk<float, WALK_EXP_GATES>(a, stream);

@@ -1848,14 +1848,16 @@ def state_walk(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, heads_per
         n_scratch, n_long = segments[2] if len(segments) > 2 else (n_segs, -1)         # (-1: not known)
         _need(0 <= n_scratch <= n_segs and n_long <= n_segs and (n_long == -1 or n_long >= n_scratch),
               "state_walk: (segments of several, long segments) of all segments wanted")
-        shape = (max(1, n_scratch),) + walk_state_shape(nh, dk, dv, mode)
-        seg_local = torch.empty(shape, dtype=torch.float32, device=proj.device)
-        seg_start = torch.empty(shape, dtype=torch.float32, device=proj.device)
-        seg_decay = torch.empty(max(1, n_scratch), nh, dtype=torch.float32, device=proj.device)
+        local = start = decay = None
+        if n_scratch:                                      # two states a segment and its heads' decays, in one piece
+            states = n_scratch * state.shape[1:].numel()
+            scratch = torch.empty(2 * states + n_scratch * nh, dtype=torch.float32, device=proj.device)
+            local = scratch.data_ptr()
+            start, decay = local + 4 * states, local + 8 * states
         _run("sharpi_state_walk_segmented", _ptr(proj), _code(proj.dtype), N, int(q_off), int(k_off), int(v_off),
              int(heads_per_group), _ptr(gates), g_stride, _ptr(p[0]), _ptr(p[1]), _ptr(p[2]), float(cap), float(q_scale),
              int(mode), _ptr(state), _ptr(ctx.state_slots), _ptr(ctx.cu_tokens), _ptr(out), ctx.n_entries, nh, dk, dv,
-             _ptr(segs), _ptr(ent_segs), n_segs, int(n_scratch), int(n_long), _ptr(seg_local), _ptr(seg_start), _ptr(seg_decay), *rot, _stream())
+             _ptr(segs), _ptr(ent_segs), n_segs, int(n_scratch), int(n_long), local, start, decay, *rot, _stream())
         return out
     _run("sharpi_state_walk", _ptr(proj), _code(proj.dtype), N, int(q_off), int(k_off), int(v_off), int(heads_per_group),
          _ptr(gates), g_stride, _ptr(p[0]), _ptr(p[1]), _ptr(p[2]), float(cap), float(q_scale), int(mode), _ptr(state),

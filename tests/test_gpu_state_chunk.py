@@ -221,11 +221,11 @@ def test_scratch_is_for_entries_of_several_segments_alone():
     out = ops.state_walk(rows, 0, H * dk, 2 * H * dk, 1, None, par, 8.0, dk ** -0.5, code, state, ctx, H, dk, dv, segments=segments,
                          inv_freq=freqs, k_scale=k_scale)
     one = state[0].numel() * 4
-    assert torch.cuda.max_memory_allocated() - before <= out.numel() * 4 + 2 * 3 * one + 65536
+    # (the allocator leaves up to a MiB behind a large tensor in its block; a place for every segment would be 106 MB)
+    assert torch.cuda.max_memory_allocated() - before <= out.numel() * 4 + 2 * 3 * one + (1 << 20)
     want, walked = _walk("fixed", lens, rows, None, modes, H, dk, dv, False)
     assert float((out.view_as(want) - want).abs().max()) <= 2e-6 * float(want.abs().max())
     assert float((state - walked).abs().max()) <= 2e-6 * float(walked.abs().max())
-
 
 
 @pytest.mark.parametrize("pad, lens", [(0, [20]), (0, [100]), (0, [300]), (0, [128, 31]), (3, [300, 20, 1])])
