@@ -38,11 +38,11 @@
 #include <type_traits>
 
 #include "common.h"
+#include "lds_loads.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
 #ifndef SHARPI_PREFILL_P_PAIR
 // 1: probabilities enter the second product as a bfloat16 pair hi + lo.  0 (hi alone) is faster, but then
@@ -88,22 +88,11 @@ struct PrefillArgs {
   int gate_stride;
 };
 
-// One load of 16 bytes a lane from `base` + the lane's offset into 64 consecutive 16-byte pieces of LDS from byte `lds` on
-// (the instruction takes the LDS address from m0).  Lanes whose offset lies at or beyond `bytes` read zeros.  Nothing
-// but lds_loads_wait waits for it.
-__device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t offset, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(offset), "s"(rsrc) : "memory");
-}
-__device__ __forceinline__ u32x4 buffer_of(const void* base, uint32_t bytes) {
-  const uint64_t a = (uint64_t)base;
-  return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, bytes, 0x00020000u};
-}
 __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
   typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
   const bf16x2 p = {(__bf16)lo, (__bf16)hi};
   return __builtin_bit_cast(uint32_t, p);
 }
-__device__ __forceinline__ void lds_loads_wait() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 template <int HD, int VD>
 constexpr int prefill_waves_a_simd() { return kPreWaves * 16 * (HD + (VD + 31) / 32 * 32) * 4 <= 80 * 1024 ? 2 : 1; }   // by the LDS two blocks need
@@ -212,7 +201,7 @@ __global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) voi
     const int d = n * 32 + (lane >> 1);
     v_off[n] = (uint32_t)(min(d, VD - 1) * page_size + ((lane & 1) ^ v_swizzle(d)) * 8) * 2;
   }
-  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)smem;
+  const uint32_t lds0 = lds_address(smem);
   auto fetch = [&](int bb, int page_raw, int buf) {   // 16-key block bb, of the page that page_at gave
     const int page = min(max(__builtin_amdgcn_readfirstlane(page_raw), 0), num_pages - 1);   // a table that is wrong reads a wrong page, never outside
     const int off = min(max((bb - page_slot(bb) * per_page) << 4, 0), page_size - 16);
@@ -221,9 +210,9 @@ __global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) voi
     const u32x4 vr = buffer_of(v_cache + head * VD * page_size + off, (uint32_t)((VD - 1) * page_size + 16) * 2);
     const uint32_t at = lds0 + buf * STAGE;
 #pragma unroll
-    for (int n = 0; n < KL; ++n) load_to_lds(kr, k_off[n], __builtin_amdgcn_readfirstlane(at + w * KB + n * 1024));
+    for (int n = 0; n < KL; ++n) load_to_lds(kr, k_off[n], 0, at + w * KB + n * 1024);
 #pragma unroll
-    for (int n = 0; n < ND; ++n) load_to_lds(vr, v_off[n], __builtin_amdgcn_readfirstlane(at + WAVES * KB + w * VB + n * 1024));
+    for (int n = 0; n < ND; ++n) load_to_lds(vr, v_off[n], 0, at + WAVES * KB + w * VB + n * 1024);
   };
 
   // where this lane reads its operands (bytes): piece 2j + g of key row r, half g of value column r

@@ -2,29 +2,27 @@
 //   out[row, :] = x[a_rows[row], :] * W[e]^T   for the rows of expert e in the expert-sorted list,
 // bfloat16 inputs, float accumulation on the matrix cores.
 //
-// The product is bound by reading the experts' weights while few rows share them, and by the
-// matrix cores' operand traffic once many do.  A block takes up to 128 rows of its expert against
-// 512 weight rows: an expert's weights are then read once for every 128 of its rows.  An expert
-// with more rows is cut into sibling tiles of equal height, and the blocks that multiply the SAME
-// weight rows by sibling tiles start side by side on one XCD, so that the weights cross the memory
-// interface about once all the same (grouped_plan.h says how the routing kernel lays that out;
-// the host never learns the routing).  The tile's work is compiled for every height in steps of
-// 32 rows up to 128, and a block takes the smallest that holds its rows: no branch inside a K
-// stage, nothing multiplied for 32-row pieces that hold no row (rows are staged in passes of 64).
+// The product is bound by reading the experts' weights while few rows share them, and by what a
+// compute unit can fetch and multiply once many do.  A block takes up to 256 rows of its expert against
+// 256 weight rows: an expert's weights are then read once for every 256 of its rows, and a unit fetches
+// 64 KB for 256 x 256 x 64 products (128 rows against 512 weight rows: 80 KB, and an expert of 129 to 256
+// rows pulled its weights through two units).  An expert with more rows is cut into sibling tiles of equal height, and the
+// blocks that multiply the SAME weight rows by sibling tiles start side by side on one XCD, so that the
+// weights cross the memory interface about once all the same (grouped_plan.h says how the routing kernel
+// lays that out; the host never learns the routing).  The tile's work is compiled for every height in
+// steps of 32 rows, and a block takes the one that holds its rows.
 //  * The blocks are persistent: as many as there are compute units (each holds one), every block
 //    taking the next slot of its XCD's walk from a ticket counter until none is left, then slots
 //    of other XCDs.  Experts of very different loads, whose tiles take very different times, are
 //    so levelled at run time; with blocks dealt out beforehand an XCD that drew a block more than
 //    its units can hold at once ran a second round alone.  The caller may bound the number of
 //    blocks, to leave compute units to other work that runs beside the product.
-//  * Each of the 8 waves owns 64 weight rows (4 MFMA tiles) and reads them straight from global
-//    memory into registers, a ring of 64-wide K stages ahead: a weight element is used by one wave
-//    only.  An x fragment read from LDS feeds four products (with two tiles a wave and 192-row
-//    blocks the LDS reads, one per two products, kept pace with the matrix cores and bounded them
-//    at 0.92 PFLOP/s at 8,192 tokens; four tiles reach 1.09).
-//  * The x rows (gathered through a_rows) are shared by the waves and staged through LDS, 64
-//    columns of K at a time, double-buffered and fetched two stages ahead; the 16-byte chunks of
-//    a row are swizzled so that reads and stores are free of bank conflicts.
+//  * The 8 waves stand 2 (halves of the rows) x 4 (64 weight rows each); both operands go from memory
+//    straight into LDS (loads that write LDS: no registers, so the ring is as deep as the LDS allows):
+//    weights 32 of K a step, three steps ahead, in the order the packed matrix has them (1 KB a 16-row
+//    tile and step, read back without conflicts); x rows (gathered through a_rows) 64 of K at a time, whole
+//    128-byte lines, a stage ahead, their 16-byte pieces XORed with row bits (xs_piece).  One barrier a step; a wave
+//    waits for its own loads of the step by count and the barrier makes them everyone's.
 //  * W is the A operand (rows = n), x the B operand: a lane ends up with 4 consecutive n of one
 //    row, stored as one 8-byte write.  Each output is one chain over k in ascending order, so a
 //    row's result does not depend on which other rows share its tile, nor on which block took it.
@@ -35,210 +33,212 @@
 //    rows never go to memory.
 //  * The plain form may square the relu of its results (relu2: feed-forwards without a gate), rounded to
 //    bfloat16 first (what a separate activation kernel would have read).
+// Measured, 16 experts, up (2 x 8,192 rows of 5,120) + down, us, beside tiles of 128 x 512 whose weights went straight to
+// registers: 8,192 tokens 1,346 + 666 (1,420 + 700), 2,048 tokens of uneven load 570 + 271 (587 + 264), 1,190 tokens 470 + 237
+// (488 + 250); 64 experts of 1,408 x 2,048, six picks, 3,000 tokens 292 + 144 (327 + 157), 1,664 tokens 187 + 106 (235 + 110).
+// Parts taken out, 4,096 tokens even (up, 656 us): no loads 465 (1.48 PFLOP/s), no products 538, weights and products without x rows
+// 615: the weights' 2.7 GB and the products each need about 460, and neither hides the other whole.
 // Limits: K % 64 == 0, N % 4 == 0 (N % 32 == 0 in the SwiGLU form).
 #pragma once
 #include <type_traits>
 
 #include "common.h"
 #include "grouped_plan.h"
+#include "lds_loads.h"
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
-#ifndef SHARPI_GAHEAD
-#define SHARPI_GAHEAD 2
-#endif
-#ifndef SHARPI_GQ
-#define SHARPI_GQ 4
-#endif
-#ifndef SHARPI_GK
-#define SHARPI_GK 64
-#endif
-constexpr int GM = kPlanTileRows;  // rows per tile
-static_assert(GM == kPlanTileRows, "the routing kernel's plan is made for tiles of this height");
-constexpr int GMT = GM / 16;  // 16-row groups per tile
-#ifndef SHARPI_GW
-#define SHARPI_GW 8
-#endif
-#ifndef SHARPI_GNT
-#define SHARPI_GNT 4
-#endif
-constexpr int GW = SHARPI_GW;   // waves per block
-constexpr int kMaxNT = SHARPI_GNT;  // 16-row weight tiles per wave: this many, or a half or a quarter where a slot is cut
-constexpr int columns_of(int nt) { return 16 * nt * GW; }   // weight rows (output columns) of a block
-constexpr int GK = SHARPI_GK;  // K per LDS stage
-constexpr int GPAD = GK;      // LDS row: no pad, the 16-byte chunks of a row are swizzled instead (xs_col)
-constexpr int GROWS = GW * 64 / (GK / 8);   // rows staged per pass: GK / 8 threads per row
-constexpr int GPASS = GM / GROWS;  // staging passes
-constexpr int kXcds = kPlanXcds;   // accelerator dies, each with its own L2
-constexpr int kAhead = SHARPI_GAHEAD;  // K stages of weights in flight per wave (2, 3 or 4)
-constexpr int GQ = SHARPI_GQ;       // 16-row groups whose LDS reads go out together (divides 4)
+constexpr int GM = kPlanTileRows;      // rows per tile
+constexpr int GW = 8;                  // waves per block
+constexpr int GWC = 4;                 // of them side by side along the columns, the others along the rows
+constexpr int kMaxNT = 4;              // 16-row weight tiles per wave: this many, or half where a slot is cut
+constexpr int columns_of(int nt) { return 16 * nt * GWC; }   // weight rows (output columns) of a block
+constexpr int GK = 64;                 // K of a stage of x rows: two steps of 32
+constexpr int kXcds = kPlanXcds;       // accelerator dies, each with its own L2
+// LDS: four steps of weights (16 tiles of 16 rows x 32 of K), then two stages of x rows (GM x 64 of K), then the groups' first rows.
+// (Deeper rings where a tile is low, up to 8 steps and 3 stages, gained nothing: 3.9 to 6.4 TB/s of weights as before.)
+constexpr int kWStep = 16 * 1024, kXStage = GM * GK * 2, kXAt = 4 * kWStep, kGroupedLds = kXAt + 2 * kXStage;
+constexpr int kOffsetsKept = 1025;     // of more groups the rows are read from memory
+static_assert(2 * kWStep == kXStage, "both rings turn by the same exclusive or");
+static_assert(GM == 2 * 16 * 8, "tile heights are compiled in steps of 32 rows up to 256");
 
-// Where column `col` (a multiple of 8 elements = one 16-byte chunk) of LDS row `row` is kept: the
-// chunk index is XORed with bits 1..3 of the row.  The LDS serves a 16-byte read of a wave in four
-// turns of two octets of lanes, one octet from rows 0..7 and one from rows 8..15 of the operand
-// (measured with the bank-conflict counter: rows padded to 144 bytes conflict two ways).  With the
-// swizzle the eight chunks an octet reads fall into eight different 16-byte bank groups of its half
-// (even rows use one half of the 256-byte bank space, odd rows the other), and the two octets of a
-// turn into different ones; an octet of the staging stores fills one whole row, i.e. one half.
-static_assert(GK == 64, "the swizzle assumes rows of eight 16-byte chunks");
-__device__ __forceinline__ int xs_col(int row, int col) { return col ^ (((row >> 1) & 7) << 3); }
+// Where 16-byte piece `piece` of x row `row` of a stage is kept.  The LDS serves a 16-byte read of a wave in four
+// turns of two octets of lanes, one from operand rows 0..7 and one from rows 8..15 (measured with the bank-conflict
+// counter); with the exclusive or the sixteen pieces of a turn fall into the sixteen different 16-byte groups of the bank space.
+__device__ __forceinline__ int xs_piece(int row, int piece) { return piece ^ ((row >> 1) & 7); }
 
-// A weight fragment.  STREAM: with the streaming hint (nontemporal), for a group whose weights no
-// other row tile reads: a pure read in this kernel's pattern reaches 6.9 TB/s with the hint and
-// 6.2 without.  A group cut into sibling tiles reads them without the hint: what the first
-// sibling fetches the others are to find in the L2.
-template <bool STREAM> __device__ __forceinline__ bf16x8 load_weights(const bf16_t* p) {
-  if constexpr (STREAM) return __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(p));
-  else return *reinterpret_cast<const bf16x8*>(p);
-}
-
-// The work of one tile of MT * 16 rows (the block's rows, rounded up) against 16 * NT * GW weight rows.
-template <typename TO, int MT, int NT, bool PACKED, bool ACT, bool STREAM>
-__device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, const bf16_t* __restrict__ We,
+// The work of one tile of up to MT * 32 rows against 16 * NT * GWC weight rows.
+template <typename TO, int MT, int NT, bool PACKED, bool ACT>
+__device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint32_t x_bytes, const bf16_t* __restrict__ We,
                                              TO* __restrict__ out, int N, int K, const int* __restrict__ a_rows,
-                                             const float* __restrict__ act_scale, GatedAct act, int relu2, int row0, int row_end,
-                                             int n_base, bf16_t (*xs)[GM][GPAD]) {
+                                             const float* __restrict__ act_scale, GatedAct act, int relu2, int tile_row0, int row_end,
+                                             int col_base, bool stream, const char* smem, int* counter, int& next) {
   static_assert(!ACT || NT % 2 == 0, "the SwiGLU form pairs gate tiles with up tiles");
   constexpr int HT = ACT ? NT / 2 : NT;         // tiles of distinct output columns per wave
   const int n_out = ACT ? N / 2 : N;            // output columns
-  constexpr int PASS = (MT * 16 + GROWS - 1) / GROWS;   // staging passes
-  constexpr int Q = MT % GQ == 0 ? GQ : 2;      // 16-row groups whose LDS reads go out together
-  static_assert(MT % Q == 0, "tile heights come in steps of 32 rows");
+  constexpr int TILES = NT * GWC;               // weight tiles of the block
+  constexpr int WL = (TILES + GW - 1) / GW;     // loads of weights a wave and step
+  constexpr int XL = (4 * MT + GW - 1) / GW;    // loads of x rows a wave and stage (8 rows each)
   const int lane = threadIdx.x & (kWave - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
+  const int wr = wid / GWC, wc = wid % GWC;
 
-  // 32-bit element offsets from uniform bases (the host checks that they fit): half the address registers
-  // Row layout: lane (r, g) reads 16 bytes of row n at k = c*GK + j*32 + g*8.  Packed layout (the
-  // matrix stored as [N/16][K/128][16 runs of 8 k][16 rows][8]): the same element sits at
-  // tile*16*K + c*GK*16 + j*512 + lane*8, and a wave's load is one contiguous 1 KB.
-  constexpr uint32_t kStageStep = PACKED ? GK * 16 : GK;
-  constexpr uint32_t kSubStep = PACKED ? 512 : 32;
-  static_assert(128 % GK == 0, "a K stage must not straddle a packed 128-wide unit");
-  uint32_t woff[NT];
+  // Weights: tile lt of the block is tile lt % NT of column wave lt / NT.  A tile that lies beyond the last column (or its rows that do)
+  // is read as the last that exists, never stored.
+  // Packed layout (the matrix stored as [N/16][K/128][16 runs of 8 k][16 rows][8]): a step of a tile is 1 KB in a row.
+  // Row layout: lane (row l % 16, run l / 16) reads 16 bytes of its row; in LDS both lie as [run][row].
+  constexpr uint32_t kWStepBytes = PACKED ? 1024 : 64;
+  uint32_t w_off[WL];
+  int w_tile[WL];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    // ACT: tile 0 is the gate tile of the wave's 16 columns, tile 1 the up tile of the same columns
+  for (int i = 0; i < WL; ++i) {
+    const int lt = (wid * WL + i) % TILES;      // (fewer tiles than waves: fetched twice, to the same place)
+    const int t = lt % NT;
+    int n = col_base + (lt / NT) * HT * 16 + (t % HT) * 16;
+    w_tile[i] = lt;
     if constexpr (PACKED) {
-      int n = n_base + (t % HT) * 16;
-      if (n >= n_out) n = n_out - 16;  // loaded, never stored
+      if (n >= n_out) n = n_out - 16;
       if (ACT && t >= HT) n += n_out;
-      woff[t] = (uint32_t)n * (uint32_t)K + lane * 8;
+      w_off[i] = (uint32_t)n * (uint32_t)K * 2 + lane * 16;
     } else {
-      int n = n_base + (t % HT) * 16 + r;
-      if (n >= n_out) n = n_out - 1;  // loaded, never stored
+      n += lane & 15;
+      if (n >= n_out) n = n_out - 1;
       if (ACT && t >= HT) n += n_out;
-      woff[t] = (uint32_t)n * (uint32_t)K + g * 8;
+      w_off[i] = (uint32_t)n * (uint32_t)K * 2 + (lane >> 4) * 16;
     }
   }
-  // staging role: thread loads 16 bytes of row (tid / 8 + GROWS * pass), columns (tid % 8) * 8
-  const int srow = threadIdx.x / (GK / 8), scol = (threadIdx.x % (GK / 8)) * 8;
-  uint32_t xoff[PASS];
-#pragma unroll
-  for (int ps = 0; ps < PASS; ++ps) {
-    // rows beyond the expert's last read its last row again: every load is unconditional, and what
-    // such rows produce is never stored
-    const int row = min(row0 + srow + GROWS * ps, row_end - 1);
-    xoff[ps] = (uint32_t)(a_rows ? a_rows[row] : row) * (uint32_t)K + scol;
-  }
-
   f32x4 acc[NT][MT];
 #pragma unroll
   for (int t = 0; t < NT; ++t)
 #pragma unroll
     for (int mb = 0; mb < MT; ++mb) acc[t][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  const int chunks = K / GK;
-  // The memory counter retires loads in order, so waiting for one load waits for every load issued
-  // before it.  Both streams therefore run the same distance ahead: x rows of stage c + 2 go into
-  // one of two register sets while stage c is multiplied (and into LDS one stage later), weights
-  // of stage c + kAhead into the ring slot that stage c has just used up.
-  u32x4 stage[2][PASS];
-  bf16x8 wf[kAhead][GK / 32][NT];   // weight fragments of the next kAhead stages, a ring indexed by stage % kAhead
+  const u32x4 wb = buffer_of(We, (uint32_t)N * (uint32_t)K * 2), xb = buffer_of(x, x_bytes);
+  const uint32_t lds0 = lds_address(smem);
+  const int steps = K / 32, stages = K / GK;
+  auto load_w = [&](int s) {                    // weights of step s into the ring
 #pragma unroll
-  for (int ps = 0; ps < PASS; ++ps) stage[0][ps] = *reinterpret_cast<const u32x4*>(x + xoff[ps]);
-  if (chunks > 1) {
-#pragma unroll
-    for (int ps = 0; ps < PASS; ++ps) stage[1][ps] = *reinterpret_cast<const u32x4*>(x + xoff[ps] + GK);
-  }
-  auto fill_ring = [&](auto all_tag) {
-#pragma unroll
-    for (int a = 0; a < kAhead; ++a)
-      if (decltype(all_tag)::value || a < chunks) {
-#pragma unroll
-        for (int j = 0; j < GK / 32; ++j)
-#pragma unroll
-          for (int t = 0; t < NT; ++t) wf[a][j][t] = load_weights<STREAM>(We + woff[t] + a * kStageStep + j * kSubStep);
-      }
+    for (int i = 0; i < WL; ++i) {
+      const uint32_t at = lds0 + (s & 3) * kWStep + w_tile[i] * 1024;
+      if (stream) load_to_lds<true>(wb, w_off[i], s * kWStepBytes, at);
+      else load_to_lds<false>(wb, w_off[i], s * kWStepBytes, at);
+    }
   };
-  if (chunks >= kAhead) fill_ring(std::true_type{}); else fill_ring(std::false_type{});
+  load_w(0);                                    // (on their way while the rows' places are looked up)
+  load_w(1);
+  if (steps > 2) load_w(2);
+  // x rows: a load brings 8 rows of 128 bytes, lane l row l / 8 at place l % 8.  Rows beyond the expert's last read its last row again
+  // (what such rows produce is never stored).
+  uint32_t x_off[XL];
+  int x_load[XL];
 #pragma unroll
-  for (int ps = 0; ps < PASS; ++ps) *reinterpret_cast<u32x4*>(&xs[0][srow + GROWS * ps][xs_col(srow + GROWS * ps, scol)]) = stage[0][ps];
-  __syncthreads();
+  for (int i = 0; i < XL; ++i) {
+    const int li = min(wid * XL + i, 4 * MT - 1);
+    const int lrow = li * 8 + (lane >> 3);
+    const int row = min(tile_row0 + lrow, row_end - 1);
+    x_load[i] = li;
+    x_off[i] = (uint32_t)(a_rows ? a_rows[row] : row) * (uint32_t)K * 2 + xs_piece(lrow, lane & 7) * 16;
+  }
+  // waited for here: the compiler's own waits must not fall among the loads below, which it does not know of
+#pragma unroll
+  for (int i = 0; i < XL; ++i) asm volatile("" : "+v"(x_off[i]));
+  auto load_x = [&](int c) {                    // x rows of stage c
+#pragma unroll
+    for (int i = 0; i < XL; ++i) load_to_lds<false>(xb, x_off[i], c * (GK * 2), lds0 + kXAt + (c & 1) * kXStage + x_load[i] * 1024);
+  };
+  load_x(0);
 
-  // One K stage; `slot` (the stage's place in the ring) and `par` (its parity) are compile-time
-  // constants.  `steady`: every load of the stage is known to be in range, so none sits behind a
-  // branch.  The compiler counts outstanding loads statically; a load that may or may not have been
-  // issued makes it wait for all of them, and nothing would be hidden.
-  auto stage_step = [&](int c, auto slot_tag, auto par_tag, auto steady_tag) {
-    constexpr int slot = decltype(slot_tag)::value;
-    constexpr int par = decltype(par_tag)::value;
-    constexpr bool steady = decltype(steady_tag)::value;
-    if (steady || c + 2 < chunks) {   // this stage's register set went to LDS a stage ago
+  // operand addresses (bytes): fragment t of a step lies at w_at + t * 1024, row group mb of a stage's half at x_at + mb * 2048
+  int w_at = wc * NT * 1024 + lane * 16;
+  int x_at[2];
 #pragma unroll
-      for (int ps = 0; ps < PASS; ++ps) stage[par][ps] = *reinterpret_cast<const u32x4*>(x + xoff[ps] + (c + 2) * GK);
-    }
-    // the loads above are issued here and waited for a stage later: without the fence the compiler
-    // moves each load down to the LDS store that uses it and waits for it at once
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int j = 0; j < GK / 32; ++j) {
-      // 16-row groups GQ at a time: their LDS reads go out together, then their MFMAs
-#pragma unroll
-      for (int mq = 0; mq < MT; mq += Q) {
-        bf16x8 xf[Q];
-#pragma unroll
-        for (int i = 0; i < Q; ++i) xf[i] = *reinterpret_cast<const bf16x8*>(&xs[par][(mq + i) * 16 + r][xs_col(r, j * 32 + g * 8)]);
-#pragma unroll
-        for (int i = 0; i < Q; ++i)
-#pragma unroll
-          for (int t = 0; t < NT; ++t)
-            acc[t][mq + i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[slot][j][t], xf[i], acc[t][mq + i], 0, 0, 0);
-      }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    if (steady || c + kAhead < chunks) {   // this slot's weights are used up: fetch those of kAhead stages on
-#pragma unroll
-      for (int j = 0; j < GK / 32; ++j)
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-          wf[slot][j][t] = load_weights<STREAM>(We + woff[t] + (c + kAhead) * kStageStep + j * kSubStep);
-    }
-    if (steady || c + 1 < chunks) {   // the next stage's x rows, fetched a stage ago
-#pragma unroll
-      for (int ps = 0; ps < PASS; ++ps) *reinterpret_cast<u32x4*>(&xs[par ^ 1][srow + GROWS * ps][xs_col(srow + GROWS * ps, scol)]) = stage[par ^ 1][ps];
-    }
+  for (int hh = 0; hh < 2; ++hh) x_at[hh] = kXAt + (wr * MT * 16 + r) * 128 + xs_piece(r, hh * 4 + g) * 16;
+  // LDS reads run beside products: a step begins with its weights and half of its row groups in registers, reads the
+  // other half while the first is multiplied, and the next step's first part while the other half is (with all reads of a step ahead
+  // of its products, the LDS and the matrix cores took turns).
+  constexpr int H0 = (MT + 1) / 2, H1 = MT / 2;
+  bf16x8 wf[2][NT], x0[H0], x1[H1 > 0 ? H1 : 1];
+  auto arrive = [&](int s, auto half_tag) {     // step s is in LDS, and everyone has read step s - 1
+    constexpr int hh = decltype(half_tag)::value;
+    // This step's loads: behind them were sent two steps of weights, and in a stage's second step the next stage's x rows.  (In
+    // the last two steps some of those do not exist, and the first x rows were sent last: everything is waited for.)
+    if (s > 0 && s + 2 < steps) lds_loads_wait<hh == 0 ? 2 * WL : 2 * WL + XL>();
+    else lds_loads_wait<0>();
     __syncthreads();
   };
-  // stages are unrolled over ring slot x parity, so that both are constants
-  constexpr int kUnroll = (kAhead % 2 == 0) ? kAhead : 2 * kAhead;
-  auto stage_group = [&](int c, auto steady_tag) {
-    auto one = [&](auto i_tag) {
-      constexpr int i = decltype(i_tag)::value;
-      if (decltype(steady_tag)::value || c + i < chunks)
-        stage_step(c + i, std::integral_constant<int, i % kAhead>{}, std::integral_constant<int, i % 2>{}, steady_tag);
-    };
-    // exactly kUnroll stages: the loops below advance by that many
-    one(std::integral_constant<int, 0>{}); one(std::integral_constant<int, 1>{});
-    if constexpr (kUnroll > 2) { one(std::integral_constant<int, 2>{}); one(std::integral_constant<int, 3>{}); }
-    if constexpr (kUnroll > 4) { one(std::integral_constant<int, 4>{}); one(std::integral_constant<int, 5>{}); }
-    static_assert(kUnroll == 2 || kUnroll == 4 || kUnroll == 6, "stage_group lists two, four or six stages");
+  auto send = [&](int s, auto half_tag) {       // the loads that take the place of step s - 1
+    constexpr int hh = decltype(half_tag)::value;
+    if (hh == 0 && (s >> 1) + 1 < stages) load_x((s >> 1) + 1);
+    if (s + 3 < steps) load_w(s + 3);
   };
-  int c = 0;
-  for (; c + kUnroll + kAhead <= chunks; c += kUnroll) stage_group(c, std::true_type{});   // every fetch is of a stage that exists
-  for (; c < chunks; c += kUnroll) stage_group(c, std::false_type{});                      // the last stages check each fetch
+  auto read_first = [&](auto half_tag) {
+    constexpr int hh = decltype(half_tag)::value;
+#pragma unroll
+    for (int t = 0; t < NT; ++t) wf[hh][t] = *reinterpret_cast<const bf16x8*>(smem + w_at + hh * kWStep + t * 1024);
+#pragma unroll
+    for (int mb = 0; mb < H0; ++mb) x0[mb] = *reinterpret_cast<const bf16x8*>(smem + x_at[hh] + mb * 2048);
+  };
+  // the order the compiler is to keep: a read, then its share of the products
+  auto in_turn = [&](auto reads_tag, auto products_tag) {
+    constexpr int R = decltype(reads_tag)::value, P = decltype(products_tag)::value, kShare = R > 0 && P > R ? P / (R > 0 ? R : 1) : 1;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x8, kShare, 0);
+    }
+  };
+  auto step = [&](int s, auto half_tag, auto last_tag) {
+    constexpr int hh = decltype(half_tag)::value;
+    constexpr bool last = decltype(last_tag)::value;
+#pragma unroll
+    for (int mb = 0; mb < H1; ++mb) x1[mb] = *reinterpret_cast<const bf16x8*>(smem + x_at[hh] + (H0 + mb) * 2048);
+    auto row_products = [&](const bf16x8& rows, int mb) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) acc[t][mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[hh][t], rows, acc[t][mb], 0, 0, 0);
+    };
+#pragma unroll
+    for (int mb = 0; mb < H0; ++mb) row_products(x0[mb], mb);
+    in_turn(std::integral_constant<int, H1>{}, std::integral_constant<int, H0 * NT>{});
+    if constexpr (hh == 1) {
+      w_at ^= 2 * kWStep;
+      x_at[0] ^= kXStage;
+      x_at[1] ^= kXStage;
+    }
+    if constexpr (!last) {
+      __builtin_amdgcn_sched_barrier(0);        // products of the first half stay ahead of the barrier, those of the other behind it
+      arrive(s + 1, std::integral_constant<int, hh ^ 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+      read_first(std::integral_constant<int, hh ^ 1>{});
+    }
+    // this half's products, with the reads above and, half way through, the loads that fill the place step s has left
+    constexpr int kBefore = H1 / 2;
+#pragma unroll
+    for (int mb = 0; mb < kBefore; ++mb) row_products(x1[mb], H0 + mb);
+    if constexpr (!last) {
+      in_turn(std::integral_constant<int, NT + H0>{}, std::integral_constant<int, kBefore * NT>{});
+      __builtin_amdgcn_sched_barrier(0);
+      send(s + 1, std::integral_constant<int, hh ^ 1>{});
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int mb = kBefore; mb < H1; ++mb) row_products(x1[mb], H0 + mb);
+  };
+  using Half0 = std::integral_constant<int, 0>;
+  using Half1 = std::integral_constant<int, 1>;
+  arrive(0, Half0{});
+  send(0, Half0{});
+  read_first(Half0{});
+  for (int c = 0; c + 1 < stages; ++c) {
+    step(2 * c, Half0{}, std::false_type{});
+    step(2 * c + 1, Half1{}, std::false_type{});
+  }
+  step(steps - 2, Half0{}, std::false_type{});
+  step(steps - 1, Half1{}, std::true_type{});
 
+  if (threadIdx.x == 0) next = atomicAdd(counter, 1);   // the block's next slot: on its way while the results are stored
+  const int n_base = col_base + wc * HT * 16, row0 = tile_row0 + wr * MT * 16;
   // lane holds out[row0 + mb*16 + r][n_base + t*16 + 4g + 0..3]
   auto store = [&](TO* dst, const f32x4& v) {
     if constexpr (sizeof(TO) == 4) {
@@ -285,12 +285,13 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, const
 
 template <typename TO, int NT, bool PACKED, bool ACT>
 __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
-    const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, TO* __restrict__ out, int N, int K,
+    const bf16_t* __restrict__ x, uint32_t x_bytes, const bf16_t* __restrict__ W, TO* __restrict__ out, int N, int K,
     const int* __restrict__ a_rows, const float* __restrict__ act_scale, GatedAct act, int relu2,
     const int* __restrict__ group_offsets, const int* __restrict__ plan, int n_groups, int nb) {
-  __shared__ __attribute__((aligned(16))) bf16_t xs[2][GM][GPAD];
+  __shared__ __attribute__((aligned(1024))) char smem[kGroupedLds];
   __shared__ int s_slot, s_total[kXcds], s_taken[kXcds];
   __shared__ int4 s_unit[kWave + 1];
+  __shared__ int s_offset[kOffsetsKept];
   constexpr int GN = columns_of(NT);
   constexpr int kCols = ACT ? GN / 2 : GN;   // output columns of a block
   const int n_out = ACT ? N / 2 : N;
@@ -300,17 +301,14 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
   // siblings, the siblings of a column block side by side.  The slots of an XCD are handed out by a
   // ticket counter; when its own XCD's are gone a block takes slots of the next XCD's walk.
   //
-  // A slot takes a block about as long whatever its rows (it streams the same weights), and a walk
-  // is only a few slots per block long: slots that fill no whole round of the XCD's blocks would
-  // leave most of them idle for a slot's time at the end.  Those last slots are therefore cut by
-  // columns into 2 or 4 narrower ones (2 or 1 weight tiles a wave), as many as spread them over
-  // the blocks; a walk of fewer slots than blocks is cut the same way.
+  // A walk is only a few slots per block long: slots that fill no whole round of the XCD's blocks would leave most of them idle for
+  // a slot's time at the end.  Those last slots are therefore cut by columns into two (16 experts of 13 to 396 rows, 8,192 ->
+  // 5,120: 313 us where they were cut only if the halves fitted one round, 294 always; quarters, 318, read the x rows too often).
   // The unit lists are read by waves, a unit a lane (every thread after the other through the 16 units of each XCD
   // that 64 groups make cost 40 us a product: 16 rows an expert, 64 experts of 2,816 x 2,048: 173 -> 135 us).
   int* counters = const_cast<int*>(plan) + plan_counters_at(n_groups);
   const int home = blockIdx.x % kXcds;
   const int per_xcd = ((int)gridDim.x + kXcds - 1) / kXcds;   // blocks whose first walk is one XCD's
-  constexpr int kMaxCut = ACT ? NT / 2 : NT;                  // the gated form keeps a gate and an up tile a wave
   const int lane = threadIdx.x & (kWave - 1);
   auto unit_slots = [&](const int* pu) { return (plan_part_first(pu[1] + 1, pu[2], nb) - plan_part_first(pu[1], pu[2], nb)) * pu[3]; };
   // units j0 .. j0 + 63 of a walk into LDS: (slots before it, group, siblings, first column block), and all their slots
@@ -331,6 +329,8 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     }
     __syncthreads();
   };
+  if (n_groups < kOffsetsKept)
+    for (int i = threadIdx.x; i <= n_groups; i += GW * kWave) s_offset[i] = group_offsets[i];
   static_assert(GW == kXcds, "a wave counts the slots of one XCD's walk");
   {
     const int x = threadIdx.x >> 6;
@@ -350,8 +350,7 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     const int total = __builtin_amdgcn_readfirstlane(s_total[xcd]);   // slots of this walk
     const int whole = total / per_xcd * per_xcd;   // slots of whole rounds: taken as they are
     const int rest = total - whole;
-    int cut = 1;
-    if (rest > 0 && 2 * rest <= per_xcd) cut = (4 * rest <= per_xcd && kMaxCut >= 4) ? 4 : (kMaxCut >= 2 ? 2 : 1);
+    const int cut = rest > 0 ? 2 : 1;
     const int tickets = whole + rest * cut;
     if (q == 1) {                                  // its own walk is done: which others still have slots
       if (threadIdx.x < kXcds) s_taken[threadIdx.x] = __hip_atomic_load(&counters[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -359,8 +358,10 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     }
     if (q > 0 && s_taken[xcd] >= tickets) continue;
     if (n_units > 0 && n_units <= kWave) list_units(px, n_units, 0);
+    int next = -1;                                 // thread 0: the ticket taken at the end of the slot before, if there was one
     for (;;) {
-      if (threadIdx.x == 0) s_slot = atomicAdd(&counters[xcd], 1);
+      if (threadIdx.x == 0) s_slot = next >= 0 ? next : atomicAdd(&counters[xcd], 1);
+      next = -1;
       __syncthreads();
       const int ticket = __builtin_amdgcn_readfirstlane(s_slot);      // (what is found through LDS is the same for all lanes: scalars again)
       __syncthreads();
@@ -389,38 +390,24 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
       const int nblock = col0 + slot / n_sib;
       const int col_base = nblock * kCols + piece * (kCols / width);
       if (col_base >= n_out) continue;
-      const int first_row = group_offsets[e];
-      const int last_row = group_offsets[e + 1];
+      const int first_row = n_groups < kOffsetsKept ? s_offset[e] : group_offsets[e];
+      const int last_row = n_groups < kOffsetsKept ? s_offset[e + 1] : group_offsets[e + 1];
       const int height = plan_height(last_row - first_row, n_sib);
       const int row0 = first_row + sib * height;
       const int row_end = min(last_row, row0 + height);
       const int n_rows = row_end - row0;
       if (n_rows <= 0) continue;
-      const int wave_cols = (ACT ? 8 * NT : 16 * NT) / width;   // output columns of a wave
-      const int n_base = col_base + (threadIdx.x >> 6) * wave_cols;
       const bf16_t* We = W + (size_t)e * N * K;
-      static_assert(GM == 128, "tile heights are compiled in steps of 32 rows up to 128");
-#define GT1(MTV, NTV, ST) grouped_tile<TO, MTV, NTV, PACKED, ACT, ST>(x, We, out, N, K, a_rows, act_scale, act, relu2, row0, row_end, n_base, xs)
-      // (the hint only for weights stored tile by tile, the order the served model keeps them in)
-#define GT2(MTV, NTV)                                \
-  do {                                               \
-    if (PACKED && n_sib == 1) GT1(MTV, NTV, PACKED); \
-    else GT1(MTV, NTV, false);                       \
-  } while (0)
-#define GT(NTV)                     \
-  do {                              \
-    if (n_rows <= 32) GT2(2, NTV);  \
-    else if (n_rows <= 64) GT2(4, NTV); \
-    else if (n_rows <= 96) GT2(6, NTV); \
-    else GT2(8, NTV);               \
-  } while (0)
-      if (width == 1) GT(NT);
-      else if constexpr (kMaxCut >= 2) {
-        if (width == 2) GT(NT / 2);
-        else if constexpr (kMaxCut >= 4) GT(NT / 4);
-      }
+      // (the streaming hint only where no sibling reads the same weights: a pure read reaches 6.9 TB/s with it, 6.2 without)
+#define GT1(MTV, NTV) \
+  case MTV: grouped_tile<TO, MTV, NTV, PACKED, ACT>(x, x_bytes, We, out, N, K, a_rows, act_scale, act, relu2, row0, row_end, col_base, n_sib == 1, smem, &counters[xcd], next); break
+#define GT(NTV)                                                                                                  \
+  switch ((n_rows + 31) >> 5) {                                                                                  \
+    GT1(1, NTV); GT1(2, NTV); GT1(3, NTV); GT1(4, NTV); GT1(5, NTV); GT1(6, NTV); GT1(7, NTV); GT1(8, NTV);      \
+  }
+      if (width == 1) GT(NT)
+      else GT(NT / 2)
 #undef GT
-#undef GT2
 #undef GT1
     }
   }
@@ -441,6 +428,11 @@ static bool grouped_args_ok(int x_rows, int n_rows, int N, int K, int n_groups, 
   return (long long)N * K <= 0x7fffffffLL && x_rows > 0 && (long long)x_rows * K <= 0x7fffffffLL;
 }
 
+static uint32_t grouped_x_bytes(int x_rows, int K) {
+  const unsigned long long bytes = 2ull * x_rows * K;       // below 2^32: grouped_args_ok
+  return (uint32_t)bytes;
+}
+
 static int compute_units() {
   static int units[64] = {0};
   int dev = 0;
@@ -454,10 +446,10 @@ static int compute_units() {
 }
 
 // As many blocks as stay at once (one to a compute unit), fewer if there is less work (a slot may
-// be cut in up to four) or if the caller bounds them (max_blocks > 0: the compute units left over
+// be cut in two) or if the caller bounds them (max_blocks > 0: the compute units left over
 // are for other work).
 static dim3 grouped_grid(int n_rows, int n_groups, int nb, int max_blocks) {
-  long long blocks = 4LL * kXcds * plan_slots_bound(n_rows, n_groups, nb);
+  long long blocks = 2LL * kXcds * plan_slots_bound(n_rows, n_groups, nb);
   const long long stay = compute_units();
   if (blocks > stay) blocks = stay;
   if (max_blocks > 0 && blocks > max_blocks) blocks = max_blocks;
