@@ -478,7 +478,7 @@ def gemm_tiled(x: torch.Tensor, w: torch.Tensor, out_dtype: Optional[torch.dtype
     M, K = x.shape
     N = w.shape[0]
     out = torch.empty(M, N, dtype=out_dtype, device=x.device)
-    _run("sharpi_gemm_tiled", _ptr(x), _ptr(w), _ptr(out), _code(x.dtype), _code(out_dtype), M, N, K, None, None, 0,
+    _run("sharpi_gemm_tiled", _ptr(x), _ptr(w), _ptr(out), _code(x.dtype), _code(out_dtype), M, N, K, None, None, 0, M,
          _stream())
     return out
 
@@ -1047,7 +1047,7 @@ def grouped_gemm(x: torch.Tensor, w: torch.Tensor, offsets: torch.Tensor, a_rows
         _need(x.shape[0] == n_rows, "grouped_gemm: x must have n_rows rows when not gathered")
     out = torch.empty(n_rows, N, dtype=x.dtype, device=x.device)
     _run("sharpi_gemm_tiled", _ptr(x), _ptr(w), _ptr(out), _code(x.dtype), _code(x.dtype), n_rows, N, K, _ptr(a_rows),
-         _ptr(offsets), E, _stream())
+         _ptr(offsets), E, x.shape[0], _stream())
     return out
 
 

@@ -32,7 +32,7 @@ _SIGNATURES = {
     "sharpi_attention_decode": [P, P, P, P, P, P, P, P, P, P, I, I, F, I, I, I, I, I, I, I, I, F, I, P, P],
     "sharpi_attention_decode_values": [P, P, P, P, P, P, P, P, P, P, I, I, F, I, I, I, I, I, I, I, I, I, F, I, P, I, P, I, P],
     "sharpi_attention_prefill": [P, P, P, P, P, P, P, I, I, I, I, F, I, I, I, I, I, I, I, F, I, P, I, P, I, P],
-    "sharpi_gemm_tiled": [P, P, P, I, I, I, I, I, P, P, I, P],
+    "sharpi_gemm_tiled": [P, P, P, I, I, I, I, I, P, P, I, I, P],
     "sharpi_gemm_skinny": [P, P, P, I, I, I, I, P, P, I, I, I, I, I, I, P],
     "sharpi_gemm_skinny_swiglu": [P, P, P, I, I, I, P, P, I, P, I, I, I, I, I, F, P],
     "sharpi_gemm_skinny_picked": [P, P, P, I, I, I, P, P, I, I, I, I, I, I, F, I, I, I, I, P],
