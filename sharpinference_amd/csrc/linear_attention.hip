@@ -14,7 +14,8 @@
 // after the other from the slot's state; phase 2 walks every segment again from its start state, now
 // writing outputs, and the last segment leaves the entry's new state in the slot.  Twice the sums
 // on as many times the blocks as an entry has segments; the results differ from the unsegmented
-// walk's by rounding only (the state at a segment's start is summed in another order).
+// walk's by rounding only (the state at a segment's start is summed in another order).  Heads of 64 or 128 key and value channels
+// whose rows lie on 16-byte borders take both phases as matrix products (gla_chunk.hip).
 //
 // Three forms: stages of 16 tokens (8 for the widest heads) for whole entries of steps that bring
 // portions of prompts; stages of 8 tokens for the segmented walk, whose many blocks then sit six to a
@@ -38,6 +39,7 @@
 // The decays are made from their logits once per (token, channel) by a kernel of their own, in
 // float: alpha = exp(log_sigmoid(z + bias) / tau), in place over the logits.
 #include "common.h"
+#include "gla_chunk.h"
 
 constexpr int kCols = 8;                 // value columns a walking wave owns
 constexpr int kGroups = kWave / kCols;   // row groups
@@ -387,12 +389,17 @@ static int launch_segmented(const void* proj, int stride, int q_off, int k_off, 
   gla_walk_kernel<T, RPL, VEC, 8><<<grid, 2 * kWave, 0, stream>>>(                                         \
       (const T*)proj, stride, q_off, k_off, v_off, alpha, q_scale, state, state_slots, cu_tokens, out, nh, dk, dv, ncb, segs, PH, \
       seg_state, seg_decay)
+  const int dtype = sizeof(T) == 4 ? DT_F32 : DT_BF16;
+  const GlaChunkArgs chunk{proj, stride, q_off, k_off, v_off, alpha, q_scale, state, state_slots, out, nh, segs, seg_state, seg_decay};
+  const bool products = gla_chunk_takes(dtype, stride, q_off, k_off, v_off, chunk, dk, dv);
 #define SEGMENTED(RPL)                                                                                       \
   do {                                                                                                       \
-    if (vec) PHASE(RPL, true, 1);                                                                            \
+    if (products) gla_chunk_launch(dtype, chunk, dk, dv, n_segs, false, stream);                             \
+    else if (vec) PHASE(RPL, true, 1);                                                                       \
     else PHASE(RPL, false, 1);                                                                               \
     gla_combine_kernel<RPL><<<cgrid, kWave, 0, stream>>>(state, state_slots, ent_segs, seg_state, seg_decay, nh); \
-    if (vec) PHASE(RPL, true, 2);                                                                            \
+    if (products) gla_chunk_launch(dtype, chunk, dk, dv, n_segs, true, stream);                              \
+    else if (vec) PHASE(RPL, true, 2);                                                                       \
     else PHASE(RPL, false, 2);                                                                               \
   } while (0)
   if (dk <= 32) SEGMENTED(4);

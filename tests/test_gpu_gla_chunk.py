@@ -1,0 +1,104 @@
+"""Gated linear attention's segments as matrix products: against the recurrence in 64 bits, no further from it than the walk, at
+the edges of blocks of 16 tokens and of segments, with decays of 0 and 1, and with values that are no number, which stay with their
+token and later ones."""
+import types
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def recurrence(q, k, v, alpha, S):
+    out = []
+    for t in range(q.shape[0]):
+        S = alpha[t][:, :, None] * S + k[t][:, :, None] * v[t][:, None, :]
+        out.append((S * q[t][:, :, None]).sum(1))
+    return torch.stack(out), S
+
+
+def step(lens, slots):
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    return types.SimpleNamespace(n_entries=len(lens), n_tokens=int(cu[-1]), max_entry_len=max(lens), cu=cu,
+                                 state_slots=torch.tensor(slots, dtype=torch.int32, device=DEV), cu_tokens=torch.from_numpy(cu).to(DEV))
+
+
+def run(proj, alpha, state, ctx, H, dk, dv, pad, segmented=True):
+    from sharpinference_amd import ops
+    lens = np.diff(ctx.cu).tolist()
+    segments = tuple(torch.from_numpy(x).to(DEV) for x in ops.gla_segments(lens, ctx.cu)) if segmented else None
+    state = state.clone()
+    o = ops.gla_walk(proj, pad, pad + H * dk, pad + 2 * H * dk, alpha, dk ** -0.5, state, ctx, H, dk, dv, segments=segments)
+    return o, state
+
+
+def inputs(lens, H, dk, dv, pad, dtype, tau, seed):
+    from sharpinference_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    T = sum(lens)
+    proj = torch.randn(T, pad + H * (2 * dk + dv) + 8, device=DEV, generator=g).to(dtype)
+    alpha = torch.sigmoid(2 * torch.randn(T, H * dk, device=DEV, generator=g) + 1) ** (1 / tau)
+    some = torch.rand(T, H * dk, device=DEV, generator=g)
+    alpha = torch.where(some < 0.01, torch.zeros_like(alpha), torch.where(some > 0.99, torch.ones_like(alpha), alpha))
+    state = torch.randn(len(lens) + 1, *ops.gla_state_shape(H, dk, dv), device=DEV, generator=g)
+    return proj, alpha.contiguous(), state
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H, dk, dv, tau", [(2, 128, 128, 16.0), (3, 64, 128, 1.0), (1, 128, 64, 0.3), (2, 64, 64, 40.0)])
+@pytest.mark.parametrize("lens", [[128], [1, 15, 16, 17], [129, 2], [33, 127, 260], [400]])
+def test_segments_as_products_are_no_further_from_64_bits_than_the_walk(dtype, H, dk, dv, tau, lens):
+    from sharpinference_amd import ops
+    pad = 8
+    proj, alpha, state = inputs(lens, H, dk, dv, pad, dtype, tau, sum(lens) + dk)
+    ctx = step(lens, [i + 1 for i in range(len(lens))])
+    got, left = run(proj, alpha, state, ctx, H, dk, dv, pad)
+    walk, walk_left = run(proj, alpha, state, ctx, H, dk, dv, pad, segmented=False)
+    assert torch.equal(left[0], state[0])                                # nobody's slot
+    p = proj.double()
+    part = lambda a, n: p[:, a:a + H * n].reshape(-1, H, n)
+    q, k, v, a = part(pad, dk) * dk ** -0.5, part(pad + H * dk, dk), part(pad + 2 * H * dk, dv), alpha.double().view(-1, H, dk)
+    S0 = ops.gla_state_matrices(state, dk, dv).double()
+    errors = np.zeros((2, 2))
+    for e in range(len(lens)):
+        rows = slice(int(ctx.cu[e]), int(ctx.cu[e + 1]))
+        want, S = recurrence(q[rows], k[rows], v[rows], a[rows], S0[e + 1])
+        for i, (o, st) in enumerate(((got, left), (walk, walk_left))):
+            errors[i] += [float((o[rows].double().view(want.shape) - want).pow(2).sum() / want.pow(2).mean()),
+                          float((ops.gla_state_matrices(st[e + 1:e + 2], dk, dv)[0].double() - S).pow(2).sum() / S.pow(2).mean())]
+    count = np.array([got.numel(), len(lens) * H * dk * dv])
+    ours, walks = np.sqrt(errors / count)
+    # a score's decays are products of up to 128 factors here as there; one rounding of float more is 2.4e-8
+    assert (ours <= 1.1 * walks + 3e-8).all(), (ours, walks)
+    assert (ours <= 4e-7).all(), ours
+
+
+@pytest.mark.parametrize("what", ["v", "k", "q", "alpha"])
+@pytest.mark.parametrize("at", [3, 40, 127, 128, 200])
+def test_what_is_no_number_stays_with_its_token_and_later_ones(what, at):
+    H, dk, dv, pad, lens = 2, 128, 64, 8, [260, 20]
+    proj, alpha, state = inputs(lens, H, dk, dv, pad, torch.bfloat16, 16.0, 5)
+    ctx = step(lens, [0, 1])
+    clean, left = run(proj, alpha, state, ctx, H, dk, dv, pad)
+    for bad in (float("inf"), float("nan")):
+        p, a = proj.clone(), alpha.clone()
+        if what == "alpha":
+            a[at, 7] = bad
+        else:
+            p[at, pad + {"q": 0, "k": H * dk, "v": 2 * H * dk}[what] + 7] = bad
+        o, st = run(p, a, state, ctx, H, dk, dv, pad)
+        assert torch.equal(o[:at], clean[:at]) and torch.equal(o[260:], clean[260:])
+        assert torch.equal(o[:, dv:], clean[:, dv:])                     # the other head
+        assert not bool(o[at, :dv].isfinite().all())
+        assert torch.equal(st[1], left[1]) and (what == "q") == bool(st[0].isfinite().all())
+
+
+def test_rows_off_the_borders_are_walked():
+    H, dk, dv, lens = 2, 64, 64, [300]
+    proj, alpha, state = inputs(lens, H, dk, dv, 8, torch.bfloat16, 4.0, 9)
+    ctx = step(lens, [0])
+    want, left = run(proj, alpha, state, ctx, H, dk, dv, 8)
+    got, st = run(torch.cat([proj[:, 5:], proj[:, :5]], 1).contiguous(), alpha, state, ctx, H, dk, dv, 3)
+    assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max()) and float((st - left).abs().max()) <= 1e-5 * float(left.abs().max())
