@@ -31,4 +31,4 @@ SHARPI_EXPORT int sharpi_gemm_grouped(const void* x, int x_rows, const void* W, 
   return SHARPI_OK;
 }
 
-SHARPI_EXPORT int sharpi_gemm_grouped_tile_rows() { return GM; }
+SHARPI_EXPORT int sharpi_gemm_grouped_tile_rows() { return kPlanTileRows; }

@@ -34,8 +34,8 @@
 //  * The plain form may square the relu of its results (relu2: feed-forwards without a gate), rounded to
 //    bfloat16 first (what a separate activation kernel would have read).
 // Measured, 16 experts, up (2 x 8,192 rows of 5,120) + down, us, beside tiles of 128 x 512 whose weights went straight to
-// registers: 8,192 tokens 1,346 + 666 (1,420 + 700), 2,048 tokens of uneven load 570 + 271 (587 + 264), 1,190 tokens 470 + 237
-// (488 + 250); 64 experts of 1,408 x 2,048, six picks, 3,000 tokens 292 + 144 (327 + 157), 1,664 tokens 187 + 106 (235 + 110).
+// registers: 8,192 tokens 1,328 + 647 (1,420 + 700), 2,048 tokens of uneven load 576 + 269 (587 + 264), 1,190 tokens 463 + 241
+// (488 + 250); 64 experts of 1,408 x 2,048, six picks, 3,000 tokens 291 + 137 (327 + 157), 1,664 tokens 192 + 100 (235 + 110).
 // Parts taken out, 4,096 tokens even (up, 656 us): no loads 465 (1.48 PFLOP/s), no products 538, weights and products without x rows
 // 615: the weights' 2.7 GB and the products each need about 460, and neither hides the other whole.
 // Limits: K % 64 == 0, N % 4 == 0 (N % 32 == 0 in the SwiGLU form).
@@ -49,7 +49,8 @@
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
 
-constexpr int GM = kPlanTileRows;      // rows per tile
+constexpr int GM = 256;                // rows per tile: two of the plan's
+static_assert(GM % kPlanTileRows == 0, "the plan's units stay level");
 constexpr int GW = 8;                  // waves per block
 constexpr int GWC = 4;                 // of them side by side along the columns, the others along the rows
 constexpr int kMaxNT = 4;              // 16-row weight tiles per wave: this many, or half where a slot is cut
@@ -304,19 +305,26 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
   // A walk is only a few slots per block long: slots that fill no whole round of the XCD's blocks would leave most of them idle for
   // a slot's time at the end.  Those last slots are therefore cut by columns into two (16 experts of 13 to 396 rows, 8,192 ->
   // 5,120: 313 us where they were cut only if the halves fitted one round, 294 always; quarters, 318, read the x rows too often).
+  if (n_groups < kOffsetsKept)
+    for (int i = threadIdx.x; i <= n_groups; i += GW * kWave) s_offset[i] = group_offsets[i];
+  __syncthreads();
   // The unit lists are read by waves, a unit a lane (every thread after the other through the 16 units of each XCD
   // that 64 groups make cost 40 us a product: 16 rows an expert, 64 experts of 2,816 x 2,048: 173 -> 135 us).
   int* counters = const_cast<int*>(plan) + plan_counters_at(n_groups);
   const int home = blockIdx.x % kXcds;
   const int per_xcd = ((int)gridDim.x + kXcds - 1) / kXcds;   // blocks whose first walk is one XCD's
   const int lane = threadIdx.x & (kWave - 1);
-  auto unit_slots = [&](const int* pu) { return (plan_part_first(pu[1] + 1, pu[2], nb) - plan_part_first(pu[1], pu[2], nb)) * pu[3]; };
+  // The plan counts siblings of kPlanTileRows rows; here a group's rows are cut into tiles of GM (the deal stays level, and
+  // the tall tiles, which take longest, still come first in a walk).
+  auto offset_of = [&](int e) { return n_groups < kOffsetsKept ? s_offset[e] : group_offsets[e]; };
+  auto siblings_of = [&](int e) { return (offset_of(e + 1) - offset_of(e) + GM - 1) / GM; };
+  auto unit_slots = [&](const int* pu) { return (plan_part_first(pu[1] + 1, pu[2], nb) - plan_part_first(pu[1], pu[2], nb)) * siblings_of(pu[0]); };
   // units j0 .. j0 + 63 of a walk into LDS: (slots before it, group, siblings, first column block), and all their slots
   auto list_units = [&](const int* px, int n_units, int j0) {
     __syncthreads();
     if (threadIdx.x < kWave) {
       const int* pu = px + 1 + 4 * min(j0 + lane, n_units - 1);
-      const int u_group = pu[0], u_sib = pu[3], u_col = plan_part_first(pu[1], pu[2], nb);
+      const int u_group = pu[0], u_sib = siblings_of(pu[0]), u_col = plan_part_first(pu[1], pu[2], nb);
       const int slots = j0 + lane < n_units ? unit_slots(pu) : 0;
       int upto = slots;
 #pragma unroll
@@ -329,8 +337,6 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     }
     __syncthreads();
   };
-  if (n_groups < kOffsetsKept)
-    for (int i = threadIdx.x; i <= n_groups; i += GW * kWave) s_offset[i] = group_offsets[i];
   static_assert(GW == kXcds, "a wave counts the slots of one XCD's walk");
   {
     const int x = threadIdx.x >> 6;
@@ -390,8 +396,7 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
       const int nblock = col0 + slot / n_sib;
       const int col_base = nblock * kCols + piece * (kCols / width);
       if (col_base >= n_out) continue;
-      const int first_row = n_groups < kOffsetsKept ? s_offset[e] : group_offsets[e];
-      const int last_row = n_groups < kOffsetsKept ? s_offset[e + 1] : group_offsets[e + 1];
+      const int first_row = offset_of(e), last_row = offset_of(e + 1);
       const int height = plan_height(last_row - first_row, n_sib);
       const int row0 = first_row + sib * height;
       const int row_end = min(last_row, row0 + height);

@@ -21,10 +21,12 @@
 // plan (int32), per XCD x at plan + x * plan_stride(G), G groups:
 //   [0]                      units of this XCD
 //   [1 + 4j .. 4 + 4j]       unit j: group, part, parts, siblings
+// The product of bfloat16 rows reads the units and their order, and cuts a group's rows into tiles of its own, twice as tall: the
+// tall ones come first in a walk either way, and units of three or four siblings here have as many slots as those of one.
 #pragma once
 
 constexpr int kPlanXcds = 8;
-constexpr int kPlanTileRows = 256;
+constexpr int kPlanTileRows = 128;
 constexpr int kPlanMaxParts = 16;
 
 __host__ __device__ inline int plan_siblings(int rows) { return (rows + kPlanTileRows - 1) / kPlanTileRows; }
@@ -33,9 +35,6 @@ __host__ __device__ inline int plan_height(int rows, int n_sib) { return ((rows 
 __host__ __device__ inline int plan_parts(int n_sib) { return n_sib <= 2 ? 2 : n_sib <= 4 ? 4 : n_sib <= 8 ? 8 : kPlanMaxParts; }
 // what a unit weighs when units are dealt to the XCDs: its share of the group's (siblings x column blocks)
 __host__ __device__ inline int plan_weight(int n_sib) { return n_sib * (kPlanMaxParts / plan_parts(n_sib)); }
-// the order in which units are dealt, the greatest first: by weight, units of one weight by the height of their tiles, so that the
-// long slots of a walk begin early (16 experts of 13 to 396 rows, 8,192 -> 5,120: 295 us without the second)
-__host__ __device__ inline int plan_order(int rows, int n_sib) { return plan_weight(n_sib) * 16 + plan_height(rows, n_sib) / 32; }
 // column blocks [first, first + count) of part `part` of `parts`, of nb column blocks in all
 // (parts is a power of two)
 __host__ __device__ inline int plan_part_first(int part, int parts, int nb) { return (int)((unsigned)part * (unsigned)nb / (unsigned)parts); }

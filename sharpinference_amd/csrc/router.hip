@@ -639,22 +639,22 @@ __device__ void permute_block(const int* __restrict__ topk_ids, const float* __r
   if (plan) {
     // The plan of the grouped product (grouped_plan.h).  Groups: the experts, and the always-on
     // group (every token once) if there is one.  Every group with rows gives plan_parts units;
-    // units in the order of their weight (then of their tiles' height, of group and part) are dealt to the XCDs row by
+    // units in the order of their weight (then of group and part) are dealt to the XCDs row by
     // row, rows alternating in direction so that the XCDs' loads stay level.
     const int n_groups = n_experts + (shared_group ? 1 : 0);
     const int stride = plan_stride(n_groups);
     __syncthreads();
-    // a group's place in the order and its units as one number that orders groups as the deal does and tells their units; 0: no rows
+    // a group's weight and units as one number that orders groups as the deal does and tells their units; 0: no rows
     int* rank = plan_scratch;
     for (int g = threadIdx.x; g < n_groups; g += step) {
       const int sg = plan_siblings(count[g]);
-      rank[g] = count[g] == 0 ? 0 : plan_order(count[g], sg) * (int)kPlanRankParts + plan_parts(sg);
+      rank[g] = count[g] == 0 ? 0 : plan_weight(sg) * (int)kPlanRankParts + plan_parts(sg);
     }
     __syncthreads();
     for (int g = threadIdx.x; g < n_groups; g += step) {
       if (count[g] == 0) continue;
       const int sg = plan_siblings(count[g]);
-      const int wg = plan_order(count[g], sg), pg = plan_parts(sg);
+      const int wg = plan_weight(sg), pg = plan_parts(sg);
       // units that come before this group's: of heavier groups all, of equally heavy ones those of lower index
       int before = 0;
 #pragma unroll 8
