@@ -2,38 +2,31 @@
 // over the paged cache, causal and window masks applied per element.
 //
 // A block owns a tile of up to 128 consecutive tokens of one entry and one query head; each of its
-// four waves takes 32 of the tokens (or, for tiles of up to 64 tokens, two waves: the keys of a tile
-// are walked one chunk after the other, so a short prompt, whose last tiles alone decide how long the
-// launch takes, is served faster by twice the blocks of half the rows; a row's sums are the same
+// four waves takes 32 of the tokens (or, for tiles of up to 64 tokens, 16: a row's sums are the same
 // either way).  As in the decode kernel everything is transposed:
 //   S^T[key, q]  = K[key, :] . Q[q, :]          A = K block, B = Q^T
 //   O^T[d, q]   += V^T[d, key] * P^T[key, q]    A = V^T block (values are stored transposed
 //                                               inside a page), B = P^T
-// on 32x32x16 products, and the S^T accumulator of a lane is the B operand of the second product once
-// exponentiated and split into a bfloat16 pair hi + lo (two products: the probabilities keep ~16
-// bits; the row's sum is taken from the unrounded values).  Softmax state (a reference maximum and
-// the sum per query) is float, kept in base-2 units (scores times log2 e, the hardware's exp2).
-// The keys of a query are always visited in the same chunks (32 keys at absolute positions),
-// whatever tile it sits in and however many waves the tile has.
+// and the S^T accumulator of a lane is the B operand of the second product once exponentiated
+// and split into a bfloat16 pair hi + lo (two products: the probabilities keep ~16 bits; the row's
+// sum is taken from the unrounded values).  Softmax state (a reference maximum and the sum per query)
+// is float, kept in base-2 units (scores times log2 e, the hardware's exp2).
+// The keys of a query are always visited in the same chunks (pairs of 16-key blocks at absolute
+// positions), whatever tile it sits in.
 //
-// Keys and values go from the cache straight into LDS (loads that write LDS, no registers between),
-// a stage of 16 keys a wave ahead: wave w fetches the stage's 16-key block w, so a stage needs one
-// page number a wave, itself requested a stage earlier.  The cache's order is kept in 16-byte pieces;
-// where a piece goes is chosen by the lane that fetches it:
-//  * key rows are stored in the order in which the product's accumulator hands keys to lanes: row
-//    rho of a 16-key block holds the key with bits 2 and 3 of rho exchanged, so that a lane ends up
-//    with eight consecutive keys of a 16-key block, which is what the second product reads of the
-//    values with one 16-byte load;
-//  * a row's 16-byte pieces, and the two halves of a value row, are XORed with row bits so that the
-//    operand reads are free of bank conflicts (k_swizzle, v_swizzle).
+// Keys and values go from the cache straight into LDS (loads that write LDS, no registers between), a
+// stage of 64 keys ahead: wave w fetches the stage's 16-key block w, so a stage needs one page number a
+// wave, itself requested a stage earlier, and a barrier covers 96 products of a wave.  The cache's order
+// is kept in 16-byte pieces; a key row's are XORed with row bits so that the operand reads are free
+// of bank conflicts (k_swizzle).  Heads of one kv head run on one die and share its L2.
 //
-// What bounds it: per 32 keys and 32 rows a wave issues 24 products of 32 cycles (128-wide heads) and about
+// What bounds it: per 32 keys and 32 rows a wave issues 48 products of 16 cycles (128-wide heads) and about
 // 150 vector instructions a lane for the softmax, on one SIMD that two waves share.
-// 40 heads of 128 sharing 8 key heads, 8,192 tokens: 904 us (761 TFLOP/s, the pair's second product not counted; with it the
-// matrix cores run at 1.14 PFLOP/s, a large plain product reaches 1.35); 1,452 us with 16x16x32 products, chunks on their way
-// through registers, and two divisions by the page size a chunk.  2,048 tokens: 76 us (133); 64 heads of 192 / 128, window
-// 1,024, 2,048 tokens: 111 us (180); 16 heads, 1,900 tokens: 47 us (75), where a compute unit has one block and the chain of
-// a wave's products and softmax is what is left.  Three prompts of 400 tokens in tiles of 64: 32 us (34).
+// 40 heads of 128 sharing 8 key heads, 8,192 tokens: 1,041 us (660 TFLOP/s, the pair's second product not counted); 1,452 us with
+// 32-key chunks on their way through registers and divisions by the page size in every chunk.  2,048 tokens: 98 us (133); 64 heads of
+// 192 / 128, window 1,024, 2,048 tokens: 139 us (180); 16 heads, 1,900 tokens: 49 us (75).  Three prompts of 400 tokens in
+// tiles of 64: 30 us (34).  On 32x32x16 products, eight consecutive keys a lane, it took 904, 76, 111 and 47 us: other sums of the
+// same exactness, whose roundings turned routers' near ties in whole models; these are the bits of the kernel before.
 #pragma once
 #include <type_traits>
 
@@ -42,7 +35,6 @@
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) float f32x4;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 #ifndef SHARPI_PREFILL_P_PAIR
 // 1: probabilities enter the second product as a bfloat16 pair hi + lo.  0 (hi alone) is faster, but then
@@ -51,22 +43,18 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 // up to a quarter in 4 of 60, none with the pair.
 #define SHARPI_PREFILL_P_PAIR 1
 #endif
-constexpr int kPreWaves = 4;                         // waves of a whole tile (half as many for tiles of half the rows)
-constexpr int kWaveTokens = 32;                      // query rows of a wave
-constexpr int kTileTokens = kWaveTokens * kPreWaves; // 128 tokens per block at most
+constexpr int kPreWaves = 4;
+constexpr int kTileTokens = 32 * kPreWaves;          // 128 tokens per block at most
 
 // LDS layouts.  The LDS serves a 16-byte read of a wave in four turns of two octets of lanes: one
-// octet holding operand rows 0..7 and one holding rows 24..31 (or 8..15 and 16..23; measured with the
-// bank-conflict counter on operands of 16 rows: octets l..l+7 and l+24..l+31).  The 16 pieces of 16
+// octet holding operand rows 0..7 and one holding rows 8..15 of the neighbouring lane group (measured
+// with the bank-conflict counter).  The 16 pieces of 16
 // bytes that a turn reads must fall into the 16 different 16-byte groups of the 256-byte bank space:
 // a piece's number is XORed with row bits, as many as rows share a group.
 template <int HD> __device__ __forceinline__ constexpr int k_swizzle(int row) {
   return HD % 128 == 0 ? (row & 15) : HD % 64 == 0 ? ((row >> 1) & 7) : ((row >> 2) & 3);
 }
-// values: a 16-key block is kept as rows of 32 bytes, one a value column; the halves of eight
-// neighbouring columns fill the bank space, and the octets of a turn, 16 columns apart, take opposite halves.
-__device__ __forceinline__ constexpr int v_swizzle(int d) { return (d >> 4) & 1; }
-__device__ __forceinline__ constexpr int k_key(int row) { return (row & ~12) | ((row & 4) << 1) | ((row & 8) >> 1); }   // key of LDS row `row`
+// values: a 16-key block is kept as rows of 32 bytes, one a value column: a wave's 8-byte reads are 512 bytes in a row.
 
 constexpr float kLazyMax = 8.0f;                     // how far the row maximum may outgrow its reference
 // the reference before a row has seen a key: finite, so that a masked score (-inf) minus it is
@@ -97,18 +85,20 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
 template <int HD, int VD>
 constexpr int prefill_waves_a_simd() { return kPreWaves * 16 * (HD + (VD + 31) / 32 * 32) * 4 <= 80 * 1024 ? 2 : 1; }   // by the LDS two blocks need
 
-template <int HD, int VD, int WAVES>
-__global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) void attn_prefill_kernel(
+template <int HD, int VD, int kQT>
+__global__ __launch_bounds__(kPreWaves* kWave, (prefill_waves_a_simd<HD, VD>())) void attn_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ block_table, const int* __restrict__ positions, const int* __restrict__ tiles,
     bf16_t* __restrict__ out, int window_kind, int window, float scale, int nh, int nkv, int page_size,
     int max_blocks, int num_pages, float softcap, int sink, const float* __restrict__ sink_vals, int keep,
     const bf16_t* __restrict__ gate, int gate_stride) {
-  constexpr int NJ = HD / 16;                       // product steps of a score
-  constexpr int ND = (VD + 31) / 32;                // 32-column tiles of the values (the last may be half one: its rest is never stored)
+  constexpr int WAVES = kPreWaves, kWaveTokens = 16 * kQT;
+  constexpr int NJ = HD / 32;                       // product steps of a score
+  constexpr int ND = VD / 16;                       // 16-column tiles of the values
+  constexpr int VL = (VD + 31) / 32;                // loads of a 16-key block of values (32 columns each; half of the last may be idle)
   constexpr int CH = HD / 8;                        // 16-byte pieces of a key row
-  constexpr int KL = HD / 32;                       // loads of a 16-key block of keys (64 pieces each), and of values: ND
-  constexpr int KB = 16 * HD * 2, VB = ND * 1024;   // LDS bytes of a 16-key block
+  constexpr int KL = HD / 32;                       // loads of a 16-key block of keys (64 pieces each)
+  constexpr int KB = 16 * HD * 2, VB = VL * 1024;   // LDS bytes of a 16-key block
   constexpr int STAGE = WAVES * (KB + VB);          // a stage: WAVES blocks of keys, then as many of values
   constexpr int SUBS = WAVES / 2;                   // 32-key chunks of a stage
   static_assert(HD % 32 == 0 && VD % 16 == 0 && WAVES % 2 == 0, "sizes the layouts are made for");
@@ -117,7 +107,7 @@ __global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) voi
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r = lane & 31, g = lane >> 5;
+  const int r = lane & 15, g = lane >> 4;
   // Tiles run from the last backwards (later tiles of a prompt see more keys, and the longest blocks should start first),
   // heads fastest.  Blocks go to the 8 dies round-robin, so where the heads divide by 8 a die takes neighbouring
   // heads: those of one kv head read the same keys and values out of one L2.
@@ -135,23 +125,28 @@ __global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) voi
     return 0;
   };
 
-  // this wave's 32 tokens: the lane's query row, its position, its first key
+  // this wave's tokens: per column tile, the lane's query row, its position, its first key
   const int wrow0 = w * kWaveTokens;
-  const int row = wrow0 + r;
-  const bool qok = row < rows;
-  const int qpos = pos0 + row;
-  const int qstart = first_key(qpos);
-  bf16x8 qf[NJ];
-  {
+  int qpos[kQT], qstart[kQT];
+  bool qok[kQT];
+  bf16x8 qf[kQT][NJ];
+#pragma unroll
+  for (int c = 0; c < kQT; ++c) {
+    const int row = wrow0 + c * 16 + r;
+    qok[c] = row < rows;
+    qpos[c] = pos0 + row;
+    qstart[c] = first_key(qpos[c]);
     // rows beyond the tile's last read its last row; their scores are masked and their output is never stored
     const bf16_t* src = q + ((size_t)(tok0 + min(row, rows - 1)) * nh + h) * HD + g * 8;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) qf[j] = *reinterpret_cast<const bf16x8*>(src + j * 16);
-    // waited for here: the compiler would wait where they are first used, inside the loop, and so in every
-    // stage for the loads of the next one, which it does not know of
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(qf[j]));
+    for (int j = 0; j < NJ; ++j) qf[c][j] = *reinterpret_cast<const bf16x8*>(src + j * 32);
   }
+  // waited for here: the compiler would wait where they are first used, inside the loop, and so in every
+  // stage for the loads of the next one, which it does not know of
+#pragma unroll
+  for (int c = 0; c < kQT; ++c)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(qf[c][j]));
   const bool wave_has_rows = wrow0 < rows;
   const bool wave_full = wrow0 + kWaveTokens <= rows;                 // all 32 rows exist
   const int wave_first_pos = pos0 + wrow0;
@@ -161,11 +156,6 @@ __global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) voi
   const float scale_log2 = scale * 1.4426950408889634f;               // softmax in base 2: exp(x) = 2^(x log2 e)
   const float cap_log2 = softcap * 1.4426950408889634f;               // capped scores: cap * tanh(score / cap), in base-2 units
   const float scale_by_cap = softcap > 0.f ? scale / softcap : 0.f;
-  // Scores are scaled where the reference is taken off (one multiply-add) and the maximum is taken of unscaled ones,
-  // unless they are capped or a scale that is not positive would turn their order.
-  const bool scaled_first = softcap > 0.f || !(scale > 0.f);
-  const float sc = scaled_first ? 1.0f : scale_log2;
-
   // Stages are WAVES 16-key blocks aligned to absolute positions; blocks count from the sequence's start.
   const int first = first_key(pos0);                // the first key of the tile's first row
   const int b_first_seen = first >> 4;
@@ -193,13 +183,13 @@ __global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) voi
 #pragma unroll
   for (int n = 0; n < KL; ++n) {
     const int f = n * kWave + lane, lrow = f / CH, piece = f % CH;
-    k_off[n] = (uint32_t)(k_key(lrow) * HD + (piece ^ k_swizzle<HD>(lrow)) * 8) * 2;
+    k_off[n] = (uint32_t)(lrow * HD + (piece ^ k_swizzle<HD>(lrow)) * 8) * 2;
   }
-  uint32_t v_off[ND];
+  uint32_t v_off[VL];
 #pragma unroll
-  for (int n = 0; n < ND; ++n) {
+  for (int n = 0; n < VL; ++n) {
     const int d = n * 32 + (lane >> 1);
-    v_off[n] = (uint32_t)(min(d, VD - 1) * page_size + ((lane & 1) ^ v_swizzle(d)) * 8) * 2;
+    v_off[n] = (uint32_t)(min(d, VD - 1) * page_size + (lane & 1) * 8) * 2;
   }
   const uint32_t lds0 = lds_address(smem);
   auto fetch = [&](int bb, int page_raw, int buf) {   // 16-key block bb, of the page that page_at gave
@@ -212,99 +202,131 @@ __global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) voi
 #pragma unroll
     for (int n = 0; n < KL; ++n) load_to_lds(kr, k_off[n], 0, at + w * KB + n * 1024);
 #pragma unroll
-    for (int n = 0; n < ND; ++n) load_to_lds(vr, v_off[n], 0, at + WAVES * KB + w * VB + n * 1024);
+    for (int n = 0; n < VL; ++n) load_to_lds(vr, v_off[n], 0, at + WAVES * KB + w * VB + n * 1024);
   };
 
-  // where this lane reads its operands (bytes): piece 2j + g of key row r, half g of value column r
-  constexpr int KX = HD % 128 == 0 ? 8 : HD % 64 == 0 ? 4 : 2;        // different XORed places; further ones lie 32 * KX bytes on
-  int k_at[KX];
+  // where this lane reads its operands (bytes): piece 4j + g of key row r, keys 4g .. 4g + 3 of value column r
+  int k_at[NJ];
 #pragma unroll
-  for (int j = 0; j < KX; ++j) k_at[j] = r * HD * 2 + ((2 * j + g) ^ k_swizzle<HD>(r)) * 16;
-  const int v_at = WAVES * KB + r * 32 + (g ^ v_swizzle(r)) * 16;
+  for (int j = 0; j < NJ; ++j) k_at[j] = r * HD * 2 + ((4 * j + g) ^ k_swizzle<HD>(r)) * 16;
+  const int v_at = WAVES * KB + r * 32 + g * 8;
 
-  float m = kNoMax, l = 0.f;
-  f32x16 acc[ND];
+  float m[kQT], l[kQT];
+  f32x4 acc[kQT][ND];
 #pragma unroll
-  for (int d = 0; d < ND; ++d)
+  for (int c = 0; c < kQT; ++c) {
+    m[c] = kNoMax;
+    l[c] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[d][i] = 0.f;
+    for (int d = 0; d < ND; ++d) acc[c][d] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
 
   // One 32-key chunk: keys (b0 << 4) .. + 31, chunk `sub` of the stage in the buffer at `buf`.
   auto chunk = [&](int b0, const char* buf, auto sub_tag, bool whole) {
     constexpr int sub = decltype(sub_tag)::value;
-    f32x16 s;
+    f32x4 s[kQT][2];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) s[i] = 0.f;
+    for (int u = 0; u < 2; ++u) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const bf16x8 kf = *reinterpret_cast<const bf16x8*>(buf + k_at[j % KX] + (j / KX) * 32 * KX + sub * 2 * KB);
-      s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[j], s, 0, 0, 0);
-    }
-    // the lane holds S^T[key = 16 * (b0 + i / 8) + 8g + i % 8][query row r]
-    if (scaled_first) {
-      if (softcap > 0.f) {
+      for (int c = 0; c < kQT; ++c) s[c][u] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = cap_log2 * tanhf(s[i] * scale_by_cap);
-      } else {
+      for (int j = 0; j < NJ; ++j) {
+        const bf16x8 kf = *reinterpret_cast<const bf16x8*>(buf + k_at[j] + (sub * 2 + u) * KB);
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] *= scale_log2;
+        for (int c = 0; c < kQT; ++c) s[c][u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[c][j], s[c][u], 0, 0, 0);
       }
+    }
+    // the lane holds S^T[key = 16 * (b0 + u) + 4g + i][query row c * 16 + r]; scores go to base-2 units
+    if (softcap > 0.f) {
+#pragma unroll
+      for (int c = 0; c < kQT; ++c)
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) s[c][u][i] = cap_log2 * tanhf(s[c][u][i] * scale_by_cap);
+    } else {
+#pragma unroll
+      for (int c = 0; c < kQT; ++c)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) s[c][u] *= scale_log2;
     }
     if (!whole) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int key = (b0 << 4) + 16 * (i >> 3) + 8 * g + (i & 7);
-        const bool ok = qok && (key >= qstart || key < keep) && key <= qpos;
-        s[i] = ok ? s[i] : -INFINITY;
-      }
-    }
-    float lm = s[0];
+      for (int c = 0; c < kQT; ++c)
 #pragma unroll
-    for (int i = 1; i < 16; ++i) lm = fmaxf(lm, s[i]);
-    lm *= sc;
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int key = ((b0 + u) << 4) + 4 * g + i;
+            const bool ok = qok[c] && (key >= qstart[c] || key < keep) && key <= qpos[c];
+            s[c][u][i] = ok ? s[c][u][i] : -INFINITY;
+          }
+    }
+    float lmax[kQT];
+    bool grown = false;
+#pragma unroll
+    for (int c = 0; c < kQT; ++c) {
+      float lm = s[c][0][0];
+#pragma unroll
+      for (int x = 1; x < 8; ++x) lm = fmaxf(lm, s[c][x >> 2][x & 3]);
+      lmax[c] = lm;
+      grown = grown || lm - m[c] > kLazyMax;
+    }
     // m is a reference, not the running maximum: a row moves it only when the chunk's largest
     // score lies more than kLazyMax (base-2 units) above it.  Probabilities then reach 2^kLazyMax
     // at most, which float sums carry easily.  Most chunks move no row of the wave: they need
-    // no exchange between lanes and no rescaling.  The rule is the row's own (its two lanes
+    // no exchange between lanes and no rescaling.  The rule is the row's own (its four lanes
     // hold the same m and, once exchanged, the same maximum), so what a row ends up with does
     // not depend on the rows it shares a wave with.
-    if (__builtin_amdgcn_ballot_w64(lm - m > kLazyMax) != 0) {   // wave-uniform
-      const float cm = fmaxf(lm, __shfl_xor(lm, 32, kWave));
-      const bool move = cm - m > kLazyMax;
-      const float corr = move ? __builtin_amdgcn_exp2f(m - cm) : 1.0f;
-      m = move ? cm : m;
-      l *= corr;
+    if (__builtin_amdgcn_ballot_w64(grown) != 0) {   // wave-uniform
 #pragma unroll
-      for (int d = 0; d < ND; ++d) acc[d] *= corr;
+      for (int c = 0; c < kQT; ++c) {
+        float cm = lmax[c];
+        cm = fmaxf(cm, __shfl_xor(cm, 16, kWave));
+        cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
+        const bool move = cm - m[c] > kLazyMax;
+        const float corr = move ? __builtin_amdgcn_exp2f(m[c] - cm) : 1.0f;
+        m[c] = move ? cm : m[c];
+        l[c] *= corr;
+#pragma unroll
+        for (int d = 0; d < ND; ++d) acc[c][d] *= corr;
+      }
     }
-    u32x4 pf[2];
+    u32x4 pf[kQT];
 #if SHARPI_PREFILL_P_PAIR
-    u32x4 pf_lo[2];
+    u32x4 pf_lo[kQT];
 #endif
-    float ls = 0.f;
 #pragma unroll
-    for (int i = 0; i < 16; i += 2) {
-      const float e0 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i], sc, -m));       // masked: 2^-inf = 0
-      const float e1 = __builtin_amdgcn_exp2f(__builtin_fmaf(s[i + 1], sc, -m));
-      ls += e0;
-      ls += e1;
-      const uint32_t hi = bf16_pair(e0, e1);                                       // round to nearest even
-      pf[i >> 3][(i & 7) >> 1] = hi;
+    for (int c = 0; c < kQT; ++c) {
+      float ls = 0.f;
+#pragma unroll
+      for (int x = 0; x < 8; x += 2) {
+        const float e0 = __builtin_amdgcn_exp2f(s[c][x >> 2][x & 3] - m[c]);              // masked: 2^-inf = 0
+        const float e1 = __builtin_amdgcn_exp2f(s[c][x >> 2][(x & 3) + 1] - m[c]);
+        ls += e0;
+        ls += e1;
+        const uint32_t hi = bf16_pair(e0, e1);                                            // round to nearest even
+        pf[c][x >> 1] = hi;
 #if SHARPI_PREFILL_P_PAIR
-      pf_lo[i >> 3][(i & 7) >> 1] = bf16_pair(e0 - __uint_as_float(hi << 16), e1 - __uint_as_float(hi & 0xffff0000u));
-#endif
-    }
-    l += ls;
-#pragma unroll
-    for (int u = 0; u < 2; ++u)
-#pragma unroll
-      for (int d = 0; d < ND; ++d) {
-        const bf16x8 vf = *reinterpret_cast<const bf16x8*>(buf + v_at + (sub * 2 + u) * VB + d * 1024);
-        acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8, pf[u]), acc[d], 0, 0, 0);
-#if SHARPI_PREFILL_P_PAIR
-        acc[d] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, __builtin_bit_cast(bf16x8, pf_lo[u]), acc[d], 0, 0, 0);
+        pf_lo[c][x >> 1] = bf16_pair(e0 - __uint_as_float(hi << 16), e1 - __uint_as_float(hi & 0xffff0000u));
 #endif
       }
+      l[c] += ls;
+    }
+#pragma unroll
+    for (int d = 0; d < ND; ++d) {
+      // lane (column r, group g): keys 4g..4g+3 of the chunk's first block, then of its second
+      const uint2 v0 = *reinterpret_cast<const uint2*>(buf + v_at + (sub * 2) * VB + d * 512);
+      const uint2 v1 = *reinterpret_cast<const uint2*>(buf + v_at + (sub * 2 + 1) * VB + d * 512);
+      const bf16x8 vf = __builtin_bit_cast(bf16x8, u32x4{v0.x, v0.y, v1.x, v1.y});
+#pragma unroll
+      for (int c = 0; c < kQT; ++c) {
+        acc[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8, pf[c]), acc[c][d], 0, 0, 0);
+#if SHARPI_PREFILL_P_PAIR
+        acc[c][d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf, __builtin_bit_cast(bf16x8, pf_lo[c]), acc[c][d], 0, 0, 0);
+#endif
+      }
+    }
   };
 
   int b_next = after(b_first);
@@ -340,39 +362,41 @@ __global__ __launch_bounds__(WAVES* kWave, (prefill_waves_a_simd<HD, VD>())) voi
     b_next = b_two;
   }
 
-  float L = l + __shfl_xor(l, 32, kWave);
-  if (!qok) return;
-  // a key of score 0 (or of the head's learned score) without a value: 2^(score log2 e - reference) more
-  if (sink) L += __builtin_amdgcn_exp2f((sink_vals ? sink_vals[h] * 1.4426950408889634f : 0.f) - m);
-  float inv = L > 0.f ? 1.0f / L : 0.f;
-  const size_t token = tok0 + row;
-  if (gate) inv *= 1.0f / (1.0f + expf(-bf16_to_f32(gate[token * gate_stride + h])));
-  bf16_t* orow = out + (token * nh + h) * VD;
 #pragma unroll
-  for (int d = 0; d < ND; ++d)
+  for (int c = 0; c < kQT; ++c) {
+    float L = l[c];
+    L += __shfl_xor(L, 16, kWave);
+    L += __shfl_xor(L, 32, kWave);
+    if (!qok[c]) continue;
+    // a key of score 0 (or of the head's learned score) without a value: 2^(score log2 e - reference) more
+    if (sink) L += __builtin_amdgcn_exp2f((sink_vals ? sink_vals[h] * 1.4426950408889634f : 0.f) - m[c]);
+    float inv = L > 0.f ? 1.0f / L : 0.f;
+    const size_t token = tok0 + wrow0 + c * 16 + r;
+    if (gate) inv *= 1.0f / (1.0f + expf(-bf16_to_f32(gate[token * gate_stride + h])));
+    bf16_t* orow = out + (token * nh + h) * VD;
 #pragma unroll
-    for (int i = 0; i < 16; i += 4) {
-      // the lane holds O^T[32d + 8 * (i / 4) + 4g + 0..3][query row r]
-      const int col = d * 32 + 2 * i + 4 * g;
-      if (VD % 32 != 0 && col >= VD) continue;
+    for (int d = 0; d < ND; ++d) {
+      // lane holds O^T[d*16 + 4g + i][query row]
+      const f32x4 o = acc[c][d] * inv;
       uint2 packed;
-      packed.x = (uint32_t)f32_to_bf16(acc[d][i] * inv).bits | ((uint32_t)f32_to_bf16(acc[d][i + 1] * inv).bits << 16);
-      packed.y = (uint32_t)f32_to_bf16(acc[d][i + 2] * inv).bits | ((uint32_t)f32_to_bf16(acc[d][i + 3] * inv).bits << 16);
-      *reinterpret_cast<uint2*>(orow + col) = packed;
+      packed.x = (uint32_t)f32_to_bf16(o[0]).bits | ((uint32_t)f32_to_bf16(o[1]).bits << 16);
+      packed.y = (uint32_t)f32_to_bf16(o[2]).bits | ((uint32_t)f32_to_bf16(o[3]).bits << 16);
+      *reinterpret_cast<uint2*>(orow + d * 16 + 4 * g) = packed;
     }
+  }
 }
 
 template <int HD, int VD>
 static int launch_prefill(const PrefillArgs& a, hipStream_t stream) {
   dim3 grid(a.nh, a.n_tiles);
-#define PRE_WAVES(W)                                                                                                     \
-  attn_prefill_kernel<HD, VD, W><<<grid, W * kWave, 0, stream>>>(                                                       \
+#define PRE_QT(QTV)                                                                                                     \
+  attn_prefill_kernel<HD, VD, QTV><<<grid, kPreWaves * kWave, 0, stream>>>(                                                    \
       (const bf16_t*)a.q, (const bf16_t*)a.k_cache, (const bf16_t*)a.v_cache, a.block_table, a.positions, a.tiles,        \
       (bf16_t*)a.out, a.window_kind, a.window, a.scale, a.nh, a.nkv, a.page_size, a.max_blocks, a.num_pages, a.softcap,   \
       a.sink, a.sink_vals, a.keep, (const bf16_t*)a.gate, a.gate_stride)
-  if (a.tile_tokens == kTileTokens) PRE_WAVES(kPreWaves);
-  else PRE_WAVES(kPreWaves / 2);
-#undef PRE_WAVES
+  if (a.tile_tokens == kTileTokens) PRE_QT(2);
+  else PRE_QT(1);
+#undef PRE_QT
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
 }
