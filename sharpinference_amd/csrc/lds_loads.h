@@ -18,15 +18,19 @@ __device__ __forceinline__ uint32_t lds_address(const char* p) {
   return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const char*)p;
 }
 // Lane l's 16 bytes at offset + step (step and lds the same for all lanes) go to LDS byte lds + 16 l (the instruction takes the LDS
-// address from m0).  STREAM: with the streaming hint, for data that nobody else reads.
+// address from m0: an operand, so that the compiler knows what m0 holds).  STREAM: with the streaming hint, for data that nobody else
+// reads.  The compiler keeps dependent instructions apart where the hardware does not, but does not look inside the statement.  Two
+// such distances end at this load: five wait states from a vector instruction that writes a scalar register (readfirstlane, or a
+// spilled scalar read back from a lane) to a memory instruction that reads it as descriptor or step, and one from a write of m0.
+// s_nop 4 is five.
 template <bool STREAM = false>
 __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t offset, uint32_t step, uint32_t lds) {
   lds = __builtin_amdgcn_readfirstlane(lds);
   step = __builtin_amdgcn_readfirstlane(step);
   if constexpr (STREAM)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"s"(lds), "v"(offset), "s"(rsrc), "s"(step) : "memory");
+    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"{m0}"(lds), "v"(offset), "s"(rsrc), "s"(step) : "memory");
   else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(offset), "s"(rsrc), "s"(step) : "memory");
+    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(offset), "s"(rsrc), "s"(step) : "memory");
 }
 template <int LEFT = 0> __device__ __forceinline__ void lds_loads_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory");
