@@ -7,21 +7,27 @@
 // border between s and t: D_ts = (product from the border to t) (product from s + 1 to the border), both at most 1.  A wave
 // has 16 tokens in registers (lane (i, g): a quarter of token i's channels); inside them the borders are those of halves of 2, 4,
 // 8 and 16 tokens, a product of the 16 x 16 tile each, of which the pairs with that border are kept (X: from the start of the
-// token's half, Y: behind the token to its end; both double their reach by exchanges inside 16 lanes).  Between the waves' tokens the
-// border is the later block's start: keys times Y lie in LDS for all, queries times X take on the decays of the blocks
-// between from block to block.
+// token's half, Y: behind the token to its end; both double their reach by the product of the other half's decays).  Between the
+// waves' tokens the border is the later block's start: keys times Y lie in LDS for all, queries times X take on the decays of the
+// blocks between from block to block.
 //
-// Decays, products of them, scores and states are float as in the walk (v_mfma_f32_16x16x4_f32); what is summed over tokens or over a
+// Decays, scores and states are float as in the walk (v_mfma_f32_16x16x4_f32); what is summed over tokens or over a
 // state is summed in double (v_mfma_f64_16x16x4_f64: products of floats are exact, half the rate; with float sums the errors
 // against 64 bits were 1.1 to 3 times the walk's, whose sums are short).  Scores come transposed (keys down, queries across) and are the next product's operand in their registers; the columns of values are dealt to the
 // tiles so that a lane's reads of values and states are four neighbours.  A zero weight times a value that is no number
 // would spoil earlier tokens: where a wave's tokens hold one, their own pairs are summed one by one.
 //
-// Bound: one block a unit (100 KB of LDS) and what its waves do one after the other: 0.3 k double products of 64 cycles and 0.3 k
-// float ones of 32 a wave, the exchanges, and the registers: queries, keys, X, Y and the halves' products fill 160 of 256, so that
-// outputs of 128 columns spill a hundred.  All launches of a call, us before (the walk's phases) and now: 16 heads of 128 x 128, 1,900
-// tokens 224 -> 124 (32 local, 5 between, 78 outputs), 512 tokens 113 -> 109; 32 heads, 4,096 tokens 727 -> 481; 16 heads of 64 x 64, two
-// of 1,024 79 -> 48.  Errors against 64 bits, 1,900 tokens: outputs 1.25e-7 -> 1.14e-7, state 7.9e-8 -> 6.9e-8.
+// The products of decays are formed in double and rounded once: of halves for X and Y, of blocks for the queries on their way, of a whole
+// segment for its state, which keeps them in double.  A product of floats 1 - a and 1 - b drops a b where that is less than half a
+// place of the result, always to the same side: with products of floats, doubled from pairs on, the state's error after 1,900
+// tokens of decays 1 - 2e-4 was 1.7e-5 (the walk's 7.5e-7, now 1.7e-7), of decays about 1 - 2.5e-4 1.07e-6 (5.3e-7, now 8.6e-8).
+//
+// Bound: what a block's waves do one after the other, and how many blocks a unit holds.  A wave makes, for 128 x 128, 400 double
+// products of 64 cycles on average (32 a block of tokens up to its own, 256 for the state) and 270 float ones of 32; outputs of 128
+// key channels keep 28 to 41 of their 256 registers a lane in scratch, those of 64 none.  LDS: 608 bytes a key channel and 256 or 512
+// (float) a value column, 59 KB (bf16, 64 x 64: two blocks a unit) to 152 (float, 128 x 128).  All launches of a call, bf16, us of the
+// walk's phases and of the products: 16 heads of 128 x 128, 1,900 tokens 216 -> 115, 512 tokens 110 -> 104; 32 heads, 4,000 tokens 711 ->
+// 382; 16 heads of 64 x 64, two of 600 72 -> 40.  Errors against 64 bits, 1,900 tokens: outputs 1.25e-7 -> 1.07e-7, state 7.7e-8 -> 4.6e-8.
 #include "gla_chunk.h"
 
 #include <type_traits>
@@ -35,10 +41,9 @@ constexpr int kSliceCols = 8;            // value columns of a state slice (line
 
 __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
 
-// the value of the lane in the neighbouring half of 2 H lanes (of any of its lanes: the value is the same in a half)
-template <int H> __device__ __forceinline__ float other_half(float x) {
-  constexpr int ctrl = H == 1 ? 0xB1 : H == 2 ? 0x4E : H == 4 ? 0x141 : 0x140;      // quad permutations, mirrors of 8 and 16 lanes
-  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), ctrl, 0xF, 0xF, true));
+// the neighbouring lane's value
+__device__ __forceinline__ float neighbour(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, true));
 }
 
 // A score is eight chains of channels: a sum's rounding grows with its length.
@@ -67,9 +72,12 @@ template <typename T, int DK, int DV, bool FINAL>
 __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs a) {
   constexpr int CH = DK / 4, RPL = DK / 8, NH = DV / 64, NT = DV / 16;
   constexpr int LDV = DV + 16;
-  __shared__ __attribute__((aligned(16))) float ks[kSeg][DK];          // keys times Y; 16-byte pieces swizzled (k_piece)
+  // keys times Y; before, of every block of 16 tokens the products of the decays of its pairs (rows 0 .. 7 of the block), fours (8 .. 11)
+  // and eights (12, 13); 16-byte pieces swizzled (k_piece)
+  __shared__ __attribute__((aligned(16))) float ks[kSeg][DK];
   __shared__ __attribute__((aligned(16))) T vs[kSeg][LDV];
-  __shared__ __attribute__((aligned(16))) float bt[kGlaWaves][DK];     // the products of the blocks' decays
+  __shared__ __attribute__((aligned(16))) float bt[kGlaWaves][DK];     // the products of the blocks' decays,
+  __shared__ double bd[kGlaWaves][DK];                                 // and before they are rounded
   __shared__ int odd[kGlaWaves];                                       // whether a block's values hold one that is no number
   const int seg = blockIdx.x, h = blockIdx.y;
   const int e = a.segs[4 * seg], t0 = a.segs[4 * seg + 1], nt = min(a.segs[4 * seg + 2], kSeg);
@@ -85,12 +93,39 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
   const int t = I * kBlockTokens + i;
   const bool live = t < nt;
   const size_t row = (size_t)(t0 + min(t, nt - 1));
+  // a block's decays of one channel a thread, for their products
+  constexpr int COLUMNS = kGlaWaves * DK / kGlaThreads;
+  float f[COLUMNS][kBlockTokens];
+#pragma unroll
+  for (int n = 0; n < COLUMNS; ++n) {
+    const int J = (tid + n * kGlaThreads) / DK, ch = tid % DK;
+#pragma unroll
+    for (int x = 0; x < kBlockTokens; ++x) {
+      const int tx = J * kBlockTokens + x;
+      f[n][x] = a.alpha[(size_t)(t0 + min(tx, nt - 1)) * (size_t)(a.nh * DK) + h * DK + ch];
+      f[n][x] = tx < nt ? f[n][x] : 1.f;
+    }
+  }
   float k[CH], X[CH], Y[CH], q[FINAL ? CH : 1];
 #pragma unroll
   for (int m = 0; m < CH; m += 8) {
     load8(proj + row * a.stride + a.k_off + h * DK + CH * g + m, k + m);
     load8(a.alpha + row * (size_t)(a.nh * DK) + h * DK + CH * g + m, X + m);
     if constexpr (FINAL) load8(proj + row * a.stride + a.q_off + h * DK + CH * g + m, q + m);
+  }
+#pragma unroll
+  for (int n = 0; n < COLUMNS; ++n) {
+    const int J = (tid + n * kGlaThreads) / DK, ch = tid % DK;
+    auto put = [&](int node, double d) { ks[J * kBlockTokens + node][k_piece(node, ch >> 2) * 4 + (ch & 3)] = (float)d; };
+    double d[8];
+#pragma unroll
+    for (int x = 0; x < 8; ++x) put(x, d[x] = (double)f[n][2 * x] * (double)f[n][2 * x + 1]);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) put(8 + x, d[x] = d[2 * x] * d[2 * x + 1]);
+#pragma unroll
+    for (int x = 0; x < 2; ++x) put(12 + x, d[x] = d[2 * x] * d[2 * x + 1]);
+    bd[J][ch] = d[0] * d[1];
+    bt[J][ch] = (float)(d[0] * d[1]);
   }
   __syncthreads();
   // values into LDS
@@ -110,13 +145,11 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
     }
     if (bad) odd[tv / kBlockTokens] = 1;
   }
-  float tot[CH];
 #pragma unroll
   for (int m = 0; m < CH; ++m) {
     k[m] = live ? k[m] : 0.f;
     X[m] = live ? X[m] : 1.f;
     Y[m] = 1.f;
-    tot[m] = X[m];
     if constexpr (FINAL) q[m] = live ? q[m] * a.q_scale : 0.f;
   }
   // the pairs of the wave's own tokens: lane (i, g) gets query i with keys 4 g + 0..3
@@ -152,13 +185,18 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
       }
     }
     const bool up = i & H;
+    const int node = (H == 2 ? 0 : H == 4 ? 8 : 12) + ((i / H) ^ 1);   // the other half
 #pragma unroll
-    for (int m = 0; m < CH; ++m) {
-      const float p = other_half<H>(tot[m]);
-      X[m] *= up ? p : 1.f;
-      Y[m] *= up ? 1.f : p;
-      tot[m] *= p;
-      asm volatile("" : "+v"(X[m]), "+v"(Y[m]), "+v"(tot[m]));         // (one channel after the other, for the registers' sake)
+    for (int m = 0; m < CH; m += 4) {
+      f32x4 p;
+      if constexpr (H == 1) p = f32x4{neighbour(X[m]), neighbour(X[m + 1]), neighbour(X[m + 2]), neighbour(X[m + 3])};
+      else p = *reinterpret_cast<const f32x4*>(&ks[I * kBlockTokens + node][k_piece(node, (CH * g + m) / 4) * 4]);
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        X[m + x] *= up ? p[x] : 1.f;
+        Y[m + x] *= up ? 1.f : p[x];
+        asm volatile("" : "+v"(X[m + x]), "+v"(Y[m + x]));             // (a few channels after the others, for the registers' sake)
+      }
     }
   };
   level(std::integral_constant<int, 1>{});
@@ -168,7 +206,6 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
 #pragma unroll
   for (int m = 0; m < CH; m += 4) {
     *reinterpret_cast<f32x4*>(&ks[t][k_piece(t, (CH * g + m) / 4) * 4]) = f32x4{k[m] * Y[m], k[m + 1] * Y[m + 1], k[m + 2] * Y[m + 2], k[m + 3] * Y[m + 3]};
-    if (i == 0) *reinterpret_cast<f32x4*>(&bt[I][CH * g + m]) = f32x4{tot[m], tot[m + 1], tot[m + 2], tot[m + 3]};
   }
   __syncthreads();
 
@@ -269,18 +306,18 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
     f64x4 acc[4];
 #pragma unroll
     for (int c = 0; c < 4; ++c) acc[c] = f64x4{0.0, 0.0, 0.0, 0.0};
-    float keep = 1.f;                                                  // the decays of the blocks behind J
+    double keep = 1.0;                                                 // the decays of the blocks behind J
     for (int J = blocks - 1; J >= 0; --J) {
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
         const int tk = J * kBlockTokens + 4 * u + g;
-        const float kv = ks[tk][k_piece(tk, ch >> 2) * 4 + (ch & 3)] * keep;
+        const double kv = (double)ks[tk][k_piece(tk, ch >> 2) * 4 + (ch & 3)] * keep;
         float v[4];
         read4<T>(&vs[tk][64 * hi + 4 * i], v);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) acc[c] = mfma4((double)v[c], (double)kv, acc[c]);
+        for (int c = 0; c < 4; ++c) acc[c] = mfma4((double)v[c], kv, acc[c]);
       }
-      keep *= bt[J][ch];
+      keep *= bd[J][ch];
     }
 #pragma unroll
     for (int v = 0; v < 4; ++v) {
@@ -289,11 +326,11 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
       if constexpr (FINAL) {
         const f32x4 s0 = *reinterpret_cast<const f32x4*>(S_seg + at);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) s[c] += (double)keep * (double)s0[c];
+        for (int c = 0; c < 4; ++c) s[c] += keep * (double)s0[c];
       }
       *reinterpret_cast<f32x4*>(S_to + at) = f32x4{(float)s[0], (float)s[1], (float)s[2], (float)s[3]};
     }
-    if (!FINAL && hi == 0 && g == 0) a.seg_decay[((size_t)seg * a.nh + h) * DK + ch] = keep;
+    if (!FINAL && hi == 0 && g == 0) a.seg_decay[((size_t)seg * a.nh + h) * DK + ch] = (float)keep;
   }
 }
 
