@@ -24,10 +24,10 @@
 //
 // Bound: what a block's waves do one after the other, and how many blocks a unit holds.  A wave makes, for 128 x 128, 400 double
 // products of 64 cycles on average (32 a block of tokens up to its own, 256 for the state) and 270 float ones of 32; outputs of 128
-// key channels keep 28 to 41 of their 256 registers a lane in scratch, those of 64 none.  LDS: 608 bytes a key channel and 256 or 512
+// key channels keep 34 to 48 of their 256 registers a lane in scratch, those of 64 none.  LDS: 608 bytes a key channel and 256 or 512
 // (float) a value column, 59 KB (bf16, 64 x 64: two blocks a unit) to 152 (float, 128 x 128).  All launches of a call, bf16, us of the
-// walk's phases and of the products: 16 heads of 128 x 128, 1,900 tokens 216 -> 115, 512 tokens 110 -> 104; 32 heads, 4,000 tokens 711 ->
-// 382; 16 heads of 64 x 64, two of 600 72 -> 40.  Errors against 64 bits, 1,900 tokens: outputs 1.25e-7 -> 1.07e-7, state 7.7e-8 -> 4.6e-8.
+// walk's phases and of the products: 16 heads of 128 x 128, 1,900 tokens 216 -> 116, 512 tokens 110 -> 105; 32 heads, 4,000 tokens 711 ->
+// 386; 16 heads of 64 x 64, two of 600 72 -> 41.  Errors against 64 bits, 1,900 tokens: outputs 1.25e-7 -> 1.07e-7, state 7.7e-8 -> 4.6e-8.
 #include "gla_chunk.h"
 
 #include <type_traits>
@@ -66,10 +66,10 @@ template <typename T> __device__ __forceinline__ void read4(const T* p, float* v
   }
 }
 
-// FINAL: outputs, and the state in its slot where the segment is its entry's last; else what the segment makes of nothing and
-// the product of its decays.
+// Tokens t0 .. t0 + nt - 1 (kSeg at most) of segment `seg`: `begins` and `ends` where they are its first and its last, `last` where the
+// segment is its entry's last.
 template <typename T, int DK, int DV, bool FINAL>
-__global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs a) {
+__device__ __forceinline__ void gla_chunk(const GlaChunkArgs& a, int seg, int h, int e, int t0, int nt, bool begins, bool ends, bool last) {
   constexpr int CH = DK / 4, RPL = DK / 8, NH = DV / 64, NT = DV / 16;
   constexpr int LDV = DV + 16;
   // keys times Y; before, of every block of 16 tokens the products of the decays of its pairs (rows 0 .. 7 of the block), fours (8 .. 11)
@@ -79,11 +79,9 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
   __shared__ __attribute__((aligned(16))) float bt[kGlaWaves][DK];     // the products of the blocks' decays,
   __shared__ double bd[kGlaWaves][DK];                                 // and before they are rounded
   __shared__ int odd[kGlaWaves];                                       // whether a block's values hold one that is no number
-  const int seg = blockIdx.x, h = blockIdx.y;
-  const int e = a.segs[4 * seg], t0 = a.segs[4 * seg + 1], nt = min(a.segs[4 * seg + 2], kSeg);
-  const bool last = a.segs[4 * seg + 3] != 0;
-  if (!FINAL && last) return;                                          // (nobody reads it)
-  const int tid = threadIdx.x, lane = tid & (kWave - 1), wid = tid >> 6, i = lane & 15, g = lane >> 4;
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));        // (a chunk's addresses are formed in it: kept from one to the next they would fill the registers)
+  const int lane = tid & (kWave - 1), wid = __builtin_amdgcn_readfirstlane(tid >> 6), i = lane & 15, g = lane >> 4;
   const f32x4 zero = f32x4{0.f, 0.f, 0.f, 0.f};
   const int I = wid < 4 ? wid : 11 - wid;                              // blocks of 16 tokens: waves of one SIMD get an early and a late one
   auto k_piece = [](int t, int piece) { return piece ^ (t & 7); };
@@ -92,7 +90,7 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
   const T* proj = (const T*)a.proj;
   const int t = I * kBlockTokens + i;
   const bool live = t < nt;
-  const size_t row = (size_t)(t0 + min(t, nt - 1));
+  const size_t row = (size_t)max(t0 + min(t, nt - 1), 0);              // (no token: one that exists, unused)
   // a block's decays of one channel a thread, for their products
   constexpr int COLUMNS = kGlaWaves * DK / kGlaThreads;
   float f[COLUMNS][kBlockTokens];
@@ -102,7 +100,7 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
 #pragma unroll
     for (int x = 0; x < kBlockTokens; ++x) {
       const int tx = J * kBlockTokens + x;
-      f[n][x] = a.alpha[(size_t)(t0 + min(tx, nt - 1)) * (size_t)(a.nh * DK) + h * DK + ch];
+      f[n][x] = a.alpha[(size_t)max(t0 + min(tx, nt - 1), 0) * (size_t)(a.nh * DK) + h * DK + ch];
       f[n][x] = tx < nt ? f[n][x] : 1.f;
     }
   }
@@ -296,12 +294,14 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
           *reinterpret_cast<f32x4*>(o + 64 * hi + 16 * v) = f32x4{(float)acc[4 * hi][v], (float)acc[4 * hi + 1][v], (float)acc[4 * hi + 2][v], (float)acc[4 * hi + 3][v]};
     }
   }
-  if (FINAL && !last) return;
+  const bool to_slot = FINAL && ends && last;
+  if (FINAL && ends && !last) return;
+  if (FINAL && !ends) __syncthreads();                                 // (the outputs above have read what is written below)
 
   // The state: a wave has 16 rows of it (two neighbouring places of all eight row groups) and 64 columns at a time.
   constexpr int RW = DK / 16;                                          // waves over the rows, the others over the columns
   const int r = 2 * (wid % RW) + (i >> 3), g8 = i & 7, ch = g8 * RPL + r;
-  float* S_to = FINAL ? a.state + ((size_t)a.state_slots[e] * a.nh + h) * seg_floats : S_seg;
+  float* S_to = to_slot ? a.state + ((size_t)a.state_slots[e] * a.nh + h) * seg_floats : S_seg;
   for (int hi = wid / RW; hi < NH; hi += kGlaWaves / RW) {
     f64x4 acc[4];
 #pragma unroll
@@ -323,14 +323,34 @@ __global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs 
     for (int v = 0; v < 4; ++v) {
       const size_t at = ((size_t)(8 * hi + 2 * v + (g >> 1)) * DK + r * 8 + g8) * kSliceCols + 4 * (g & 1);
       double s[4] = {acc[0][v], acc[1][v], acc[2][v], acc[3][v]};
-      if constexpr (FINAL) {
+      if (FINAL || !begins) {
         const f32x4 s0 = *reinterpret_cast<const f32x4*>(S_seg + at);
 #pragma unroll
         for (int c = 0; c < 4; ++c) s[c] += keep * (double)s0[c];
       }
       *reinterpret_cast<f32x4*>(S_to + at) = f32x4{(float)s[0], (float)s[1], (float)s[2], (float)s[3]};
     }
-    if (!FINAL && hi == 0 && g == 0) a.seg_decay[((size_t)seg * a.nh + h) * DK + ch] = (float)keep;
+    if (!FINAL && hi == 0 && g == 0) {
+      float* d = a.seg_decay + ((size_t)seg * a.nh + h) * DK + ch;
+      *d = begins ? (float)keep : (float)(keep * (double)*d);
+    }
+  }
+}
+
+// FINAL: outputs, and the state in its slot where the segment is its entry's last; else what the segment makes of nothing and
+// the product of its decays.  The step's own lists cut segments to kSeg tokens; a longer one, of a caller's own list, goes in
+// chunks of so many, the state between them where the segment's state is kept.
+template <typename T, int DK, int DV, bool FINAL>
+__global__ __launch_bounds__(kGlaThreads, 2) void gla_chunk_kernel(GlaChunkArgs a) {
+  const int seg = blockIdx.x, h = blockIdx.y;
+  const int e = a.segs[4 * seg], first = a.segs[4 * seg + 1], tokens = a.segs[4 * seg + 2];
+  const bool last = a.segs[4 * seg + 3] != 0;
+  if (!FINAL && last) return;                                          // (nobody reads it)
+  for (int done = 0;; done += kSeg) {
+    const bool ends = tokens - done <= kSeg;
+    gla_chunk<T, DK, DV, FINAL>(a, seg, h, e, first + done, ends ? max(tokens - done, 0) : kSeg, done == 0, ends, last);
+    if (ends) return;
+    __syncthreads();
   }
 }
 

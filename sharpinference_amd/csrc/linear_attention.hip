@@ -415,7 +415,7 @@ static int launch_segmented(const void* proj, int stride, int q_off, int k_off, 
 
 // The walk of gla_walk with long entries cut into segments that are walked side by side (see the head of
 // this file).  segs int [n_segs, 4] = (entry, first token of the step's rows, tokens, 1 if the entry's last
-// segment), an entry's segments consecutive and in order; ent_segs int [n_entries, 2] = (first segment,
+// segment), an entry's segments consecutive and in order, of any length (gla_segments cuts to 128 tokens); ent_segs int [n_entries, 2] = (first segment,
 // segments); seg_state float [n_segs, nh, ceil(dv / 8), DKP, 8] and seg_decay float [n_segs, nh, DKP]: scratch.
 SHARPI_EXPORT int sharpi_gla_walk_segmented(const void* proj, int dtype, int stride, int q_off, int k_off, int v_off,
                                             const float* alpha, float q_scale, float* state, const int* state_slots,

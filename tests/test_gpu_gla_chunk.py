@@ -118,3 +118,30 @@ def test_rows_off_the_borders_are_walked():
     want, left = run(proj, alpha, state, ctx, H, dk, dv, 8)
     got, st = run(torch.cat([proj[:, 5:], proj[:, :5]], 1).contiguous(), alpha, state, ctx, H, dk, dv, 3)
     assert float((got - want).abs().max()) <= 1e-5 * float(want.abs().max()) and float((st - left).abs().max()) <= 1e-5 * float(left.abs().max())
+
+
+@pytest.mark.parametrize("H, dk, dv", [(2, 128, 64), (1, 64, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("cuts", [[[129]], [[300], [0], [7]], [[128, 257, 31], [1]], [[400, 16], [128]]])
+def test_a_callers_own_segments_may_be_longer_than_a_chunk(cuts, dtype, H, dk, dv):
+    """Lists that ops.gla_segments would not make: segments of more tokens than a chunk, and of none."""
+    from sharpinference_amd import ops
+    lens, pad = [sum(c) for c in cuts], 8
+    proj, alpha, state = inputs(lens, H, dk, dv, pad, dtype, 16.0, sum(lens))
+    ctx = step(lens, list(range(len(lens))))
+    segs, ents = [], []
+    for e, c in enumerate(cuts):
+        ents.append((len(segs), len(c)))
+        for n, m in enumerate(c):
+            segs.append((e, int(ctx.cu[e]) + sum(c[:n]), m, int(n == len(c) - 1)))
+    lists = tuple(torch.tensor(x, dtype=torch.int32, device=DEV) for x in (segs, ents))
+    left = state.clone()
+    got = ops.gla_walk(proj, pad, pad + H * dk, pad + 2 * H * dk, alpha, dk ** -0.5, left, ctx, H, dk, dv, segments=lists)
+    want, want_left = run(proj, alpha, state, ctx, H, dk, dv, pad, segmented=False)
+    # both within 4e-7 of 64 bits (above), the largest of some thousand differences within 6 times that
+    for a, b in ((got, want), (left, want_left)):
+        assert float((a - b).abs().max()) <= 5e-6 * float(b.pow(2).mean().sqrt())
+    assert torch.equal(left[len(lens)], state[len(lens)])                # nobody's slot
+    for e, n in enumerate(lens):
+        if n == 0:
+            assert torch.equal(left[e], state[e])
