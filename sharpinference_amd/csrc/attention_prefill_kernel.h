@@ -85,7 +85,8 @@ __device__ __forceinline__ uint32_t bf16_pair(float lo, float hi) {
 template <int HD, int VD>
 constexpr int prefill_waves_a_simd() { return kPreWaves * 16 * (HD + (VD + 31) / 32 * 32) * 4 <= 80 * 1024 ? 2 : 1; }   // by the LDS two blocks need
 
-template <int HD, int VD, int kQT>
+// DIRECT: the caches begin at 16-byte addresses.
+template <int HD, int VD, int kQT, bool DIRECT>
 __global__ __launch_bounds__(kPreWaves* kWave, (prefill_waves_a_simd<HD, VD>())) void attn_prefill_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_cache, const bf16_t* __restrict__ v_cache,
     const int* __restrict__ block_table, const int* __restrict__ positions, const int* __restrict__ tiles,
@@ -200,9 +201,9 @@ __global__ __launch_bounds__(kPreWaves* kWave, (prefill_waves_a_simd<HD, VD>()))
     const u32x4 vr = buffer_of(v_cache + head * VD * page_size + off, (uint32_t)((VD - 1) * page_size + 16) * 2);
     const uint32_t at = lds0 + buf * STAGE;
 #pragma unroll
-    for (int n = 0; n < KL; ++n) load_to_lds(kr, k_off[n], 0, at + w * KB + n * 1024);
+    for (int n = 0; n < KL; ++n) bring_to_lds<DIRECT>(kr, k_off[n], 0, at + w * KB + n * 1024);
 #pragma unroll
-    for (int n = 0; n < VL; ++n) load_to_lds(vr, v_off[n], 0, at + WAVES * KB + w * VB + n * 1024);
+    for (int n = 0; n < VL; ++n) bring_to_lds<DIRECT>(vr, v_off[n], 0, at + WAVES * KB + w * VB + n * 1024);
   };
 
   // where this lane reads its operands (bytes): piece 4j + g of key row r, keys 4g .. 4g + 3 of value column r
@@ -389,13 +390,16 @@ __global__ __launch_bounds__(kPreWaves* kWave, (prefill_waves_a_simd<HD, VD>()))
 template <int HD, int VD>
 static int launch_prefill(const PrefillArgs& a, hipStream_t stream) {
   dim3 grid(a.nh, a.n_tiles);
-#define PRE_QT(QTV)                                                                                                     \
-  attn_prefill_kernel<HD, VD, QTV><<<grid, kPreWaves * kWave, 0, stream>>>(                                                    \
+#define PRE_QT(QTV, DIR)                                                                                                 \
+  attn_prefill_kernel<HD, VD, QTV, DIR><<<grid, kPreWaves * kWave, 0, stream>>>(                                                    \
       (const bf16_t*)a.q, (const bf16_t*)a.k_cache, (const bf16_t*)a.v_cache, a.block_table, a.positions, a.tiles,        \
       (bf16_t*)a.out, a.window_kind, a.window, a.scale, a.nh, a.nkv, a.page_size, a.max_blocks, a.num_pages, a.softcap,   \
       a.sink, a.sink_vals, a.keep, (const bf16_t*)a.gate, a.gate_stride)
-  if (a.tile_tokens == kTileTokens) PRE_QT(2);
-  else PRE_QT(1);
+  const bool direct = whole_pieces(a.k_cache, a.v_cache), full = a.tile_tokens == kTileTokens;
+  if (direct && full) PRE_QT(2, true);
+  else if (direct) PRE_QT(1, true);
+  else if (full) PRE_QT(2, false);
+  else PRE_QT(1, false);
 #undef PRE_QT
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;

@@ -15,10 +15,15 @@ SHARPI_EXPORT int sharpi_gemm_grouped(const void* x, int x_rows, const void* W, 
   if (!grouped_args_ok(x_rows, n_rows, N, K, n_groups, packed, group_offsets, plan)) return SHARPI_ERR_ARG;
   const int nb = ceil_div(N, columns_of(kMaxNT));
   const dim3 grid = grouped_grid(n_rows, n_groups, nb, max_blocks), block(GW * kWave);
-#define GG_LAUNCH(TOV, PK)                                                                                             \
-  grouped_gemm_kernel<TOV, kMaxNT, PK, false><<<grid, block, 0, stream>>>((const bf16_t*)x, grouped_x_bytes(x_rows, K), (const bf16_t*)W, (TOV*)out, \
-                                                                         N, K, a_rows, nullptr, GatedAct{0, 0.f}, relu2, group_offsets, plan, \
-                                                                         n_groups, nb)
+#define GG_FORM(TOV, PK, DIR)                                                                                             \
+  grouped_gemm_kernel<TOV, kMaxNT, PK, false, DIR><<<grid, block, 0, stream>>>((const bf16_t*)x, grouped_x_bytes(x_rows, K), (const bf16_t*)W, (TOV*)out, \
+                                                                              N, K, a_rows, nullptr, GatedAct{0, 0.f}, relu2, group_offsets, plan, \
+                                                                              n_groups, nb)
+#define GG_LAUNCH(TOV, PK)                 \
+  do {                                     \
+    if (whole_pieces(x, W)) GG_FORM(TOV, PK, true); \
+    else GG_FORM(TOV, PK, false);          \
+  } while (0)
   if (out_dtype == DT_BF16) {
     if (packed) GG_LAUNCH(bf16_t, true); else GG_LAUNCH(bf16_t, false);
   } else if (out_dtype == DT_F32) {
@@ -27,6 +32,7 @@ SHARPI_EXPORT int sharpi_gemm_grouped(const void* x, int x_rows, const void* W, 
     return SHARPI_ERR_ARG;
   }
 #undef GG_LAUNCH
+#undef GG_FORM
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
 }

@@ -69,8 +69,8 @@ static_assert(GM == 2 * 16 * 8, "tile heights are compiled in steps of 32 rows u
 // counter); with the exclusive or the sixteen pieces of a turn fall into the sixteen different 16-byte groups of the bank space.
 __device__ __forceinline__ int xs_piece(int row, int piece) { return piece ^ ((row >> 1) & 7); }
 
-// The work of one tile of up to MT * 32 rows against 16 * NT * GWC weight rows.
-template <typename TO, int MT, int NT, bool PACKED, bool ACT>
+// The work of one tile of up to MT * 32 rows against 16 * NT * GWC weight rows.  DIRECT: both operands begin at 16-byte addresses.
+template <typename TO, int MT, int NT, bool PACKED, bool ACT, bool DIRECT>
 __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint32_t x_bytes, const bf16_t* __restrict__ We,
                                              TO* __restrict__ out, int N, int K, const int* __restrict__ a_rows,
                                              const float* __restrict__ act_scale, GatedAct act, int relu2, int tile_row0, int row_end,
@@ -123,8 +123,8 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
       const uint32_t at = lds0 + (s & 3) * kWStep + w_tile[i] * 1024;
-      if (stream) load_to_lds<true>(wb, w_off[i], s * kWStepBytes, at);
-      else load_to_lds<false>(wb, w_off[i], s * kWStepBytes, at);
+      if (DIRECT && stream) load_to_lds<true>(wb, w_off[i], s * kWStepBytes, at);
+      else bring_to_lds<DIRECT>(wb, w_off[i], s * kWStepBytes, at);
     }
   };
   load_w(0);                                    // (on their way while the rows' places are looked up)
@@ -147,7 +147,7 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   for (int i = 0; i < XL; ++i) asm volatile("" : "+v"(x_off[i]));
   auto load_x = [&](int c) {                    // x rows of stage c
 #pragma unroll
-    for (int i = 0; i < XL; ++i) load_to_lds<false>(xb, x_off[i], c * (GK * 2), lds0 + kXAt + (c & 1) * kXStage + x_load[i] * 1024);
+    for (int i = 0; i < XL; ++i) bring_to_lds<DIRECT>(xb, x_off[i], c * (GK * 2), lds0 + kXAt + (c & 1) * kXStage + x_load[i] * 1024);
   };
   load_x(0);
 
@@ -284,7 +284,7 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   }
 }
 
-template <typename TO, int NT, bool PACKED, bool ACT>
+template <typename TO, int NT, bool PACKED, bool ACT, bool DIRECT>
 __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     const bf16_t* __restrict__ x, uint32_t x_bytes, const bf16_t* __restrict__ W, TO* __restrict__ out, int N, int K,
     const int* __restrict__ a_rows, const float* __restrict__ act_scale, GatedAct act, int relu2,
@@ -356,7 +356,7 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     const int total = __builtin_amdgcn_readfirstlane(s_total[xcd]);   // slots of this walk
     const int whole = total / per_xcd * per_xcd;   // slots of whole rounds: taken as they are
     const int rest = total - whole;
-    const int cut = rest > 0 ? 2 : 1;
+    const int cut = DIRECT && rest > 0 ? 2 : 1;
     const int tickets = whole + rest * cut;
     if (q == 1) {                                  // its own walk is done: which others still have slots
       if (threadIdx.x < kXcds) s_taken[threadIdx.x] = __hip_atomic_load(&counters[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -404,16 +404,23 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
       if (n_rows <= 0) continue;
       const bf16_t* We = W + (size_t)e * N * K;
       // (the streaming hint only where no sibling reads the same weights: a pure read reaches 6.9 TB/s with it, 6.2 without)
-#define GT1(MTV, NTV) \
-  case MTV: grouped_tile<TO, MTV, NTV, PACKED, ACT>(x, x_bytes, We, out, N, K, a_rows, act_scale, act, relu2, row0, row_end, col_base, n_sib == 1, smem, &counters[xcd], next); break
+#define GTILE(MTV, NTV) \
+  grouped_tile<TO, MTV, NTV, PACKED, ACT, DIRECT>(x, x_bytes, We, out, N, K, a_rows, act_scale, act, relu2, row0, row_end, col_base, n_sib == 1, smem, &counters[xcd], next)
+#define GT1(MTV, NTV) case MTV: GTILE(MTV, NTV); break
 #define GT(NTV)                                                                                                  \
   switch ((n_rows + 31) >> 5) {                                                                                  \
     GT1(1, NTV); GT1(2, NTV); GT1(3, NTV); GT1(4, NTV); GT1(5, NTV); GT1(6, NTV); GT1(7, NTV); GT1(8, NTV);      \
   }
-      if (width == 1) GT(NT)
-      else GT(NT / 2)
+      if constexpr (DIRECT) {
+        if (width == 1) GT(NT)
+        else GT(NT / 2)
+      } else {                                     // (two heights are compiled: such a product waits for its operands)
+        if (n_rows <= 64) GTILE(2, NT);
+        else GTILE(8, NT);
+      }
 #undef GT
 #undef GT1
+#undef GTILE
     }
   }
   // the last block to leave sets the counters back for the next product that reads this plan

@@ -17,12 +17,15 @@ SHARPI_EXPORT int sharpi_gemm_grouped_swiglu(const void* x, int x_rows, const vo
   constexpr int GN = columns_of(kMaxNT);   // the gated form pairs gate tiles with up tiles
   const int nb = ceil_div(N / 2, GN / 2);
   const dim3 grid = grouped_grid(n_rows, n_groups, nb, max_blocks), block(GW * kWave);
-  if (packed)
-    grouped_gemm_kernel<bf16_t, kMaxNT, true, true><<<grid, block, 0, stream>>>(
-        (const bf16_t*)x, grouped_x_bytes(x_rows, K), (const bf16_t*)W, (bf16_t*)out, N, K, a_rows, act_scale, act, 0, group_offsets, plan, n_groups, nb);
-  else
-    grouped_gemm_kernel<bf16_t, kMaxNT, false, true><<<grid, block, 0, stream>>>(
-        (const bf16_t*)x, grouped_x_bytes(x_rows, K), (const bf16_t*)W, (bf16_t*)out, N, K, a_rows, act_scale, act, 0, group_offsets, plan, n_groups, nb);
+#define GS_LAUNCH(PK, DIR)                                                                                                  \
+  grouped_gemm_kernel<bf16_t, kMaxNT, PK, true, DIR><<<grid, block, 0, stream>>>(                                             \
+      (const bf16_t*)x, grouped_x_bytes(x_rows, K), (const bf16_t*)W, (bf16_t*)out, N, K, a_rows, act_scale, act, 0, group_offsets, plan, n_groups, nb)
+  if (whole_pieces(x, W)) {
+    if (packed) GS_LAUNCH(true, true); else GS_LAUNCH(false, true);
+  } else {
+    if (packed) GS_LAUNCH(true, false); else GS_LAUNCH(false, false);
+  }
+#undef GS_LAUNCH
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
 }

@@ -9,6 +9,9 @@
 
 typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 
+// Operands of such loads begin at 16-byte addresses; of others the pieces go through registers (DIRECT false), by kernels compiled apart:
+// a branch at the loads made the products 4 to 6 % slower and prompt attention 7.
+inline bool whole_pieces(const void* a, const void* b) { return (((uintptr_t)a | (uintptr_t)b) & 15) == 0; }
 // `bytes` of memory from `base` on, as the descriptor buffer loads take: lanes whose offset lies at or beyond them read zeros.
 __device__ __forceinline__ u32x4 buffer_of(const void* base, uint32_t bytes) {
   const uint64_t a = (uint64_t)base;
@@ -31,6 +34,17 @@ __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t offset, uint32_
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds" ::"{m0}"(lds), "v"(offset), "s"(rsrc), "s"(step) : "memory");
   else
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(offset), "s"(rsrc), "s"(step) : "memory");
+}
+// The same bytes by way of registers, from any address.
+__device__ __forceinline__ void copy_to_lds(u32x4 rsrc, uint32_t offset, uint32_t step, uint32_t lds) {
+  const char* base = (const char*)((uint64_t)rsrc[0] | (uint64_t)rsrc[1] << 32);
+  u32x4 piece;
+  __builtin_memcpy(&piece, base + (size_t)step + offset, 16);
+  *(__attribute__((address_space(3))) u32x4*)(uintptr_t)(lds + (threadIdx.x & (kWave - 1)) * 16) = piece;
+}
+template <bool DIRECT> __device__ __forceinline__ void bring_to_lds(u32x4 rsrc, uint32_t offset, uint32_t step, uint32_t lds) {
+  if constexpr (DIRECT) load_to_lds(rsrc, offset, step, lds);
+  else copy_to_lds(rsrc, offset, step, lds);
 }
 template <int LEFT = 0> __device__ __forceinline__ void lds_loads_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory");

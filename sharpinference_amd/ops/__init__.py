@@ -76,7 +76,8 @@ def _dev(*ts) -> None:
 
 
 def _whole_pieces(t: torch.Tensor) -> torch.Tensor:
-    """The tensor, or a copy that begins at a 16-byte address: what kernels take that load straight into LDS."""
+    """Rows, or a copy of them that begins at a 16-byte address.  Kernels that load straight into LDS take operands that begin
+    elsewhere through registers, which is slower than a copy of the rows; weights and caches are never copied."""
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
@@ -457,7 +458,6 @@ def attention_prefill(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Ten
           "attention_prefill: caches must be K [pages, nkv, page_size, hd], V [pages, nkv, hd, page_size] bfloat16")
     _need(block_table.dim() == 2 and positions.shape == (T,) and tiles.dim() == 2 and tiles.shape[1] == 3,
           "attention_prefill: block_table [entries, max_blocks], positions [T], tiles [n, 3]")
-    k_cache, v_cache = _whole_pieces(k_cache), _whole_pieces(v_cache)
     if out is None:
         out = torch.empty(T, nh * vd, dtype=q.dtype, device=q.device)
     _need(out.shape == (T, nh * vd) and out.dtype == q.dtype, "attention_prefill: out must be [T, nh*vd] of q's dtype")
@@ -1193,7 +1193,7 @@ def gemm_grouped(x: torch.Tensor, w, rt: Routing, gather: bool, out_dtype: torch
     results are the squares of their relu."""
     w, packed = _unwrap(w)
     _dev(x, w)
-    x, w = _whole_pieces(x), _whole_pieces(w)
+    x = _whole_pieces(x)
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_grouped: bfloat16 operands only")
     _need(w.dim() == 3 and w.shape[0] >= rt.n_groups and x.dim() == 2 and x.shape[1] == w.shape[2],
           f"gemm_grouped: x {tuple(x.shape)} vs w {tuple(w.shape)}")
@@ -1216,7 +1216,7 @@ def gemm_grouped_swiglu(x: torch.Tensor, w, rt: Routing, scale: Optional[torch.T
     rows.  Returns [n_rows, I] bfloat16."""
     w, packed = _unwrap(w)
     _dev(x, w, scale)
-    x, w = _whole_pieces(x), _whole_pieces(w)
+    x = _whole_pieces(x)
     _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16, "gemm_grouped_swiglu: bfloat16 operands only")
     _need(w.dim() == 3 and w.shape[0] >= rt.n_groups and x.dim() == 2 and x.shape[1] == w.shape[2],
           f"gemm_grouped_swiglu: x {tuple(x.shape)} vs w {tuple(w.shape)}")

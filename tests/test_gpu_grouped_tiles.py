@@ -47,6 +47,28 @@ def test_every_height_of_a_tile(counts, N, K):
             assert bool(((act - ref).abs() <= 2 ** -8 * ref.abs() + 1e-30).all())
 
 
+@pytest.mark.parametrize("off", [1, 2, 5])
+def test_weights_may_begin_at_any_address(off):
+    """The same bits as from an address that is a multiple of 16, and no copy of the weights."""
+    from sharpinference_amd import ops
+    g = torch.Generator().manual_seed(off)
+    counts, N, K = [3, 0, 290, 64, 31], 320, 192
+    x = torch.randn(sum(counts), K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(len(counts), N, K, generator=g) * 0.1).bfloat16().to(DEV)
+    rt = routed(counts)
+    flat = torch.empty(w.numel() + off, dtype=torch.bfloat16, device=DEV)
+    flat[off:] = w.reshape(-1)
+    own = flat[off:].view(w.shape)
+    assert own.data_ptr() % 16
+    for gather in (True, False):
+        assert torch.equal(ops.gemm_grouped(x, own, rt, gather, torch.float32), ops.gemm_grouped(x, w, rt, gather, torch.float32))
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        got = ops.gemm_grouped_swiglu(x, own, rt, None, gather)
+        assert torch.cuda.max_memory_allocated() - before < w.numel() * 2
+        assert torch.equal(got, ops.gemm_grouped_swiglu(x, w, rt, None, gather))
+
+
 def test_more_groups_than_offsets_are_kept_of():
     from sharpinference_amd import ops
     g = torch.Generator().manual_seed(3)

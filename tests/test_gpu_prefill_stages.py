@@ -1,6 +1,6 @@
 """Prompt attention where its stages and layouts can go wrong: pages whose size is no power of two, starts and ends inside
 a 16-key block, a 32-key chunk and a stage, kept tokens before a window, every swizzle of the key rows, half a tile of
-value columns, and pages behind no visible key (given back: -1 in the table, whatever page 0 holds)."""
+value columns, pages behind no visible key (given back: -1 in the table, whatever page 0 holds), and caches that begin at any address."""
 import math
 
 import pytest
@@ -61,3 +61,33 @@ def test_stages_chunks_and_pages(nh, nkv, hd, vd, ps, kind, window, keep, start,
         want = reference(q[t], k, v, start + t, first(start + t), keep, scale, cap, sink)
         # half a step of a bfloat16 result, and probabilities of 16 bits over values below 6
         assert bool(((a[t] - want).abs() <= 2 ** -8 * want.abs() + 6 * 2 ** -14).all()), (t, float((a[t] - want).abs().max()))
+
+
+@pytest.mark.parametrize("nh,nkv,hd,vd", [(8, 2, 128, 128), (2, 1, 192, 96), (3, 3, 32, 96)])
+@pytest.mark.parametrize("off", [(1, 0), (0, 2), (7, 5)])
+def test_caches_may_begin_at_any_address(nh, nkv, hd, vd, off):
+    """The same bits as from addresses that are multiples of 16, and no copy of the caches."""
+    from sharpinference_amd import ops
+    g = torch.Generator().manual_seed(hd + off[0])
+    pages, ps, rows, start = 40, 16, 130, 300
+    kc, vc = torch.randn(pages, nkv, ps, hd, generator=g).bfloat16().to(DEV), torch.randn(pages, nkv, vd, ps, generator=g).bfloat16().to(DEV)
+    q = torch.randn(rows, nh * hd, generator=g).bfloat16().to(DEV)
+    table = torch.randperm(pages, generator=g).int()[None, :27].contiguous().to(DEV)
+    positions = torch.arange(start, start + rows, dtype=torch.int32, device=DEV)
+
+    def moved(t, n):
+        flat = torch.empty(t.numel() + n, dtype=t.dtype, device=DEV)
+        flat[n:] = t.reshape(-1)
+        return flat[n:].view(t.shape)
+
+    own = moved(kc, off[0]), moved(vc, off[1])
+    assert any(t.data_ptr() % 16 for t in own)
+    for tile in (ops.PREFILL_TILE_TOKENS, ops.PREFILL_TILE_TOKENS // 2):
+        tiles = torch.tensor([(0, o, min(tile, rows - o)) for o in range(0, rows, tile)], dtype=torch.int32, device=DEV)
+        run = lambda k, v: ops.attention_prefill(q, k, v, table, positions, tiles, 0, 0, hd ** -0.5, nh, nkv, hd, tile_tokens=tile, vd=vd)
+        want = run(kc, vc)
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        got = run(*own)
+        assert torch.cuda.max_memory_allocated() - before < kc.numel() * 2
+        assert torch.equal(got, want)
