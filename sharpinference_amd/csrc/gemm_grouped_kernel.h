@@ -69,7 +69,9 @@ static_assert(GM == 2 * 16 * 8, "tile heights are compiled in steps of 32 rows u
 // counter); with the exclusive or the sixteen pieces of a turn fall into the sixteen different 16-byte groups of the bank space.
 __device__ __forceinline__ int xs_piece(int row, int piece) { return piece ^ ((row >> 1) & 7); }
 
-// The work of one tile of up to MT * 32 rows against 16 * NT * GWC weight rows.  DIRECT: both operands begin at 16-byte addresses.
+// The work of one tile of up to MT * 32 rows against 16 * NT * GWC weight rows.  DIRECT: both operands begin at 16-byte
+// addresses; else the pieces go through registers, a latency of memory a step (16 experts of 8,192 x 5,120, 2,048 rows: 433 us, 1,041
+// from an odd address).
 template <typename TO, int MT, int NT, bool PACKED, bool ACT, bool DIRECT>
 __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint32_t x_bytes, const bf16_t* __restrict__ We,
                                              TO* __restrict__ out, int N, int K, const int* __restrict__ a_rows,
@@ -403,9 +405,11 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
       const int n_rows = row_end - row0;
       if (n_rows <= 0) continue;
       const bf16_t* We = W + (size_t)e * N * K;
-      // (the streaming hint only where no sibling reads the same weights: a pure read reaches 6.9 TB/s with it, 6.2 without)
+      // The streaming hint only where no sibling reads the same weights (a pure read reaches 6.9 TB/s with it, 6.2 without), and only
+      // for weights stored tile by tile: a step takes half a line of a row's, and with the hint the other half came from memory once
+      // more (rows of 16 experts of 8,192 x 5,120, 300 tokens: 382 us with it, 308 without; 2,048 tokens 432 and 385).
 #define GTILE(MTV, NTV) \
-  grouped_tile<TO, MTV, NTV, PACKED, ACT, DIRECT>(x, x_bytes, We, out, N, K, a_rows, act_scale, act, relu2, row0, row_end, col_base, n_sib == 1, smem, &counters[xcd], next)
+  grouped_tile<TO, MTV, NTV, PACKED, ACT, DIRECT>(x, x_bytes, We, out, N, K, a_rows, act_scale, act, relu2, row0, row_end, col_base, PACKED && n_sib == 1, smem, &counters[xcd], next)
 #define GT1(MTV, NTV) case MTV: GTILE(MTV, NTV); break
 #define GT(NTV)                                                                                                  \
   switch ((n_rows + 31) >> 5) {                                                                                  \
