@@ -22,7 +22,8 @@
 //    weights 32 of K a step, three steps ahead, in the order the packed matrix has them (1 KB a 16-row
 //    tile and step, read back without conflicts); x rows (gathered through a_rows) 64 of K at a time, whole
 //    128-byte lines, a stage ahead, their 16-byte pieces XORed with row bits (xs_piece).  One barrier a step; a wave
-//    waits for its own loads of the step by count and the barrier makes them everyone's.
+//    waits for its own loads of the step by count and the barrier makes them everyone's.  Tiles of up to 128 rows, whose steps are
+//    short beside a barrier and a latency, go a stage of 64 at a time, weights and rows two or three stages ahead.
 //  * W is the A operand (rows = n), x the B operand: a lane ends up with 4 consecutive n of one
 //    row, stored as one 8-byte write.  Each output is one chain over k in ascending order, so a
 //    row's result does not depend on which other rows share its tile, nor on which block took it.
@@ -36,6 +37,10 @@
 // Measured, 16 experts, up (2 x 8,192 rows of 5,120) + down, us, beside tiles of 128 x 512 whose weights went straight to
 // registers: 8,192 tokens 1,328 + 647 (1,420 + 700), 2,048 tokens of uneven load 576 + 269 (587 + 264), 1,190 tokens 463 + 241
 // (488 + 250); 64 experts of 1,408 x 2,048, six picks, 3,000 tokens 291 + 137 (327 + 157), 1,664 tokens 192 + 100 (235 + 110).
+// Tiles of up to 128 rows, a step and a stage at a time: 28 experts of 2,048 x 4,096, 43 rows each 104 -> 97, 71 rows 110 -> 104; 16 of
+// 5,120 x 8,192, 19 rows each 238 -> 223; in rows, not packed, 64 of 2,816 x 2,048, 6 rows each 184 -> 180.  Where an expert's rows about
+// fill a tile of 128 the product stays behind tiles of 128 x 512: 64 of 2,048 x 1,408, 111 rows 97 (90), 32 of 4,096 x 2,048,
+// 75 rows 114 (106), 28 of 2,048 x 4,096, 71 rows 104 (92).
 // Parts taken out, 4,096 tokens even (up, 656 us): no loads 465 (1.48 PFLOP/s), no products 538, weights and products without x rows
 // 615: the weights' 2.7 GB and the products each need about 460, and neither hides the other whole.
 // Limits: K % 64 == 0, N % 4 == 0 (N % 32 == 0 in the SwiGLU form).
@@ -57,11 +62,9 @@ constexpr int kMaxNT = 4;              // 16-row weight tiles per wave: this man
 constexpr int columns_of(int nt) { return 16 * nt * GWC; }   // weight rows (output columns) of a block
 constexpr int GK = 64;                 // K of a stage of x rows: two steps of 32
 constexpr int kXcds = kPlanXcds;       // accelerator dies, each with its own L2
-// LDS: four steps of weights (16 tiles of 16 rows x 32 of K), then two stages of x rows (GM x 64 of K), then the groups' first rows.
-// (Deeper rings where a tile is low, up to 8 steps and 3 stages, gained nothing: 3.9 to 6.4 TB/s of weights as before.)
-constexpr int kWStep = 16 * 1024, kXStage = GM * GK * 2, kXAt = 4 * kWStep, kGroupedLds = kXAt + 2 * kXStage;
+// LDS: rings of weights (steps of 32 of K) and x rows (stages of 64), see grouped_tile.
+constexpr int kGroupedLds = 144 * 1024;
 constexpr int kOffsetsKept = 1025;     // of more groups the rows are read from memory
-static_assert(2 * kWStep == kXStage, "both rings turn by the same exclusive or");
 static_assert(GM == 2 * 16 * 8, "tile heights are compiled in steps of 32 rows up to 256");
 
 // Where 16-byte piece `piece` of x row `row` of a stage is kept.  The LDS serves a 16-byte read of a wave in four
@@ -83,6 +86,14 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   constexpr int TILES = NT * GWC;               // weight tiles of the block
   constexpr int WL = (TILES + GW - 1) / GW;     // loads of weights a wave and step
   constexpr int XL = (4 * MT + GW - 1) / GW;    // loads of x rows a wave and stage (8 rows each)
+  // The rings: of tall tiles two stages of x rows (32 KB each) and four steps of weights (16 KB), filled a step at a time, weights three
+  // steps ahead; of tiles of up to 128 rows (half as much of x) three stages of both, of which a cut slot's (half of the weights, too)
+  // has four, filled a stage at a time.
+  constexpr int RS = MT > 4 ? 2 : NT == kMaxNT ? 3 : 4;
+  constexpr bool STAGED = RS > 2;
+  constexpr int kWStep = 1024 * (MT > 4 ? 16 : TILES), kXStage = MT > 4 ? 32768 : 16384, kXAt = 2 * RS * kWStep;
+  constexpr int GL = XL + 2 * WL;               // a wave's loads of a stage
+  static_assert(TILES * 1024 <= kWStep && MT * 32 * GK * 2 <= kXStage && kXAt + RS * kXStage <= kGroupedLds, "the rings hold a tile");
   const int lane = threadIdx.x & (kWave - 1);
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -121,17 +132,17 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   const u32x4 wb = buffer_of(We, (uint32_t)N * (uint32_t)K * 2), xb = buffer_of(x, x_bytes);
   const uint32_t lds0 = lds_address(smem);
   const int steps = K / 32, stages = K / GK;
-  auto load_w = [&](int s) {                    // weights of step s into the ring
+  auto load_w = [&](int s, int place) {         // weights of step s into the ring
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
-      const uint32_t at = lds0 + (s & 3) * kWStep + w_tile[i] * 1024;
+      const uint32_t at = lds0 + place * kWStep + w_tile[i] * 1024;
       if (DIRECT && stream) load_to_lds<true>(wb, w_off[i], s * kWStepBytes, at);
       else bring_to_lds<DIRECT>(wb, w_off[i], s * kWStepBytes, at);
     }
   };
-  load_w(0);                                    // (on their way while the rows' places are looked up)
-  load_w(1);
-  if (steps > 2) load_w(2);
+#pragma unroll
+  for (int s = 0; s < (STAGED ? 2 * RS - 2 : 3); ++s)   // (on their way while the rows' places are looked up)
+    if (s < 2 || s < steps) load_w(s, s);
   // x rows: a load brings 8 rows of 128 bytes, lane l row l / 8 at place l % 8.  Rows beyond the expert's last read its last row again
   // (what such rows produce is never stored).
   uint32_t x_off[XL];
@@ -147,11 +158,13 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   // waited for here: the compiler's own waits must not fall among the loads below, which it does not know of
 #pragma unroll
   for (int i = 0; i < XL; ++i) asm volatile("" : "+v"(x_off[i]));
-  auto load_x = [&](int c) {                    // x rows of stage c
+  auto load_x = [&](int c, int place) {         // x rows of stage c
 #pragma unroll
-    for (int i = 0; i < XL; ++i) bring_to_lds<DIRECT>(xb, x_off[i], c * (GK * 2), lds0 + kXAt + (c & 1) * kXStage + x_load[i] * 1024);
+    for (int i = 0; i < XL; ++i) bring_to_lds<DIRECT>(xb, x_off[i], c * (GK * 2), lds0 + kXAt + place * kXStage + x_load[i] * 1024);
   };
-  load_x(0);
+#pragma unroll
+  for (int c = 0; c < RS - 1; ++c)
+    if (c == 0 || c < stages) load_x(c, c);
 
   // operand addresses (bytes): fragment t of a step lies at w_at + t * 1024, row group mb of a stage's half at x_at + mb * 2048
   int w_at = wc * NT * 1024 + lane * 16;
@@ -163,18 +176,36 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   // of its products, the LDS and the matrix cores took turns).
   constexpr int H0 = (MT + 1) / 2, H1 = MT / 2;
   bf16x8 wf[2][NT], x0[H0], x1[H1 > 0 ? H1 : 1];
+  int place = 0;                                // of this stage in the rings
   auto arrive = [&](int s, auto half_tag) {     // step s is in LDS, and everyone has read step s - 1
     constexpr int hh = decltype(half_tag)::value;
-    // This step's loads: behind them were sent two steps of weights, and in a stage's second step the next stage's x rows.  (In
-    // the last two steps some of those do not exist, and the first x rows were sent last: everything is waited for.)
-    if (s > 0 && s + 2 < steps) lds_loads_wait<hh == 0 ? 2 * WL : 2 * WL + XL>();
-    else lds_loads_wait<0>();
+    // This step's loads: counted is what was sent behind them.  (The first x rows were sent last: everything is waited for.)
+    if constexpr (STAGED) {                     // whole stages: those behind it
+      if (hh == 1) return;                      // (came with the step before)
+      const int behind = stages - 1 - (s >> 1);
+      if (s == 0) lds_loads_wait<0>();
+      else if (RS == 4 && behind >= 2) lds_loads_wait<2 * GL>();
+      else if (behind >= 1) lds_loads_wait<GL>();
+      else lds_loads_wait<0>();
+    } else {                                    // two steps of weights and, in a stage's second step, the next stage's x rows
+      if (s > 0 && s + 2 < steps) lds_loads_wait<hh == 0 ? 2 * WL : 2 * WL + XL>();
+      else lds_loads_wait<0>();
+    }
     __syncthreads();
   };
-  auto send = [&](int s, auto half_tag) {       // the loads that take the place of step s - 1
+  auto send = [&](int s, auto half_tag) {       // the loads that take the place of step s - 1, or of the stage before
     constexpr int hh = decltype(half_tag)::value;
-    if (hh == 0 && (s >> 1) + 1 < stages) load_x((s >> 1) + 1);
-    if (s + 3 < steps) load_w(s + 3);
+    if constexpr (STAGED) {
+      const int c = (s >> 1) + RS - 1, to = place == 0 ? RS - 1 : place - 1;
+      if (hh == 0 && c < stages) {
+        load_x(c, to);
+        load_w(2 * c, 2 * to);
+        load_w(2 * c + 1, 2 * to + 1);
+      }
+    } else {
+      if (hh == 0 && (s >> 1) + 1 < stages) load_x((s >> 1) + 1, place ^ 1);
+      if (s + 3 < steps) load_w(s + 3, (s + 3) & 3);
+    }
   };
   auto read_first = [&](auto half_tag) {
     constexpr int hh = decltype(half_tag)::value;
@@ -205,9 +236,11 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
     for (int mb = 0; mb < H0; ++mb) row_products(x0[mb], mb);
     in_turn(std::integral_constant<int, H1>{}, std::integral_constant<int, H0 * NT>{});
     if constexpr (hh == 1) {
-      w_at ^= 2 * kWStep;
-      x_at[0] ^= kXStage;
-      x_at[1] ^= kXStage;
+      const int turn = place == RS - 1 ? 1 - RS : 1;
+      place += turn;
+      w_at += turn * 2 * kWStep;
+      x_at[0] += turn * kXStage;
+      x_at[1] += turn * kXStage;
     }
     if constexpr (!last) {
       __builtin_amdgcn_sched_barrier(0);        // products of the first half stay ahead of the barrier, those of the other behind it
@@ -292,7 +325,7 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     const int* __restrict__ a_rows, const float* __restrict__ act_scale, GatedAct act, int relu2,
     const int* __restrict__ group_offsets, const int* __restrict__ plan, int n_groups, int nb) {
   __shared__ __attribute__((aligned(1024))) char smem[kGroupedLds];
-  __shared__ int s_slot, s_total[kXcds], s_taken[kXcds];
+  __shared__ int s_slot, s_total[kXcds], s_rows[kXcds], s_taken[kXcds];
   __shared__ int4 s_unit[kWave + 1];
   __shared__ int s_offset[kOffsetsKept];
   constexpr int GN = columns_of(NT);
@@ -306,7 +339,11 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
   //
   // A walk is only a few slots per block long: slots that fill no whole round of the XCD's blocks would leave most of them idle for
   // a slot's time at the end.  Those last slots are therefore cut by columns into two (16 experts of 13 to 396 rows, 8,192 ->
-  // 5,120: 313 us where they were cut only if the halves fitted one round, 294 always; quarters, 318, read the x rows too often).
+  // 5,120: 313 us where they were cut only if the halves fitted one round, 294 always; quarters, 318, read the x rows too often;
+  // a first round nearly full, 28 experts of 2,048 x 4,096, 71 rows each, 104 halved, 112 whole).
+  // A walk with work for a quarter of its blocks cuts its groups into tiles of half the rows: twice as many blocks, and the deeper rings
+  // (one matrix of 2,048 x 4,096, 130 rows 53 -> 37 us, 700 rows 58 -> 40; 8 groups of 512 x 512, 250 rows each 18.8 -> 16.0;
+  // from half of the blocks on nothing changed).
   if (n_groups < kOffsetsKept)
     for (int i = threadIdx.x; i <= n_groups; i += GW * kWave) s_offset[i] = group_offsets[i];
   __syncthreads();
@@ -319,15 +356,17 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
   // The plan counts siblings of kPlanTileRows rows; here a group's rows are cut into tiles of GM (the deal stays level, and
   // the tall tiles, which take longest, still come first in a walk).
   auto offset_of = [&](int e) { return n_groups < kOffsetsKept ? s_offset[e] : group_offsets[e]; };
-  auto siblings_of = [&](int e) { return (offset_of(e + 1) - offset_of(e) + GM - 1) / GM; };
-  auto unit_slots = [&](const int* pu) { return (plan_part_first(pu[1] + 1, pu[2], nb) - plan_part_first(pu[1], pu[2], nb)) * siblings_of(pu[0]); };
+  auto siblings_of = [&](int e, int rows) { return (offset_of(e + 1) - offset_of(e) + rows - 1) / rows; };
+  auto unit_slots = [&](const int* pu, int rows) {
+    return (plan_part_first(pu[1] + 1, pu[2], nb) - plan_part_first(pu[1], pu[2], nb)) * siblings_of(pu[0], rows);
+  };
   // units j0 .. j0 + 63 of a walk into LDS: (slots before it, group, siblings, first column block), and all their slots
-  auto list_units = [&](const int* px, int n_units, int j0) {
+  auto list_units = [&](const int* px, int n_units, int j0, int rows) {
     __syncthreads();
     if (threadIdx.x < kWave) {
       const int* pu = px + 1 + 4 * min(j0 + lane, n_units - 1);
-      const int u_group = pu[0], u_sib = siblings_of(pu[0]), u_col = plan_part_first(pu[1], pu[2], nb);
-      const int slots = j0 + lane < n_units ? unit_slots(pu) : 0;
+      const int u_group = pu[0], u_sib = siblings_of(pu[0], rows), u_col = plan_part_first(pu[1], pu[2], nb);
+      const int slots = j0 + lane < n_units ? unit_slots(pu, rows) : 0;
       int upto = slots;
 #pragma unroll
       for (int o = 1; o < kWave; o <<= 1) {
@@ -344,11 +383,21 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     const int x = threadIdx.x >> 6;
     const int* px = plan + x * plan_stride(n_groups);
     const int n_units = px[0];
-    int total = 0;
-    for (int j = lane; j < n_units; j += kWave) total += unit_slots(px + 1 + 4 * j);
+    int total = 0, total_low = 0;
+    for (int j = lane; j < n_units; j += kWave) {
+      total += unit_slots(px + 1 + 4 * j, GM);
+      total_low += unit_slots(px + 1 + 4 * j, GM / 2);
+    }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) total += __shfl_xor(total, o, kWave);
-    if (lane == 0) s_total[x] = total;
+    for (int o = 32; o > 0; o >>= 1) {
+      total += __shfl_xor(total, o, kWave);
+      total_low += __shfl_xor(total_low, o, kWave);
+    }
+    if (lane == 0) {
+      const bool low = 4 * total <= per_xcd;
+      s_total[x] = low ? total_low : total;
+      s_rows[x] = low ? GM / 2 : GM;
+    }
   }
   __syncthreads();
   for (int q = 0; q < kXcds; ++q) {
@@ -359,13 +408,14 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
     const int whole = total / per_xcd * per_xcd;   // slots of whole rounds: taken as they are
     const int rest = total - whole;
     const int cut = DIRECT && rest > 0 ? 2 : 1;
+    const int rows_most = __builtin_amdgcn_readfirstlane(s_rows[xcd]);
     const int tickets = whole + rest * cut;
     if (q == 1) {                                  // its own walk is done: which others still have slots
       if (threadIdx.x < kXcds) s_taken[threadIdx.x] = __hip_atomic_load(&counters[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       __syncthreads();
     }
     if (q > 0 && s_taken[xcd] >= tickets) continue;
-    if (n_units > 0 && n_units <= kWave) list_units(px, n_units, 0);
+    if (n_units > 0 && n_units <= kWave) list_units(px, n_units, 0, rows_most);
     int next = -1;                                 // thread 0: the ticket taken at the end of the slot before, if there was one
     for (;;) {
       if (threadIdx.x == 0) s_slot = next >= 0 ? next : atomicAdd(&counters[xcd], 1);
@@ -379,7 +429,7 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
       const int piece = ticket < whole ? 0 : (ticket - whole) % width;
       int e = -1, n_sib = 1, col0 = 0;
       for (int j0 = 0; j0 < n_units && e < 0; j0 += kWave) {
-        if (n_units > kWave) list_units(px, n_units, j0);
+        if (n_units > kWave) list_units(px, n_units, j0, rows_most);
         const int mine = s_unit[lane].x;             // this lane's unit begins behind so many slots (of these units)
         const int last = __builtin_amdgcn_readfirstlane(s_unit[kWave].x);
         if (slot < last) {

@@ -18,7 +18,7 @@ HEIGHTS = [1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 224, 225
 
 
 @pytest.mark.parametrize("counts", [HEIGHTS, HEIGHTS[::-1], [700], [0, 256, 0, 0, 9]])
-@pytest.mark.parametrize("N,K", [(20, 64), (264, 128), (320, 192), (272, 320), (1056, 128)])
+@pytest.mark.parametrize("N,K", [(20, 64), (264, 128), (320, 192), (272, 320), (1056, 128), (96, 1152), (32, 576)])
 def test_every_height_of_a_tile(counts, N, K):
     from sharpinference_amd import ops
     g = torch.Generator().manual_seed(N + K)
