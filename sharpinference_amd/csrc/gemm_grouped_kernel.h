@@ -38,7 +38,7 @@
 // registers: 8,192 tokens 1,328 + 647 (1,420 + 700), 2,048 tokens of uneven load 576 + 269 (587 + 264), 1,190 tokens 463 + 241
 // (488 + 250); 64 experts of 1,408 x 2,048, six picks, 3,000 tokens 291 + 137 (327 + 157), 1,664 tokens 192 + 100 (235 + 110).
 // Tiles of up to 128 rows, a step and a stage at a time: 28 experts of 2,048 x 4,096, 43 rows each 104 -> 97, 71 rows 110 -> 104; 16 of
-// 5,120 x 8,192, 19 rows each 238 -> 223; in rows, not packed, 64 of 2,816 x 2,048, 6 rows each 184 -> 180.  Where an expert's rows about
+// 5,120 x 8,192, 19 rows each 238 -> 223.  Where an expert's rows about
 // fill a tile of 128 the product stays behind tiles of 128 x 512: 64 of 2,048 x 1,408, 111 rows 97 (90), 32 of 4,096 x 2,048,
 // 75 rows 114 (106), 28 of 2,048 x 4,096, 71 rows 104 (92).
 // Parts taken out, 4,096 tokens even (up, 656 us): no loads 465 (1.48 PFLOP/s), no products 538, weights and products without x rows
@@ -102,9 +102,14 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   // Weights: tile lt of the block is tile lt % NT of column wave lt / NT.  A tile that lies beyond the last column (or its rows that do)
   // is read as the last that exists, never stored.
   // Packed layout (the matrix stored as [N/16][K/128][16 runs of 8 k][16 rows][8]): a step of a tile is 1 KB in a row.
-  // Row layout: lane (row l % 16, run l / 16) reads 16 bytes of its row; in LDS both lie as [run][row].
+  // Row layout: lane (row l % 16, run l / 16) reads 16 bytes of its row; in LDS both lie as [run][row].  Where weights come a stage at a
+  // time a load takes whole lines, 8 rows of 128 bytes, as those of x rows do.  The streaming hint goes with whole lines only: of half a
+  // line the other half came from memory once more.  us with tiles of 128 x 512, half lines and the hint, half lines without, lines
+  // without and lines with it: 16 experts of 8,192 x 5,120, 300 rows 281, 382, 308, 259, 234; 64 of 2,816 x 2,048, 300 tokens 186,
+  // 234, 187, 172, 162; 20 of 1,408 x 960 (caches hold them from call to call) 33, 33, 25, 23, 26.
+  constexpr bool LINES = STAGED && !PACKED;
   constexpr uint32_t kWStepBytes = PACKED ? 1024 : 64;
-  uint32_t w_off[WL];
+  uint32_t w_off[LINES ? 2 : 1][WL];
   int w_tile[WL];
 #pragma unroll
   for (int i = 0; i < WL; ++i) {
@@ -115,12 +120,13 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
     if constexpr (PACKED) {
       if (n >= n_out) n = n_out - 16;
       if (ACT && t >= HT) n += n_out;
-      w_off[i] = (uint32_t)n * (uint32_t)K * 2 + lane * 16;
+      w_off[0][i] = (uint32_t)n * (uint32_t)K * 2 + lane * 16;
     } else {
-      n += lane & 15;
-      if (n >= n_out) n = n_out - 1;
-      if (ACT && t >= HT) n += n_out;
-      w_off[i] = (uint32_t)n * (uint32_t)K * 2 + (lane >> 4) * 16;
+#pragma unroll
+      for (int u = 0; u < (LINES ? 2 : 1); ++u) {
+        const int row = LINES ? u * 8 + (lane >> 3) : lane & 15, piece = LINES ? xs_piece(row, lane & 7) : lane >> 4;
+        w_off[u][i] = (uint32_t)(min(n + row, n_out - 1) + (ACT && t >= HT ? n_out : 0)) * (uint32_t)K * 2 + piece * 16;
+      }
     }
   }
   f32x4 acc[NT][MT];
@@ -135,9 +141,11 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   auto load_w = [&](int s, int place) {         // weights of step s into the ring
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
-      const uint32_t at = lds0 + place * kWStep + w_tile[i] * 1024;
-      if (DIRECT && stream) load_to_lds<true>(wb, w_off[i], s * kWStepBytes, at);
-      else bring_to_lds<DIRECT>(wb, w_off[i], s * kWStepBytes, at);
+      const int u = LINES ? s & 1 : 0;
+      const uint32_t at = lds0 + (LINES ? (place >> 1) * 2 * kWStep + w_tile[i] * 2048 + u * 1024 : place * kWStep + w_tile[i] * 1024);
+      const uint32_t off = LINES ? (u ? w_off[LINES][i] : w_off[0][i]) : w_off[0][i], step = LINES ? (s >> 1) * (GK * 2) : s * kWStepBytes;
+      if (DIRECT && stream && (PACKED || LINES)) load_to_lds<true>(wb, off, step, at);
+      else bring_to_lds<DIRECT>(wb, off, step, at);
     }
   };
 #pragma unroll
@@ -166,8 +174,11 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   for (int c = 0; c < RS - 1; ++c)
     if (c == 0 || c < stages) load_x(c, c);
 
-  // operand addresses (bytes): fragment t of a step lies at w_at + t * 1024, row group mb of a stage's half at x_at + mb * 2048
-  int w_at = wc * NT * 1024 + lane * 16;
+  // operand addresses (bytes): fragment t of a step lies at w_at + t * 1024 (lines: 2048), row group mb of a stage's half at x_at + mb * 2048
+  int w_at[2];
+#pragma unroll
+  for (int hh = 0; hh < 2; ++hh)
+    w_at[hh] = LINES ? wc * NT * 2048 + r * 128 + xs_piece(r, hh * 4 + g) * 16 : wc * NT * 1024 + lane * 16 + hh * kWStep;
   int x_at[2];
 #pragma unroll
   for (int hh = 0; hh < 2; ++hh) x_at[hh] = kXAt + (wr * MT * 16 + r) * 128 + xs_piece(r, hh * 4 + g) * 16;
@@ -210,7 +221,7 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   auto read_first = [&](auto half_tag) {
     constexpr int hh = decltype(half_tag)::value;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) wf[hh][t] = *reinterpret_cast<const bf16x8*>(smem + w_at + hh * kWStep + t * 1024);
+    for (int t = 0; t < NT; ++t) wf[hh][t] = *reinterpret_cast<const bf16x8*>(smem + w_at[hh] + t * (LINES ? 2048 : 1024));
 #pragma unroll
     for (int mb = 0; mb < H0; ++mb) x0[mb] = *reinterpret_cast<const bf16x8*>(smem + x_at[hh] + mb * 2048);
   };
@@ -238,7 +249,8 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
     if constexpr (hh == 1) {
       const int turn = place == RS - 1 ? 1 - RS : 1;
       place += turn;
-      w_at += turn * 2 * kWStep;
+      w_at[0] += turn * 2 * kWStep;
+      w_at[1] += turn * 2 * kWStep;
       x_at[0] += turn * kXStage;
       x_at[1] += turn * kXStage;
     }
@@ -455,11 +467,9 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
       const int n_rows = row_end - row0;
       if (n_rows <= 0) continue;
       const bf16_t* We = W + (size_t)e * N * K;
-      // The streaming hint only where no sibling reads the same weights (a pure read reaches 6.9 TB/s with it, 6.2 without), and only
-      // for weights stored tile by tile: a step takes half a line of a row's, and with the hint the other half came from memory once
-      // more (rows of 16 experts of 8,192 x 5,120, 300 tokens: 382 us with it, 308 without; 2,048 tokens 432 and 385).
+      // (the streaming hint only where no sibling reads the same weights: a pure read reaches 6.9 TB/s with it, 6.2 without)
 #define GTILE(MTV, NTV) \
-  grouped_tile<TO, MTV, NTV, PACKED, ACT, DIRECT>(x, x_bytes, We, out, N, K, a_rows, act_scale, act, relu2, row0, row_end, col_base, PACKED && n_sib == 1, smem, &counters[xcd], next)
+  grouped_tile<TO, MTV, NTV, PACKED, ACT, DIRECT>(x, x_bytes, We, out, N, K, a_rows, act_scale, act, relu2, row0, row_end, col_base, n_sib == 1, smem, &counters[xcd], next)
 #define GT1(MTV, NTV) case MTV: GTILE(MTV, NTV); break
 #define GT(NTV)                                                                                                  \
   switch ((n_rows + 31) >> 5) {                                                                                  \
