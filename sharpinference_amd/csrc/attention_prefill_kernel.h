@@ -25,7 +25,7 @@
 // 40 heads of 128 sharing 8 key heads, 8,192 tokens: 1,041 us (660 TFLOP/s, the pair's second product not counted); 1,452 us with
 // 32-key chunks on their way through registers and divisions by the page size in every chunk.  2,048 tokens: 98 us (133); 64 heads of
 // 192 / 128, window 1,024, 2,048 tokens: 139 us (180); 16 heads, 1,900 tokens: 49 us (75).  Three prompts of 400 tokens in
-// tiles of 64: 30 us (34).  On 32x32x16 products, eight consecutive keys a lane, it took 904, 76, 111 and 47 us: other sums of the
+// tiles of 64: 32 us (35).  On 32x32x16 products, eight consecutive keys a lane, it took 904, 76, 111 and 47 us: other sums of the
 // same exactness, whose roundings turned routers' near ties in whole models; these are the bits of the kernel before.
 #pragma once
 #include <type_traits>

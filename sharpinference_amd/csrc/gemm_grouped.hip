@@ -37,4 +37,5 @@ SHARPI_EXPORT int sharpi_gemm_grouped(const void* x, int x_rows, const void* W, 
   return SHARPI_OK;
 }
 
+// rows of the tiles that the plan counts in
 SHARPI_EXPORT int sharpi_gemm_grouped_tile_rows() { return kPlanTileRows; }

@@ -365,8 +365,8 @@ __global__ __launch_bounds__(GW* kWave, 2) void grouped_gemm_kernel(
   const int home = blockIdx.x % kXcds;
   const int per_xcd = ((int)gridDim.x + kXcds - 1) / kXcds;   // blocks whose first walk is one XCD's
   const int lane = threadIdx.x & (kWave - 1);
-  // The plan counts siblings of kPlanTileRows rows; here a group's rows are cut into tiles of GM (the deal stays level, and
-  // the tall tiles, which take longest, still come first in a walk).
+  // The plan counts siblings of kPlanTileRows rows; here a group's rows are cut into tiles of GM, or half of that where the
+  // walk has little work (the deal stays level, and the tall tiles, which take longest, still come first in a walk).
   auto offset_of = [&](int e) { return n_groups < kOffsetsKept ? s_offset[e] : group_offsets[e]; };
   auto siblings_of = [&](int e, int rows) { return (offset_of(e + 1) - offset_of(e) + rows - 1) / rows; };
   auto unit_slots = [&](const int* pu, int rows) {

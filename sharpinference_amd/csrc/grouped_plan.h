@@ -2,12 +2,16 @@
 // kernel and read by the product's blocks; the host never learns the routing.
 //
 // A *group* is an expert (or the always-on expert that shares the experts' tensor, or a dense
-// matrix taken as a single group).  A group's rows are cut into as few row tiles of at most
-// kPlanTileRows as hold them, all of one height (a multiple of 32): its *siblings*.  Its column
-// blocks are cut into `parts` ranges, more of them the more siblings it has (plan_parts), and a
-// *unit* is (group, part): the blocks of a unit multiply the same weight rows by the group's
-// sibling tiles.  Units are dealt to the 8 XCDs (each with an L2 of its own), the heaviest first,
-// and every XCD walks its units one after the other; inside a unit the siblings of one column
+// matrix taken as a single group).  What a group weighs in the deal is counted in row tiles of at
+// most kPlanTileRows, as few as hold its rows: its *siblings*.  Its column blocks are cut into
+// `parts` ranges, more of them the more siblings it has (plan_parts), and a *unit* is (group,
+// part): the blocks of a unit multiply the same weight rows by the group's row tiles.  Units are
+// dealt to the 8 XCDs (each with an L2 of its own), the heaviest first, and every XCD walks its
+// units one after the other.
+//
+// The product reads the units and their order and cuts a group's rows into tiles of its own, of
+// twice that height (or of that height, gemm_grouped_kernel.h), all of a group's of one height (a
+// multiple of 32): the tall ones come first in a walk either way.  Inside a unit the tiles of one column
 // block are neighbours.  Blocks go to XCDs round-robin by their linear id, so block b is slot
 // b / 8 of XCD b % 8: sibling blocks start together on one XCD and stream the same weight rows at
 // the same pace, and what the first fetches from memory the others find in that XCD's L2.
@@ -20,9 +24,7 @@
 //
 // plan (int32), per XCD x at plan + x * plan_stride(G), G groups:
 //   [0]                      units of this XCD
-//   [1 + 4j .. 4 + 4j]       unit j: group, part, parts, siblings
-// The product of bfloat16 rows reads the units and their order, and cuts a group's rows into tiles of its own, twice as tall: the
-// tall ones come first in a walk either way, and units of three or four siblings here have as many slots as those of one.
+//   [1 + 4j .. 4 + 4j]       unit j: group, part, parts, siblings (what the deal was weighed by)
 #pragma once
 
 constexpr int kPlanXcds = 8;

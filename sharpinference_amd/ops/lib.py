@@ -208,8 +208,8 @@ def delta_chunk_floats(n_chunks: int, nh: int, dk: int, dv: int) -> int:
 
 
 def grouped_tile_rows() -> int:
-    """Rows of the tallest tile of the grouped product for many rows (an expert with more rows is
-    cut into sibling tiles): the library says what it was built with."""
+    """Rows of the tiles that the plan of the grouped product for many rows counts a group's load in (the product itself
+    cuts tiles of its own, up to twice as tall): the library says what it was built with."""
     if "tile_rows" not in _takes:
         fn = load().sharpi_gemm_grouped_tile_rows
         fn.argtypes, fn.restype = [], c_int

@@ -13,8 +13,9 @@ from ..ops.profile import section
 from ..cache.spec import KVSpec, MixedSpec, StateSpec, kv_of, WINDOW_CHUNK, WINDOW_NONE, WINDOW_SLIDING  # noqa: F401
 from .base import INIT_NORM_WEIGHT, HostStep, LayerCache, ParamSpec, Part, StepContext, StepPlanner, TensorSource
 
-SHORT_PROMPT_TOKENS = 1536   # up to so many prompt tokens in a step, tiles of half as many tokens (measured:
-                             # 20-25 % less attention time from 512 to 1,536 tokens, 6 % more at 2,048)
+SHORT_PROMPT_TOKENS = 1536   # up to so many prompt tokens in a step, tiles of half as many tokens.  Measured at 16 heads of 128,
+                             # us of tiles of 64 and of 128: 200 tokens 12 / 16, 1,000 41 / 55, 1,536 57 / 65; eight sizes of 8 to 40
+                             # heads: 14 to 65 % more with 128, but level for 40 heads from 1,200 tokens on (72 / 73 at 1,536).
 
 
 def prompt_tile_tokens(lens) -> int:

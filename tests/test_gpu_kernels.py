@@ -353,8 +353,8 @@ def test_router_and_permute(T, E, k, H, dtype):
 
 
 def _check_plan(ops, rt, counts):
-    """The plan of the grouped product for many rows: every group with rows is cut into sibling
-    row tiles (as few of the library's tile height as hold its rows) and its column blocks into
+    """The plan of the grouped product for many rows: every group with rows is weighed by its sibling
+    row tiles (as few of the plan's tile height as hold its rows; the product cuts its own) and its column blocks are cut into
     parts (2, 4, 8 or 16: more the more siblings); every (group, part) unit appears once, on one of
     the 8 XCDs, the heaviest units dealt first so that the XCDs' loads stay level.  Behind the
     units lie the ticket counters of the product's blocks, zero when the plan is made."""
