@@ -14,7 +14,10 @@ from .base import INIT_NORM_WEIGHT, HostStep, LayerCache, ParamSpec, Part, StepC
 CHUNK_FROM_TOKENS = 64        # a step whose longest entry has this many tokens gets the segments' work lists of layers that
                               # may run segments as matrix products
 SEGMENT_FROM_TOKENS = 512     # ... layers that walk segments token by token take them from this many tokens on,
-SEGMENT_UP_TO_BLOCKS = 2048   # ... while whole entries would give fewer blocks than this
+SEGMENT_UP_TO_BLOCKS = 2048   # ... while whole entries would give fewer blocks than this.  Both lines are those of segments that are walked;
+                              # gated linear attention's as products win on either side (16 heads of 128, us walked whole and as
+                              # products: 384 tokens 148 / 103, 512 194 / 105; 1,900 beside 7 single tokens, 2,048 blocks, 698 / 167), but
+                              # lose below 256 tokens (128: 53 / 74) and short of 512 behind many single ones (384 and 31: 149 / 174)
 
 
 class EntrySpans(NamedTuple):
