@@ -14,6 +14,7 @@
 // value column); slot = page * page_size + offset;
 // a negative slot means "do not store" (the layer reads another layer's cache).
 #include "common.h"
+#include "value_pages.h"
 
 template <typename T>
 __global__ void rope_kv_kernel(const T* __restrict__ qkv, T* __restrict__ q_out, T* __restrict__ k_cache,
@@ -124,36 +125,70 @@ __global__ void rope_kv_kernel(const T* __restrict__ qkv, T* __restrict__ q_out,
   }
 }
 
-// The same for head sizes 32, 64, 128, 256 with interleaved pairs and a rotary width that is a
-// multiple of 8 (runs beyond it pass through): a thread per run of 8 elements (4 rotary pairs),
-// 16-byte accesses; the hd/8 lanes of a head are neighbours in a wave and sum their squares with
-// shuffles.  Blocks (token, y) share a token's heads between them, 256 runs each, so that a
-// handful of decode tokens still spreads over many compute units.
+// The same for head sizes 32, 64, 128, 256 whose rotary width is a multiple of 8 (pairs split in halves: of 16; runs beyond it
+// pass through): a thread per run of 8 elements, 16-byte accesses; the hd/8 lanes of a head are neighbours in a wave, sum their
+// squares with shuffles and hand each other the partners of split pairs.  Blocks (token, y) share a token's heads between
+// them, 256 runs each, so that a handful of decode tokens still spreads over many compute units.  The token's angles are the
+// same for every head: a block computes each of them once, into LDS (four sines and cosines in every thread were the kernel's
+// time).  Steps of many tokens leave the values to blocks of their own behind the tokens' (value_pages.h).
+// Bound: the rows' bytes.  40 + 8 heads of 128 and 8 of values, us: 2,048 tokens 30 -> 17.8, 8,192 104 -> 54.7 (235 MB: 4.3 TB/s, about
+// a copy's rate); 16 + 4 heads with split pairs, 1,950 tokens (a wave a head before) 20.9 -> 12.2.
+constexpr int kRopeMaxAngles = 128;              // hd <= 256
+constexpr int kRopeSplitTokens = 64;             // up to so many tokens a step, a token's heads lie in several blocks
+
 template <typename T>
 __global__ __launch_bounds__(256) void rope_kv_vec_kernel(
     const T* __restrict__ qkv, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache,
     const int* __restrict__ slot_mapping, const int* __restrict__ positions, const float* __restrict__ inv_freq,
     const float* __restrict__ bias, int qk_norm, float eps, int temp_tuning, float floor_scale, float attn_scale,
-    int nh, int nkv, int hd, int page_size, int rotary_dim, int row_stride) {
+    int n_tokens, int nh, int nkv, int hd, int vd, int page_size, int half_split, int rotary_dim, int row_stride, int values_apart) {
+  __shared__ __attribute__((aligned(16))) char tile[kValueLds<T>];
+  __shared__ int tile_slots[kValueTokens];
+  __shared__ float cs_tab[kRopeMaxAngles], sn_tab[kRopeMaxAngles];
+  if (blockIdx.x >= n_tokens) {                    // (values_apart: the blocks behind the tokens')
+    const size_t v_at = (size_t)(nh + nkv) * hd;
+    values_to_pages<T>(blockIdx.x - n_tokens, n_tokens, nkv, vd, page_size, slot_mapping, v_cache, reinterpret_cast<T*>(tile), tile_slots,
+                       [&](int t, int c, float* v) {
+      load8(qkv + (size_t)t * row_stride + v_at + c, v);
+      if (bias) {
+        float b8[8];
+        load8(bias + v_at + c, b8);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] += b8[j];
+      }
+    });
+    return;
+  }
   const int t = blockIdx.x;
   const int per_head = hd >> 3;                    // lanes per head: 4, 8, 16 or 32
-  const int chunks = (nh + 2 * nkv) * per_head;
+  const int chunks = (nh + (values_apart ? nkv : 2 * nkv)) * per_head;
   const int pos = positions[t];
   const int slot = slot_mapping[t];
   const T* src = qkv + (size_t)t * row_stride;
   float post = 1.0f;
   if (temp_tuning) post = 1.0f + attn_scale * logf(floorf(((float)pos + 1.0f) / floor_scale) + 1.0f);
+  if (inv_freq) {
+    if (threadIdx.x < rotary_dim / 2) {
+      const float ang = (float)pos * inv_freq[threadIdx.x];
+      cs_tab[threadIdx.x] = cosf(ang);
+      sn_tab[threadIdx.x] = sinf(ang);
+    }
+    __syncthreads();
+  }
   // a thread's run within a head is the same in every turn of the loop (the block size is a multiple
-  // of the lanes per head), and so are its four angles: their sines and cosines are computed once
+  // of the lanes per head), and so are its angles: x becomes x cs + (its partner) sn
   const int run = threadIdx.x % per_head;
-  float cs[4], sn[4];
+  const int half_runs = rotary_dim / 16;           // (split pairs: runs of the low half)
+  float cs[8], sn[8];
   const bool rotates = inv_freq != nullptr && run * 8 < rotary_dim;
+  const bool low = run < half_runs;
+  const int mate = (threadIdx.x & (kWave - 1)) + (low ? half_runs : -half_runs);
   if (rotates) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const float ang = (float)pos * inv_freq[run * 4 + j];
-      cs[j] = cosf(ang);
-      sn[j] = sinf(ang);
+    for (int j = 0; j < 8; ++j) {
+      const int i = half_split ? (low ? run : run - half_runs) * 8 + j : run * 4 + j / 2;
+      cs[j] = cs_tab[i];
+      sn[j] = (half_split ? low : j % 2 == 0) ? -sn_tab[i] : sn_tab[i];
     }
   }
   for (int base = blockIdx.y * blockDim.x; base < chunks; base += gridDim.y * blockDim.x) {
@@ -173,19 +208,25 @@ __global__ __launch_bounds__(256) void rope_kv_vec_kernel(
       }
     }
     float ss = 0.f;
-    if (valid && (is_q || is_k)) {
-      if (rotates) {
+    if (half_split && inv_freq) {      // every lane takes part in the shuffles
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float a = x[2 * j], b = x[2 * j + 1];
-          x[2 * j] = a * cs[j] - b * sn[j];
-          x[2 * j + 1] = a * sn[j] + b * cs[j];
-        }
+      for (int j = 0; j < 8; ++j) {
+        const float other = __shfl(x[j], mate & (kWave - 1), kWave);
+        if (rotates && (is_q || is_k)) x[j] = x[j] * cs[j] + other * sn[j];
       }
+    } else if (rotates && (is_q || is_k)) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
+      for (int j = 0; j < 4; ++j) {
+        const float a = x[2 * j], b = x[2 * j + 1];
+        x[2 * j] = a * cs[2 * j] + b * sn[2 * j];
+        x[2 * j + 1] = a * sn[2 * j + 1] + b * cs[2 * j];
+      }
     }
-    if (qk_norm) {   // every lane takes part in the shuffles
+    if (qk_norm) {
+      if (valid && (is_q || is_k)) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
+      }
       for (int off = per_head >> 1; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
       const float mul = 1.0f / sqrtf(ss / (float)hd + eps);
       if (is_q || is_k) {
@@ -233,21 +274,21 @@ SHARPI_EXPORT int sharpi_rope_kv(const void* qkv, void* q_out, void* k_cache, vo
   if (temp_tuning && !(floor_scale > 0.f)) return SHARPI_ERR_ARG;
   dim3 grid(n_tokens, nh + 2 * nkv), block(kWave);
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
-  if ((hd == 32 || hd == 64 || hd == 128 || hd == 256) && vd == hd && pair_layout == 0 && (rotary_dim & 7) == 0 &&
-      (row_stride & 7) == 0) {
-    // a few tokens (decode): a token's heads over several blocks, for the compute units' sake;
-    // many tokens: one block per token, which then computes its angles once for all heads
-    const dim3 vgrid(n_tokens, n_tokens <= 64 ? ceil_div((nh + 2 * nkv) * (hd >> 3), 256) : 1);
-    if (dtype == DT_F32)
-      rope_kv_vec_kernel<float><<<vgrid, 256, 0, stream>>>((const float*)qkv, (float*)q_out, (float*)k_cache,
-                                                             (float*)v_cache, slot_mapping, positions, inv_freq,
-                                                             bias, qk_norm, eps, temp_tuning, floor_scale, attn_scale,
-                                                             nh, nkv, hd, page_size, rotary_dim, row_stride);
-    else
-      rope_kv_vec_kernel<bf16_t><<<vgrid, 256, 0, stream>>>((const bf16_t*)qkv, (bf16_t*)q_out,
-                                                              (bf16_t*)k_cache, (bf16_t*)v_cache, slot_mapping,
-                                                              positions, inv_freq, bias, qk_norm, eps, temp_tuning,
-                                                              floor_scale, attn_scale, nh, nkv, hd, page_size, rotary_dim, row_stride);
+  // few tokens (decode): a token's heads over several blocks, for the compute units' sake; many tokens: one block
+  // per token, which then computes its angles once for all heads, and blocks of their own for the values
+  const bool many = n_tokens > kRopeSplitTokens;
+  const auto at16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  if ((hd == 32 || hd == 64 || hd == 128 || hd == 256) && (vd == hd || (many && vd % 8 == 0)) &&
+      rotary_dim % (pair_layout ? 16 : 8) == 0 && (row_stride & 7) == 0 && at16(qkv) && at16(q_out) && at16(k_cache) && at16(bias)) {
+    const int tiles = many ? value_tiles(n_tokens, nkv * vd) : 0;
+    const dim3 vgrid(n_tokens + tiles, many ? 1 : ceil_div((nh + 2 * nkv) * (hd >> 3), 256));
+#define ROPE_GO(T)                                                                                                               \
+  rope_kv_vec_kernel<T><<<vgrid, 256, 0, stream>>>((const T*)qkv, (T*)q_out, (T*)k_cache, (T*)v_cache, slot_mapping, positions, inv_freq, \
+                                                   bias, qk_norm, eps, temp_tuning, floor_scale, attn_scale, n_tokens, nh, nkv, hd, vd,   \
+                                                   page_size, pair_layout, rotary_dim, row_stride, many)
+    if (dtype == DT_F32) ROPE_GO(float);
+    else ROPE_GO(bf16_t);
+#undef ROPE_GO
     SHARPI_CHECK_LAUNCH();
     return SHARPI_OK;
   }

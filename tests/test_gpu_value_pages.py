@@ -1,0 +1,55 @@
+"""Steps of many tokens turn their values into the cache's pages in blocks of their own: the same bits as the same tokens in
+portions small enough to go token by token."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+DT = {"float32": torch.float32, "bfloat16": torch.bfloat16}
+
+
+def _slots(kind, T, pages, ps, g):
+    """A prompt's pages in shuffled order from the first place on, or from another, tokens anywhere, or some not stored."""
+    if kind in ("pages", "shifted"):
+        first = 0 if kind == "pages" else 5
+        order = torch.randperm(pages, generator=g)
+        place = torch.arange(T) + first
+        return (order[place // ps] * ps + place % ps).to(torch.int32)
+    slots = torch.randperm(pages * ps, generator=g)[:T].to(torch.int32)
+    if kind == "holes":
+        slots[torch.rand(T, generator=g) < 0.4] = -1
+    return slots if kind != "none" else torch.full((T,), -1, dtype=torch.int32)
+
+
+CASES = [("pages", 65, 16, 128), ("pages", 200, 32, 64), ("shifted", 83, 16, 128), ("shifted", 131, 48, 72), ("anywhere", 96, 16, 136),
+         ("holes", 79, 16, 8), ("none", 70, 16, 128), ("pages", 130, 16, 24)]
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("kind, T, ps, vd", CASES)
+@pytest.mark.parametrize("layout", [0, 1])
+def test_rotated_heads_and_values_of_a_long_step(kind, T, ps, vd, layout, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(T + vd)
+    nh, nkv, hd, r, pages = 5, 3, 128, 32, T // ps + 3
+    width = (nh + nkv) * hd + nkv * vd
+    qkv = torch.randn(T, width + 8, generator=g).to(DT[dtype]).to(DEV)
+    bias = torch.randn(width, generator=g).to(DEV) if T % 2 else None
+    freq = torch.tensor([300.0 ** (-2.0 * i / r) for i in range(r // 2)], device=DEV)
+    slots = _slots(kind, T, pages, ps, g).to(DEV)
+    pos = (torch.arange(T) * 7).to(torch.int32).to(DEV)
+    got, caches = [], []
+    for portion in (T, 50):
+        kc = torch.zeros(pages, nkv, ps, hd, dtype=DT[dtype], device=DEV)
+        vc = torch.zeros(pages, nkv, vd, ps, dtype=DT[dtype], device=DEV)
+        out = [ops.rope_kv(qkv[i:i + portion], kc, vc, slots[i:i + portion], pos[i:i + portion], freq, True, 1e-5, (40.0, 0.1), nh, nkv, hd,
+                           layout, bias, vd, 8) for i in range(0, T, portion)]
+        got.append(torch.cat(out).float())
+        caches.append((kc.float(), vc.float()))
+    assert torch.equal(caches[0][1], caches[1][1])
+    # where heads and values differ in width the portions take the general kernel, which sums the squares in another order: eight
+    # roundings of the sum, halved by the root, and in bfloat16 (8 bits) two sides of a boundary: one place, 2^-7 of a value
+    tol = 0.0 if vd == hd else 8 * 2.0 ** -24 if dtype == "float32" else 2.0 ** -7
+    for a, b in ((got[0], got[1]), (caches[0][0], caches[1][0])):
+        assert bool(((a - b).abs() <= tol * (a.abs() + a.abs().max() * 2.0 ** -4)).all())
