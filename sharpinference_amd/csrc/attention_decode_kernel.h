@@ -174,8 +174,8 @@ __global__ __launch_bounds__(kDecWaves* kWave) void attn_decode_kernel(
         s[u][i] = ok ? sc : -INFINITY;
         cm = fmaxf(cm, s[u][i]);
       }
-    cm = fmaxf(cm, __shfl_xor(cm, 16, kWave));
-    cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
+    cm = reduce16(cm, MaxOf{});
+    cm = reduce32(cm, MaxOf{});
     const float m_new = fmaxf(m, cm);
     float corr = 1.0f;
     bf16x8 pf, pf_lo;   // probabilities as a bfloat16 pair hi + lo: ~16 bits survive the product

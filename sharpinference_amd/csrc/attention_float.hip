@@ -124,8 +124,8 @@ __global__ __launch_bounds__(kFlWaves* kWave) void attn_float_kernel(FloatAttent
       hidden |= seen ? 0 : 1 << x;
       mb = fmaxf(mb, sc[x]);
     }
-    mb = fmaxf(mb, __shfl_xor(mb, 16, kWave));
-    mb = fmaxf(mb, __shfl_xor(mb, 32, kWave));
+    mb = reduce16(mb, MaxOf{});
+    mb = reduce32(mb, MaxOf{});
     const float m_new = fmaxf(m, mb);
     const float ref = m_new > -INFINITY ? m_new : 0.f;         // (nothing seen yet: every term is exp(-inf) = 0)
     const float corr = expf(m - ref);
@@ -169,8 +169,8 @@ __global__ __launch_bounds__(kFlWaves* kWave) void attn_float_kernel(FloatAttent
 #pragma unroll
       for (int x = 0; x < 4; ++x) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[d][x], pe[x], acc[d], 0, 0, 0);
   }
-  l += __shfl_xor(l, 16, kWave);                               // the row's four lanes hold a quarter of its keys each
-  l += __shfl_xor(l, 32, kWave);
+  l = reduce16(l, SumOf{});                               // the row's four lanes hold a quarter of its keys each
+  l = reduce32(l, SumOf{});
 #pragma unroll
   for (int d = 0; d < ND; ++d) acc_s[w][d][lane] = acc[d];
   if (g == 0) {

@@ -43,7 +43,7 @@ struct LmGeom {
 };
 
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-  return (uint32_t)f32_to_bf16(a).bits | ((uint32_t)f32_to_bf16(b).bits << 16);
+  return f32_to_bf16_pair(a, b);
 }
 
 // the first key a query at position p sees (window 0: all earlier ones)
@@ -215,8 +215,8 @@ __global__ __launch_bounds__(kLmWaves* kWave, S == 8 ? 4 : 2) void attn_latent_m
         sv[4 * u + i] = ok ? s[u][i] * scale : -INFINITY;
         mx = fmaxf(mx, sv[4 * u + i]);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, kWave));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+    mx = reduce16(mx, MaxOf{});
+    mx = reduce32(mx, MaxOf{});
     const float m_new = fmaxf(m_run, mx);
     const float corr = m_run > -INFINITY ? expf(m_run - m_new) : 0.f;
     float pe[8], ps = 0.f;
@@ -225,8 +225,8 @@ __global__ __launch_bounds__(kLmWaves* kWave, S == 8 ? 4 : 2) void attn_latent_m
       pe[i] = sv[i] > -INFINITY ? expf(sv[i] - m_new) : 0.f;
       ps += pe[i];
     }
-    ps += __shfl_xor(ps, 16, kWave);
-    ps += __shfl_xor(ps, 32, kWave);
+    ps = reduce16(ps, SumOf{});
+    ps = reduce32(ps, SumOf{});
     l_run = l_run * corr + ps;
     m_run = m_new;
     uint4 hi, lo;

@@ -283,8 +283,8 @@ __global__ __launch_bounds__(kPreWaves* kWave, (prefill_waves_a_simd<HD, VD>()))
 #pragma unroll
       for (int c = 0; c < kQT; ++c) {
         float cm = lmax[c];
-        cm = fmaxf(cm, __shfl_xor(cm, 16, kWave));
-        cm = fmaxf(cm, __shfl_xor(cm, 32, kWave));
+        cm = reduce16(cm, MaxOf{});
+        cm = reduce32(cm, MaxOf{});
         const bool move = cm - m[c] > kLazyMax;
         const float corr = move ? __builtin_amdgcn_exp2f(m[c] - cm) : 1.0f;
         m[c] = move ? cm : m[c];
@@ -366,8 +366,8 @@ __global__ __launch_bounds__(kPreWaves* kWave, (prefill_waves_a_simd<HD, VD>()))
 #pragma unroll
   for (int c = 0; c < kQT; ++c) {
     float L = l[c];
-    L += __shfl_xor(L, 16, kWave);
-    L += __shfl_xor(L, 32, kWave);
+    L = reduce16(L, SumOf{});
+    L = reduce32(L, SumOf{});
     if (!qok[c]) continue;
     // a key of score 0 (or of the head's learned score) without a value: 2^(score log2 e - reference) more
     if (sink) L += __builtin_amdgcn_exp2f((sink_vals ? sink_vals[h] * 1.4426950408889634f : 0.f) - m[c]);
@@ -380,8 +380,8 @@ __global__ __launch_bounds__(kPreWaves* kWave, (prefill_waves_a_simd<HD, VD>()))
       // lane holds O^T[d*16 + 4g + i][query row]
       const f32x4 o = acc[c][d] * inv;
       uint2 packed;
-      packed.x = (uint32_t)f32_to_bf16(o[0]).bits | ((uint32_t)f32_to_bf16(o[1]).bits << 16);
-      packed.y = (uint32_t)f32_to_bf16(o[2]).bits | ((uint32_t)f32_to_bf16(o[3]).bits << 16);
+      packed.x = f32_to_bf16_pair(o[0], o[1]);
+      packed.y = f32_to_bf16_pair(o[2], o[3]);
       *reinterpret_cast<uint2*>(orow + d * 16 + 4 * g) = packed;
     }
   }

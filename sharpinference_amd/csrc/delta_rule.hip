@@ -129,8 +129,8 @@ __global__ __launch_bounds__(256) void lowrank_kernel(const float* __restrict__ 
         *reinterpret_cast<f32x4*>((float*)jb.out + at) = acc[a];
       } else {
         uint2 o;
-        o.x = (uint32_t)f32_to_bf16(acc[a][0]).bits | ((uint32_t)f32_to_bf16(acc[a][1]).bits << 16);
-        o.y = (uint32_t)f32_to_bf16(acc[a][2]).bits | ((uint32_t)f32_to_bf16(acc[a][3]).bits << 16);
+        o.x = f32_to_bf16_pair(acc[a][0], acc[a][1]);
+        o.y = f32_to_bf16_pair(acc[a][2], acc[a][3]);
         *reinterpret_cast<uint2*>((T*)jb.out + at) = o;
       }
       continue;
@@ -293,10 +293,10 @@ __global__ __launch_bounds__(512, NT <= 8 ? 4 : 2) void delta_step_kernel(DeltaI
       }
       if (n % 2) __builtin_amdgcn_sched_barrier(0);      // (all tiles' operands read ahead would not fit the registers)
     }
-    dotk += __shfl_xor(dotk, 16, kWave);
-    dotq += __shfl_xor(dotq, 16, kWave);
-    dotk += __shfl_xor(dotk, 32, kWave);
-    dotq += __shfl_xor(dotq, 32, kWave);
+    dotk = reduce16(dotk, SumOf{});
+    dotq = reduce16(dotq, SumOf{});
+    dotk = reduce32(dotk, SumOf{});
+    dotq = reduce32(dotq, SumOf{});
     const int c = strip * 16 + j;
     const float u = c < a.dv ? beta * (vo_s[c] - dotk * ks) : 0.f;
     if (g == 0 && c < a.dv) o_s[c] = fmaf(u, kq, dotq * qs);

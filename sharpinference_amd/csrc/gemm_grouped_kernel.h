@@ -293,8 +293,8 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
       *reinterpret_cast<f32x4*>(dst) = v;
     } else {
       uint2 packed;
-      packed.x = (uint32_t)f32_to_bf16(v[0]).bits | ((uint32_t)f32_to_bf16(v[1]).bits << 16);
-      packed.y = (uint32_t)f32_to_bf16(v[2]).bits | ((uint32_t)f32_to_bf16(v[3]).bits << 16);
+      packed.x = f32_to_bf16_pair(v[0], v[1]);
+      packed.y = f32_to_bf16_pair(v[2], v[3]);
       *reinterpret_cast<uint2*>(dst) = packed;
     }
   };

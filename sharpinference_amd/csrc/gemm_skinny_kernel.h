@@ -50,8 +50,8 @@ template <> __device__ __forceinline__ void store4<float>(float* p, f32x4 v) {
 }
 template <> __device__ __forceinline__ void store4<bf16_t>(bf16_t* p, f32x4 v) {
   uint2 packed;
-  packed.x = (uint32_t)f32_to_bf16(v[0]).bits | ((uint32_t)f32_to_bf16(v[1]).bits << 16);
-  packed.y = (uint32_t)f32_to_bf16(v[2]).bits | ((uint32_t)f32_to_bf16(v[3]).bits << 16);
+  packed.x = f32_to_bf16_pair(v[0], v[1]);
+  packed.y = f32_to_bf16_pair(v[2], v[3]);
   *reinterpret_cast<uint2*>(p) = packed;
 }
 

@@ -338,8 +338,8 @@ __global__ __launch_bounds__(256) void head_gemm_mfma_kernel(const bf16_t* __res
         for (int i = 0; i < 4; ++i) v[i] *= 1.0f / (1.0f + expf(-bf16_to_f32(gate[(size_t)t * ldg + (size_t)h * N + n + i])));
       }
       uint2 o;
-      o.x = (uint32_t)f32_to_bf16(v[0]).bits | ((uint32_t)f32_to_bf16(v[1]).bits << 16);
-      o.y = (uint32_t)f32_to_bf16(v[2]).bits | ((uint32_t)f32_to_bf16(v[3]).bits << 16);
+      o.x = f32_to_bf16_pair(v[0], v[1]);
+      o.y = f32_to_bf16_pair(v[2], v[3]);
       *reinterpret_cast<uint2*>(out + (size_t)t * ldo + (size_t)h * so + n) = o;
     }
   }

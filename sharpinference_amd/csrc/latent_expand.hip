@@ -136,8 +136,8 @@ __global__ __launch_bounds__(kExpThreads, 2) void latent_expand_kernel(
   };
   auto pack = [](const f32x4& v) {
     uint2 o;
-    o.x = (uint32_t)f32_to_bf16(v[0]).bits | ((uint32_t)f32_to_bf16(v[1]).bits << 16);
-    o.y = (uint32_t)f32_to_bf16(v[2]).bits | ((uint32_t)f32_to_bf16(v[3]).bits << 16);
+    o.x = f32_to_bf16_pair(v[0], v[1]);
+    o.y = f32_to_bf16_pair(v[2], v[3]);
     return o;
   };
   if (values) {                                     // (the same for the whole block)
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(256) void latent_queries_kernel(const bf16_t* __res
         const int pair = (c - dn) / 2 + i;
         if (pair < n_pairs) {
           const float a = bf16_bits_to_f32(x[i] & 0xffffu), b = bf16_bits_to_f32(x[i] >> 16);
-          x[i] = (uint32_t)f32_to_bf16(a * cs[pair] - b * sn[pair]).bits | ((uint32_t)f32_to_bf16(b * cs[pair] + a * sn[pair]).bits << 16);
+          x[i] = f32_to_bf16_pair(a * cs[pair] - b * sn[pair], b * cs[pair] + a * sn[pair]);
         }
       }
     }

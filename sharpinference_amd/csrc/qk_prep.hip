@@ -395,7 +395,7 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_run_kernel(PrepArgs a, i
       float ss = 0.f;
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss = fmaf(x[j], x[j], ss);
-      for (int o = lanes >> 1; o > 0; o >>= 1) ss += __shfl_xor(ss, o, kWave);
+      ss = group_sum(ss, lanes);
       const float inv = rsqrtf(ss / (float)a.hd + a.eps);
       if (live) {
 #pragma unroll

@@ -227,7 +227,7 @@ __global__ __launch_bounds__(256) void rope_kv_vec_kernel(
 #pragma unroll
         for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
       }
-      for (int off = per_head >> 1; off > 0; off >>= 1) ss += __shfl_xor(ss, off, kWave);
+      ss = group_sum(ss, per_head);
       const float mul = 1.0f / sqrtf(ss / (float)hd + eps);
       if (is_q || is_k) {
 #pragma unroll

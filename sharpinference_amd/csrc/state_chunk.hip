@@ -235,8 +235,8 @@ __device__ __forceinline__ void segment_state(const SegWeights& w, const KT* k_s
     *reinterpret_cast<float4*>(to + at + (size_t)(2 * ct) * slice) = x;
   }
   if (MODE == WALK_EXP_GATES && ct0 == 0) {
-    nsum += __shfl_xor(nsum, 16, kWave);
-    nsum += __shfl_xor(nsum, 32, kWave);
+    nsum = reduce16(nsum, SumOf{});
+    nsum = reduce32(nsum, SumOf{});
     const int n_at = NOFF + ((r >> 2) * 8 + g8) * 4 + (r & 3);
     if (from) nsum = fmaf(keep, from[n_at], nsum);
     for (int cb = g; cb < 2 * NCT; cb += 4) to[(size_t)cb * slice + n_at] = nsum;     // (every slice has its copy)
@@ -442,8 +442,8 @@ __device__ __forceinline__ void state_chunk_final_block(const WalkArgs& a) {
     if (plain < qt) keys(qt, std::true_type{});
     float inv = 1.f;
     if (MODE == WALK_EXP_GATES) {
-      den += __shfl_xor(den, 16, kWave);
-      den += __shfl_xor(den, 32, kWave);
+      den = reduce16(den, SumOf{});
+      den = reduce32(den, SumOf{});
       inv = fmaxf(fabsf(den), w.e[t]) + kWalkFloor;
     }
     if (t < nt) {

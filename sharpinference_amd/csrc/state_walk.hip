@@ -274,14 +274,14 @@ __global__ __launch_bounds__(kWave) void state_walk_kernel(
         }
       }
       if (PHASE == WALK_LOCAL) continue;
-      acc += __shfl_xor(acc, 8, kWave);
-      acc += __shfl_xor(acc, 16, kWave);
-      acc += __shfl_xor(acc, 32, kWave);
+      acc += row_rotated<8>(acc);
+      acc = reduce16(acc, SumOf{});
+      acc = reduce32(acc, SumOf{});
       float y;
       if (MODE == WALK_EXP_GATES) {
-        nq += __shfl_xor(nq, 8, kWave);
-        nq += __shfl_xor(nq, 16, kWave);
-        nq += __shfl_xor(nq, 32, kWave);
+        nq += row_rotated<8>(nq);
+        nq = reduce16(nq, SumOf{});
+        nq = reduce32(nq, SumOf{});
         y = acc / (fmaxf(fabsf(nq), e_s[tt]) + kWalkFloor);
       } else if (MODE == WALK_FIXED_DECAY) {
         y = acc;
