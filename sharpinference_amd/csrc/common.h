@@ -72,6 +72,24 @@ __device__ __forceinline__ void store8(bf16_t* p, const float* v) {
   *reinterpret_cast<uint4*>(p) = o;
 }
 
+// Eight neighbouring elements as they lie in memory.
+template <typename T> struct Run8;
+template <> struct Run8<float> {
+  float4 a, b;
+  __device__ __forceinline__ void load(const float* p) {
+    a = *reinterpret_cast<const float4*>(p);
+    b = *reinterpret_cast<const float4*>(p + 4);
+  }
+  __device__ __forceinline__ void floats(float (&v)[8]) const {
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  }
+};
+template <> struct Run8<bf16_t> {
+  uint4 a;
+  __device__ __forceinline__ void load(const bf16_t* p) { a = *reinterpret_cast<const uint4*>(p); }
+  __device__ __forceinline__ void floats(float (&v)[8]) const { load8(reinterpret_cast<const bf16_t*>(&a), v); }
+};
+
 // The gated unit of a feed-forward, one element: act(s g) * (s u), with the activation a code that
 // the caller passes (shared with the Python side): SiLU x / (1 + exp(-x)), or GELU in its tanh form
 // 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3))).  One definition for the activation kernel and

@@ -13,6 +13,7 @@
 // attention kernel over keys of the head's width computes each map's scores on its own; and values mixed with
 // those of another layer, (1 - c) v + c v_other, in float on their way into the cache.
 //
+// Rows of widths and offsets that are multiples of 8 go to qk_prep_run_kernel; the others, and norms over more than 1,024 runs of 8, as follows.
 // One block per token, or, in steps of few tokens, one per (token, kv head): the block then takes
 // that kv head's key and value and the query heads that read it, so that a decode step still fills
 // the chip (what a row's sums are made of and their order do not depend on the split).  The token's
@@ -21,6 +22,7 @@
 // sums of squares are taken in an order that depends on the row alone, and everything after the
 // projection is float arithmetic rounded once, on the way out.
 #include "common.h"
+#include "value_pages.h"
 
 constexpr int kPrepThreads = 256;
 constexpr int kPrepMaxTaps = 8;
@@ -60,17 +62,90 @@ struct PrepArgs {
   const void* v_other;     // another layer's projections of the same tokens (null: values as they are)
   int v_other_stride, v_other_off;
   float v_mix;             // c
-  int taps4;               // four taps, their weights on multiples of 16 bytes (with by8)
+  int values_apart;        // values go in blocks of their own behind the tokens' (value_pages.h)
+  int n_tokens;
   int by8;                 // every offset, stride and width a multiple of 8 (and split halves): eight channels a thread
 };
 
 constexpr int kPrepMaxTurns = 256;    // rotary pairs whose cosines and sines a block keeps (a map of up to 512 elements)
+static_assert(kPrepThreads == kValueThreads, "a block of either kind");
 
+// Channels c .. c + 7 of q | k | v of token t, column col of its projected row, through the convolution or with the bias (wide
+// rows).  TAPS: 0 none, 4 four with their weights on multiples of 32 bytes, -1 any number.
+template <typename T, int TAPS>
+__device__ __forceinline__ void prep_gather8(const PrepArgs& a, int t, int c, int col, int C, float* y) {
+  const T* proj = (const T*)a.proj;
+  if constexpr (TAPS != 0) {
+    const int e = a.entry_of_token[t];
+    const int li = t - a.cu_tokens[e];                 // the token's place in its entry
+    if (TAPS == 4 && li >= 3) {
+      // The four rows, as they lie in memory, and the eight channels' weights (32 floats on end, 16 bytes a load) are all requested
+      // before the first is used; a weight and a row at a time the loads' number and latency were the kernel's time
+      // (1900 tokens of 4096 channels: 62 -> 35 us).
+      Run8<T> u[4];
+      float4 cw[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) u[j].load(proj + (size_t)(t - 3 + j) * a.stride + col);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) cw[i] = *reinterpret_cast<const float4*>(a.conv_w + (size_t)(c + i) * 4);
+      float v[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        u[j].floats(v);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) y[i] = fmaf(j == 0 ? cw[i].x : j == 1 ? cw[i].y : j == 2 ? cw[i].z : cw[i].w, v[i], j == 0 ? 0.f : y[i]);
+      }
+      return;
+    }
+    const float* tail = a.tail + (size_t)a.state_slots[e] * (a.taps - 1) * C;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] = 0.f;
+#pragma unroll 1
+    for (int j = 0; j < a.taps; ++j) {
+      const int back = a.taps - 1 - j;                 // this tap reads the row `back` tokens ago
+      float u[8];
+      if (back <= li) load8(proj + (size_t)(t - back) * a.stride + col, u);
+      else load8(tail + (size_t)(a.taps - 1 + li - back) * C + c, u);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) y[i] = fmaf(a.conv_w[(size_t)(c + i) * a.taps + j], u[i], y[i]);
+    }
+    return;
+  }
+  load8(proj + (size_t)t * a.stride + col, y);
+  if (a.bias) {
+    float b8[8];
+    load8(a.bias + c, b8);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) y[i] += b8[i];
+  }
+}
+
+// Values mixed with another layer's: channels c .. c + 7 of the values of token t.
 template <typename T>
+__device__ __forceinline__ void prep_mix8(const PrepArgs& a, int t, int c, float* v) {
+  if (!a.v_other) return;
+  const T* other = (const T*)a.v_other + (size_t)t * a.v_other_stride + a.v_other_off + c;
+  float u[8];
+  load8(other, u);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] = fmaf(1.0f - a.v_mix, v[j], a.v_mix * u[j]);
+}
+
+template <typename T, int TAPS>
 __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
-  extern __shared__ __attribute__((aligned(32))) float row[];          // q | k | v of the token, as floats
+  extern __shared__ __attribute__((aligned(32))) float row[];          // q | k | v of the token, as floats (values apart: q | k)
   __shared__ float red[16];
   __shared__ float inv[kPrepMaxHeads];
+  if (blockIdx.x >= a.n_tokens) {          // (values_apart: the blocks behind the tokens')
+    const bool own = a.v_off >= 0;
+    const int v0 = own ? (a.nh + a.nkv) * a.hd : a.nh * a.hd, all_c = (a.nh + a.nkv) * a.hd + (own ? a.nkv * a.vd : 0);
+    values_to_pages<T>(blockIdx.x - a.n_tokens, a.n_tokens, a.nkv, a.vd, a.page_size, a.slot_mapping, (T*)a.v_cache,
+                       reinterpret_cast<T*>(row), reinterpret_cast<int*>(inv), [&](int tt, int c, float* v) {
+      prep_gather8<T, TAPS>(a, tt, v0 + c, (own ? a.v_off : a.k_off) + c, all_c, v);
+      prep_mix8<T>(a, tt, c, v);
+    });
+    return;
+  }
   const int t = blockIdx.x;
   // the heads this block takes: all, or kv head blockIdx.y with its query heads
   const int per_kv = a.nh / a.nkv;
@@ -91,58 +166,21 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
   };
 
   // 1. gather, through the convolution where there is one
+  const int upto = a.values_apart ? qn + kn : C;
   if (a.by8) {
     // eight consecutive channels a thread, 16-byte loads (the sums of a channel are those of the scalar form)
-    const int e = a.taps > 0 ? a.entry_of_token[t] : 0;
-    const int li = a.taps > 0 ? t - a.cu_tokens[e] : 0;
-    const float* tail = a.taps > 0 ? a.tail + (size_t)a.state_slots[e] * (a.taps - 1) * C : nullptr;
-    for (int c = threadIdx.x * 8; c < C; c += kPrepThreads * 8) {
+    for (int c = threadIdx.x * 8; c < upto; c += kPrepThreads * 8) {
       if (!mine(c)) continue;
       const int col = c < qn ? a.q_off + c : c < qn + kn ? a.k_off + (c - qn) : a.v_off + (c - qn - kn);
       float y[8];
-      if (a.taps4) {
-        // Four taps: the four rows and the eight channels' weights (32 floats on end, 16 bytes a load) are all requested
-        // before the first is used; a weight and a row at a time the loads' number and latency were the kernel's time
-        // (1900 tokens of 4096 channels: 62 -> 35 us).
-        float u[4][8];
-        float4 cw[8];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          if (3 - j <= li) load8(proj + (size_t)(t - 3 + j) * a.stride + col, u[j]);
-          else load8(tail + (size_t)(li + j) * C + c, u[j]);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) cw[i] = *reinterpret_cast<const float4*>(a.conv_w + (size_t)(c + i) * 4);
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          y[i] = fmaf(cw[i].w, u[3][i], fmaf(cw[i].z, u[2][i], fmaf(cw[i].y, u[1][i], fmaf(cw[i].x, u[0][i], 0.f))));
-      } else if (a.taps > 0) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) y[i] = 0.f;
-        for (int j = 0; j < a.taps; ++j) {
-          const int back = a.taps - 1 - j;
-          float u[8];
-          if (back <= li) load8(proj + (size_t)(t - back) * a.stride + col, u);
-          else load8(tail + (size_t)(a.taps - 1 + li - back) * C + c, u);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) y[i] = fmaf(a.conv_w[(size_t)(c + i) * a.taps + j], u[i], y[i]);
-        }
-      } else {
-        load8(proj + (size_t)t * a.stride + col, y);
-        if (a.bias) {
-          float b8[8];
-          load8(a.bias + c, b8);
-#pragma unroll
-          for (int i = 0; i < 8; ++i) y[i] += b8[i];
-        }
-      }
+      prep_gather8<T, TAPS>(a, t, c, col, C, y);
       store8(row + c, y);
     }
   } else if (a.taps > 0) {
     const int e = a.entry_of_token[t];
     const int li = t - a.cu_tokens[e];                 // the token's place in its entry
     const float* tail = a.tail + (size_t)a.state_slots[e] * (a.taps - 1) * C;
-    for (int c = threadIdx.x; c < C; c += kPrepThreads) {
+    for (int c = threadIdx.x; c < upto; c += kPrepThreads) {
       if (!mine(c)) continue;
       const int col = c < qn ? a.q_off + c : c < qn + kn ? a.k_off + (c - qn) : a.v_off + (c - qn - kn);
       float y = 0.f;
@@ -156,7 +194,7 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
       row[c] = y;
     }
   } else {
-    for (int c = threadIdx.x; c < C; c += kPrepThreads) {
+    for (int c = threadIdx.x; c < upto; c += kPrepThreads) {
       if (!mine(c)) continue;
       const int col = c < qn ? a.q_off + c : c < qn + kn ? a.k_off + (c - qn) : a.v_off + (c - qn - kn);
       const float u = to_f32<T>(proj[(size_t)t * a.stride + col]);
@@ -167,14 +205,14 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
 
   // 2. values leave as they are (a layer without a value projection stores its unnormed keys)
   const int slot = a.slot_mapping ? a.slot_mapping[t] : -1;
-  if (slot >= 0) {
+  if (slot >= 0 && !a.values_apart) {
     const int page = slot / a.page_size, off = slot % a.page_size;
     T* vc = (T*)a.v_cache;
     const float* vsrc = own_v ? row + qn + kn : row + qn;
     for (int i = kh0 * a.vd + threadIdx.x; i < kh1 * a.vd; i += kPrepThreads) {
       const int g = i / a.vd, d = i % a.vd;
       float v = vsrc[i];
-      if (a.v_other) v = (1.0f - a.v_mix) * v + a.v_mix * to_f32<T>(((const T*)a.v_other)[(size_t)t * a.v_other_stride + a.v_other_off + i]);
+      if (a.v_other) v = fmaf(1.0f - a.v_mix, v, a.v_mix * to_f32<T>(((const T*)a.v_other)[(size_t)t * a.v_other_stride + a.v_other_off + i]));
       vc[(((size_t)page * a.nkv + g) * a.vd + d) * a.page_size + off] = from_f32<T>(v);
     }
   }
@@ -334,106 +372,151 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
   }
 }
 
-// The same for the plain case (no convolution, one map a head, at most a norm per head, values of their own; widths and
-// offsets multiples of 8, pairs split in halves): nothing is staged.  A head lies in neighbouring lanes of a wave, eight elements
-// a lane (kLanes of them, hd / 8 rounded up to a power of two), its sum of squares and the partner run of a
-// rotation come by lane exchange, 16-byte accesses throughout.  Blocks (token, y) share a token's heads between
-// them; consecutive tokens go to one die, whose cache then gathers the values' columns (a page keeps 16 tokens or more
-// of a value channel side by side).
-template <typename T>
-__global__ __launch_bounds__(kPrepThreads) void qk_prep_run_kernel(PrepArgs a, int n_tokens, int lanes) {
+// The same for rows whose widths and offsets are multiples of 8 (pairs split in halves: the rotated width of 16): nothing is staged.  A head
+// lies in neighbouring lanes of a wave, eight elements a lane (hd / 8 of them rounded up to a power of two); its sum of
+// squares and the partner run of a split rotation come by lane exchange, 16-byte accesses throughout.  A block has a thread for
+// every run of a token's heads where that is at most 1,024 (a norm over the whole projection asks for it), else blocks (token, y) share them; steps of many
+// tokens leave the values to blocks of their own behind the tokens' (value_pages.h).
+// Bound: a block's chain of latencies, so a run is requested before the angles are formed, and the next before one is worked on.  us, staged
+// through LDS before: 16 + 4 heads of 128, 1,900 tokens, norms over the projections 30 -> 13.6, with four taps 35 -> 28.3; two maps a head, 1,664 tokens
+// 18.5 -> 12.7.  64 + 8 heads of 192, 2,048 tokens (a block of 256 for three turns, each behind the one before) 41.8 -> 40.3.
+constexpr int kRunMaxThreads = 1024;
+
+template <typename T, int TAPS>
+__global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run_kernel(PrepArgs a, int log_lanes) {
   __shared__ float cs_tab[kPrepMaxTurns], sn_tab[kPrepMaxTurns];
-  const int per_die = gridDim.x / 8;
-  const int t = (blockIdx.x % 8) * per_die + blockIdx.x / 8;
-  if (t >= n_tokens) return;
+  __shared__ __attribute__((aligned(16))) float red[2][kRunMaxThreads / kWave];
+  __shared__ __attribute__((aligned(16))) char tile[kValueLds<T>];
+  const int qn = a.nh * a.hd, kn = a.nkv * a.hd, runs = a.hd / 8, heads = a.nh + a.nkv;
+  const bool own_v = a.v_off >= 0;
+  const int v_at = own_v ? qn + kn : qn, v_col = own_v ? a.v_off : a.k_off, C = qn + kn + (own_v ? a.nkv * a.vd : 0);
+  if (blockIdx.x >= a.n_tokens) {          // (values_apart: the blocks behind the tokens', y of them side by side)
+    const int v = (blockIdx.x - a.n_tokens) * gridDim.y + blockIdx.y;
+    if (v < value_tiles(a.n_tokens, a.nkv * a.vd))
+      values_to_pages<T>(v, a.n_tokens, a.nkv, a.vd, a.page_size, a.slot_mapping, (T*)a.v_cache, reinterpret_cast<T*>(tile),
+                         reinterpret_cast<int*>(cs_tab), [&](int tt, int c, float* x) {
+        prep_gather8<T, TAPS>(a, tt, v_at + c, v_col + c, C, x);
+        prep_mix8<T>(a, tt, c, x);
+      });
+    return;
+  }
+  const int t = blockIdx.x;
+  // a thread's run inside a head is the same in every turn
+  const int li = threadIdx.x & ((1 << log_lanes) - 1);
+  const bool in = li < runs;
+  int base = blockIdx.y * blockDim.x;
+  Run8<T> raw;                             // (without a convolution) the next turn's run, on its way
+  const auto column = [&](int h) { return (h < a.nh ? a.q_off + h * a.hd : a.k_off + (h - a.nh) * a.hd) + li * 8; };
+  const auto request = [&]() {
+    const int h = (base + (int)threadIdx.x) >> log_lanes;
+    if (TAPS == 0 && in && h < heads) raw.load((const T*)a.proj + (size_t)t * a.stride + column(h));
+  };
+  request();
   const float pos = (float)a.positions[t];
-  const int half_runs = a.rotary_dim / 16;               // runs of the low half of the rotated part
+  const int slot = a.slot_mapping ? a.slot_mapping[t] : -1;
   if (a.inv_freq) {
-    for (int i = threadIdx.x; i < a.rotary_dim / 2; i += kPrepThreads) {
-      const float ang = pos * a.inv_freq[i];
-      cs_tab[i] = cosf(ang) * a.magnitude;
-      sn_tab[i] = sinf(ang) * a.magnitude;
+    for (int i = threadIdx.x; i < a.rotary_dim / 2; i += blockDim.x) {
+      float sn, cs;
+      sincosf(pos * a.inv_freq[i], &sn, &cs);
+      cs_tab[i] = cs * a.magnitude;
+      sn_tab[i] = sn * a.magnitude;
     }
     __syncthreads();
   }
-  const int qn = a.nh * a.hd, kn = a.nkv * a.hd, runs = a.hd / 8, heads = a.nh + a.nkv;
-  const T* src = (const T*)a.proj + (size_t)t * a.stride;
-  const int slot = a.slot_mapping ? a.slot_mapping[t] : -1;
   const int page = slot >= 0 ? slot / a.page_size : 0, off = slot >= 0 ? slot % a.page_size : 0;
   const float temp = a.temp_on ? 1.0f + a.temp_scale * logf(floorf((pos + 1.0f) / a.temp_floor) + 1.0f) : 1.0f;
-  // a thread's run inside a head is the same in every turn: its angles and norm weights stay in registers
-  const int li = threadIdx.x % lanes;
-  const bool in = li < runs, turns = a.inv_freq && li < 2 * half_runs;
-  const int mate = li < half_runs ? (int)threadIdx.x + half_runs : (int)threadIdx.x - half_runs;
-  float c8[8], s8[8], wq[8], wk[8];
-  if (turns) {
-    const int i0 = (li < half_runs ? li : li - half_runs) * 8;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      c8[j] = cs_tab[i0 + j];
-      s8[j] = li < half_runs ? -sn_tab[i0 + j] : sn_tab[i0 + j];
-    }
-  }
-  if (a.norm_mode != NORM_NONE && in) {
-    load8(a.q_norm_w + li * 8, wq);
-    load8(a.k_norm_w + li * 8, wk);
-  }
-  for (int base = blockIdx.y * kPrepThreads; base < heads * lanes; base += gridDim.y * kPrepThreads) {
-    const int h = (base + (int)threadIdx.x) / lanes;
+  const int map_runs = a.maps > 1 ? runs / a.maps : runs, mp = a.maps > 1 ? li / map_runs : 0, lm = li - mp * map_runs;
+  const int half_runs = a.rotary_dim / 16;               // split pairs: runs of the low half of the rotated part
+  const bool low = lm < half_runs, turns = a.inv_freq && in && lm * 8 < a.rotary_dim;
+  const int mate = (int)threadIdx.x + (low ? half_runs : -half_runs);
+  const int ang = a.half_split ? (low ? lm : lm - half_runs) * 8 : lm * 4;     // the run's first angle
+  for (;;) {
+    const int h = (base + (int)threadIdx.x) >> log_lanes;
     const bool is_q = h < a.nh, live = in && h < heads;
     float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if (live) {
-      load8(src + (is_q ? a.q_off + h * a.hd : a.k_off + (h - a.nh) * a.hd) + li * 8, x);
-      if (a.bias) {
-        float b8[8];
-        load8(a.bias + (size_t)h * a.hd + li * 8, b8);
+      if constexpr (TAPS == 0) {
+        raw.floats(x);
+        if (a.bias) {
+          float b8[8];
+          load8(a.bias + h * a.hd + li * 8, b8);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] += b8[j];
+          for (int j = 0; j < 8; ++j) x[j] += b8[j];
+        }
+      } else {
+        prep_gather8<T, TAPS>(a, t, h * a.hd + li * 8, column(h), C, x);
       }
     }
-    if (a.norm_mode != NORM_NONE) {                      // every lane takes part in the exchanges
-      float ss = 0.f;
+    base += gridDim.y * blockDim.x;
+    const bool more = base < (heads << log_lanes);
+    if (more) request();
+    if (a.norm_mode != NORM_NONE) {                      // every lane takes part in the exchanges (a lane without a run holds zeros)
+      float w8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      if (live) load8((is_q ? a.q_norm_w : a.k_norm_w) + (a.norm_mode == NORM_WHOLE ? (is_q ? h : h - a.nh) * a.hd : 0) + li * 8, w8);
+      float ss = 0.f, inv;
 #pragma unroll
       for (int j = 0; j < 8; ++j) ss = fmaf(x[j], x[j], ss);
-      ss = group_sum(ss, lanes);
-      const float inv = rsqrtf(ss / (float)a.hd + a.eps);
-      if (live) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) x[j] = x[j] * inv * (is_q ? wq[j] : wk[j]);
+      if (a.norm_mode == NORM_PER_HEAD) {
+        inv = rsqrtf(group_sum(ss, 1 << log_lanes) / (float)a.hd + a.eps);
+      } else {                                           // (one turn)
+        const float sq = wave_sum(is_q ? ss : 0.f), sk = wave_sum(is_q ? 0.f : ss);
+        if (threadIdx.x % kWave == 0) {
+          red[0][threadIdx.x / kWave] = sq;
+          red[1][threadIdx.x / kWave] = sk;
+        }
+        if (threadIdx.x < kRunMaxThreads / kWave && threadIdx.x >= blockDim.x / kWave) red[0][threadIdx.x] = red[1][threadIdx.x] = 0.f;
+        __syncthreads();
+        float total = 0.f;
+#pragma unroll 1
+        for (int i = 0; i < (int)blockDim.x / kWave; i += 4) {
+          const float4 part = *reinterpret_cast<const float4*>(&red[is_q ? 0 : 1][i]);   // (a block's waves beyond the last: zeros)
+          total = total + part.x + part.y + part.z + part.w;
+        }
+        inv = rsqrtf(total / (float)(is_q ? qn : kn) + a.eps);
       }
+#pragma unroll
+      for (int j = 0; j < 8; ++j) x[j] = x[j] * inv * w8[j];
     }
     if (a.inv_freq) {
+      if (a.half_split) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float other = __shfl(x[j], mate & (kWave - 1), kWave);
-        if (turns) x[j] = x[j] * c8[j] + other * s8[j];
+        for (int j = 0; j < 8; ++j) {
+          const float other = __shfl(x[j], mate & (kWave - 1), kWave);
+          if (turns) x[j] = x[j] * cs_tab[ang + j] + other * (low ? -sn_tab[ang + j] : sn_tab[ang + j]);
+        }
+      } else if (turns) {
+#pragma unroll
+        for (int j = 0; j < 8; j += 2) {
+          const float lo = x[j], hi = x[j + 1], c = cs_tab[ang + j / 2], sn = sn_tab[ang + j / 2];
+          x[j] = lo * c - hi * sn;
+          x[j + 1] = hi * c + lo * sn;
+        }
       }
     }
-    if (!live) continue;
-    if (is_q) {
+    if (live) {
+      if (is_q) {
+        if (a.temp_on) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) x[j] *= temp;
-      store8((T*)a.q_out + (size_t)t * qn + (size_t)h * a.hd + li * 8, x);
-    } else if (slot >= 0) {
-      store8((T*)a.k_cache + (((size_t)page * a.nkv + (h - a.nh)) * a.page_size + off) * a.hd + li * 8, x);
+          for (int j = 0; j < 8; ++j) x[j] *= temp;
+        }
+        T* q = (T*)a.q_out + ((size_t)t * a.nh + h) * a.maps * a.hd + li * 8;
+        if (a.maps == 1) {
+          store8(q, x);
+        } else {                                         // the map's own row of the head's width, zeros in the other maps' rows
+          const float zero[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+          for (int mm = 0; mm < a.maps; ++mm) store8(q + (size_t)mm * a.hd, mm == mp ? x : zero);
+        }
+      } else if (slot >= 0) {
+        store8((T*)a.k_cache + (((size_t)page * a.nkv + (h - a.nh)) * a.page_size + off) * a.hd + li * 8, x);
+      }
     }
+    if (!more) break;
   }
-  if (slot < 0) return;
-  for (int i = (blockIdx.y * kPrepThreads + threadIdx.x) * 8; i < a.nkv * a.vd; i += gridDim.y * kPrepThreads * 8) {
+  if (slot < 0 || a.values_apart) return;
+  for (int i = (blockIdx.y * blockDim.x + threadIdx.x) * 8; i < a.nkv * a.vd; i += gridDim.y * blockDim.x * 8) {
     float v[8];
-    load8(src + a.v_off + i, v);
-    if (a.bias) {
-      float b8[8];
-      load8(a.bias + qn + kn + i, b8);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] += b8[j];
-    }
-    if (a.v_other) {
-      float u[8];
-      load8((const T*)a.v_other + (size_t)t * a.v_other_stride + a.v_other_off + i, u);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) v[j] = (1.0f - a.v_mix) * v[j] + a.v_mix * u[j];
-    }
+    prep_gather8<T, TAPS>(a, t, v_at + i, v_col + i, C, v);
+    prep_mix8<T>(a, t, i, v);
     const int g = i / a.vd, d = i % a.vd;
     T* dst = (T*)a.v_cache + (((size_t)page * a.nkv + g) * a.vd + d) * a.page_size + off;
 #pragma unroll
@@ -499,32 +582,54 @@ SHARPI_EXPORT int sharpi_qk_prep(const void* proj, int dtype, int stride, int q_
   const int parts = (n_tokens <= kPrepSplitTokens && nkv > 1 && nkv <= 65535 && nh % nkv == 0) ? nkv : 1;
   auto at16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 32 == 0; };
   const int sd = hd / maps;
-  const int by8 = (half_split || rotary_dim == 0) && rotary_dim % 16 == 0 && sd % 8 == 0 && vd % 8 == 0 &&
-                  stride % 8 == 0 && q_off % 8 == 0 && k_off % 8 == 0 && (v_off < 0 || v_off % 8 == 0) && at16(proj) && at16(q_out) &&
-                  at16(k_cache) && at16(tail) && at16(bias) && rotary_dim / 2 <= kPrepMaxTurns;
   if (rotary_dim / 2 > kPrepMaxTurns) return SHARPI_ERR_ARG;
+  const bool wide = sd % 8 == 0 && vd % 8 == 0 && stride % 8 == 0 && q_off % 8 == 0 && k_off % 8 == 0 && (v_off < 0 || v_off % 8 == 0) &&
+                    at16(proj) && at16(q_out) && at16(k_cache) && at16(tail) && at16(bias);
+  const bool other_wide = !v_other || (at16(v_other) && v_other_stride % 8 == 0 && v_other_off % 8 == 0);
+  const int by8 = wide && (half_split || rotary_dim == 0) && rotary_dim % 16 == 0;
+  // (a step stores all its tokens or, without slots, none)
+  const bool v_apart = wide && other_wide && n_tokens > kPrepSplitTokens && slot_mapping != nullptr;
+  const int tiles = v_apart ? value_tiles(n_tokens, nkv * vd) : 0;
   PrepArgs a{proj, stride, q_off, k_off, v_off, nh, nkv, hd, vd, conv_w, taps, tail, state_slots, entry_of_token,
              cu_tokens, positions, norm_mode, q_norm_w, k_norm_w, eps, rotary_dim > 0 ? inv_freq : nullptr, rotary_dim,
              half_split, magnitude, q_out, k_cache, v_cache, slot_mapping, page_size, parts, bias, temp_on, temp_floor,
-             temp_scale, maps, v_other, v_other_stride, v_other_off, v_mix, taps == 4 && at16(conv_w), by8};
+             temp_scale, maps, v_other, v_other_stride, v_other_off, v_mix, v_apart, n_tokens, by8};
   const int lanes = hd <= 64 ? (hd <= 8 ? 1 : hd <= 16 ? 2 : hd <= 32 ? 4 : 8) : hd <= 128 ? 16 : hd <= 256 ? 32 : 64;
-  if (by8 && taps == 0 && maps == 1 && norm_mode != NORM_WHOLE && v_off >= 0 && hd <= 512 && at16(q_norm_w) && at16(k_norm_w) &&
-      (!v_other || (at16(v_other) && v_other_stride % 8 == 0 && v_other_off % 8 == 0))) {
-    // few tokens: a block a turn; many: four turns or so a block, to share the angles
-    const int all_turns = ceil_div((nh + nkv) * lanes, kPrepThreads);
-    const int y = n_tokens <= kPrepSplitTokens ? all_turns : ceil_div(all_turns, 4);
-    dim3 rgrid(8 * ceil_div(n_tokens, 8), y);
-    if (dtype == DT_F32) qk_prep_run_kernel<float><<<rgrid, kPrepThreads, 0, stream>>>(a, n_tokens, lanes);
-    else if (dtype == DT_BF16) qk_prep_run_kernel<bf16_t><<<rgrid, kPrepThreads, 0, stream>>>(a, n_tokens, lanes);
-    else return SHARPI_ERR_ARG;
+  const int items = (nh + nkv) * lanes;
+  // a thread for every run where a block can have them; of a few tokens 256 a block, or the launch would leave the chip empty (a
+  // norm over the projection aside, whose sums need them together)
+  const bool together = items <= kRunMaxThreads && (norm_mode == NORM_WHOLE || n_tokens > kPrepSplitTokens);
+  const bool by_runs = wide && other_wide && rotary_dim % (half_split ? 16 : 8) == 0 && hd <= 512 && at16(q_norm_w) && at16(k_norm_w) &&
+                       (norm_mode != NORM_WHOLE || together);
+  if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
+  const bool taps4 = taps == 4 && at16(conv_w);
+#define PREP_BY_TAPS(GO)                                                    \
+  do {                                                                      \
+    if (dtype == DT_F32) {                                                  \
+      if (taps == 0) GO(float, 0); else if (taps4) GO(float, 4); else GO(float, -1);    \
+    } else {                                                                \
+      if (taps == 0) GO(bf16_t, 0); else if (taps4) GO(bf16_t, 4); else GO(bf16_t, -1); \
+    }                                                                       \
+  } while (0)
+  if (by_runs) {
+    const int threads = together ? max(kValueThreads, ceil_div(items, kWave) * kWave) : kPrepThreads;
+    // not together: a block a turn of few tokens; of many four turns or so a block, to share the angles
+    const int turns = ceil_div(items, threads), y = n_tokens <= kPrepSplitTokens ? turns : ceil_div(turns, 4);
+    const dim3 rgrid(n_tokens + ceil_div(tiles, y), y);
+#define RUN_GO(T, TAPSV) qk_prep_run_kernel<T, TAPSV><<<rgrid, threads, 0, stream>>>(a, __builtin_ctz(lanes))
+    PREP_BY_TAPS(RUN_GO);
+#undef RUN_GO
     SHARPI_CHECK_LAUNCH();
-    return SHARPI_OK;
+  } else {
+    dim3 pgrid(n_tokens + tiles, parts);               // (values apart: one part)
+    const size_t row_lds = v_apart ? (size_t)(qn + kn) * sizeof(float) : lds, tile_lds = dtype == DT_F32 ? kValueLds<float> : kValueLds<bf16_t>;
+    const size_t prep_lds = v_apart && row_lds < tile_lds ? tile_lds : row_lds;
+#define PREP_GO(T, TAPSV) qk_prep_kernel<T, TAPSV><<<pgrid, kPrepThreads, prep_lds, stream>>>(a)
+    PREP_BY_TAPS(PREP_GO);
+#undef PREP_GO
+    SHARPI_CHECK_LAUNCH();
   }
-  dim3 pgrid(n_tokens, parts);
-  if (dtype == DT_F32) qk_prep_kernel<float><<<pgrid, kPrepThreads, lds, stream>>>(a);
-  else if (dtype == DT_BF16) qk_prep_kernel<bf16_t><<<pgrid, kPrepThreads, lds, stream>>>(a);
-  else return SHARPI_ERR_ARG;
-  SHARPI_CHECK_LAUNCH();
+#undef PREP_BY_TAPS
   if (taps > 0 && update_tail) {
     dim3 grid(ceil_div(qn + kn + vn, 256), n_entries);
     if (dtype == DT_F32)

@@ -291,24 +291,6 @@ __device__ __forceinline__ void wave_dot_rows(const T* const (&xr)[TT], const TW
   for (int i = 0; i < TT; ++i) out[i] = wave_sum(s[i]);
 }
 
-// Eight neighbouring elements as they lie in memory.
-template <typename T> struct Run8;
-template <> struct Run8<float> {
-  float4 a, b;
-  __device__ __forceinline__ void load(const float* p) {
-    a = *reinterpret_cast<const float4*>(p);
-    b = *reinterpret_cast<const float4*>(p + 4);
-  }
-  __device__ __forceinline__ void floats(float (&v)[8]) const {
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-  }
-};
-template <> struct Run8<bf16_t> {
-  uint4 a;
-  __device__ __forceinline__ void load(const bf16_t* p) { a = *reinterpret_cast<const uint4*>(p); }
-  __device__ __forceinline__ void floats(float (&v)[8]) const { load8(reinterpret_cast<const bf16_t*>(&a), v); }
-};
-
 // One wave: the EE x TT products of EE router rows and TT token rows, bit for bit those of wave_dot_rows (the same chain
 // a lane, the lanes added in the same pairs); hidden % 8 == 0.  What bounds it: a row read for one product
 // costs the cache's 64 bytes a cycle more than its eight multiply-adds a lane, so a row is read for EE or TT of them,

@@ -20,7 +20,7 @@ __host__ __device__ inline int value_tiles(int n_tokens, int channels) {
 }
 
 // Tile `tile` of value_tiles(n_tokens, nkv * vd); vd % 8 == 0.  gather(t, c, v) gives channels c .. c + 7 of the nkv * vd of token t as
-// floats.  lds: kValueLds<T> bytes, slots: LDS of kValueTokens ints.  Every thread of the block calls it.
+// floats.  lds: kValueLds<T> bytes, slots: LDS of kValueTokens ints.  Every thread of a block of kValueThreads or more calls it.
 template <typename T, typename G>
 __device__ __forceinline__ void values_to_pages(int tile, int n_tokens, int nkv, int vd, int page_size, const int* __restrict__ slot_mapping,
                                                 T* __restrict__ v_cache, T* lds, int* slots, const G& gather) {
@@ -31,7 +31,7 @@ __device__ __forceinline__ void values_to_pages(int tile, int n_tokens, int nkv,
   if (threadIdx.x < kValueTokens && t0 + (int)threadIdx.x < n_tokens) own = slot_mapping[t0 + threadIdx.x];
   if (threadIdx.x < kValueTokens) slots[threadIdx.x] = own;
   if (!__syncthreads_or(own >= 0)) return;         // (a layer that reads another's cache)
-  {
+  if (threadIdx.x < kValueThreads) {
     const int tok = threadIdx.x >> 4, run = threadIdx.x & 15;
     const int t = t0 + tok, c = c0 + run * 8;
     if (t < n_tokens && c < nkv * vd) {
@@ -43,7 +43,7 @@ __device__ __forceinline__ void values_to_pages(int tile, int n_tokens, int nkv,
   }
   __syncthreads();
   const int col = threadIdx.x >> 1, first = (threadIdx.x & 1) * 8, c = c0 + col;
-  if (c >= nkv * vd) return;
+  if (threadIdx.x >= kValueThreads || c >= nkv * vd) return;
   int s[8];
   bool run = true;
 #pragma unroll
