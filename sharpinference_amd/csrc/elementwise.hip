@@ -439,10 +439,34 @@ __global__ void add_bias_kernel(T* __restrict__ x, const float* __restrict__ bia
     x[i] = from_f32<T>(to_f32<T>(x[i]) + bias[i % N]);
 }
 
+// eight columns a thread, rows by blockIdx.y (the flat index took a 64-bit division an element: 1,950 rows of 2,048 7.1 -> 5.5 us)
+template <typename T>
+__global__ __launch_bounds__(256) void add_bias8_kernel(T* __restrict__ x, const float* __restrict__ bias, int n_rows, int N) {
+  const int c = (blockIdx.x * 256 + threadIdx.x) * 8;
+  if (c >= N) return;
+  float b[8];
+  load8(bias + c, b);
+  for (int t = blockIdx.y; t < n_rows; t += gridDim.y) {
+    T* p = x + (size_t)t * N + c;
+    float v[8];
+    load8(p, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) v[j] += b[j];
+    store8(p, v);
+  }
+}
+
 SHARPI_EXPORT int sharpi_add_bias(void* x, int dtype, const float* bias, int n_rows, int N, hipStream_t stream) {
   if (n_rows <= 0) return SHARPI_OK;
   if (N <= 0 || !bias) return SHARPI_ERR_ARG;
   const size_t total = (size_t)n_rows * N;
+  if (N % 8 == 0 && (((uintptr_t)x | (uintptr_t)bias) & 15) == 0 && (dtype == DT_F32 || dtype == DT_BF16)) {
+    const dim3 grid8(ceil_div(N / 8, 256), min(n_rows, 65535));
+    if (dtype == DT_F32) add_bias8_kernel<float><<<grid8, 256, 0, stream>>>((float*)x, bias, n_rows, N);
+    else add_bias8_kernel<bf16_t><<<grid8, 256, 0, stream>>>((bf16_t*)x, bias, n_rows, N);
+    SHARPI_CHECK_LAUNCH();
+    return SHARPI_OK;
+  }
   const dim3 block(256), grid((unsigned)min((size_t)4096, (total + 255) / 256));
   if (dtype == DT_F32) add_bias_kernel<float><<<grid, block, 0, stream>>>((float*)x, bias, n_rows, N);
   else if (dtype == DT_BF16) add_bias_kernel<bf16_t><<<grid, block, 0, stream>>>((bf16_t*)x, bias, n_rows, N);

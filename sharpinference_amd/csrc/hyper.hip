@@ -245,12 +245,61 @@ __global__ __launch_bounds__(256) void map_difference_kernel(const T* __restrict
   }
 }
 
+// The same for heads of up to 512 values, a multiple of 8: a head in neighbouring lanes, eight values a lane (1,664 tokens of 16 heads
+// 9.3 -> 5.5 us).
+template <typename T>
+__global__ __launch_bounds__(256) void map_difference8_kernel(const T* __restrict__ a, float lambda, float eps, float post,
+                                                              const T* __restrict__ proj, int stride, int g_off,
+                                                              T* __restrict__ out, int n_pairs, int H, int e, int log_lanes) {
+  const unsigned idx = blockIdx.x * 256u + threadIdx.x;
+  const int p = idx >> log_lanes, c = (idx & ((1 << log_lanes) - 1)) * 8;
+  const bool live = p < n_pairs && c < e;
+  float d[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  float mul = post, ss = 0.f;
+  if (live) {
+    float a2[8];
+    load8(a + (size_t)p * 2 * e + c, d);
+    load8(a + (size_t)p * 2 * e + e + c, a2);
+    if (proj) {
+      const int t = p / H;
+      const float z = to_f32<T>(proj[(size_t)t * stride + g_off + (p - t * H)]);
+      mul = 1.0f / (1.0f + expf(-z));
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      d[j] = d[j] - lambda * a2[j];
+      ss = fmaf(d[j], d[j], ss);
+    }
+  }
+  ss = group_sum(ss, 1 << log_lanes);
+  if (!live) return;
+  const float norm = post / sqrtf(ss / (float)e + eps);
+  mul = proj ? norm * mul : norm;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) d[j] *= mul;
+  store8(out + (size_t)p * e + c, d);
+}
+
 SHARPI_EXPORT int sharpi_map_difference(const void* a, int dtype, float lambda, float eps, float post, const void* proj,
                                         int stride, int g_off, void* out, int n_tokens, int H, int e, hipStream_t stream) {
   if (n_tokens <= 0) return SHARPI_OK;
   if (H <= 0 || e <= 0 || (proj && (g_off < 0 || g_off + H > stride))) return SHARPI_ERR_ARG;
   const long long pairs = (long long)n_tokens * H;
   if (pairs > 0x7fffffffLL) return SHARPI_ERR_ARG;
+  const auto at16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  int log_lanes = 0;
+  while ((8 << log_lanes) < e && log_lanes < 6) ++log_lanes;
+  if (e % 8 == 0 && e <= 512 && at16(a) && at16(out) && (pairs << log_lanes) < 0x7fffffffLL && (dtype == DT_F32 || dtype == DT_BF16)) {
+    const unsigned blocks = (unsigned)(((pairs << log_lanes) + 255) / 256);
+    if (dtype == DT_F32)
+      map_difference8_kernel<float><<<blocks, 256, 0, stream>>>((const float*)a, lambda, eps, post, (const float*)proj, stride, g_off,
+                                                                (float*)out, (int)pairs, H, e, log_lanes);
+    else
+      map_difference8_kernel<bf16_t><<<blocks, 256, 0, stream>>>((const bf16_t*)a, lambda, eps, post, (const bf16_t*)proj, stride, g_off,
+                                                                 (bf16_t*)out, (int)pairs, H, e, log_lanes);
+    SHARPI_CHECK_LAUNCH();
+    return SHARPI_OK;
+  }
   const dim3 block(256), grid((unsigned)((pairs + 3) / 4));
   if (dtype == DT_F32)
     map_difference_kernel<float><<<grid, block, 0, stream>>>((const float*)a, lambda, eps, post, (const float*)proj, stride, g_off,

@@ -40,6 +40,7 @@
 // float: alpha = exp(log_sigmoid(z + bias) / tau), in place over the logits.
 #include "common.h"
 #include "gla_chunk.h"
+#include "norm_gate.h"
 
 constexpr int kCols = 8;                 // value columns a walking wave owns
 constexpr int kGroups = kWave / kCols;   // row groups
@@ -316,7 +317,7 @@ __global__ __launch_bounds__(kWave) void gla_combine_kernel(const float* __restr
 }
 
 // Each head's output normed over its dv elements (learned weights shared by the heads), times
-// silu(gate): one wave a (token, head).  o float [T, nh * dv]; gate columns of proj.
+// silu(gate): one wave a (token, head), where norm_gate.h does not take the heads' width.  o float [T, nh * dv]; gate columns of proj.
 template <typename T>
 __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __restrict__ o, const float* __restrict__ w,
                                                               float eps, const T* __restrict__ proj, int stride,
@@ -494,6 +495,13 @@ SHARPI_EXPORT int sharpi_head_norm_gate(const float* o, const float* w, float ep
                                         int g_off, void* out, int n_tokens, int nh, int dv, hipStream_t stream) {
   if (n_tokens <= 0) return SHARPI_OK;
   if (nh <= 0 || dv <= 0) return SHARPI_ERR_ARG;
+  const PartNorm parts{o, w, 0, eps, proj, stride, g_off, proj ? PART_GATE_SILU_QUOTIENT : PART_GATE_NONE, 0, out, n_tokens * nh, nh, dv};
+  if ((dtype == DT_F32 || dtype == DT_BF16) && part_norm_wide(parts)) {
+    if (dtype == DT_F32) part_norm_launch<float>(parts, stream);
+    else part_norm_launch<bf16_t>(parts, stream);
+    SHARPI_CHECK_LAUNCH();
+    return SHARPI_OK;
+  }
   const int blocks = ceil_div(n_tokens * nh, 4);
   if (dtype == DT_F32)
     head_norm_gate_kernel<float><<<blocks, 256, 0, stream>>>(o, w, eps, (const float*)proj, stride, g_off, (float*)out,

@@ -37,6 +37,7 @@
 // start states one after the other (for the gates, with m' = max(F + m, m_L):
 // S' = exp(F + m - m') S + exp(m_L - m') L); WALK_FINAL walks every segment from its start state,
 // writes the outputs, and the entry's last segment leaves the new state in the slot.
+#include "norm_gate.h"
 #include "state_walk.h"
 
 enum : int { WALK_WHOLE = 0, WALK_LOCAL = 1, WALK_FINAL = 2 };
@@ -493,13 +494,8 @@ SHARPI_EXPORT int sharpi_state_walk_segmented(const void* proj, int dtype, int s
 // Behind a walk: o float [T, G * gd] in G equal parts, each divided by its root mean square, times a
 // weight per channel, times a gate act(z) read from columns g_off.. of proj [T, stride] (act: 0 none,
 // 1 SiLU, 2 sigmoid).  gate_first: the gate multiplies o BEFORE the statistics are taken (the norm
-// then sees the gated values); otherwise after the weight.  A wave a (token, part).
+// then sees the gated values); otherwise after the weight.  A wave a (token, part), where norm_gate.h does not take the parts' width.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ float gate_value(int act, float z) {
-  const float s = 1.0f / (1.0f + expf(-z));
-  return act == 1 ? z * s : s;
-}
-
 template <typename T>
 __global__ __launch_bounds__(256) void group_norm_gate_kernel(const float* __restrict__ o, const float* __restrict__ w,
                                                                float eps, const T* __restrict__ proj, int stride,
@@ -514,16 +510,16 @@ __global__ __launch_bounds__(256) void group_norm_gate_kernel(const float* __res
   float ss = 0.f;
   for (int d = lane; d < gd; d += kWave) {
     float v = x[d];
-    if (gate && gate_first) v *= gate_value(act, to_f32<T>(gate[d]));
+    if (gate && gate_first) v *= part_gate(act, to_f32<T>(gate[d]));
     ss = fmaf(v, v, ss);
   }
   ss = wave_sum(ss);
   const float inv = rsqrtf(ss / (float)gd + eps);
   for (int d = lane; d < gd; d += kWave) {
     float v = x[d];
-    if (gate && gate_first) v *= gate_value(act, to_f32<T>(gate[d]));
+    if (gate && gate_first) v *= part_gate(act, to_f32<T>(gate[d]));
     float y = w ? v * inv * w[(size_t)p * gd + d] : v * inv;      // (w null: a norm without a weight)
-    if (gate && !gate_first) y *= gate_value(act, to_f32<T>(gate[d]));
+    if (gate && !gate_first) y *= part_gate(act, to_f32<T>(gate[d]));
     out[(size_t)pair * gd + d] = from_f32<T>(y);
   }
 }
@@ -533,6 +529,13 @@ SHARPI_EXPORT int sharpi_group_norm_gate(const float* o, const float* w, float e
                                          int gd, hipStream_t stream) {
   if (n_tokens <= 0) return SHARPI_OK;
   if (G <= 0 || gd <= 0 || act < 0 || act > 2 || (act && !proj)) return SHARPI_ERR_ARG;
+  const PartNorm parts{o, w, gd, eps, proj, stride, g_off, act, gate_first, out, n_tokens * G, G, gd};
+  if ((dtype == DT_F32 || dtype == DT_BF16) && part_norm_wide(parts)) {
+    if (dtype == DT_F32) part_norm_launch<float>(parts, stream);
+    else part_norm_launch<bf16_t>(parts, stream);
+    SHARPI_CHECK_LAUNCH();
+    return SHARPI_OK;
+  }
   const int blocks = ceil_div(n_tokens * G, 4);
   if (dtype == DT_F32)
     group_norm_gate_kernel<float><<<blocks, 256, 0, stream>>>(o, w, eps, (const float*)proj, stride, g_off, act, gate_first,
@@ -579,6 +582,46 @@ __global__ __launch_bounds__(256) void short_conv_kernel(const T* __restrict__ p
   out[(size_t)t * C + ch] = from_f32<T>(acc / (1.0f + expf(-acc)));
 }
 
+// Four taps, channels by eights: a thread takes eight channels of S consecutive tokens, so that their weights (128 bytes) and the rows
+// that several of them read are read once (one channel and tap at a time: 1,950 tokens of 6,144 channels 75.4 -> 21.4 us).
+template <typename T, int S>
+__global__ __launch_bounds__(256) void short_conv4_kernel(const T* __restrict__ proj, int stride, int c_off, const float* __restrict__ w,
+                                                           const float* __restrict__ bias, const float* __restrict__ tail,
+                                                           const int* __restrict__ state_slots, const int* __restrict__ entry_of_token,
+                                                           const int* __restrict__ cu_tokens, T* __restrict__ out, int n_tokens, int C) {
+  const int t0 = blockIdx.x * S, ch = (blockIdx.y * 256 + threadIdx.x) * 8;
+  if (ch >= C) return;
+  const T* src = proj + c_off + ch;
+  Run8<T> row[S + 3];                              // rows t0 - 3 ..
+#pragma unroll
+  for (int i = 0; i < S + 3; ++i) row[i].load(src + (size_t)min(max(t0 - 3 + i, 0), n_tokens - 1) * stride);
+  float4 wv[8];
+  float b8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int j = 0; j < 8; ++j) wv[j] = *reinterpret_cast<const float4*>(w + (size_t)(ch + j) * 4);
+  if (bias) load8(bias + ch, b8);
+#pragma unroll
+  for (int i = 0; i < S; ++i) {
+    const int t = t0 + i;
+    if (t >= n_tokens) break;
+    const int e = entry_of_token[t], local = t - cu_tokens[e];
+    float acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = b8[j];
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {                  // 3 - x tokens back
+      float u[8];
+      if (3 - x <= local) row[i + x].floats(u);
+      else load8(tail + ((size_t)state_slots[e] * 3 + local + x) * C + ch, u);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[j] = fmaf(x == 0 ? wv[j].x : x == 1 ? wv[j].y : x == 2 ? wv[j].z : wv[j].w, u[j], acc[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[j] = acc[j] / (1.0f + expf(-acc[j]));
+    store8(out + (size_t)t * C + ch, acc);
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void short_conv_tail_kernel(const T* __restrict__ proj, int stride, int c_off, int taps,
                                                                float* __restrict__ tail, const int* __restrict__ state_slots,
@@ -605,7 +648,28 @@ SHARPI_EXPORT int sharpi_short_conv(const void* proj, int dtype, int stride, int
   if (C <= 0 || taps < 1 || taps > kConvMaxTaps || (taps > 1 && !tail) || n_entries <= 0 || ceil_div(C, 256) > 65535) return SHARPI_ERR_ARG;
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
   dim3 grid(n_tokens, ceil_div(C, 256)), tgrid(n_entries, ceil_div(C, 256));
-  if (dtype == DT_F32) {
+  const auto at16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  if (taps == 4 && C % 8 == 0 && stride % 8 == 0 && c_off % 8 == 0 && at16(proj) && at16(w) && at16(bias) && at16(tail) && at16(out)) {
+    // (few tokens: one a thread, or a handful of blocks would go through them)
+    const int s = n_tokens > 256 ? 4 : 1;
+    const dim3 grid8(ceil_div(n_tokens, s), ceil_div(C / 8, 256));
+#define CONV4(T, SV)                                                                                                           \
+  short_conv4_kernel<T, SV><<<grid8, 256, 0, stream>>>((const T*)proj, stride, c_off, w, bias, tail, state_slots, entry_of_token, \
+                                                       cu_tokens, (T*)out, n_tokens, C)
+    if (dtype == DT_F32) {
+      if (s == 4) CONV4(float, 4); else CONV4(float, 1);
+    } else {
+      if (s == 4) CONV4(bf16_t, 4); else CONV4(bf16_t, 1);
+    }
+#undef CONV4
+    SHARPI_CHECK_LAUNCH();
+    if (update_tail) {
+      if (dtype == DT_F32)
+        short_conv_tail_kernel<float><<<tgrid, 256, 0, stream>>>((const float*)proj, stride, c_off, taps, tail, state_slots, cu_tokens, C);
+      else
+        short_conv_tail_kernel<bf16_t><<<tgrid, 256, 0, stream>>>((const bf16_t*)proj, stride, c_off, taps, tail, state_slots, cu_tokens, C);
+    }
+  } else if (dtype == DT_F32) {
     short_conv_kernel<float><<<grid, 256, 0, stream>>>((const float*)proj, stride, c_off, w, bias, taps, tail, state_slots,
                                                         entry_of_token, cu_tokens, (float*)out, C);
     SHARPI_CHECK_LAUNCH();

@@ -1,0 +1,100 @@
+"""Row kernels that take eight channels a thread: the bits of the forms that take any width, or the plain arithmetic in double."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+DT = {"float32": torch.float32, "bfloat16": torch.bfloat16}
+# float: a sum of squares over at most 16 terms a lane and 6 of the lanes, halved by the root, and five roundings behind it; bfloat16: its own
+TOL = {"float32": 16 * 2.0 ** -24, "bfloat16": 2.0 ** -8}
+
+
+class _Step:
+    def __init__(self, lens, slots):
+        i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+        cu = [0]
+        for n in lens:
+            cu.append(cu[-1] + n)
+        self.n_entries, self.n_tokens = len(lens), cu[-1]
+        self.cu_tokens, self.state_slots = i32(cu), i32(slots)
+        self.entry_of_token = i32([e for e, n in enumerate(lens) for _ in range(n)])
+        self.positions = i32([p for n in lens for p in range(n)])
+
+
+def _shifted(x):
+    """The same values two columns further on, in rows too wide to be read by eights."""
+    wide = torch.zeros(x.shape[0], x.shape[1] + 3, dtype=x.dtype, device=x.device)
+    wide[:, 2:2 + x.shape[1]] = x
+    return wide
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("lens, C", [([1], 8), ([2, 1, 3, 4], 2056), ([1] * 20, 64), ([3, 250, 1, 2, 9], 264), ([300], 2048), ([5, 4, 257], 40)])
+def test_four_taps_by_eights_give_the_bits_of_a_channel_at_a_time(lens, C, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(C + len(lens))
+    T = sum(lens)
+    u = (torch.randn(T, C, generator=g) * 2).to(DT[dtype]).to(DEV)
+    w, b = torch.randn(C, 4, generator=g).to(DEV), torch.randn(C, generator=g).to(DEV) if C != 64 else None
+    held = torch.randn(len(lens) + 2, 3, C, generator=g).to(DEV)
+    ctx, out = _Step(lens, list(range(len(lens), 0, -1))), []
+    for rows, off in ((u, 0), (_shifted(u), 2)):
+        tail = held.clone()
+        out.append((ops.short_conv(rows, off, C, w, b, tail, ctx), tail))
+    assert torch.equal(out[0][0], out[1][0]) and torch.equal(out[0][1], out[1][1])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T, groups, size", [(1, 1, 8), (70, 5, 24), (3, 16, 128), (33, 2, 192), (9, 3, 512), (5, 2, 520), (2, 3, 1024)])
+@pytest.mark.parametrize("act, first, weighted", [("silu", False, True), ("silu", True, True), ("sigmoid", False, False)])
+def test_parts_in_neighbouring_lanes(T, groups, size, act, first, weighted, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(T + size)
+    N, off, eps = groups * size, 16, 1e-3
+    o = (torch.randn(T, N, generator=g) * 5).to(DEV)
+    w = torch.randn(N, generator=g).to(DEV) if weighted else None
+    gp = (torch.randn(T, off + N + 8, generator=g) * 2).to(DT[dtype]).to(DEV)
+    got = ops.group_norm_gate(o, w, eps, groups, DT[dtype], gp, off, ops.GATE_SILU if act == "silu" else ops.GATE_SIGMOID_ACT, gate_first=first)
+    z = gp.double()[:, off:off + N]
+    gate = torch.sigmoid(z) * (z if act == "silu" else 1.0)
+    x = o.double() * gate if first else o.double()
+    x = x.view(T, groups, size)
+    want = (x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + eps)).reshape(T, N) * (w.double() if weighted else 1.0) * (1.0 if first else gate)
+    assert float(((got.double() - want).abs() - TOL[dtype] * want.abs()).max()) <= 2.0 ** -60
+    if not first:
+        heads = ops.head_norm_gate(o, w[:size].contiguous() if weighted else torch.ones(size, device=DEV), eps, groups, size, DT[dtype], gp, off)
+        want = (x / torch.sqrt(x.pow(2).mean(-1, keepdim=True) + eps) * (w.double()[:size] if weighted else 1.0)).reshape(T, N) * torch.sigmoid(z) * z
+        assert float(((heads.double() - want).abs() - TOL[dtype] * want.abs()).max()) <= 2.0 ** -60
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T, H, e, gate", [(1, 1, 8, True), (70, 8, 128, False), (3, 5, 136, True), (9, 2, 512, True), (4, 3, 520, True)])
+def test_differences_of_maps_in_neighbouring_lanes(T, H, e, gate, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(T + e)
+    a = torch.randn(T, H, 2, e, generator=g).to(DT[dtype]).to(DEV)
+    proj = torch.randn(T, 11 + H, generator=g).to(DT[dtype]).to(DEV)
+    lam, eps, post = 0.62, 1e-5, 0.7
+    d = a[:, :, 0].double() - lam * a[:, :, 1].double()
+    mul = post / torch.sqrt(d.pow(2).mean(-1, keepdim=True) + eps)
+    if gate:
+        mul = mul * torch.sigmoid(proj[:, 11:].double())[:, :, None]
+    want = d * mul
+    got = ops.map_difference(a.reshape(T, -1), H, e, lam, eps, post, proj if gate else None, 11).double().view(T, H, e)
+    # (a difference keeps the error of its two terms and of lambda's float)
+    terms = (a[:, :, 0].double().abs() + a[:, :, 1].double().abs()) * mul * 2.0 ** -23
+    assert float(((got - want).abs() - TOL[dtype] * want.abs() - terms).max()) <= 2.0 ** -60
+
+
+@pytest.mark.parametrize("T, N", [(1, 8), (70, 2056), (5, 1000), (3, 12)])
+def test_columns_side_by_side_add_as_one_by_one(T, N):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(T + N)
+    x, b = (torch.randn(T, N, generator=g) * 3).to(DEV), torch.randn(N, generator=g).to(DEV)
+    for dtype in DT.values():
+        y = x.to(dtype)
+        assert torch.equal(ops.add_bias(y.clone(), b), (y.float() + b).to(dtype))
