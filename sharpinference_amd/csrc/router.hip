@@ -1,6 +1,6 @@
 // MoE routing on the device: router logits, gate, top-k, and the expert-sorted row list.
 //
-// router_topk: one block per token, or per four tokens when there are many.
+// router_topk: one block per token, or per two or four tokens when there are many.
 // logits[e] = Wr[e, :] . x[t, :] in float (each wave owns experts e = wave, wave + nwaves, ...;
 // lanes stride over the hidden width, so the order of the additions depends on the width only).
 // gate 0 = sigmoid over every expert, gate 1 = softmax over every expert.  The k picks scan
@@ -140,17 +140,23 @@ __device__ __forceinline__ int wave_argmax(const float* v, int n, int lane, uint
       best = i;
     }
   }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) {
-    const int oi = __shfl_xor(best, off, kWave);
-    const float ov = __shfl_xor(bv, off, kWave);
-    if (oi >= 0 && (best < 0 || ov > bv || (ov == bv && oi < best))) {
-      bv = ov;
-      best = oi;
-    }
+  // the lanes that hold the largest; of several the one of the lowest index (none equal to it: only values that are no number are left)
+  const float mx = wave_max(best >= 0 ? bv : -INFINITY);
+  unsigned long long at = __ballot(best >= 0 && bv == mx);
+  if (at == 0) at = __ballot(best >= 0);
+  if (at == 0) {
+    *best_v = -INFINITY;
+    return -1;
   }
-  best = __shfl(best, 0, kWave);           // (one answer for all lanes, whatever the values were)
-  *best_v = __shfl(bv, 0, kWave);
+  if (n > kWave && (at & (at - 1)) != 0) {
+    int low = (at >> lane & 1) != 0 ? best : 0x7fffffff;
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) low = min(low, __shfl_xor(low, off, kWave));
+    at = __ballot(best == low);
+  }
+  const int src = __ffsll((long long)at) - 1;
+  *best_v = __shfl(bv, src, kWave);
+  best = __shfl(best, src, kWave);
   return best;
 }
 
@@ -352,8 +358,14 @@ __device__ __forceinline__ float wave_dots(const T* const (&xr)[TT], const TW* c
     const bool high = lane & off;
 #pragma unroll
     for (int v = 0; v < m; ++v) {
-      const float other = __shfl_xor(high ? s[v] : s[v + m], off, kWave);
-      s[v] = (high ? s[v + m] : s[v]) + other;
+      if (off >= 16) {                  // (a swap leaves each lane both terms of its product's sum)
+        const auto p = off == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(s[v]), __float_as_uint(s[v + m]), false, false)
+                                 : __builtin_amdgcn_permlane16_swap(__float_as_uint(s[v]), __float_as_uint(s[v + m]), false, false);
+        s[v] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+      } else {
+        const float other = __shfl_xor(high ? s[v] : s[v + m], off, kWave);
+        s[v] = (high ? s[v + m] : s[v]) + other;
+      }
     }
   }
   for (; off > 0; off >>= 1) s[0] += __shfl_xor(s[0], off, kWave);
@@ -369,8 +381,10 @@ __global__ __launch_bounds__(1024) void router_topk_kernel(const T* __restrict__
                                                            const float* __restrict__ corr, int n_groups, int keep,
                                                            int split_choice, const float* __restrict__ bias, float w_scale, int group_top) {
   // TT tokens per block: a router row is fetched once for all of them.
-  __shared__ float g[TT][kMaxExperts];
-  extern __shared__ float choice_s[];        // [TT][n_experts + n_groups] when the choice has scores of its own
+  extern __shared__ float router_lds[];
+  float* const g_s = router_lds;             // [TT][n_experts]: logits, then gates
+  float* const choice_s = g_s + TT * n_experts;   // [TT][n_experts + n_groups] when the choice has scores of its own
+  const auto g = [&](int i) { return g_s + i * n_experts; };
   const int t0 = blockIdx.x * TT;
   const int lane = threadIdx.x & (kWave - 1);
   const int w = threadIdx.x >> 6;
@@ -386,27 +400,27 @@ __global__ __launch_bounds__(1024) void router_topk_kernel(const T* __restrict__
       for (int x = 0; x < EE; ++x) wrow[x] = wr + (size_t)min(e0 + x, n_experts - 1) * hidden;
       const float v = wave_dots<T, TW, EE, TT>(xr, wrow, hidden, lane);
       const int e = e0 + lane / W / TT;
-      if (lane % W == 0 && e < n_experts) g[lane / W % TT][e] = bias ? v + bias[e] : v;
+      if (lane % W == 0 && e < n_experts) g(lane / W % TT)[e] = bias ? v + bias[e] : v;
     }
   } else for (int e = w; e < n_experts; e += nw) {
     float v[TT];
     wave_dot_rows<T, TW, TT>(xr, wr + (size_t)e * hidden, hidden, lane, v);
     if (lane == 0) {
 #pragma unroll
-      for (int i = 0; i < TT; ++i) g[i][e] = bias ? v[i] + bias[e] : v[i];
+      for (int i = 0; i < TT; ++i) g(i)[e] = bias ? v[i] + bias[e] : v[i];
     }
   }
   __syncthreads();
   if (k <= kWave) {                          // a wave a token
-    if (w < TT && t0 + w < n_tokens) {
-      const int t = t0 + w;
-      gate_and_pick_wave(g[w], n_experts, k, gate, renorm, topk_ids + (size_t)t * k, topk_w + (size_t)t * k,
+    for (int i = w; i < TT && t0 + i < n_tokens; i += nw) {
+      const int t = t0 + i;
+      gate_and_pick_wave(g(i), n_experts, k, gate, renorm, topk_ids + (size_t)t * k, topk_w + (size_t)t * k,
                          gate_out ? gate_out + (size_t)t * n_experts : nullptr,
-                         split_choice ? choice_s + (size_t)w * (n_experts + n_groups) : nullptr, corr, n_groups, keep, w_scale, lane, group_top);
+                         split_choice ? choice_s + (size_t)i * (n_experts + n_groups) : nullptr, corr, n_groups, keep, w_scale, lane, group_top);
     }
   } else if (threadIdx.x < TT && t0 + threadIdx.x < n_tokens) {
     const int t = t0 + threadIdx.x;
-    gate_and_pick(g[threadIdx.x], n_experts, k, gate, renorm, topk_ids + (size_t)t * k, topk_w + (size_t)t * k,
+    gate_and_pick(g(threadIdx.x), n_experts, k, gate, renorm, topk_ids + (size_t)t * k, topk_w + (size_t)t * k,
                   gate_out ? gate_out + (size_t)t * n_experts : nullptr,
                   split_choice ? choice_s + (size_t)threadIdx.x * (n_experts + n_groups) : nullptr, corr, n_groups, keep, group_top);
     if (w_scale != 1.0f)
@@ -521,34 +535,35 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
   if (n_groups < 1 || keep < 1 || keep > n_groups || n_experts % n_groups != 0 || k > keep * (n_experts / n_groups)) return SHARPI_ERR_ARG;
   if (group_top < 1 || group_top > kMaxGroupTop) return SHARPI_ERR_ARG;
   const int split_choice = corr != nullptr || keep < n_groups;
-  // What it measured (one expert a wave, four tokens a block from 64 tokens before): 3000 rows 2048 wide of 128 experts
-  // 90 -> 56 us, 64 rows 4096 wide 47 -> 19, 1660 rows 2048 wide of 64 experts with float weights 36 -> 32; 16 experts the same (latency).
-  // Few tokens, or rows that cannot be read in runs of 8: a block a token, a wave an expert at a time (enough waves for the
-  // experts, at most 16).  From 64 tokens: four experts a wave (one where there are fewer than 64 experts: a wave has
-  // few then), for four tokens a block where a token a block would be more than one block a compute unit.  Four tokens of few
-  // experts are bound by the loads of the tokens' rows: two runs on their way at a time (wave_dot_rows) are faster than one
-  // (wave_dots) where those rows are floats (12,000 rows 1024 wide of 16 experts 45 / 65 us, of 63 130 / 148; 3,000 rows
-  // 2048 wide of 32 34 / 37) or the experts at most 16 (3,000 bfloat16 rows 5120 wide of 8: 15.6 / 16.7), else not
-  // (12,000 bfloat16 rows 1024 wide of 32: 77 / 68).
-  const bool runs = (hidden & 7) == 0 && n_tokens >= 64;
-  const int tt = runs ? (n_tokens > 256 ? 4 : 1) : n_tokens >= 64 ? 4 : 1;
-  const int ee = !runs ? 0 : n_experts >= 64 ? 4 : tt == 4 && (x_dtype == DT_F32 || n_experts <= 16) ? 0 : 1;
-  dim3 grid(ceil_div(n_tokens, tt)), block(kWave * (n_experts >= 16 ? 16 : n_experts >= 8 ? 8 : 4));
-  const size_t lds = split_choice ? (size_t)tt * (n_experts + n_groups) * sizeof(float) : 0;
+  // Rows read in runs of 8: four experts a wave (two where there are at most 8, or 16 and few tokens), and as few waves as that makes, or
+  // the rows of a token would be read and turned into floats by more waves than its products need.  Several tokens a block share
+  // the experts' rows, as soon as the blocks still fill the chip: four from 1,024 tokens, two from 257 (four of floats: their rows cost
+  // no conversions).  Up to 8 waves a block of four tokens (a wave then takes several turns), 16 of fewer.
+  // us, with one expert a wave of sixteen, or four of sixteen from 64 experts, before: 8,192 rows 5,120 wide of 16 experts 78 -> 33.9,
+  // 1,600 21 -> 11.5, 300 10.7 -> 7.2; 2,048 rows 4,096 wide of 32 34 -> 16.1; 3,000 rows 2,048 wide of 64 37 -> 25.4, 64 of them 10.0 -> 7.7;
+  // 4,096 of 128 80 -> 57; floats: 12,000 rows 1,024 wide of 16 45 -> 24, 3,000 rows 2,048 wide of 32 34 -> 22.  The same tried with tiles of
+  // 16 x 16 on the bfloat16 matrix instruction: 3,000 rows of 64 15.9, but errors against 64 bits 1.15 to 1.3 times these.
+  const bool runs = (hidden & 7) == 0, halves = x_dtype == DT_BF16 && w_dtype == DT_BF16;
+  const int tt = !runs ? (n_tokens >= 64 ? 4 : 1) : n_tokens <= 256 ? 1 : halves && n_tokens < 1024 ? 2 : 4;
+  const int ee = !runs ? 0 : n_experts <= 8 || (n_experts <= 16 && n_tokens <= 64) ? 2 : 4;
+  const int waves = !runs ? (n_experts >= 16 ? 16 : n_experts >= 8 ? 8 : 4) : min(tt == 4 ? 8 : 16, ceil_div(n_experts, ee));
+  dim3 grid(ceil_div(n_tokens, tt)), block(kWave * waves);
+  const size_t lds = (size_t)tt * (n_experts + (split_choice ? n_experts + n_groups : 0)) * sizeof(float);
 #define ROUTER_LAUNCH_AT(TX, TWT, EEV, TTV)                                                                      \
   router_topk_kernel<TX, TWT, EEV, TTV><<<grid, block, lds, stream>>>((const TX*)x, (const TWT*)wr, topk_ids, topk_w, \
                                                                       gate_out, n_tokens, hidden, n_experts, k, gate, \
                                                                       renorm, corr, n_groups, keep, split_choice, bias, w_scale, group_top)
+#define ROUTER_LAUNCH_TT(TX, TWT, EEV)                                                                           \
+  do {                                                                                                           \
+    if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, EEV, 4);                                                              \
+    else if (tt == 1) ROUTER_LAUNCH_AT(TX, TWT, EEV, 1);                                                         \
+    else if constexpr (EEV > 0 && sizeof(TX) == 2 && sizeof(TWT) == 2) ROUTER_LAUNCH_AT(TX, TWT, EEV, 2);        \
+  } while (0)
 #define ROUTER_LAUNCH(TX, TWT)                                                                                   \
   do {                                                                                                           \
-    if (ee == 4) {                                                                                               \
-      if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, 4, 4); else ROUTER_LAUNCH_AT(TX, TWT, 4, 1);                        \
-    } else if (ee == 1) {                                                                                        \
-      if (tt == 1) ROUTER_LAUNCH_AT(TX, TWT, 1, 1);                                                              \
-      else if constexpr (sizeof(TX) == 2) ROUTER_LAUNCH_AT(TX, TWT, 1, 4);                                       \
-    } else {                                                                                                     \
-      if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, 0, 4); else ROUTER_LAUNCH_AT(TX, TWT, 0, 1);                        \
-    }                                                                                                            \
+    if (ee == 4) ROUTER_LAUNCH_TT(TX, TWT, 4);                                                                   \
+    else if (ee == 2) ROUTER_LAUNCH_TT(TX, TWT, 2);                                                              \
+    else ROUTER_LAUNCH_TT(TX, TWT, 0);                                                                           \
   } while (0)
   if (x_dtype == DT_F32 && w_dtype == DT_F32) ROUTER_LAUNCH(float, float);
   else if (x_dtype == DT_BF16 && w_dtype == DT_BF16) ROUTER_LAUNCH(bf16_t, bf16_t);
@@ -556,6 +571,7 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
   else if (x_dtype == DT_F32 && w_dtype == DT_BF16) ROUTER_LAUNCH(float, bf16_t);
   else return SHARPI_ERR_ARG;
 #undef ROUTER_LAUNCH
+#undef ROUTER_LAUNCH_TT
 #undef ROUTER_LAUNCH_AT
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
