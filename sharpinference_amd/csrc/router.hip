@@ -577,54 +577,135 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
   return SHARPI_OK;
 }
 
-// One block: the expert-sorted list of the (token, pick) pairs; cursor is LDS of n_experts ints, count and
-// plan_scratch of one more.  Every thread of the block calls it; the pairs must be visible to the block.
+// One block: the expert-sorted list of the (token, pick) pairs.  Every thread of the block calls it; the pairs must be visible to the block.
 //
-// Bound: latency, one block's chain of loads, counters and sums.  So a thread has eight pairs in flight, one wave
-// makes the prefix sum, and every group counts the units before its own from one number a group (one thread's
-// walks over the groups and a pair a round trip: 18000 pairs of 128 experts 48 -> 32, 512 pairs 26 -> 13 us).
+// Bound: latency, one block's chain of loads, counters and sums, and its scattered stores: a wave that stores to 64 lines takes 64 cycles and more of
+// its unit, so the list is put in order in LDS, a window of rows after the other, and leaves by whole lines.  A thread requests all its pairs (and
+// up to 24 weights) at once and keeps them (KEEP a thread; 0: more pairs than it can, read again for the second pass and stored one by one); an
+// expert has up to 16 counters, a lane takes the one of its number, and what the counter held is the pair's place behind the counter's first row;
+// every group counts the units before its own from one number a group.
+// us, pairs read, counted and stored one by one in two passes before: 18,000 pairs of 64 experts 24.8 -> 17.5, 9,984 17.5 -> 13.0, 8,192 of 28 and of
+// 16 10.7 -> 8.4 and 10.8 -> 7.8.
 constexpr unsigned kPlanRankParts = 32;        // (above kPlanMaxParts)
+constexpr int kPermuteThreads = 1024;
+constexpr int kPermuteCounters = 1024;         // counters of all experts
+constexpr int kMaxCopies = 16;                 // counters an expert
+template <int KEEP> constexpr int kPermuteWindow = KEEP <= 1 ? 1 : KEEP <= 8 ? KEEP * 1024 : 16384;    // rows put in order at a time
+static_assert(kPermuteCounters >= kMaxExperts && kPermuteCounters <= kPermuteThreads, "a counter for every expert, a thread for every counter");
+
+template <int KEEP>
 __device__ void permute_block(const int* __restrict__ topk_ids, const float* __restrict__ topk_w,
                               int* __restrict__ offsets, int* __restrict__ sorted_token,
                               float* __restrict__ sorted_w, int* __restrict__ inv_pos, int* __restrict__ plan,
-                              int n_pairs, int k, int n_experts, int shared_group, int* count, int* cursor,
-                              int* plan_scratch) {
-  constexpr int kAhead = 8;                  // pairs a thread has in flight: one block is alone with its loads' latency
-  const int step = blockDim.x;
-  for (int e = threadIdx.x; e < n_experts; e += step) count[e] = 0;
+                              int n_pairs, int k, int n_experts, int shared_group, int* count, int* counters, int* spare,
+                              int* plan_scratch, int* row_token, float* row_weight) {
+  constexpr int kAhead = 8;                  // pairs a thread has in flight where it does not keep them
+  constexpr bool kWeights = KEEP > 0 && KEEP <= 24;
+  constexpr int step = kPermuteThreads;
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  int log_copies = 0;
+  if (KEEP > 0)
+    while ((2 << log_copies) <= kMaxCopies && (n_experts << (log_copies + 1)) <= kPermuteCounters) ++log_copies;
+  const int n_counters = n_experts << log_copies, copy = lane & ((1 << log_copies) - 1);
+  const auto counter = [&](int id) { return (id << log_copies) + copy; };
+  // i / k by a product: exact while i k < 2^32 (kept pairs are fewer than 2^15, k at most 2^10)
+  const unsigned part_k = k > 1 ? (unsigned)(0xffffffffu / (unsigned)k + 1) : 0;
+  const auto token_of = [&](int i) { return k > 1 ? (int)__umulhi((unsigned)i, part_k) : i; };
+  int pair[KEEP > 0 ? KEEP : 1];             // the pair's expert, then its counter and (times kPermuteCounters) what that held; -1: no row
+  float weight[kWeights ? KEEP : 1];
+  if constexpr (KEEP > 0) {
+#pragma unroll
+    for (int x = 0; x < KEEP; ++x) {
+      if (x % kAhead == 0 && x * step >= n_pairs) break;
+      const int i = min(tid + x * step, n_pairs - 1);
+      pair[x] = topk_ids[i];
+      if (kWeights) weight[x] = topk_w[i];
+    }
+  }
+  counters[tid] = 0;
   __syncthreads();
-  for (int i0 = threadIdx.x; i0 < n_pairs; i0 += kAhead * step) {
-    int id[kAhead];
+  if constexpr (KEEP > 0) {
+    int* const mine = spare + tid;           // (pairs without a row count here: no branch, all on their way together)
 #pragma unroll
-    for (int x = 0; x < kAhead; ++x) id[x] = topk_ids[min(i0 + x * step, n_pairs - 1)];
+    for (int x = 0; x < KEEP; ++x) {
+      if (x % kAhead == 0 && x * step >= n_pairs) break;
+      const bool real = tid + x * step < n_pairs && pair[x] < n_experts;
+      const int c = counter(pair[x]);
+      const int was = atomicAdd(real ? counters + c : mine, 1);
+      pair[x] = real ? was * kPermuteCounters + c : -1;
+    }
+  } else {
+    for (int i0 = tid; i0 < n_pairs; i0 += kAhead * step) {
+      int id[kAhead];
 #pragma unroll
-    for (int x = 0; x < kAhead; ++x)
-      if (i0 + x * step < n_pairs && id[x] < n_experts) atomicAdd(&count[id[x]], 1);
+      for (int x = 0; x < kAhead; ++x) id[x] = topk_ids[min(i0 + x * step, n_pairs - 1)];
+#pragma unroll
+      for (int x = 0; x < kAhead; ++x)
+        if (i0 + x * step < n_pairs && id[x] < n_experts) atomicAdd(counters + counter(id[x]), 1);
+    }
   }
   __syncthreads();
-  if (threadIdx.x < kWave) {                 // one wave's prefix sum: a lane a run of neighbouring experts
-    const int per = (n_experts + kWave - 1) / kWave, e0 = min((int)threadIdx.x * per, n_experts), e1 = min(e0 + per, n_experts);
-    int mine = 0;
-    for (int e = e0; e < e1; ++e) mine += count[e];
-    int run = mine;                          // inclusive over the lanes, then what lies before the lane's own
+  // the rows before each counter's: a sum over the wave's counters, then over the waves before it
+  const int held = tid < n_counters ? counters[tid] : 0;
+  int upto = held;
 #pragma unroll
-    for (int off = 1; off < kWave; off <<= 1) {
-      const int o = __shfl_up(run, off, kWave);
-      if ((int)threadIdx.x >= off) run += o;
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int o = __shfl_up(upto, off, kWave);
+    if (lane >= off) upto += o;
+  }
+  if (lane == kWave - 1) plan_scratch[tid / kWave] = upto;
+  __syncthreads();
+  int before = 0, all = 0;
+#pragma unroll
+  for (int w = 0; w < kPermuteThreads / kWave; ++w) {
+    const int sum = plan_scratch[w];
+    before += w < tid / kWave ? sum : 0;
+    all += sum;
+  }
+  if (tid < n_counters) {
+    counters[tid] = before + upto - held;
+    if (copy == 0) offsets[tid >> log_copies] = before + upto - held;
+  }
+  if (tid == 0) {
+    offsets[n_experts] = all;
+    // an always-on expert as one more group: every token once, in token order, with weight 1
+    if (shared_group) {
+      offsets[n_experts + 1] = all + n_pairs / k;
+      count[n_experts] = n_pairs / k;
     }
-    const int all = __shfl(run, kWave - 1, kWave);
-    run -= mine;
-    for (int e = e0; e < e1; ++e) {
-      offsets[e] = run;
-      cursor[e] = run;
-      run += count[e];
+  }
+  __syncthreads();
+  for (int e = tid; e < n_experts; e += step) count[e] = (e + 1 < n_experts ? counters[(e + 1) << log_copies] : all) - counters[e << log_copies];
+  // (an identity expert: no product, no row; whoever sums the pairs asks the id)
+  if constexpr (KEEP > 0) {
+    constexpr int W = kPermuteWindow<KEEP>;
+#pragma unroll
+    for (int x = 0; x < KEEP; ++x) {
+      if (x % kAhead == 0 && x * step >= n_pairs) break;
+      const int i = tid + x * step;
+      if (pair[x] >= 0) pair[x] = counters[(unsigned)pair[x] % kPermuteCounters] + (unsigned)pair[x] / kPermuteCounters;
+      if (i < n_pairs) inv_pos[i] = max(pair[x], 0);
     }
-    if (threadIdx.x == 0) {
-      offsets[n_experts] = all;
-      // an always-on expert as one more group: every token once, in token order, with weight 1
-      if (shared_group) {
-        offsets[n_experts + 1] = all + n_pairs / k;
-        count[n_experts] = n_pairs / k;
+    if constexpr (KEEP == 1) {               // (a store a thread: no order to wait for)
+      if (n_pairs > 0 && pair[0] >= 0) {
+        sorted_token[pair[0]] = token_of(tid);
+        sorted_w[pair[0]] = weight[0];
+      }
+    } else for (int w0 = 0; w0 < all; w0 += W) {
+      if (w0 > 0) __syncthreads();           // (the window before has left)
+#pragma unroll
+      for (int x = 0; x < KEEP; ++x) {
+        if (x % kAhead == 0 && x * step >= n_pairs) break;
+        const int r = pair[x] - w0, i = tid + x * step;
+        if (pair[x] >= 0 && r >= 0 && r < W) {
+          row_token[r] = token_of(i);
+          row_weight[r] = kWeights ? weight[x] : topk_w[i];
+        }
+      }
+      __syncthreads();
+      for (int r = tid; r < min(W, all - w0); r += step) {
+        sorted_token[w0 + r] = row_token[r];
+        sorted_w[w0 + r] = row_weight[r];
       }
     }
   }
@@ -685,33 +766,35 @@ __device__ void permute_block(const int* __restrict__ topk_ids, const float* __r
     }
     if (threadIdx.x < kPlanCounters) plan[plan_counters_at(n_groups) + threadIdx.x] = 0;
   }
-  __syncthreads();
-  for (int i0 = threadIdx.x; i0 < n_pairs; i0 += kAhead * step) {
-    int id[kAhead], row[kAhead];
-    float wt[kAhead];
+  if constexpr (KEEP == 0) {
+    __syncthreads();                         // (the counts are taken: the counters go on as the next rows)
+    for (int i0 = tid; i0 < n_pairs; i0 += kAhead * step) {
+      int id[kAhead], row[kAhead];
+      float wt[kAhead];
 #pragma unroll
-    for (int x = 0; x < kAhead; ++x) {
-      const int i = min(i0 + x * step, n_pairs - 1);
-      id[x] = topk_ids[i];
-      wt[x] = topk_w[i];
-    }
-#pragma unroll
-    for (int x = 0; x < kAhead; ++x)
-      row[x] = i0 + x * step < n_pairs && id[x] < n_experts ? atomicAdd(&cursor[id[x]], 1) : -1;
-#pragma unroll
-    for (int x = 0; x < kAhead; ++x) {
-      const int i = i0 + x * step;
-      if (i >= n_pairs) break;
-      if (row[x] >= 0) {
-        sorted_token[row[x]] = (unsigned)i / (unsigned)k;
-        sorted_w[row[x]] = wt[x];
+      for (int x = 0; x < kAhead; ++x) {
+        const int i = min(i0 + x * step, n_pairs - 1);
+        id[x] = topk_ids[i];
+        wt[x] = topk_w[i];
       }
-      inv_pos[i] = max(row[x], 0);       // (an identity expert: no product, no row; whoever sums the pairs asks the id)
+#pragma unroll
+      for (int x = 0; x < kAhead; ++x)
+        row[x] = i0 + x * step < n_pairs && id[x] < n_experts ? atomicAdd(counters + counter(id[x]), 1) : -1;
+#pragma unroll
+      for (int x = 0; x < kAhead; ++x)
+        if (const int i = i0 + x * step; i < n_pairs) {
+          if (row[x] >= 0) {
+            sorted_token[row[x]] = (unsigned)i / (unsigned)k;
+            sorted_w[row[x]] = wt[x];
+          }
+          inv_pos[i] = max(row[x], 0);
+        }
     }
   }
 }
 
-__global__ __launch_bounds__(1024) void moe_permute_kernel(const int* __restrict__ topk_ids,
+template <int KEEP>
+__global__ __launch_bounds__(kPermuteThreads) void moe_permute_kernel(const int* __restrict__ topk_ids,
                                                            const float* __restrict__ topk_w,
                                                            int* __restrict__ offsets,
                                                            int* __restrict__ sorted_token,
@@ -719,10 +802,13 @@ __global__ __launch_bounds__(1024) void moe_permute_kernel(const int* __restrict
                                                            int* __restrict__ inv_pos, int* __restrict__ plan,
                                                            int n_pairs, int k, int n_experts, int shared_group) {
   __shared__ int count[kMaxExperts + 1];
-  __shared__ int cursor[kMaxExperts];
+  __shared__ int counters[kPermuteCounters];
+  __shared__ int spare[kPermuteThreads];
   __shared__ int plan_scratch[kMaxExperts + 1];
-  permute_block(topk_ids, topk_w, offsets, sorted_token, sorted_w, inv_pos, plan, n_pairs, k, n_experts,
-                shared_group, count, cursor, plan_scratch);
+  __shared__ int row_token[kPermuteWindow<KEEP>];
+  __shared__ float row_weight[kPermuteWindow<KEEP>];
+  permute_block<KEEP>(topk_ids, topk_w, offsets, sorted_token, sorted_w, inv_pos, plan, n_pairs, k, n_experts,
+                shared_group, count, counters, spare, plan_scratch, row_token, row_weight);
 }
 
 // plan: plan_ints(n_experts + shared_group) ints (grouped_plan.h) for the grouped product of many rows, or null.
@@ -733,8 +819,15 @@ SHARPI_EXPORT int sharpi_moe_permute(const int* topk_ids, const float* topk_w, i
   if (n_experts <= 0 || n_experts > kMaxExperts || k <= 0) return SHARPI_ERR_ARG;
   if (n_tokens < 0) return SHARPI_ERR_ARG;
   if (plan && plan_len < plan_ints(n_experts + (shared_group ? 1 : 0))) return SHARPI_ERR_ARG;
-  moe_permute_kernel<<<1, 1024, 0, stream>>>(topk_ids, topk_w, offsets, sorted_token, sorted_w, inv_pos, plan,
-                                             n_tokens * k, k, n_experts, shared_group);
+  const int n_pairs = n_tokens * k;
+#define PERMUTE(KEEPV)                                                                                                          \
+  moe_permute_kernel<KEEPV><<<1, kPermuteThreads, 0, stream>>>(topk_ids, topk_w, offsets, sorted_token, sorted_w, inv_pos, plan, n_pairs, k, \
+                                                    n_experts, shared_group)
+  if (n_pairs <= 1024) PERMUTE(1);
+  else if (n_pairs <= 8 * 1024) PERMUTE(8);
+  else if (n_pairs <= 24 * 1024) PERMUTE(24);
+  else PERMUTE(0);
+#undef PERMUTE
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
 }
