@@ -230,11 +230,21 @@ class CacheManager:
                 rc.reserved[g] = self.pages_to_hold(g, reserve_tokens, max_step_tokens)
                 self._reserved_total[g] += rc.reserved[g]
         rc.state_slot = self._free_state_slots.pop()
-        for per_slot in self.states:
-            for t in per_slot:
-                t[rc.state_slot].zero_()
+        self._clear_states(rc.state_slot)
         self.requests[req_id] = rc
         return rc
+
+    def _clear_states(self, slot: int) -> None:
+        """A slot's rows of every state set to zero: on a GPU in one launch (a launch a state took 4 us each, thirteen of them in a
+        model of four layers with convolutions and recurrences)."""
+        states = [t for per_slot in self.states for t in per_slot]
+        if self.device.type == "cuda" and states:
+            from .. import ops
+
+            ops.clear_row(states, slot)
+        else:
+            for t in states:
+                t[slot].zero_()
 
     def pages_needed(self, req_id, n_tokens: int) -> List[int]:
         rc = self.requests[req_id]

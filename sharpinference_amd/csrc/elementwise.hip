@@ -713,3 +713,42 @@ SHARPI_EXPORT int sharpi_post_pre_norm(float* h, const void* const* xs, const fl
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
 }
+
+// ---------------------------------------------------------------------------
+// Several pieces of memory set to zero in one launch (a request's rows of all the states a model keeps).
+// ---------------------------------------------------------------------------
+constexpr int kClearPieces = 32;
+struct ClearArgs {
+  void* at[kClearPieces];
+  long long bytes[kClearPieces];
+};
+
+__global__ __launch_bounds__(256) void clear_pieces_kernel(ClearArgs a) {
+  char* p = (char*)a.at[blockIdx.y];
+  const size_t n = (size_t)a.bytes[blockIdx.y], first = (size_t)blockIdx.x * 256 + threadIdx.x, step = (size_t)gridDim.x * 256;
+  if (((uintptr_t)p | n) % 16 == 0) {
+    for (size_t i = first; i < n / 16; i += step) reinterpret_cast<uint4*>(p)[i] = make_uint4(0, 0, 0, 0);
+  } else {
+    for (size_t i = first; i < n; i += step) p[i] = 0;
+  }
+}
+
+// at, bytes: `n` host values each
+SHARPI_EXPORT int sharpi_clear_pieces(void* const* at, const long long* bytes, int n, hipStream_t stream) {
+  for (int i0 = 0; i0 < n; i0 += kClearPieces) {
+    ClearArgs a;
+    long long most = 0;
+    const int m = min(kClearPieces, n - i0);
+    for (int i = 0; i < kClearPieces; ++i) {
+      a.at[i] = i < m ? at[i0 + i] : nullptr;
+      a.bytes[i] = i < m ? bytes[i0 + i] : 0;
+      if (a.bytes[i] < 0 || (a.bytes[i] > 0 && !a.at[i])) return SHARPI_ERR_ARG;
+      most = a.bytes[i] > most ? a.bytes[i] : most;
+    }
+    if (most == 0) continue;
+    const long long blocks = (most + 256 * 64 - 1) / (256 * 64);      // four stores a thread of the largest
+    clear_pieces_kernel<<<dim3((unsigned)(blocks < 512 ? blocks : 512), m), 256, 0, stream>>>(a);
+    SHARPI_CHECK_LAUNCH();
+  }
+  return SHARPI_OK;
+}

@@ -8,7 +8,7 @@ from __future__ import annotations
 
 import collections
 
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import torch
 
@@ -243,6 +243,22 @@ def add_bias(x: torch.Tensor, bias: torch.Tensor) -> torch.Tensor:
           and bias.is_contiguous(), "add_bias: x [T, N] contiguous and bias float32 [N] wanted")
     _run("sharpi_add_bias", _ptr(x), _code(x.dtype), _ptr(bias), x.shape[0], x.shape[1], _stream())
     return x
+
+
+def clear_row(tensors: Sequence[torch.Tensor], row: int) -> None:
+    """tensors[i][row] = 0 for all of them (contiguous, on one device), in one launch."""
+    import ctypes
+
+    if not tensors:
+        return
+    _dev(*tensors)
+    _need(all(t.is_contiguous() and t.dim() >= 1 and 0 <= row < t.shape[0] and t.device == tensors[0].device for t in tensors),
+          "clear_row: contiguous tensors of one device, each with that row")
+    sizes = [t.numel() // t.shape[0] * t.element_size() for t in tensors]
+    at = (ctypes.c_void_p * len(tensors))(*[t.data_ptr() + row * n for t, n in zip(tensors, sizes)])
+    with torch.cuda.device(tensors[0].device):
+        _run("sharpi_clear_pieces", ctypes.cast(at, ctypes.c_void_p), ctypes.cast((ctypes.c_longlong * len(sizes))(*sizes), ctypes.c_void_p),
+             len(tensors), _stream())
 
 
 def cast(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:

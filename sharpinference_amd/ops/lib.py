@@ -23,6 +23,7 @@ _SIGNATURES = {
     "sharpi_silu_mul": [P, P, P, I, I, I, I, F, P, P],
     "sharpi_moe_combine": [P, P, P, P, P, I, I, I, I, P, I, P, P],
     "sharpi_cast": [P, I, P, I, c_longlong, P],
+    "sharpi_clear_pieces": [P, P, I, P],
     "sharpi_add_bias": [P, I, P, I, I, P],
     "sharpi_peak_read": [P, c_longlong, P, P, P],
     "sharpi_peak_mfma": [P, I, I, P],
