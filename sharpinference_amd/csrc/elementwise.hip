@@ -16,10 +16,32 @@ __global__ void embed_gather_kernel(const int* __restrict__ ids, const T* __rest
   for (int i = threadIdx.x; i < hidden; i += blockDim.x) o[i] = to_f32<T>(row[i]) * scale;
 }
 
+// eight elements a thread, a row over as many blocks as that takes (one block went through a row element by element, twenty dependent turns of
+// 5,120: 1 token 9.3 -> 4.0 us, 2,048 24 -> 17.5)
+constexpr int kGatherThreads = 128;
+template <typename T>
+__global__ __launch_bounds__(kGatherThreads) void embed_gather8_kernel(const int* __restrict__ ids, const T* __restrict__ table,
+                                                                       float* __restrict__ out, int hidden, float scale) {
+  const int t = blockIdx.x, i = (blockIdx.y * kGatherThreads + threadIdx.x) * 8;
+  if (i >= hidden) return;
+  float v[8];
+  load8(table + (size_t)ids[t] * hidden + i, v);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) v[j] *= scale;
+  store8(out + (size_t)t * hidden + i, v);
+}
+
 SHARPI_EXPORT int sharpi_embed_gather(const int* ids, const void* table, int table_dtype, float* out,
                                       int n_tokens, int hidden, float scale, hipStream_t stream) {
   if (n_tokens <= 0) return SHARPI_OK;
   if (hidden <= 0) return SHARPI_ERR_ARG;
+  if (hidden % 8 == 0 && hidden <= (1 << 24) && (((uintptr_t)table | (uintptr_t)out) & 15) == 0 && (table_dtype == DT_F32 || table_dtype == DT_BF16)) {
+    const dim3 grid8(n_tokens, ceil_div(hidden / 8, kGatherThreads));
+    if (table_dtype == DT_F32) embed_gather8_kernel<float><<<grid8, kGatherThreads, 0, stream>>>(ids, (const float*)table, out, hidden, scale);
+    else embed_gather8_kernel<bf16_t><<<grid8, kGatherThreads, 0, stream>>>(ids, (const bf16_t*)table, out, hidden, scale);
+    SHARPI_CHECK_LAUNCH();
+    return SHARPI_OK;
+  }
   dim3 grid(n_tokens), block(256);
   if (table_dtype == DT_F32)
     embed_gather_kernel<float><<<grid, block, 0, stream>>>(ids, (const float*)table, out, hidden, scale);
