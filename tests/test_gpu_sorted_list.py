@@ -6,7 +6,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("T,k,E,identity", [(1024, 1, 16, 0), (1025, 1, 1024, 0), (8192, 1, 7, 0), (2731, 3, 600, 40), (4096, 6, 64, 0), (4097, 6, 64, 3), (3000, 8, 9, 9)])
+@pytest.mark.parametrize("T,k,E,identity", [(1024, 1, 16, 0), (1025, 1, 1024, 0), (1024, 2, 16, 0), (683, 3, 60, 4), (512, 8, 128, 0), (4097, 1, 16, 0), (8192, 1, 7, 0), (2731, 3, 600, 40), (4096, 6, 64, 0), (4097, 6, 64, 3), (3000, 8, 9, 9)])
 def test_every_pair_has_one_row_among_its_experts(T, k, E, identity):
     from sharpinference_amd import ops
 
