@@ -222,6 +222,7 @@ SHARPI_EXPORT int sharpi_latent_prep(const void* q, int ldq, int q_off, const vo
 }
 
 // ---------------------------------------------------------------------------
+constexpr int kHgSmall = 128;         // tiles of 64 x 64 up to which a wave takes 16 x 16
 constexpr int kHgTile = 64, kHgK = 16;
 
 template <typename T>
@@ -278,15 +279,44 @@ __global__ __launch_bounds__(256) void head_gemm_kernel(const T* __restrict__ x,
   }
 }
 
-// The same on the matrix cores (bfloat16): a block of four waves computes 64 tokens x 64 outputs of
-// one head, a wave 32 x 32 as 2 x 2 tiles of v_mfma_f32_16x16x32_bf16 with the weights as the A
+// The same on the matrix cores (bfloat16): a block of four waves computes 32 S tokens x 32 S outputs of
+// one head, a wave 16 S x 16 S as S x S tiles of v_mfma_f32_16x16x32_bf16 with the weights as the A
 // operand (out^T = W x^T); both operands come straight from memory in runs of 8 elements (a head's
 // weights are small and stay in cache).  Every output is one chain over k in the same order whatever
-// the number of tokens.  K, the heads' input stride and the row strides are multiples of 8 elements,
+// the number of tokens and S.  K, the heads' input stride and the row strides are multiples of 8 elements,
 // the output's of 4.
+//
+// Bound: few blocks, a chain of loads from memory (the weights are read once a step); many blocks, operands through L2 (64 outputs a 128 rows read).
+// With up to half of the chip's units covered by 64 x 64 tiles a wave takes 16 x 16 (four times the waves) and requests 512 of K before its first
+// product; more tiles than that read too much that way, and there two steps ahead (many waves a unit) beat four and eight.
+// us, 64 x 64 with two steps in turn for all before -> now, weights from memory, 16 heads, 512 x 128 and 128 x 512: 1 token 3.8 -> 2.6, 8.2 -> 3.7;
+// 64 tokens 4.9 -> 4.2, 11.3 -> 6.0; 300 tokens (160 tiles) 128 x 512 11.7 -> 10.8 (16 x 16: 14.1); 1,000 21.2 -> 19.8 (36.4), 20.0 -> 19.7 (31.6).
 typedef __attribute__((ext_vector_type(8))) __bf16 hg_bf16x8;
 typedef __attribute__((ext_vector_type(4))) float hg_f32x4;
 
+// U steps of 32 elements, all of them in flight before the first product
+template <int S, int U>
+__device__ __forceinline__ void head_gemm_steps(const bf16_t* const* xp, const bf16_t* const* wp, int k0, hg_f32x4 (*acc)[S]) {
+  uint4 xa[U][S], wa[U][S];
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int a = 0; a < S; ++a) {
+      xa[u][a] = *reinterpret_cast<const uint4*>(xp[a] + k0 + 32 * u);
+      wa[u][a] = *reinterpret_cast<const uint4*>(wp[a] + k0 + 32 * u);
+    }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int a = 0; a < S; ++a)
+#pragma unroll
+      for (int b = 0; b < S; ++b)
+        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<hg_bf16x8*>(&wa[u][a]),
+                                                            *reinterpret_cast<hg_bf16x8*>(&xa[u][b]), acc[a][b], 0, 0, 0);
+}
+
+template <int S, bool GATED>
 __global__ __launch_bounds__(256) void head_gemm_mfma_kernel(const bf16_t* __restrict__ x, int ldx, int sx,
                                                              const bf16_t* __restrict__ w, bf16_t* __restrict__ out,
                                                              int ldo, int so, const bf16_t* __restrict__ gate, int ldg,
@@ -294,48 +324,62 @@ __global__ __launch_bounds__(256) void head_gemm_mfma_kernel(const bf16_t* __res
   const int h = blockIdx.z;
   const int wv = threadIdx.x >> 6, lane = threadIdx.x & (kWave - 1);
   const int g = lane >> 4, m = lane & 15;
-  const int t_base = blockIdx.x * 64 + (wv >> 1) * 32, n_base = blockIdx.y * 64 + (wv & 1) * 32;
+  const int t_base = blockIdx.x * 32 * S + (wv >> 1) * 16 * S, n_base = blockIdx.y * 32 * S + (wv & 1) * 16 * S;
   if (t_base >= n_tokens || n_base >= N) return;
-  const bf16_t* xp[2];
-  const bf16_t* wp[2];
+  const bf16_t* xp[S];
+  const bf16_t* wp[S];
 #pragma unroll
-  for (int a = 0; a < 2; ++a) {
+  for (int a = 0; a < S; ++a) {
     xp[a] = x + (size_t)min(t_base + 16 * a + m, n_tokens - 1) * ldx + (size_t)h * sx + 8 * g;
     wp[a] = w + ((size_t)h * N + min(n_base + 16 * a + m, N - 1)) * K + 8 * g;
   }
-  hg_f32x4 acc[2][2];
+  hg_f32x4 acc[S][S];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < S; ++a)
 #pragma unroll
-    for (int b = 0; b < 2; ++b) acc[a][b] = hg_f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-  for (int k0 = 0; k0 < K; k0 += 32) {
+    for (int b = 0; b < S; ++b) acc[a][b] = hg_f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16_t gates[S][S][GATED ? 4 : 1];              // (requested ahead of the products)
+  if constexpr (GATED) {
+#pragma unroll
+    for (int a = 0; a < S; ++a)
+#pragma unroll
+      for (int b = 0; b < S; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          gates[a][b][i] = gate[(size_t)min(t_base + 16 * b + m, n_tokens - 1) * ldg + (size_t)h * N + min(n_base + 16 * a + 4 * g, N - 4) + i];
+  }
+  constexpr int kAhead = S == 1 ? 16 : 2;
+  int k0 = 0;
+  for (; k0 + 32 * kAhead <= K; k0 += 32 * kAhead) head_gemm_steps<S, kAhead>(xp, wp, k0, acc);
+  if (S == 1)
+    for (; k0 + 32 * 4 <= K; k0 += 32 * 4) head_gemm_steps<S, 4>(xp, wp, k0, acc);
+  for (; k0 < K; k0 += 32) {
     const bool in = k0 + 8 * g < K;
-    uint4 xa[2], wa[2];
+    uint4 xa[S], wa[S];
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
+    for (int a = 0; a < S; ++a) {
       xa[a] = in ? *reinterpret_cast<const uint4*>(xp[a] + k0) : make_uint4(0, 0, 0, 0);
       wa[a] = in ? *reinterpret_cast<const uint4*>(wp[a] + k0) : make_uint4(0, 0, 0, 0);
     }
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int a = 0; a < S; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
+      for (int b = 0; b < S; ++b)
         acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<hg_bf16x8*>(&wa[a]),
                                                             *reinterpret_cast<hg_bf16x8*>(&xa[b]), acc[a][b], 0, 0, 0);
   }
 #pragma unroll
-  for (int b = 0; b < 2; ++b) {
+  for (int b = 0; b < S; ++b) {
     const int t = t_base + 16 * b + m;
     if (t >= n_tokens) continue;
 #pragma unroll
-    for (int a = 0; a < 2; ++a) {
+    for (int a = 0; a < S; ++a) {
       const int n = n_base + 16 * a + 4 * g;
       if (n >= N) continue;                       // (N is a multiple of 4: the four outputs are in or out together)
       float v[4] = {acc[a][b][0], acc[a][b][1], acc[a][b][2], acc[a][b][3]};
-      if (gate) {
+      if constexpr (GATED) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] *= 1.0f / (1.0f + expf(-bf16_to_f32(gate[(size_t)t * ldg + (size_t)h * N + n + i])));
+        for (int i = 0; i < 4; ++i) v[i] *= 1.0f / (1.0f + expf(-bf16_to_f32(gates[a][b][i])));
       }
       uint2 o;
       o.x = f32_to_bf16_pair(v[0], v[1]);
@@ -360,10 +404,18 @@ SHARPI_EXPORT int sharpi_head_gemm(const void* x, int dtype, int ldx, int sx, co
     head_gemm_kernel<float><<<grid, block, 0, stream>>>((const float*)x, ldx, sx, (const float*)w, (float*)out, ldo, so,
                                                         (const float*)gate, ldg, n_tokens, N, K);
   else if (dtype == DT_BF16 && K % 8 == 0 && sx % 8 == 0 && ldx % 8 == 0 && N % 4 == 0 && so % 4 == 0 && ldo % 4 == 0 &&
-           ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)out & 7) == 0)
-    head_gemm_mfma_kernel<<<grid, block, 0, stream>>>((const bf16_t*)x, ldx, sx, (const bf16_t*)w, (bf16_t*)out, ldo, so,
-                                                      (const bf16_t*)gate, ldg, n_tokens, N, K);
-  else if (dtype == DT_BF16)
+           ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)out & 7) == 0) {
+    const bool small = (long)grid.x * grid.y * grid.z <= kHgSmall && ceil_div(N, 32) <= 65535;
+    if (small) grid = dim3(ceil_div(n_tokens, 32), ceil_div(N, 32), H);
+#define HEAD_GEMM(S, GATED)                                                                                               \
+  head_gemm_mfma_kernel<S, GATED><<<grid, block, 0, stream>>>((const bf16_t*)x, ldx, sx, (const bf16_t*)w, (bf16_t*)out, ldo, so, \
+                                                              (const bf16_t*)gate, ldg, n_tokens, N, K)
+    if (small && gate) HEAD_GEMM(1, true);
+    else if (small) HEAD_GEMM(1, false);
+    else if (gate) HEAD_GEMM(2, true);
+    else HEAD_GEMM(2, false);
+#undef HEAD_GEMM
+  } else if (dtype == DT_BF16)
     head_gemm_kernel<bf16_t><<<grid, block, 0, stream>>>((const bf16_t*)x, ldx, sx, (const bf16_t*)w, (bf16_t*)out, ldo,
                                                          so, (const bf16_t*)gate, ldg, n_tokens, N, K);
   else
