@@ -294,24 +294,16 @@ __global__ __launch_bounds__(kLmWaves* kWave, S == 8 ? 4 : 2) void attn_latent_m
 }
 
 // The rows with more than one run: out = sum_r o_r e^(m_r - M) / (sum_r l_r e^(m_r - M) + e^(sink - M)), a wave a
-// (token, head) row or a part of one, four waves a block.  The maximum and the denominator are taken with a lane a run
+// (token, head) row, four rows a block.  The maximum and the denominator are taken with a lane a run
 // (wave reductions in a fixed order), the output with a lane per four elements, runs in ascending order.
-//
-// Bound: one chain of reads a wave (what other dies have just written).  Rows of many runs give their pieces of 256 elements to waves of their own
-// (`parts`); the sums are the same.  us, 512 elements, a wave a row before: 16 heads, 1 token, 16 runs 5.6 -> 4.1; 64 tokens, 12 runs 5.8 -> 4.4, 40
-// runs 15.4 -> 15.0; 8 tokens of 128 heads, 100 runs 40.6 -> 36.2.  Prompts' two or three runs are bound by their bytes and stay a wave a row: 1,000
-// tokens of 64 heads 65 -> 66 (in parts 75), 300 of 16 8.2 (8.5).
 constexpr int kLmMergeWaves = 4;
-constexpr int kLmMergePart = 4 * kWave;      // elements a wave takes at a time
-constexpr int kLmMergeRowRuns = 4;           // runs up to which a wave takes the whole row
 
 __global__ __launch_bounds__(kLmMergeWaves* kWave) void attn_latent_merge_kernel(
     const float* __restrict__ part_o, const float* __restrict__ part_ml, const int* __restrict__ positions,
     const int* __restrict__ token_list, const float* __restrict__ sink, bf16_t* __restrict__ out, int H, int R,
-    int run_keys, int max_runs, int window, int parts) {
+    int run_keys, int max_runs, int window) {
   const int token = token_list ? token_list[blockIdx.x] : blockIdx.x;
-  const int wave = blockIdx.y * kLmMergeWaves + (threadIdx.x >> 6);
-  const int head = wave / parts, part = wave % parts;
+  const int head = blockIdx.y * kLmMergeWaves + (threadIdx.x >> 6);
   const int lane = threadIdx.x & (kWave - 1);
   if (head >= H) return;
   const int n_runs = positions[token] / run_keys + 1 - first_seen(positions[token], window) / run_keys;
@@ -319,7 +311,7 @@ __global__ __launch_bounds__(kLmMergeWaves* kWave) void attn_latent_merge_kernel
   const size_t rh = (size_t)token * H + head;
   bf16_t* orow = out + rh * R;
   if (n_runs > max_runs) {          // the launch was sized for fewer keys than this token sees: never a result over fewer keys
-    for (int d = part * kWave + lane; d < R; d += parts * kWave) orow[d].bits = 0x7fc0;
+    for (int d = lane; d < R; d += kWave) orow[d].bits = 0x7fc0;
     return;
   }
   const float* ml = part_ml + rh * max_runs * 2;
@@ -333,7 +325,7 @@ __global__ __launch_bounds__(kLmMergeWaves* kWave) void attn_latent_merge_kernel
   const float inv = denom > 0.f ? 1.0f / denom : 0.f;
   const float w_lane = lane < n_runs ? expf(ml[2 * lane] - M) : 0.f;     // run r's weight sits in lane r (the first 64 runs)
   const float* po = part_o + rh * max_runs * R;
-  for (int d0 = part * kLmMergePart; d0 < R; d0 += parts * kLmMergePart) {      // (every lane walks the loop: the weights come from other lanes)
+  for (int d0 = 0; d0 < R; d0 += 4 * kWave) {      // (every lane walks the loop: the weights come from other lanes)
     const int d = d0 + 4 * lane;
     const bool on = d < R;
     float4 o = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -464,10 +456,9 @@ SHARPI_EXPORT int sharpi_attention_latent_merge(const float* part_o, const float
                                                 int H, int R, int run_keys, int max_runs, int window, hipStream_t stream) {
   if (n_tokens <= 0 || max_runs <= 1) return SHARPI_OK;
   if (H <= 0 || H > 65535 || R <= 0 || R % 4 || run_keys <= 0) return SHARPI_ERR_ARG;
-  const int parts = max_runs > kLmMergeRowRuns ? min(ceil_div(R, kLmMergePart), 4) : 1;      // (4: the grid has room for any H)
-  dim3 grid(n_tokens, ceil_div(H * parts, kLmMergeWaves)), block(kLmMergeWaves * kWave);
+  dim3 grid(n_tokens, ceil_div(H, kLmMergeWaves)), block(kLmMergeWaves * kWave);
   attn_latent_merge_kernel<<<grid, block, 0, stream>>>(part_o, part_ml, positions, token_list, sink, (bf16_t*)out, H, R,
-                                                       run_keys, max_runs, window, parts);
+                                                       run_keys, max_runs, window);
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
 }
