@@ -186,6 +186,102 @@ __device__ __forceinline__ float group_sum(float v, int lanes) {
   return v;
 }
 
+// Two values of which the lanes of a pair (lane ^ 32, 16, 8) exchange one: afterwards `a` holds the lower lane's pair of values, one in each
+// lane, and `b` the upper lane's.
+template <int BIT> __device__ __forceinline__ void pair_swap(float& a, float& b) {
+  if constexpr (BIT == 8) {
+    const int ia = __builtin_bit_cast(int, a), ib = __builtin_bit_cast(int, b);
+    a = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(ia, ib, 0x118, 0xf, 0xc, false));   // (row_shr:8 into lanes 8 .. 15)
+    b = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(ib, ia, 0x108, 0xf, 0x3, false));   // (row_shl:8 into lanes 0 .. 7)
+  } else {
+    const auto p = BIT == 32 ? __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false)
+                             : __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    a = __uint_as_float(p[0]);
+    b = __uint_as_float(p[1]);
+  }
+}
+// the value of lane ^ 4, 2, 1
+template <int BIT> __device__ __forceinline__ float lane_xor(float v) {
+  const int i = __builtin_bit_cast(int, v);
+  if constexpr (BIT == 4) {
+    const int up = __builtin_amdgcn_update_dpp(0, i, 0x104, 0xf, 0x5, false);                       // (row_shl:4 into lanes 0 .. 3, 8 .. 11)
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(up, i, 0x114, 0xf, 0xa, false));   // (row_shr:4 into the others)
+  } else {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, i, BIT == 2 ? 0x4e : 0xb1, 0xf, 0xf, true));
+  }
+}
+
+// Sum of the squares of a row that lies in `lanes` neighbouring lanes (a power of two, the same for the wave), eight elements on end a lane and
+// turn, zeros behind its end; in the order of a wave that takes one element a lane and turn: a chain over the elements 64 apart, then
+// the 64 in the pairs of place ^ 32, 16, 8, 4, 2, 1.  So a row has the same bits here as in the kernels for any width.  More than one turn: 64 lanes.
+// Lanes 8 apart hold the chain's elements, in the same place of their eight: they exchange them until every lane has whole chains.
+template <int R> __device__ __forceinline__ float row_square_sum(const float (&x)[R][8], int lanes) {
+  if (R > 1 || lanes == 64) {
+    float s = 0.f;
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      float y[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) y[j] = x[u][j];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pair_swap<32>(y[j], y[j + 4]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pair_swap<16>(y[j / 2 * 4 + j % 2], y[j / 2 * 4 + j % 2 + 2]);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) pair_swap<8>(y[2 * j], y[2 * j + 1]);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) s = fmaf(y[i], y[i], s);
+    }
+    s += lane_xor<4>(s);
+    s += lane_xor<2>(s);
+    s += lane_xor<1>(s);
+    s = reduce16(reduce32(s, SumOf{}), SumOf{});
+    return s + row_rotated<8>(s);
+  }
+  float y[8], s[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) y[j] = x[0][j];
+  if (lanes == 32) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pair_swap<16>(y[j], y[j + 4]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pair_swap<8>(y[j / 2 * 4 + j % 2], y[j / 2 * 4 + j % 2 + 2]);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      s[j] = 0.f;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) s[j] = fmaf(y[2 * i + j], y[2 * i + j], s[j]);
+      s[j] += lane_xor<4>(s[j]);
+      s[j] += lane_xor<2>(s[j]);
+      s[j] += lane_xor<1>(s[j]);
+      s[j] = reduce16(s[j], SumOf{});
+      s[j] += row_rotated<8>(s[j]);
+    }
+    return s[0] + s[1];
+  }
+  if (lanes == 16) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) pair_swap<8>(y[j], y[j + 4]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      s[j] = fmaf(y[4 + j], y[4 + j], fmaf(y[j], y[j], 0.f));
+      s[j] += lane_xor<4>(s[j]);
+      s[j] += lane_xor<2>(s[j]);
+      s[j] += lane_xor<1>(s[j]);
+      s[j] += row_rotated<8>(s[j]);
+    }
+    return (s[0] + s[2]) + (s[1] + s[3]);
+  }
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    s[j] = fmaf(y[j], y[j], 0.f);
+    if (lanes >= 8) s[j] += lane_xor<4>(s[j]);
+    if (lanes >= 4) s[j] += lane_xor<2>(s[j]);
+    if (lanes >= 2) s[j] += lane_xor<1>(s[j]);
+  }
+  return ((s[0] + s[4]) + (s[2] + s[6])) + ((s[1] + s[5]) + (s[3] + s[7]));
+}
+
 // Block-wide sum for blocks of up to 1024 threads; `red` is LDS of >= 16 floats.
 // The result is the same in every thread; the order of additions is fixed.
 __device__ __forceinline__ float block_sum(float v, float* red) {

@@ -1,9 +1,9 @@
 // Behind a recurrence: every part (a head, a group of channels) of a token's row divided by its root mean square, times a weight a
 // channel, times a gate; for parts of up to 1,024 channels, a multiple of 8.  A part lies in neighbouring lanes of a wave, eight
-// channels a lane and turn, 16-byte accesses.
+// channels a lane and turn, 16-byte accesses; its squares are added in the order of the kernels for any width, so the bits are theirs.
 // Bound: the gate's exponential and division, and bytes (a wave a part, one channel a lane and turn, spent as much again on two-byte
-// loads and stores).  us: 3,000 rows of 16 x 128 23.0 -> 12.1, 1,950 rows of
-// 8 x 512, gated first 27.7 -> 14.1.
+// loads and stores).  us: 3,000 rows of 16 x 128 24.4 -> 12.6, 1,950 rows of 8 x 512, gated first 26.0 -> 13.8 (squares added as the lanes
+// come, with other bits, 11.6 and 13.4).
 #pragma once
 #include "common.h"
 
@@ -42,7 +42,6 @@ __global__ __launch_bounds__(256) void part_norm_kernel(PartNorm a, int log_lane
   const T* gate = a.act ? (const T*)a.proj + (size_t)t * a.stride + a.g_off + (size_t)p * a.gd : nullptr;
   float x[R][8];
   Run8<T> z[R];
-  float ss = 0.f;
 #pragma unroll
   for (int u = 0; u < R; ++u) {
     const int d = (li + u * kWave) * 8;
@@ -61,10 +60,8 @@ __global__ __launch_bounds__(256) void part_norm_kernel(PartNorm a, int log_lane
 #pragma unroll
       for (int j = 0; j < 8; ++j) x[u][j] *= part_gate(a.act, g[j]);
     }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) ss = fmaf(x[u][j], x[u][j], ss);
   }
-  ss = group_sum(ss, 1 << log_lanes);
+  const float ss = row_square_sum(x, 1 << log_lanes);
   const float inv = rsqrtf(ss / (float)a.gd + a.eps);
 #pragma unroll
   for (int u = 0; u < R; ++u) {

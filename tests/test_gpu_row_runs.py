@@ -70,6 +70,26 @@ def test_parts_in_neighbouring_lanes(T, groups, size, act, first, weighted, dtyp
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("size", [8, 16, 24, 64, 96, 128, 192, 256, 320, 512, 520, 1024])
+@pytest.mark.parametrize("first", [False, True])
+def test_parts_in_neighbouring_lanes_give_the_bits_of_a_wave_a_part(size, first, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(size)
+    T, groups, eps = 9, 5, 1e-3
+    N = groups * size
+    o = (torch.randn(T, N, generator=g) * 5).to(DEV)
+    w = torch.randn(N, generator=g).to(DEV)
+    gates = (torch.randn(T, N, generator=g) * 2).to(DT[dtype]).to(DEV)
+    wide = _shifted(gates)               # (gates that cannot be read by eights: a wave a part)
+    for act in (ops.GATE_SILU, ops.GATE_SIGMOID_ACT):
+        by = [ops.group_norm_gate(o, w, eps, groups, DT[dtype], x, off, act, gate_first=first) for x, off in ((gates, 0), (wide, 2))]
+        assert torch.equal(*by)
+    if not first:
+        assert torch.equal(*[ops.head_norm_gate(o, w[:size].contiguous(), eps, groups, size, DT[dtype], x, off) for x, off in ((gates, 0), (wide, 2))])
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T, H, e, gate", [(1, 1, 8, True), (70, 8, 128, False), (3, 5, 136, True), (9, 2, 512, True), (4, 3, 520, True)])
 def test_differences_of_maps_in_neighbouring_lanes(T, H, e, gate, dtype):
     from sharpinference_amd import ops
