@@ -109,6 +109,19 @@ def test_differences_of_maps_in_neighbouring_lanes(T, H, e, gate, dtype):
     assert float(((got - want).abs() - TOL[dtype] * want.abs() - terms).max()) <= 2.0 ** -60
 
 
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("e", [8, 16, 24, 64, 96, 128, 192, 256, 320, 512])
+def test_differences_of_maps_in_neighbouring_lanes_give_the_bits_of_a_wave_a_head(e, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(e)
+    T, H = 9, 5
+    flat = torch.randn(T * H * 2 * e, generator=g).to(DT[dtype]).to(DEV)
+    proj = torch.randn(T, 11 + H, generator=g).to(DT[dtype]).to(DEV)
+    moved = torch.cat([flat[:1], flat])[1:]          # (one element on: no 16-byte loads, a wave a head)
+    assert torch.equal(*[ops.map_difference(x.view(T, -1), H, e, 0.62, 1e-5, 0.7, proj, 11) for x in (flat, moved)])
+
+
 @pytest.mark.parametrize("T, N", [(1, 8), (70, 2056), (5, 1000), (3, 12)])
 def test_columns_side_by_side_add_as_one_by_one(T, N):
     from sharpinference_amd import ops
