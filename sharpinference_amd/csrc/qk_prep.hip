@@ -377,15 +377,21 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
 // squares and the partner run of a split rotation come by lane exchange, 16-byte accesses throughout.  A block has a thread for
 // every run of a token's heads where that is at most 1,024 (a norm over the whole projection asks for it), else blocks (token, y) share them; steps of many
 // tokens leave the values to blocks of their own behind the tokens' (value_pages.h).
-// Bound: a block's chain of latencies, so a run is requested before the angles are formed, and the next before one is worked on.  us, staged
-// through LDS before: 16 + 4 heads of 128, 1,900 tokens, norms over the projections 30 -> 13.6, with four taps 35 -> 28.3; two maps a head, 1,664 tokens
-// 18.5 -> 12.7.  64 + 8 heads of 192, 2,048 tokens (a block of 256 for three turns, each behind the one before) 41.8 -> 40.3.
+// Bound: a block's chain of latencies, so a run is requested before the angles are formed, and the next before one is worked on.  us, 16 + 4 heads
+// of 128, staged through LDS before: 1,900 tokens, norms over the projections 22.3 -> 12.4 (their squares added as the lanes come, with other bits,
+// 11.7), two maps a head 22.0 -> 12.5, four taps with the tail's launch 38.0 -> 29.0.  64 + 8 heads of 192, 2,048 tokens (a block of 256 for three turns, each
+// behind the one before) 40.2 -> 34.7.
 constexpr int kRunMaxThreads = 1024;
 
-template <typename T, int TAPS>
+// How the squares of a norm are added.  RUN_LANES: eight a lane, then the lanes.  RUN_ROW and RUN_WHOLE, a norm over the projection: in the staged
+// form's order, with its bits.  (Plain rows had the first before the others came here, and keep it.)
+enum : int { RUN_LANES = 0, RUN_ROW = 1, RUN_WHOLE = 2 };
+
+template <typename T, int TAPS, int SUMS>
 __global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run_kernel(PrepArgs a, int log_lanes) {
   __shared__ float cs_tab[kPrepMaxTurns], sn_tab[kPrepMaxTurns];
-  __shared__ __attribute__((aligned(16))) float red[2][kRunMaxThreads / kWave];
+  __shared__ float red[2][kPrepThreads / kWave];
+  extern __shared__ __attribute__((aligned(32))) float row[];          // (a norm over the whole projection: q | k of the token)
   __shared__ __attribute__((aligned(16))) char tile[kValueLds<T>];
   const int qn = a.nh * a.hd, kn = a.nkv * a.hd, runs = a.hd / 8, heads = a.nh + a.nkv;
   const bool own_v = a.v_off >= 0;
@@ -433,7 +439,8 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run
   for (;;) {
     const int h = (base + (int)threadIdx.x) >> log_lanes;
     const bool is_q = h < a.nh, live = in && h < heads;
-    float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float xs[1][8] = {{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
+    float(&x)[8] = xs[0];
     if (live) {
       if constexpr (TAPS == 0) {
         raw.floats(x);
@@ -452,26 +459,38 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run
     if (more) request();
     if (a.norm_mode != NORM_NONE) {                      // every lane takes part in the exchanges (a lane without a run holds zeros)
       float w8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (live) load8((is_q ? a.q_norm_w : a.k_norm_w) + (a.norm_mode == NORM_WHOLE ? (is_q ? h : h - a.nh) * a.hd : 0) + li * 8, w8);
-      float ss = 0.f, inv;
+      if (live) load8((is_q ? a.q_norm_w : a.k_norm_w) + (SUMS == RUN_WHOLE ? (is_q ? h : h - a.nh) * a.hd : 0) + li * 8, w8);
+      float inv;
+      if constexpr (SUMS != RUN_WHOLE) {
+        float ss = 0.f;
+        if constexpr (SUMS == RUN_LANES) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) ss = fmaf(x[j], x[j], ss);
-      if (a.norm_mode == NORM_PER_HEAD) {
-        inv = rsqrtf(group_sum(ss, 1 << log_lanes) / (float)a.hd + a.eps);
-      } else {                                           // (one turn)
-        const float sq = wave_sum(is_q ? ss : 0.f), sk = wave_sum(is_q ? 0.f : ss);
-        if (threadIdx.x % kWave == 0) {
-          red[0][threadIdx.x / kWave] = sq;
-          red[1][threadIdx.x / kWave] = sk;
+          for (int j = 0; j < 8; ++j) ss = fmaf(x[j], x[j], ss);
+          ss = group_sum(ss, 1 << log_lanes);
+        } else {
+          ss = row_square_sum(xs, 1 << log_lanes);
         }
-        if (threadIdx.x < kRunMaxThreads / kWave && threadIdx.x >= blockDim.x / kWave) red[0][threadIdx.x] = red[1][threadIdx.x] = 0.f;
+        inv = rsqrtf(ss / (float)a.hd + a.eps);
+      } else {                                           // (one turn)
+        if (live) store8(row + h * a.hd + li * 8, x);
+        __syncthreads();
+        if (threadIdx.x < kPrepThreads) {                // (the staged form's threads, chains and pairs)
+          float sq = 0.f, sk = 0.f;
+#pragma unroll 4
+          for (int c = threadIdx.x; c < qn; c += kPrepThreads) sq = fmaf(row[c], row[c], sq);
+#pragma unroll 4
+          for (int c = threadIdx.x; c < kn; c += kPrepThreads) sk = fmaf(row[qn + c], row[qn + c], sk);
+          sq = wave_sum(sq);
+          sk = wave_sum(sk);
+          if (threadIdx.x % kWave == 0) {
+            red[0][threadIdx.x / kWave] = sq;
+            red[1][threadIdx.x / kWave] = sk;
+          }
+        }
         __syncthreads();
         float total = 0.f;
-#pragma unroll 1
-        for (int i = 0; i < (int)blockDim.x / kWave; i += 4) {
-          const float4 part = *reinterpret_cast<const float4*>(&red[is_q ? 0 : 1][i]);   // (a block's waves beyond the last: zeros)
-          total = total + part.x + part.y + part.z + part.w;
-        }
+#pragma unroll
+        for (int i = 0; i < kPrepThreads / kWave; ++i) total += red[is_q ? 0 : 1][i];
         inv = rsqrtf(total / (float)(is_q ? qn : kn) + a.eps);
       }
 #pragma unroll
@@ -603,12 +622,12 @@ SHARPI_EXPORT int sharpi_qk_prep(const void* proj, int dtype, int stride, int q_
                        (norm_mode != NORM_WHOLE || together);
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
   const bool taps4 = taps == 4 && at16(conv_w);
-#define PREP_BY_TAPS(GO)                                                    \
+#define PREP_BY_TAPS(GO, ...)                                               \
   do {                                                                      \
     if (dtype == DT_F32) {                                                  \
-      if (taps == 0) GO(float, 0); else if (taps4) GO(float, 4); else GO(float, -1);    \
+      if (taps == 0) GO(float, 0, ##__VA_ARGS__); else if (taps4) GO(float, 4, ##__VA_ARGS__); else GO(float, -1, ##__VA_ARGS__);    \
     } else {                                                                \
-      if (taps == 0) GO(bf16_t, 0); else if (taps4) GO(bf16_t, 4); else GO(bf16_t, -1); \
+      if (taps == 0) GO(bf16_t, 0, ##__VA_ARGS__); else if (taps4) GO(bf16_t, 4, ##__VA_ARGS__); else GO(bf16_t, -1, ##__VA_ARGS__); \
     }                                                                       \
   } while (0)
   if (by_runs) {
@@ -616,8 +635,13 @@ SHARPI_EXPORT int sharpi_qk_prep(const void* proj, int dtype, int stride, int q_
     // not together: a block a turn of few tokens; of many four turns or so a block, to share the angles
     const int turns = ceil_div(items, threads), y = n_tokens <= kPrepSplitTokens ? turns : ceil_div(turns, 4);
     const dim3 rgrid(n_tokens + ceil_div(tiles, y), y);
-#define RUN_GO(T, TAPSV) qk_prep_run_kernel<T, TAPSV><<<rgrid, threads, 0, stream>>>(a, __builtin_ctz(lanes))
-    PREP_BY_TAPS(RUN_GO);
+    const size_t row_lds = norm_mode == NORM_WHOLE ? (size_t)(qn + kn) * sizeof(float) : 0;
+    const bool plain = (half_split || rotary_dim == 0) && taps == 0 && maps == 1 && v_off >= 0;
+#define RUN_GO(T, TAPSV, SUMSV) qk_prep_run_kernel<T, TAPSV, SUMSV><<<rgrid, threads, row_lds, stream>>>(a, __builtin_ctz(lanes))
+    if (norm_mode == NORM_WHOLE) PREP_BY_TAPS(RUN_GO, RUN_WHOLE);
+    else if (!plain) PREP_BY_TAPS(RUN_GO, RUN_ROW);
+    else if (dtype == DT_F32) RUN_GO(float, 0, RUN_LANES);
+    else RUN_GO(bf16_t, 0, RUN_LANES);
 #undef RUN_GO
     SHARPI_CHECK_LAUNCH();
   } else {

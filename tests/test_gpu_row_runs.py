@@ -131,3 +131,37 @@ def test_columns_side_by_side_add_as_one_by_one(T, N):
     for dtype in DT.values():
         y = x.to(dtype)
         assert torch.equal(ops.add_bias(y.clone(), b), (y.float() + b).to(dtype))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T", [9, 70])
+@pytest.mark.parametrize("hd", [16, 64, 96, 128, 192, 256, 512])
+@pytest.mark.parametrize("form", ["pairs", "conv", "conv3", "keys", "maps", "maps conv", "whole", "whole conv", "whole keys pairs"])
+def test_heads_by_runs_give_the_bits_of_the_staged_form(form, hd, T, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(hd + T + len(form))
+    nh, nkv, vd, r, ps = (4, 2, 40, 16, 16) if hd > 256 else (6, 2, 40, 16, 16)
+    keys, whole, maps = "keys" in form, "whole" in form, 2 if "maps" in form else 1
+    r, vd = min(r, hd // maps), hd if keys else vd
+    if r < 16 and "pairs" not in form:
+        r = 0
+    qn, kn, vn, pages = nh * hd, nkv * hd, 0 if keys else nkv * vd, T // ps + 3
+    C, taps = qn + kn + vn, 3 if form == "conv3" else 4 if "conv" in form else 0
+    proj = torch.randn(T, C + 8, generator=g).to(DT[dtype]).to(DEV)
+    wq, wk = (torch.rand(n, generator=g).to(DEV) + 0.5 for n in ((qn, kn) if whole else (hd, hd)))
+    conv = torch.randn(C, taps, generator=g).to(DEV) if taps else None
+    freq = torch.tensor([300.0 ** (-2.0 * i / r) for i in range(r // 2)], device=DEV) if r else None
+    slots = torch.randperm(pages * ps, generator=g)[:T].to(torch.int32).to(DEV)
+    held = torch.randn(2, max(taps - 1, 1), C, generator=g).to(DEV)
+    ctx, results = _Step([3, T - 3], [1, 0]), []
+    for rows, off in ((proj, 0), (_shifted(proj), 2)):           # (rows that cannot be read by eights are staged)
+        kc = torch.zeros(pages, nkv, ps, hd, dtype=DT[dtype], device=DEV)
+        vc = torch.zeros(pages, nkv, vd, ps, dtype=DT[dtype], device=DEV)
+        tail = held.clone() if taps else None
+        q = ops.qk_prep(rows, off, off + qn, None if keys else off + qn + kn, nh, nkv, hd, vd, ctx, kc, vc, slots,
+                        ops.NORM_WHOLE if whole else ops.NORM_PER_HEAD, wq, wk, 1e-5, freq,
+                        ops.PAIRS_INTERLEAVED if "pairs" in form else ops.PAIRS_HALF_SPLIT, 1.0, conv, tail, maps=maps)
+        results.append((q, kc, vc) + ((tail,) if taps else ()))
+    for a, b in zip(*results):
+        assert torch.equal(a, b)
