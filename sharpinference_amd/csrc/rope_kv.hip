@@ -80,14 +80,14 @@ __global__ void rope_kv_kernel(const T* __restrict__ qkv, T* __restrict__ q_out,
         const float ang = (float)pos * inv_freq[i];
         const float c = cosf(ang);
         const float s = sinf(ang);
-        const float ra = a * c - b * s;
-        const float rb = a * s + b * c;
+        const float ra = fmaf(a, c, -(b * s));       // (written out: the vector form below has the same bits)
+        const float rb = fmaf(b, c, a * s);
         a = ra;
         b = rb;
       }
       x0[j] = a;
       x1[j] = b;
-      ss += a * a + b * b;
+      ss += fmaf(b, b, a * a);
     }
   }
   float mul = 1.0f;
@@ -131,20 +131,33 @@ __global__ void rope_kv_kernel(const T* __restrict__ qkv, T* __restrict__ q_out,
 // them, 256 runs each, so that a handful of decode tokens still spreads over many compute units.  The token's angles are the
 // same for every head: a block computes each of them once, into LDS (four sines and cosines in every thread were the kernel's
 // time).  Steps of many tokens leave the values to blocks of their own behind the tokens' (value_pages.h).
-// Bound: the rows' bytes.  40 + 8 heads of 128 and 8 of values, us: 2,048 tokens 30 -> 17.8, 8,192 104 -> 54.7 (235 MB: 4.3 TB/s, about
-// a copy's rate); 16 + 4 heads with split pairs, 1,950 tokens (a wave a head before) 20.9 -> 12.2.
+// Interleaved pairs of heads as wide as their values (PAIRS false) keep the sums this form always had: eight squares a lane, then the lanes.  The
+// others (PAIRS) add their squares pair by pair in the general kernel's order, through LDS, and have its bits, so that a row has the same
+// bits however many tokens come with it (heads and values of two widths come here in steps of many tokens alone).
+// Bound: the rows' bytes.  40 + 8 heads of 128 and 8 of values, us: 2,048 tokens 24.2 -> 12.6 (104 -> 54.7 for 8,192, 235 MB: 4.3 TB/s, about
+// a copy's rate); 1,950 tokens with split pairs (a wave a head before), 16 + 8 heads 25.3 -> 12.3, 16 + 4 19.2 -> 10.8 (with the lanes' order of
+// the sum, other bits than a wave a head, 10.9 and 9.7).
 constexpr int kRopeMaxAngles = 128;              // hd <= 256
+// A wave's sums of a pair's two squares: a head of L lanes has 4 L, at 5 L from the head before (neighbouring heads' reads in different banks).
+constexpr int kRopeWavePairs = 5 * kWave;
 constexpr int kRopeSplitTokens = 64;             // up to so many tokens a step, a token's heads lie in several blocks
 
-template <typename T>
+// what a wave's lanes stored to LDS is there for its other lanes (a wave's LDS accesses stay in their order; the compiler has to keep it)
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <typename T, bool PAIRS>
 __global__ __launch_bounds__(256) void rope_kv_vec_kernel(
     const T* __restrict__ qkv, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache,
     const int* __restrict__ slot_mapping, const int* __restrict__ positions, const float* __restrict__ inv_freq,
     const float* __restrict__ bias, int qk_norm, float eps, int temp_tuning, float floor_scale, float attn_scale,
     int n_tokens, int nh, int nkv, int hd, int vd, int page_size, int half_split, int rotary_dim, int row_stride, int values_apart) {
-  __shared__ __attribute__((aligned(16))) char tile[kValueLds<T>];
+  constexpr size_t kTile = kValueLds<T> > 4 * kRopeWavePairs * sizeof(float) ? kValueLds<T> : 4 * kRopeWavePairs * sizeof(float);
+  __shared__ __attribute__((aligned(16))) char tile[kTile];     // (value blocks: their tile; the others: their waves' pairs of squares)
   __shared__ int tile_slots[kValueTokens];
-  __shared__ float cs_tab[kRopeMaxAngles], sn_tab[kRopeMaxAngles];
+  __shared__ __attribute__((aligned(16))) float cs_tab[kRopeMaxAngles], sn_tab[kRopeMaxAngles];
   if (blockIdx.x >= n_tokens) {                    // (values_apart: the blocks behind the tokens')
     const size_t v_at = (size_t)(nh + nkv) * hd;
     values_to_pages<T>(blockIdx.x - n_tokens, n_tokens, nkv, vd, page_size, slot_mapping, v_cache, reinterpret_cast<T*>(tile), tile_slots,
@@ -176,20 +189,18 @@ __global__ __launch_bounds__(256) void rope_kv_vec_kernel(
     __syncthreads();
   }
   // a thread's run within a head is the same in every turn of the loop (the block size is a multiple
-  // of the lanes per head), and so are its angles: x becomes x cs + (its partner) sn
+  // of the lanes per head), and so are its angles
   const int run = threadIdx.x % per_head;
   const int half_runs = rotary_dim / 16;           // (split pairs: runs of the low half)
-  float cs[8], sn[8];
   const bool rotates = inv_freq != nullptr && run * 8 < rotary_dim;
   const bool low = run < half_runs;
   const int mate = (threadIdx.x & (kWave - 1)) + (low ? half_runs : -half_runs);
-  if (rotates) {
+  const int ang = !rotates ? 0 : PAIRS && half_split ? (low ? run : run - half_runs) * 8 : run * 4;      // the run's first angle
+  float cs4[4], sn4[4];                            // (interleaved pairs keep their four)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int i = half_split ? (low ? run : run - half_runs) * 8 + j : run * 4 + j / 2;
-      cs[j] = cs_tab[i];
-      sn[j] = (half_split ? low : j % 2 == 0) ? -sn_tab[i] : sn_tab[i];
-    }
+  for (int j = 0; j < 4; ++j) {
+    cs4[j] = rotates ? cs_tab[ang + j] : 1.f;
+    sn4[j] = rotates ? sn_tab[ang + j] : 0.f;
   }
   for (int base = blockIdx.y * blockDim.x; base < chunks; base += gridDim.y * blockDim.x) {
     const int ci = base + threadIdx.x;
@@ -207,25 +218,50 @@ __global__ __launch_bounds__(256) void rope_kv_vec_kernel(
         for (int j = 0; j < 8; ++j) x[j] += b8[j];
       }
     }
-    float ss = 0.f;
-    if (half_split && inv_freq) {      // every lane takes part in the shuffles
+    [[maybe_unused]] float other[8];   // (PAIRS: split pairs' partners, turned as x is)
+    if (PAIRS && half_split && inv_freq) {      // every lane takes part in the shuffles
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const float other = __shfl(x[j], mate & (kWave - 1), kWave);
-        if (rotates && (is_q || is_k)) x[j] = x[j] * cs[j] + other * sn[j];
+      for (int j = 0; j < 8; ++j) other[j] = __shfl(x[j], mate & (kWave - 1), kWave);
+      if (rotates && (is_q || is_k)) {
+        float c[8], sn[8];
+        load8(cs_tab + ang, c);
+        load8(sn_tab + ang, sn);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float own = x[j];
+          x[j] = fmaf(own, c[j], low ? -(other[j] * sn[j]) : other[j] * sn[j]);
+          other[j] = fmaf(other[j], c[j], low ? own * sn[j] : -(own * sn[j]));
+        }
       }
     } else if (rotates && (is_q || is_k)) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float a = x[2 * j], b = x[2 * j + 1];
-        x[2 * j] = a * cs[2 * j] + b * sn[2 * j];
-        x[2 * j + 1] = a * sn[2 * j + 1] + b * cs[2 * j];
+        x[2 * j] = fmaf(a, cs4[j], -(b * sn4[j]));
+        x[2 * j + 1] = PAIRS ? fmaf(b, cs4[j], a * sn4[j]) : fmaf(a, sn4[j], b * cs4[j]);
       }
     }
     if (qk_norm) {
-      if (valid && (is_q || is_k)) {
+      float ss = 0.f;
+      if constexpr (PAIRS) {
+        float* const head_pairs = reinterpret_cast<float*>(tile) + threadIdx.x / kWave * kRopeWavePairs + (threadIdx.x & (kWave - 1)) / per_head * 5 * per_head;
+        if (!(half_split && rotates)) {
+          *reinterpret_cast<float4*>(head_pairs + 4 * run) = make_float4(fmaf(x[1], x[1], x[0] * x[0]), fmaf(x[3], x[3], x[2] * x[2]),
+                                                                         fmaf(x[5], x[5], x[4] * x[4]), fmaf(x[7], x[7], x[6] * x[6]));
+        } else if (low) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ss += x[j] * x[j];
+          for (int j = 0; j < 8; j += 4)
+            *reinterpret_cast<float4*>(head_pairs + 8 * run + j) =
+                make_float4(fmaf(other[j], other[j], x[j] * x[j]), fmaf(other[j + 1], other[j + 1], x[j + 1] * x[j + 1]),
+                            fmaf(other[j + 2], other[j + 2], x[j + 2] * x[j + 2]), fmaf(other[j + 3], other[j + 3], x[j + 3] * x[j + 3]));
+        }
+        wave_lds_fence();
+        ss = (head_pairs[run] + head_pairs[run + 2 * per_head]) + (head_pairs[run + per_head] + head_pairs[run + 3 * per_head]);
+        wave_lds_fence();
+      } else if (valid && (is_q || is_k)) {
+        ss = fmaf(x[0], x[0], x[1] * x[1]);
+#pragma unroll
+        for (int j = 2; j < 8; ++j) ss = fmaf(x[j], x[j], ss);
       }
       ss = group_sum(ss, per_head);
       const float mul = 1.0f / sqrtf(ss / (float)hd + eps);
@@ -282,12 +318,15 @@ SHARPI_EXPORT int sharpi_rope_kv(const void* qkv, void* q_out, void* k_cache, vo
       rotary_dim % (pair_layout ? 16 : 8) == 0 && (row_stride & 7) == 0 && at16(qkv) && at16(q_out) && at16(k_cache) && at16(bias)) {
     const int tiles = many ? value_tiles(n_tokens, nkv * vd) : 0;
     const dim3 vgrid(n_tokens + tiles, many ? 1 : ceil_div((nh + 2 * nkv) * (hd >> 3), 256));
-#define ROPE_GO(T)                                                                                                               \
-  rope_kv_vec_kernel<T><<<vgrid, 256, 0, stream>>>((const T*)qkv, (T*)q_out, (T*)k_cache, (T*)v_cache, slot_mapping, positions, inv_freq, \
+#define ROPE_GO(T, PAIRS)                                                                                                               \
+  rope_kv_vec_kernel<T, PAIRS><<<vgrid, 256, 0, stream>>>((const T*)qkv, (T*)q_out, (T*)k_cache, (T*)v_cache, slot_mapping, positions, inv_freq, \
                                                    bias, qk_norm, eps, temp_tuning, floor_scale, attn_scale, n_tokens, nh, nkv, hd, vd,   \
                                                    page_size, pair_layout, rotary_dim, row_stride, many)
-    if (dtype == DT_F32) ROPE_GO(float);
-    else ROPE_GO(bf16_t);
+    const bool pairs = pair_layout || vd != hd;
+    if (dtype == DT_F32 && pairs) ROPE_GO(float, true);
+    else if (dtype == DT_F32) ROPE_GO(float, false);
+    else if (pairs) ROPE_GO(bf16_t, true);
+    else ROPE_GO(bf16_t, false);
 #undef ROPE_GO
     SHARPI_CHECK_LAUNCH();
     return SHARPI_OK;

@@ -165,3 +165,28 @@ def test_heads_by_runs_give_the_bits_of_the_staged_form(form, hd, T, dtype):
         results.append((q, kc, vc) + ((tail,) if taps else ()))
     for a, b in zip(*results):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("hd, r, vd, layout", [(128, 128, 128, 1), (128, 32, 128, 1), (32, 16, 32, 1), (64, 64, 64, 1), (256, 96, 256, 1), (256, 256, 256, 1),
+                                               (64, 0, 64, 1), (128, 32, 40, 0), (64, 64, 72, 0), (256, 128, 8, 0), (32, 8, 24, 0), (128, 64, 72, 1)])
+@pytest.mark.parametrize("T", [7, 70])
+@pytest.mark.parametrize("norm", [True, False])
+def test_rotated_heads_by_runs_give_the_bits_of_a_wave_a_head(norm, T, hd, r, vd, layout, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(hd + r + T)
+    nh, nkv, ps = 5, 3, 16
+    width, pages = (nh + nkv) * hd + nkv * vd, T // ps + 3
+    rows = torch.randn(T, width, generator=g).to(DT[dtype]).to(DEV)
+    bias = torch.randn(width, generator=g).to(DEV)
+    freq = torch.tensor([300.0 ** (-2.0 * i / r) for i in range(r // 2)], device=DEV) if r else None
+    slots = torch.randperm(pages * ps, generator=g)[:T].to(torch.int32).to(DEV)
+    pos, out = (torch.arange(T) * 7).to(torch.int32).to(DEV), []
+    for extra in (0, 3):                 # (rows of another stride: a wave a head)
+        qkv = torch.nn.functional.pad(rows, (0, extra)) if extra else rows
+        kc = torch.zeros(pages, nkv, ps, hd, dtype=DT[dtype], device=DEV)
+        vc = torch.zeros(pages, nkv, vd, ps, dtype=DT[dtype], device=DEV)
+        out.append((ops.rope_kv(qkv, kc, vc, slots, pos, freq, norm, 1e-5, (40.0, 0.1), nh, nkv, hd, layout, bias, vd, extra), kc, vc))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
