@@ -133,13 +133,14 @@ __global__ void rope_kv_kernel(const T* __restrict__ qkv, T* __restrict__ q_out,
 // time).  Steps of many tokens leave the values to blocks of their own behind the tokens' (value_pages.h).
 // Interleaved pairs of heads as wide as their values (PAIRS false) keep the sums this form always had: eight squares a lane, then the lanes.  The
 // others (PAIRS) add their squares pair by pair in the general kernel's order, through LDS, and have its bits, so that a row has the same
-// bits however many tokens come with it (heads and values of two widths come here in steps of many tokens alone).
+// bits however many tokens come with it (they come here in steps of many tokens alone).
 // Bound: the rows' bytes.  40 + 8 heads of 128 and 8 of values, us: 2,048 tokens 24.2 -> 12.6 (104 -> 54.7 for 8,192, 235 MB: 4.3 TB/s, about
 // a copy's rate); 1,950 tokens with split pairs (a wave a head before), 16 + 8 heads 25.3 -> 12.3, 16 + 4 19.2 -> 10.8 (with the lanes' order of
 // the sum, other bits than a wave a head, 10.9 and 9.7).
 constexpr int kRopeMaxAngles = 128;              // hd <= 256
 // A wave's sums of a pair's two squares: a head of L lanes has 4 L, at 5 L from the head before (neighbouring heads' reads in different banks).
 constexpr int kRopeWavePairs = 5 * kWave;
+constexpr int kRopeChipWaves = 256 * 32;         // 256 compute units of 32 waves
 constexpr int kRopeSplitTokens = 64;             // up to so many tokens a step, a token's heads lie in several blocks
 
 // what a wave's lanes stored to LDS is there for its other lanes (a wave's LDS accesses stay in their order; the compiler has to keep it)
@@ -314,7 +315,11 @@ SHARPI_EXPORT int sharpi_rope_kv(const void* qkv, void* q_out, void* k_cache, vo
   // per token, which then computes its angles once for all heads, and blocks of their own for the values
   const bool many = n_tokens > kRopeSplitTokens;
   const auto at16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  if ((hd == 32 || hd == 64 || hd == 128 || hd == 256) && (vd == hd || (many && vd % 8 == 0)) &&
+  const bool pairs = pair_layout || vd != hd;
+  // (the forms that have the general kernel's bits go there until its waves are more than the chip holds at once: us, a wave a head / runs, split
+  // pairs: 1 token of 16 + 4 heads 2.8 / 3.6, 64 3.3 / 4.0, 200 4.3 / 4.8, 400 6.0 / 5.3; 100 tokens of 40 + 8 4.4 / 5.8, 200 6.6 / 6.1)
+  const bool by_runs = !pairs || (many && (long long)n_tokens * (nh + 2 * nkv) > kRopeChipWaves);
+  if (by_runs && (hd == 32 || hd == 64 || hd == 128 || hd == 256) && vd % 8 == 0 &&
       rotary_dim % (pair_layout ? 16 : 8) == 0 && (row_stride & 7) == 0 && at16(qkv) && at16(q_out) && at16(k_cache) && at16(bias)) {
     const int tiles = many ? value_tiles(n_tokens, nkv * vd) : 0;
     const dim3 vgrid(n_tokens + tiles, many ? 1 : ceil_div((nh + 2 * nkv) * (hd >> 3), 256));
@@ -322,7 +327,6 @@ SHARPI_EXPORT int sharpi_rope_kv(const void* qkv, void* q_out, void* k_cache, vo
   rope_kv_vec_kernel<T, PAIRS><<<vgrid, 256, 0, stream>>>((const T*)qkv, (T*)q_out, (T*)k_cache, (T*)v_cache, slot_mapping, positions, inv_freq, \
                                                    bias, qk_norm, eps, temp_tuning, floor_scale, attn_scale, n_tokens, nh, nkv, hd, vd,   \
                                                    page_size, pair_layout, rotary_dim, row_stride, many)
-    const bool pairs = pair_layout || vd != hd;
     if (dtype == DT_F32 && pairs) ROPE_GO(float, true);
     else if (dtype == DT_F32) ROPE_GO(float, false);
     else if (pairs) ROPE_GO(bf16_t, true);

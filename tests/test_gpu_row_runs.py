@@ -170,7 +170,7 @@ def test_heads_by_runs_give_the_bits_of_the_staged_form(form, hd, T, dtype):
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("hd, r, vd, layout", [(128, 128, 128, 1), (128, 32, 128, 1), (32, 16, 32, 1), (64, 64, 64, 1), (256, 96, 256, 1), (256, 256, 256, 1),
                                                (64, 0, 64, 1), (128, 32, 40, 0), (64, 64, 72, 0), (256, 128, 8, 0), (32, 8, 24, 0), (128, 64, 72, 1)])
-@pytest.mark.parametrize("T", [7, 70])
+@pytest.mark.parametrize("T", [7, 70, 744, 746])       # (eleven heads: 8,184 and 8,206 waves, on both sides of the choice)
 @pytest.mark.parametrize("norm", [True, False])
 def test_rotated_heads_by_runs_give_the_bits_of_a_wave_a_head(norm, T, hd, r, vd, layout, dtype):
     from sharpinference_amd import ops
