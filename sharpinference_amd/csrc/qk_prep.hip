@@ -63,6 +63,7 @@ struct PrepArgs {
   int v_other_stride, v_other_off;
   float v_mix;             // c
   int values_apart;        // values go in blocks of their own behind the tokens' (value_pages.h)
+  int values_beside;       // (runs) few tokens: a token's values go in a block of their own, the last of its column
   int n_tokens;
   int by8;                 // every offset, stride and width a multiple of 8 (and split halves): eight channels a thread
 };
@@ -76,27 +77,48 @@ template <typename T, int TAPS>
 __device__ __forceinline__ void prep_gather8(const PrepArgs& a, int t, int c, int col, int C, float* y) {
   const T* proj = (const T*)a.proj;
   if constexpr (TAPS != 0) {
-    const int e = a.entry_of_token[t];
-    const int li = t - a.cu_tokens[e];                 // the token's place in its entry
-    if (TAPS == 4 && li >= 3) {
-      // The four rows, as they lie in memory, and the eight channels' weights (32 floats on end, 16 bytes a load) are all requested
-      // before the first is used; a weight and a row at a time the loads' number and latency were the kernel's time
-      // (1900 tokens of 4096 channels: 62 -> 35 us).
-      Run8<T> u[4];
+    if constexpr (TAPS == 4) {
+      // The four rows, as they lie in memory or, of an entry's first three tokens, in the tail, and the eight channels' weights (32 floats on
+      // end, 16 bytes a load) are all requested before the first is used; a weight and a row at a time the loads' number and latency were
+      // the kernel's time (1900 tokens of 4096 channels: 62 -> 35 us).
       float4 cw[8];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) u[j].load(proj + (size_t)(t - 3 + j) * a.stride + col);
-#pragma unroll
       for (int i = 0; i < 8; ++i) cw[i] = *reinterpret_cast<const float4*>(a.conv_w + (size_t)(c + i) * 4);
-      float v[8];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        u[j].floats(v);
+      const auto add = [&](int j, const float* v) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) y[i] = fmaf(j == 0 ? cw[i].x : j == 1 ? cw[i].y : j == 2 ? cw[i].z : cw[i].w, v[i], j == 0 ? 0.f : y[i]);
+      };
+      const int e = a.entry_of_token[t], li = t - a.cu_tokens[e];          // (the token's place in its entry)
+      const T* rows = proj + (size_t)t * a.stride + col;
+      if (li >= 3) {
+        Run8<T> u[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) u[j].load(rows - (size_t)(3 - j) * a.stride);
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          u[j].floats(v);
+          add(j, v);
+        }
+      } else {
+        const float* tail = a.tail + ((size_t)a.state_slots[e] * 3 + li) * C + c;
+        Run8<T> own;
+        float v[3][8];
+        own.load(rows);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+          if (3 - j > li) load8(tail + (size_t)j * C, v[j]);
+          else load8(rows - (size_t)(3 - j) * a.stride, v[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < 3; ++j) add(j, v[j]);
+        own.floats(v[0]);
+        add(3, v[0]);
       }
       return;
     }
+    const int e = a.entry_of_token[t];
+    const int li = t - a.cu_tokens[e];                 // the token's place in its entry
     const float* tail = a.tail + (size_t)a.state_slots[e] * (a.taps - 1) * C;
 #pragma unroll
     for (int i = 0; i < 8; ++i) y[i] = 0.f;
@@ -377,10 +399,12 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
 // squares and the partner run of a split rotation come by lane exchange, 16-byte accesses throughout.  A block has a thread for
 // every run of a token's heads where that is at most 1,024 (a norm over the whole projection asks for it), else blocks (token, y) share them; steps of many
 // tokens leave the values to blocks of their own behind the tokens' (value_pages.h).
-// Bound: a block's chain of latencies, so a run is requested before the angles are formed, and the next before one is worked on.  us, 16 + 4 heads
-// of 128, staged through LDS before: 1,900 tokens, norms over the projections 22.3 -> 12.4 (their squares added as the lanes come, with other bits,
-// 11.7), two maps a head 22.0 -> 12.5, four taps with the tail's launch 38.0 -> 29.0.  64 + 8 heads of 192, 2,048 tokens (a block of 256 for three turns, each
-// behind the one before) 40.2 -> 34.7.
+// Bound: a block's chain of latencies, so a run and its norm's weights are requested before the angles are formed, and the next before one is
+// worked on; in short steps the values of a token, another chain, go in a block beside those of its heads.  us, 16 + 4 heads
+// of 128, staged through LDS before: 1,900 tokens, norms over the projections 22.3 -> 12.7 (their squares added as the lanes come, with other bits,
+// 11.7), two maps a head 21.9 -> 13.0, four taps with the tail's launch 37.9 -> 28.1; 8 tokens, a norm a head 4.6 -> 4.4 (weights and values behind
+// the rest: 5.0), over the projections 7.7 -> 5.1, four taps 11.4 -> 7.9 (a tap of the tail at a time: 14.2).  64 + 8 heads of 192, 2,048 tokens (a block of
+// 256 for three turns, each behind the one before) 40.9 -> 35.
 constexpr int kRunMaxThreads = 1024;
 
 // How the squares of a norm are added.  RUN_LANES: eight a lane, then the lanes.  RUN_ROW and RUN_WHOLE, a norm over the projection: in the staged
@@ -407,20 +431,26 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run
     return;
   }
   const int t = blockIdx.x;
+  const int slot = a.slot_mapping ? a.slot_mapping[t] : -1;
   // a thread's run inside a head is the same in every turn
   const int li = threadIdx.x & ((1 << log_lanes) - 1);
   const bool in = li < runs;
+  const int parts = gridDim.y - a.values_beside, step = parts * blockDim.x;
+  const bool values_only = (int)blockIdx.y >= parts;
   int base = blockIdx.y * blockDim.x;
-  Run8<T> raw;                             // (without a convolution) the next turn's run, on its way
+  constexpr bool kAhead = TAPS == 0 && SUMS != RUN_WHOLE;
+  Run8<T> raw;                             // (without a convolution) the next turn's run, on its way, and a head's norm weights
+  Run8<float> weight;
   const auto column = [&](int h) { return (h < a.nh ? a.q_off + h * a.hd : a.k_off + (h - a.nh) * a.hd) + li * 8; };
   const auto request = [&]() {
     const int h = (base + (int)threadIdx.x) >> log_lanes;
-    if (TAPS == 0 && in && h < heads) raw.load((const T*)a.proj + (size_t)t * a.stride + column(h));
+    if (!in || h >= heads) return;
+    if (TAPS == 0) raw.load((const T*)a.proj + (size_t)t * a.stride + column(h));
+    if (kAhead && a.norm_mode != NORM_NONE) weight.load((h < a.nh ? a.q_norm_w : a.k_norm_w) + li * 8);
   };
-  request();
+  if (!values_only) request();
   const float pos = (float)a.positions[t];
-  const int slot = a.slot_mapping ? a.slot_mapping[t] : -1;
-  if (a.inv_freq) {
+  if (a.inv_freq && !values_only) {
     for (int i = threadIdx.x; i < a.rotary_dim / 2; i += blockDim.x) {
       float sn, cs;
       sincosf(pos * a.inv_freq[i], &sn, &cs);
@@ -436,7 +466,7 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run
   const bool low = lm < half_runs, turns = a.inv_freq && in && lm * 8 < a.rotary_dim;
   const int mate = (int)threadIdx.x + (low ? half_runs : -half_runs);
   const int ang = a.half_split ? (low ? lm : lm - half_runs) * 8 : lm * 4;     // the run's first angle
-  for (;;) {
+  for (bool more = !values_only; more;) {
     const int h = (base + (int)threadIdx.x) >> log_lanes;
     const bool is_q = h < a.nh, live = in && h < heads;
     float xs[1][8] = {{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
@@ -454,12 +484,13 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run
         prep_gather8<T, TAPS>(a, t, h * a.hd + li * 8, column(h), C, x);
       }
     }
-    base += gridDim.y * blockDim.x;
-    const bool more = base < (heads << log_lanes);
+    base += step;
+    more = base < (heads << log_lanes);
+    float w8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    if (kAhead && live && a.norm_mode != NORM_NONE) weight.floats(w8);
     if (more) request();
     if (a.norm_mode != NORM_NONE) {                      // every lane takes part in the exchanges (a lane without a run holds zeros)
-      float w8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      if (live) load8((is_q ? a.q_norm_w : a.k_norm_w) + (SUMS == RUN_WHOLE ? (is_q ? h : h - a.nh) * a.hd : 0) + li * 8, w8);
+      if (!kAhead && live) load8((is_q ? a.q_norm_w : a.k_norm_w) + (SUMS == RUN_WHOLE ? (is_q ? h : h - a.nh) * a.hd : 0) + li * 8, w8);
       float inv;
       if constexpr (SUMS != RUN_WHOLE) {
         float ss = 0.f;
@@ -529,10 +560,10 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run
         store8((T*)a.k_cache + (((size_t)page * a.nkv + (h - a.nh)) * a.page_size + off) * a.hd + li * 8, x);
       }
     }
-    if (!more) break;
   }
-  if (slot < 0 || a.values_apart) return;
-  for (int i = (blockIdx.y * blockDim.x + threadIdx.x) * 8; i < a.nkv * a.vd; i += gridDim.y * blockDim.x * 8) {
+  if (slot < 0 || a.values_apart || (a.values_beside && !values_only)) return;
+  const int v_part = a.values_beside ? 0 : blockIdx.y, v_parts = a.values_beside ? 1 : gridDim.y;
+  for (int i = (v_part * blockDim.x + threadIdx.x) * 8; i < a.nkv * a.vd; i += v_parts * blockDim.x * 8) {
     float v[8];
     prep_gather8<T, TAPS>(a, t, v_at + i, v_col + i, C, v);
     prep_mix8<T>(a, t, i, v);
@@ -612,7 +643,7 @@ SHARPI_EXPORT int sharpi_qk_prep(const void* proj, int dtype, int stride, int q_
   PrepArgs a{proj, stride, q_off, k_off, v_off, nh, nkv, hd, vd, conv_w, taps, tail, state_slots, entry_of_token,
              cu_tokens, positions, norm_mode, q_norm_w, k_norm_w, eps, rotary_dim > 0 ? inv_freq : nullptr, rotary_dim,
              half_split, magnitude, q_out, k_cache, v_cache, slot_mapping, page_size, parts, bias, temp_on, temp_floor,
-             temp_scale, maps, v_other, v_other_stride, v_other_off, v_mix, v_apart, n_tokens, by8};
+             temp_scale, maps, v_other, v_other_stride, v_other_off, v_mix, v_apart, 0, n_tokens, by8};
   const int lanes = hd <= 64 ? (hd <= 8 ? 1 : hd <= 16 ? 2 : hd <= 32 ? 4 : 8) : hd <= 128 ? 16 : hd <= 256 ? 32 : 64;
   const int items = (nh + nkv) * lanes;
   // a thread for every run where a block can have them; of a few tokens 256 a block, or the launch would leave the chip empty (a
@@ -634,7 +665,8 @@ SHARPI_EXPORT int sharpi_qk_prep(const void* proj, int dtype, int stride, int q_
     const int threads = together ? max(kValueThreads, ceil_div(items, kWave) * kWave) : kPrepThreads;
     // not together: a block a turn of few tokens; of many four turns or so a block, to share the angles
     const int turns = ceil_div(items, threads), y = n_tokens <= kPrepSplitTokens ? turns : ceil_div(turns, 4);
-    const dim3 rgrid(n_tokens + ceil_div(tiles, y), y);
+    a.values_beside = !v_apart && slot_mapping != nullptr;
+    const dim3 rgrid(n_tokens + ceil_div(tiles, y), y + a.values_beside);
     const size_t row_lds = norm_mode == NORM_WHOLE ? (size_t)(qn + kn) * sizeof(float) : 0;
     const bool plain = (half_split || rotary_dim == 0) && taps == 0 && maps == 1 && v_off >= 0;
 #define RUN_GO(T, TAPSV, SUMSV) qk_prep_run_kernel<T, TAPSV, SUMSV><<<rgrid, threads, row_lds, stream>>>(a, __builtin_ctz(lanes))

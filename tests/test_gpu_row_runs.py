@@ -153,8 +153,8 @@ def test_heads_by_runs_give_the_bits_of_the_staged_form(form, hd, T, dtype):
     conv = torch.randn(C, taps, generator=g).to(DEV) if taps else None
     freq = torch.tensor([300.0 ** (-2.0 * i / r) for i in range(r // 2)], device=DEV) if r else None
     slots = torch.randperm(pages * ps, generator=g)[:T].to(torch.int32).to(DEV)
-    held = torch.randn(2, max(taps - 1, 1), C, generator=g).to(DEV)
-    ctx, results = _Step([3, T - 3], [1, 0]), []
+    held = torch.randn(4, max(taps - 1, 1), C, generator=g).to(DEV)
+    ctx, results = _Step([1, 2, T - 4, 1], [3, 0, 2, 1]), []
     for rows, off in ((proj, 0), (_shifted(proj), 2)):           # (rows that cannot be read by eights are staged)
         kc = torch.zeros(pages, nkv, ps, hd, dtype=DT[dtype], device=DEV)
         vc = torch.zeros(pages, nkv, vd, ps, dtype=DT[dtype], device=DEV)
