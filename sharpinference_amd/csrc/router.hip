@@ -1,8 +1,8 @@
 // MoE routing on the device: router logits, gate, top-k, and the expert-sorted row list.
 //
 // router_topk: one block per token, or per two or four tokens when there are many.
-// logits[e] = Wr[e, :] . x[t, :] in float (each wave owns experts e = wave, wave + nwaves, ...;
-// lanes stride over the hidden width, so the order of the additions depends on the width only).
+// logits[e] = Wr[e, :] . x[t, :] in float (a wave takes two or four neighbouring experts at a time, or one, and goes on behind
+// those of the block's other waves; lanes stride over the hidden width, so the order of the additions depends on the width only).
 // gate 0 = sigmoid over every expert, gate 1 = softmax over every expert.  The k picks scan
 // ascending with a strict >, so the lowest index wins a tie; the weight of a pick is its gate
 // value; renorm divides the k weights by their sum.
@@ -519,6 +519,41 @@ SHARPI_EXPORT int sharpi_add_rmsnorm_router(float* h, const void* delta, const v
   return SHARPI_OK;
 }
 
+// The experts a wave takes together (0: one at a time, with several runs of its row on their way), the tokens a block, the waves a block.  Every
+// choice gives the same bits.
+// Up to 256 tokens a block each: the chip has a unit for every one.  Behind that tokens share the experts' rows, two a block up to 512
+// (where those rows are bfloat16; floats fill the registers), then four.  While the blocks still have a unit each, many waves
+// hide each other's loads, so few experts are dealt to more of them; behind 1,024 tokens blocks share units, and four experts a wave with half of
+// the waves cost the fewest loads and conversions a product.  Many float rows want the waves back there: their tokens' rows leave the
+// cache before the next turn.
+// Chosen from 2,737 sizes (1 to 1,024 experts, 1 to 8,192 tokens, widths of 512 to 5,120, the four pairs of types) and compared on 2,620 others with one
+// expert a wave of sixteen, four from 64 experts, and four tokens from 257 on: none more than 6 % slower, 1.35 times as fast in the mean; with two
+// tokens up to 1,023 and eight waves of four at every number of experts, up to 1.9 times slower than that: 1.09.  us, the one / the other / now: bfloat16, 1,000 rows 2,048 wide of 512
+// experts 53 / 76 / 53, 600 of 96 13.4 / 21.2 / 13.4, 1,024 of 2 5.4 / 9.6 / 5.4, 8,192 rows 5,120 wide of 16 78 / 34 / 34, 300 of 16 10.7 / 7.2 / 7.2;
+// floats, 1,024 wide, 600 of 2 4.9 / 9.0 / 4.9.  The same tried with tiles of 16 x 16 on the bfloat16 matrix instruction: 3,000 rows of 64 15.9
+// for 25, but errors against 64 bits 1.15 to 1.3 times these.
+struct RouterShape {
+  int ee, tt, waves;
+};
+static RouterShape router_shape(int n_tokens, int hidden, int n_experts, bool x_float, bool w_float) {
+  if (hidden & 7) return {0, n_tokens >= 64 ? 4 : 1, n_experts >= 16 ? 16 : n_experts >= 8 ? 8 : 4};       // (no runs of 8)
+  const bool shared = n_tokens > 1024;               // blocks of four tokens share a unit
+  int ee, tt = n_tokens <= 256 ? 1 : n_tokens <= 512 && !w_float ? 2 : 4;
+  if (n_experts <= 2) ee = 0;
+  else if (n_experts <= 4) ee = shared ? 2 : 0;
+  else if (n_experts <= 8) ee = shared ? (w_float && !x_float ? 4 : 2) : tt == 2 ? 2 : 0;
+  else if (shared || n_experts > 24) ee = 4;
+  else if (tt == 1) ee = n_experts <= 16 && !x_float ? 0 : 4;
+  else ee = x_float || w_float ? 4 : 2;
+  if (tt == 2 && ee == 0) tt = 4;
+  if (shared && n_experts <= 4 && ee == 2) tt = 2;   // (a wave a token for the picks)
+  int most = 16;
+  if (shared) most = x_float && n_tokens > 2048 && hidden >= 2048 && hidden * n_experts >= 3 << 17 ? 16 : 8;
+  else if (x_float && w_float && n_tokens > 256 && hidden > 1024) most = 8;
+  const int full = ceil_div(n_experts, ee ? ee : 1);
+  return {ee, tt, min(most, max(ee == 0 ? 4 : tt, full))};
+}
+
 // corr (float [n_experts] or null): added to the gate values for the choice only.  n_groups, keep:
 // picks come from the `keep` best of n_groups equal groups of neighbouring experts (1, 1: no groups), a group
 // ranked by the sum of its group_top (1 or 2) largest choice scores.
@@ -535,18 +570,8 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
   if (n_groups < 1 || keep < 1 || keep > n_groups || n_experts % n_groups != 0 || k > keep * (n_experts / n_groups)) return SHARPI_ERR_ARG;
   if (group_top < 1 || group_top > kMaxGroupTop) return SHARPI_ERR_ARG;
   const int split_choice = corr != nullptr || keep < n_groups;
-  // Rows read in runs of 8: four experts a wave (two where there are at most 8, or 16 and few tokens), and as few waves as that makes, or
-  // the rows of a token would be read and turned into floats by more waves than its products need.  Several tokens a block share
-  // the experts' rows, as soon as the blocks still fill the chip: four from 1,024 tokens, two from 257 (four of floats: their rows cost
-  // no conversions).  Up to 8 waves a block of four tokens (a wave then takes several turns), 16 of fewer.
-  // us, with one expert a wave of sixteen, or four of sixteen from 64 experts, before: 8,192 rows 5,120 wide of 16 experts 78 -> 33.9,
-  // 1,600 21 -> 11.5, 300 10.7 -> 7.2; 2,048 rows 4,096 wide of 32 34 -> 16.1; 3,000 rows 2,048 wide of 64 37 -> 25.4, 64 of them 10.0 -> 7.7;
-  // 4,096 of 128 80 -> 57; floats: 12,000 rows 1,024 wide of 16 45 -> 24, 3,000 rows 2,048 wide of 32 34 -> 22.  The same tried with tiles of
-  // 16 x 16 on the bfloat16 matrix instruction: 3,000 rows of 64 15.9, but errors against 64 bits 1.15 to 1.3 times these.
-  const bool runs = (hidden & 7) == 0, halves = x_dtype == DT_BF16 && w_dtype == DT_BF16;
-  const int tt = !runs ? (n_tokens >= 64 ? 4 : 1) : n_tokens <= 256 ? 1 : halves && n_tokens < 1024 ? 2 : 4;
-  const int ee = !runs ? 0 : n_experts <= 8 || (n_experts <= 16 && n_tokens <= 64) ? 2 : 4;
-  const int waves = !runs ? (n_experts >= 16 ? 16 : n_experts >= 8 ? 8 : 4) : min(tt == 4 ? 8 : 16, ceil_div(n_experts, ee));
+  const RouterShape shape = router_shape(n_tokens, hidden, n_experts, x_dtype == DT_F32, w_dtype == DT_F32);
+  const int ee = shape.ee, tt = shape.tt, waves = shape.waves;
   dim3 grid(ceil_div(n_tokens, tt)), block(kWave * waves);
   const size_t lds = (size_t)tt * (n_experts + (split_choice ? n_experts + n_groups : 0)) * sizeof(float);
 #define ROUTER_LAUNCH_AT(TX, TWT, EEV, TTV)                                                                      \
@@ -557,7 +582,7 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
   do {                                                                                                           \
     if (tt == 4) ROUTER_LAUNCH_AT(TX, TWT, EEV, 4);                                                              \
     else if (tt == 1) ROUTER_LAUNCH_AT(TX, TWT, EEV, 1);                                                         \
-    else if constexpr (EEV > 0 && sizeof(TX) == 2 && sizeof(TWT) == 2) ROUTER_LAUNCH_AT(TX, TWT, EEV, 2);        \
+    else if constexpr (EEV == 2 || (EEV == 4 && sizeof(TWT) == 2)) ROUTER_LAUNCH_AT(TX, TWT, EEV, 2);            \
   } while (0)
 #define ROUTER_LAUNCH(TX, TWT)                                                                                   \
   do {                                                                                                           \
