@@ -308,7 +308,7 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float c = cs_tab[wi * 8 + j], sn = sn_tab[wi * 8 + j];
-          const float y0 = x0[j] * c - x1[j] * sn, y1 = x1[j] * c + x0[j] * sn;
+          const float y0 = fmaf(x0[j], c, -(x1[j] * sn)), y1 = fmaf(x0[j], sn, x1[j] * c);
           x0[j] = y0;
           x1[j] = y1;
         }
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
     }
     if (turns && a.inv_freq) {
       const float c = cs_tab[pi], s = sn_tab[pi];
-      const float y0 = x0 * c - x1 * s, y1 = x1 * c + x0 * s;
+      const float y0 = fmaf(x0, c, -(x1 * s)), y1 = fmaf(x1, c, x0 * s);
       x0 = y0;
       x1 = y1;
     }
@@ -408,7 +408,8 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
 constexpr int kRunMaxThreads = 1024;
 
 // How the squares of a norm are added.  RUN_LANES: eight a lane, then the lanes.  RUN_ROW and RUN_WHOLE, a norm over the projection: in the staged
-// form's order, with its bits.  (Plain rows had the first before the others came here, and keep it.)
+// form's order, with its bits.  (Plain rows had the first before the others came here, and keep it.)  A rotation's multiply-adds are
+// written out in every form: of the two products of a split pair's high half the one that is rounded is the one that the staged form by eights rounds.
 enum : int { RUN_LANES = 0, RUN_ROW = 1, RUN_WHOLE = 2 };
 
 template <typename T, int TAPS, int SUMS>
@@ -532,14 +533,17 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS == 4 ? 5 : 8) void qk_prep_run
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float other = __shfl(x[j], mate & (kWave - 1), kWave);
-          if (turns) x[j] = x[j] * cs_tab[ang + j] + other * (low ? -sn_tab[ang + j] : sn_tab[ang + j]);
+          if (turns) {
+            const float c = cs_tab[ang + j], sn = low ? -sn_tab[ang + j] : sn_tab[ang + j];
+            x[j] = SUMS == RUN_LANES || low ? fmaf(x[j], c, other * sn) : fmaf(other, sn, x[j] * c);
+          }
         }
       } else if (turns) {
 #pragma unroll
         for (int j = 0; j < 8; j += 2) {
           const float lo = x[j], hi = x[j + 1], c = cs_tab[ang + j / 2], sn = sn_tab[ang + j / 2];
-          x[j] = lo * c - hi * sn;
-          x[j + 1] = hi * c + lo * sn;
+          x[j] = fmaf(lo, c, -(hi * sn));
+          x[j + 1] = fmaf(hi, c, lo * sn);
         }
       }
     }
