@@ -273,36 +273,43 @@ __global__ __launch_bounds__(2 * kWave) void gla_walk_kernel(
 
 // Between the two phases of a segmented walk: an entry's segments one after the other.  The state at the
 // first segment's start is the slot's; S_start(n + 1) = D_n S_start(n) + S_local(n).  seg_state holds
-// S_local on entry and S_start on exit.  A thread keeps one element of a head's state and asks for eight segments' local
-// values and decays before it uses the first (a wave with sixteen rows a lane, one segment ahead, left 256 waves to wait: 15 segments
-// of 16 heads of 128 x 128: 12.0 -> 9.3 us).
+// S_local on entry and S_start on exit.  A thread keeps four neighbouring columns of a row of a head's state and asks for eight segments' local
+// values and decays (those there are) before it uses the first.  A wave with sixteen rows a lane, one segment ahead, left 256 waves to wait in a step
+// of one long entry; one element a thread made six times the blocks for entries of one segment.  us, 16 heads of 128 x 128, the one / the
+// other / now: 15 segments 11.6 / 9.5 / 8.1, with seven single tokens 12.8 / 20.6 / 9.5, six entries of 130 tokens and one 8.0 / 18.3 / 11.0.
 constexpr int kCombineThreads = 256;
 constexpr int kCombineAhead = 8;
+constexpr int kCombineCols = 4;
 __global__ __launch_bounds__(kCombineThreads) void gla_combine_kernel(const float* __restrict__ state, const int* __restrict__ state_slots,
                                                                       const int* __restrict__ ent_segs, float* __restrict__ seg_state,
                                                                       const float* __restrict__ seg_decay, int nh, int ncb, int rpl) {
   const int e = blockIdx.z, h = blockIdx.y, dkp = rpl * kGroups;
-  const int at = blockIdx.x * kCombineThreads + threadIdx.x;         // over the head's column slices, [ncb][dkp][kCols]
+  const int at = (blockIdx.x * kCombineThreads + threadIdx.x) * kCombineCols;      // over the head's column slices, [ncb][dkp][kCols]
   if (at >= ncb * dkp * kCols) return;
   const int place = at / kCols % dkp, row = place % kGroups * rpl + place / kGroups;
   const int seg0 = ent_segs[2 * e], n = ent_segs[2 * e + 1];
   const size_t per_head = (size_t)ncb * dkp * kCols, per_seg = nh * per_head;
-  float cur = state[((size_t)state_slots[e] * nh + h) * per_head + at];
+  typedef __attribute__((ext_vector_type(kCombineCols))) float cols;
+  cols cur = *reinterpret_cast<const cols*>(state + ((size_t)state_slots[e] * nh + h) * per_head + at);
   float* mine = seg_state + ((size_t)seg0 * nh + h) * per_head + at;
   const float* decay = seg_decay + ((size_t)seg0 * nh + h) * dkp + row;
   for (int i0 = 0; i0 < n; i0 += kCombineAhead) {
-    float local[kCombineAhead], dec[kCombineAhead];
+    cols local[kCombineAhead];
+    float dec[kCombineAhead];
 #pragma unroll
     for (int u = 0; u < kCombineAhead; ++u) {
-      const int i = max(min(i0 + u, n - 2), 0);                      // (the last segment's local state is nobody's start)
-      local[u] = mine[(size_t)i * per_seg];
-      dec[u] = decay[(size_t)i * nh * dkp];
+      local[u] = 0.f;
+      dec[u] = 0.f;
+      if (i0 + u + 1 >= n) continue;                                 // (the last segment's local state is nobody's start; n is the block's)
+      local[u] = *reinterpret_cast<const cols*>(mine + (size_t)(i0 + u) * per_seg);
+      dec[u] = decay[(size_t)(i0 + u) * nh * dkp];
     }
 #pragma unroll
     for (int u = 0; u < kCombineAhead; ++u) {
       if (i0 + u >= n) break;
-      mine[(size_t)(i0 + u) * per_seg] = cur;
-      cur = fmaf(dec[u], cur, local[u]);
+      *reinterpret_cast<cols*>(mine + (size_t)(i0 + u) * per_seg) = cur;
+#pragma unroll
+      for (int j = 0; j < kCombineCols; ++j) cur[j] = fmaf(dec[u], cur[j], local[u][j]);
     }
   }
 }
@@ -389,7 +396,7 @@ static int launch_segmented(const void* proj, int stride, int q_off, int k_off, 
     if (products) gla_chunk_launch(dtype, chunk, dk, dv, n_segs, false, stream);                             \
     else if (vec) PHASE(RPL, true, 1);                                                                       \
     else PHASE(RPL, false, 1);                                                                               \
-    gla_combine_kernel<<<dim3(ceil_div(ncb * RPL * kGroups * kCols, kCombineThreads), nh, n_entries), kCombineThreads, 0, stream>>>(     \
+    gla_combine_kernel<<<dim3(ceil_div(ncb * RPL * kGroups * kCols, kCombineThreads * kCombineCols), nh, n_entries), kCombineThreads, 0, stream>>>(     \
         state, state_slots, ent_segs, seg_state, seg_decay, nh, ncb, RPL);                                   \
     if (products) gla_chunk_launch(dtype, chunk, dk, dv, n_segs, true, stream);                              \
     else if (vec) PHASE(RPL, true, 2);                                                                       \
