@@ -289,7 +289,7 @@ __global__ __launch_bounds__(kCombineThreads) void gla_combine_kernel(const floa
   const int place = at / kCols % dkp, row = place % kGroups * rpl + place / kGroups;
   const int seg0 = ent_segs[2 * e], n = ent_segs[2 * e + 1];
   const size_t per_head = (size_t)ncb * dkp * kCols, per_seg = nh * per_head;
-  typedef __attribute__((ext_vector_type(kCombineCols))) float cols;
+  typedef __attribute__((ext_vector_type(kCombineCols), aligned(4))) float cols;     // (states at any address: one load all the same)
   cols cur = *reinterpret_cast<const cols*>(state + ((size_t)state_slots[e] * nh + h) * per_head + at);
   float* mine = seg_state + ((size_t)seg0 * nh + h) * per_head + at;
   const float* decay = seg_decay + ((size_t)seg0 * nh + h) * dkp + row;
