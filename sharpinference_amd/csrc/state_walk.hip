@@ -583,15 +583,21 @@ __global__ __launch_bounds__(256) void short_conv_kernel(const T* __restrict__ p
 }
 
 // Four taps, channels by eights: a thread takes eight channels of S consecutive tokens, so that their weights (128 bytes) and the rows
-// that several of them read are read once (one channel and tap at a time: 1,950 tokens of 6,144 channels 75.4 -> 21.4 us).
+// that several of them read are read once (one channel and tap at a time: 1,950 tokens of 6,144 channels 75.4 -> 21.4 us).  A block's
+// threads are 2^log_cols runs of channels by as many groups of tokens as that leaves room for.
+constexpr int kConvThreads = 256;
 template <typename T, int S>
-__global__ __launch_bounds__(256) void short_conv4_kernel(const T* __restrict__ proj, int stride, int c_off, const float* __restrict__ w,
+__global__ __launch_bounds__(kConvThreads) void short_conv4_kernel(const T* __restrict__ proj, int stride, int c_off, const float* __restrict__ w,
                                                            const float* __restrict__ bias, const float* __restrict__ tail,
                                                            const int* __restrict__ state_slots, const int* __restrict__ entry_of_token,
-                                                           const int* __restrict__ cu_tokens, T* __restrict__ out, int n_tokens, int C) {
-  const int t0 = blockIdx.x * S, ch = (blockIdx.y * 256 + threadIdx.x) * 8;
-  if (ch >= C) return;
+                                                           const int* __restrict__ cu_tokens, T* __restrict__ out, int n_tokens, int C, int log_cols) {
+  const int run = threadIdx.x & ((1 << log_cols) - 1), group = threadIdx.x >> log_cols;
+  const int t0 = (blockIdx.x * (kConvThreads >> log_cols) + group) * S, ch = ((blockIdx.y << log_cols) + run) * 8;
+  if (ch >= C || t0 >= n_tokens) return;
   const T* src = proj + c_off + ch;
+  int e[S], local[S];
+#pragma unroll
+  for (int i = 0; i < S; ++i) e[i] = entry_of_token[min(t0 + i, n_tokens - 1)];
   Run8<T> row[S + 3];                              // rows t0 - 3 ..
 #pragma unroll
   for (int i = 0; i < S + 3; ++i) row[i].load(src + (size_t)min(max(t0 - 3 + i, 0), n_tokens - 1) * stride);
@@ -601,18 +607,28 @@ __global__ __launch_bounds__(256) void short_conv4_kernel(const T* __restrict__ 
   for (int j = 0; j < 8; ++j) wv[j] = *reinterpret_cast<const float4*>(w + (size_t)(ch + j) * 4);
   if (bias) load8(bias + ch, b8);
 #pragma unroll
+  for (int i = 0; i < S; ++i) local[i] = t0 + i - cu_tokens[e[i]];
+#pragma unroll
   for (int i = 0; i < S; ++i) {
     const int t = t0 + i;
     if (t >= n_tokens) break;
-    const int e = entry_of_token[t], local = t - cu_tokens[e];
+    float held[3][8];                              // (an entry's first three tokens: what its tail holds of the rows before, requested together)
+    if (local[i] < 3) {
+      const float* tl = tail + ((size_t)state_slots[e[i]] * 3 + local[i]) * C + ch;
+#pragma unroll
+      for (int x = 0; x < 3; ++x)
+        if (3 - x > local[i]) load8(tl + (size_t)x * C, held[x]);
+    }
     float acc[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = b8[j];
 #pragma unroll
     for (int x = 0; x < 4; ++x) {                  // 3 - x tokens back
       float u[8];
-      if (3 - x <= local) row[i + x].floats(u);
-      else load8(tail + ((size_t)state_slots[e] * 3 + local + x) * C + ch, u);
+      row[i + x].floats(u);
+      if (x < 3 && 3 - x > local[i])
+#pragma unroll
+        for (int j = 0; j < 8; ++j) u[j] = held[x][j];
 #pragma unroll
       for (int j = 0; j < 8; ++j) acc[j] = fmaf(x == 0 ? wv[j].x : x == 1 ? wv[j].y : x == 2 ? wv[j].z : wv[j].w, u[j], acc[j]);
     }
@@ -649,17 +665,24 @@ SHARPI_EXPORT int sharpi_short_conv(const void* proj, int dtype, int stride, int
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
   dim3 grid(n_tokens, ceil_div(C, 256)), tgrid(n_entries, ceil_div(C, 256));
   const auto at16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  if (taps == 4 && C % 8 == 0 && stride % 8 == 0 && c_off % 8 == 0 && at16(proj) && at16(w) && at16(bias) && at16(tail) && at16(out)) {
-    // (few tokens: one a thread, or a handful of blocks would go through them)
-    const int s = n_tokens > 256 ? 4 : 1;
-    const dim3 grid8(ceil_div(n_tokens, s), ceil_div(C / 8, 256));
+  // Four taps by eights where there is enough for it: a channel a lane has an eighth of a thread's exponentials and its weights' lines to itself, and a step of single
+  // tokens reads three rows of floats a token whatever the form.  us, a channel a lane / two tokens a thread / four: 1 token of 6,144 channels
+  // 5.0 / 6.2 / 6.3, 64 6.6 / 7.2 / 9.0, 100 8.2 / 7.3 / 9.1, 500 22 / 11.0 / 11.9, 5,000 187 / 51.7 / 50.6; 2,048 tokens of 64 5.4 / 6.3 / 8.0, of 512 9.4 / 6.7 /
+  // 8.4; single tokens, 6,144 channels: 200 18.9 / 23.4 / 23.9, 300 26.9 / 25.7 / 26.5, 500 42 / 35.3 / 35.3.
+  const long long many = (long long)n_tokens * C;
+  const bool by_eights = many >> (n_tokens < 8LL * n_entries ? 21 : 19) != 0;
+  if (by_eights && taps == 4 && C % 8 == 0 && stride % 8 == 0 && c_off % 8 == 0 && at16(proj) && at16(w) && at16(bias) && at16(tail) && at16(out)) {
+    const int s = many >> 22 ? 4 : 2;
+    int log_cols = 0;
+    while ((1 << log_cols) < C / 8 && (1 << log_cols) < kConvThreads) ++log_cols;
+    const dim3 grid8(ceil_div(n_tokens, s * (kConvThreads >> log_cols)), ceil_div(C / 8, 1 << log_cols));
 #define CONV4(T, SV)                                                                                                           \
-  short_conv4_kernel<T, SV><<<grid8, 256, 0, stream>>>((const T*)proj, stride, c_off, w, bias, tail, state_slots, entry_of_token, \
-                                                       cu_tokens, (T*)out, n_tokens, C)
+  short_conv4_kernel<T, SV><<<grid8, kConvThreads, 0, stream>>>((const T*)proj, stride, c_off, w, bias, tail, state_slots, entry_of_token, \
+                                                       cu_tokens, (T*)out, n_tokens, C, log_cols)
     if (dtype == DT_F32) {
-      if (s == 4) CONV4(float, 4); else CONV4(float, 1);
+      if (s == 4) CONV4(float, 4); else CONV4(float, 2);
     } else {
-      if (s == 4) CONV4(bf16_t, 4); else CONV4(bf16_t, 1);
+      if (s == 4) CONV4(bf16_t, 4); else CONV4(bf16_t, 2);
     }
 #undef CONV4
     SHARPI_CHECK_LAUNCH();

@@ -46,6 +46,13 @@ def test_four_taps_by_eights_give_the_bits_of_a_channel_at_a_time(lens, C, dtype
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("lens, C", [([3, 250, 1, 2, 9], 2056), ([100, 1, 3], 6144), ([8000, 1, 300], 64), ([700, 1, 3], 6000), ([70000], 8), ([1] * 300, 7048), ([1, 2] * 300, 7000)])
+def test_four_taps_by_eights_in_longer_steps(lens, C, dtype):
+    """Two and four tokens a thread, narrow rows side by side in a block; single tokens, whose rows before are all in the tail."""
+    test_four_taps_by_eights_give_the_bits_of_a_channel_at_a_time(lens, C, dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T, groups, size", [(1, 1, 8), (70, 5, 24), (3, 16, 128), (33, 2, 192), (9, 3, 512), (5, 2, 520), (2, 3, 1024)])
 @pytest.mark.parametrize("act, first, weighted", [("silu", False, True), ("silu", True, True), ("sigmoid", False, False)])
 def test_parts_in_neighbouring_lanes(T, groups, size, act, first, weighted, dtype):
