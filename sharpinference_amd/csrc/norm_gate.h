@@ -26,8 +26,13 @@ struct PartNorm {
   int pairs, G, gd;
 };
 
+constexpr int kPartChipWaves = 256 * 24;   // 256 compute units of 24 waves
+
 inline bool part_norm_wide(const PartNorm& a) {
   const auto at16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  // (parts of up to 64 channels, an element a lane of a wave: until those waves are most of what the chip holds at once, a lane's eight exponentials one
+  // after the other take longer: us, a wave a part / here, 4 parts of 64: 1 token 2.5 / 3.2, 500 2.9 / 3.6, 1,000 3.3 / 3.7, 2,048 4.2 / 4.0, 5,000 7.3 / 5.0)
+  if (a.gd <= kWave && a.pairs <= kPartChipWaves) return false;
   return a.gd % 8 == 0 && a.gd <= 1024 && a.pairs <= (1 << 25) && at16(a.o) && at16(a.w) && at16(a.out) &&
          (a.act == PART_GATE_NONE || (a.stride % 8 == 0 && a.g_off % 8 == 0 && at16(a.proj)));
 }

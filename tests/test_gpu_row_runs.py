@@ -97,6 +97,21 @@ def test_parts_in_neighbouring_lanes_give_the_bits_of_a_wave_a_part(size, first,
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T, groups, size", [(1229, 5, 8), (6145, 1, 16), (770, 8, 24), (410, 15, 64), (2049, 3, 40)])
+@pytest.mark.parametrize("first", [False, True])
+def test_many_parts_of_up_to_64_channels(T, groups, size, first, dtype):
+    """More parts than go a wave each: the same parts in portions that do, for their bits."""
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(T)
+    N, cut = groups * size, T // 2
+    o, w = (torch.randn(T, N, generator=g) * 5).to(DEV), torch.randn(N, generator=g).to(DEV)
+    gates = (torch.randn(T, N, generator=g) * 2).to(DT[dtype]).to(DEV)
+    go = lambda a, b: ops.group_norm_gate(o[a:b].contiguous(), w, 1e-3, groups, DT[dtype], gates[a:b].contiguous(), 0, ops.GATE_SILU, gate_first=first)
+    assert torch.equal(go(0, T), torch.cat([go(0, cut), go(cut, T)]))
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T, H, e, gate", [(1, 1, 8, True), (70, 8, 128, False), (3, 5, 136, True), (9, 2, 512, True), (4, 3, 520, True)])
 def test_differences_of_maps_in_neighbouring_lanes(T, H, e, gate, dtype):
     from sharpinference_amd import ops
