@@ -144,7 +144,7 @@ def test_differences_of_maps_in_neighbouring_lanes_give_the_bits_of_a_wave_a_hea
     assert torch.equal(*[ops.map_difference(x.view(T, -1), H, e, 0.62, 1e-5, 0.7, proj, 11) for x in (flat, moved)])
 
 
-@pytest.mark.parametrize("T, N", [(1, 8), (70, 2056), (5, 1000), (3, 12)])
+@pytest.mark.parametrize("T, N", [(1, 8), (70, 2056), (5, 1000), (3, 12), (5000, 8), (301, 72), (257, 24)])
 def test_columns_side_by_side_add_as_one_by_one(T, N):
     from sharpinference_amd import ops
 
