@@ -222,7 +222,7 @@ SHARPI_EXPORT int sharpi_latent_prep(const void* q, int ldq, int q_off, const vo
 }
 
 // ---------------------------------------------------------------------------
-constexpr int kHgSmall = 128;         // tiles of 64 x 64 up to which a wave takes 16 x 16
+constexpr int kHgSmall = 64;          // tiles of 64 x 64 up to which a wave takes 16 x 16 (of up to 32 tokens, half tiles: twice as many)
 constexpr int kHgTile = 64, kHgK = 16;
 
 template <typename T>
@@ -287,8 +287,9 @@ __global__ __launch_bounds__(256) void head_gemm_kernel(const T* __restrict__ x,
 // the output's of 4.
 //
 // Bound: few blocks, a chain of loads from memory (the weights are read once a step); many blocks, operands through L2 (64 outputs a 128 rows read).
-// With up to half of the chip's units covered by 64 x 64 tiles a wave takes 16 x 16 (four times the waves) and requests 512 of K before its first
-// product; more tiles than that read too much that way, and there two steps ahead (many waves a unit) beat four and eight.
+// With up to a quarter of the chip's units covered by 64 x 64 tiles, or half of them by tiles of at most 32 tokens, a wave takes 16 x 16 (four times the
+// waves) and requests 512 of K before its first product; more tiles than that read too much that way, and there two steps ahead (many waves a unit) beat
+// four and eight.  (128 tiles, 64 heads, 512 x 128, 16 x 16 / 32 x 32 a wave: 9 tokens 3.4 / 4.6, 32 5.5 / 5.6, 33 9.2 / 7.8, 64 9.5 / 9.1.)
 // us, 64 x 64 with two steps in turn for all before -> now, weights from memory, 16 heads, 512 x 128 and 128 x 512: 1 token 3.8 -> 2.6, 8.2 -> 3.7;
 // 64 tokens 4.9 -> 4.2, 11.3 -> 6.0; 300 tokens (160 tiles) 128 x 512 11.7 -> 10.8 (16 x 16: 14.1); 1,000 21.2 -> 19.8 (36.4), 20.0 -> 19.7 (31.6).
 typedef __attribute__((ext_vector_type(8))) __bf16 hg_bf16x8;
@@ -405,7 +406,8 @@ SHARPI_EXPORT int sharpi_head_gemm(const void* x, int dtype, int ldx, int sx, co
                                                         (const float*)gate, ldg, n_tokens, N, K);
   else if (dtype == DT_BF16 && K % 8 == 0 && sx % 8 == 0 && ldx % 8 == 0 && N % 4 == 0 && so % 4 == 0 && ldo % 4 == 0 &&
            ((uintptr_t)x & 15) == 0 && ((uintptr_t)w & 15) == 0 && ((uintptr_t)out & 7) == 0) {
-    const bool small = (long)grid.x * grid.y * grid.z <= kHgSmall && ceil_div(N, 32) <= 65535;
+    const long tiles = (long)grid.x * grid.y * grid.z;
+    const bool small = tiles <= (n_tokens <= 32 ? 2 * kHgSmall : kHgSmall) && ceil_div(N, 32) <= 65535;
     if (small) grid = dim3(ceil_div(n_tokens, 32), ceil_div(N, 32), H);
 #define HEAD_GEMM(S, GATED)                                                                                               \
   head_gemm_mfma_kernel<S, GATED><<<grid, block, 0, stream>>>((const bf16_t*)x, ldx, sx, (const bf16_t*)w, (bf16_t*)out, ldo, so, \
