@@ -155,22 +155,18 @@ def test_columns_side_by_side_add_as_one_by_one(T, N):
         assert torch.equal(ops.add_bias(y.clone(), b), (y.float() + b).to(dtype))
 
 
-@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
-@pytest.mark.parametrize("T", [9, 70])
-@pytest.mark.parametrize("hd", [16, 64, 96, 128, 192, 256, 512])
-@pytest.mark.parametrize("form", ["conv", "conv3", "keys", "maps", "maps conv", "whole", "whole conv", "whole keys"])
-@pytest.mark.parametrize("turn", ["none", "pairs", "halves"])
-def test_heads_by_runs_give_the_bits_of_the_staged_form(turn, form, hd, T, dtype):
+def _prepared_by_eights_and_one_by_one(turn, form, nh, nkv, hd, T, dtype):
+    """The same rows aligned for runs of eight and shifted, so that they are staged an element at a time: the same bits."""
     from sharpinference_amd import ops
 
     g = torch.Generator().manual_seed(hd + T + len(form))
-    nh, nkv, vd, r, ps = (4, 2, 40, 16, 16) if hd > 256 else (6, 2, 40, 16, 16)
+    vd, r, ps = 40, 16, 16
     keys, whole, maps = "keys" in form, "whole" in form, 2 if "maps" in form else 1
     r, vd = min(r, hd // maps), hd if keys else vd
     if turn == "none" or (r < 16 and turn == "halves"):
         r = 0
     qn, kn, vn, pages = nh * hd, nkv * hd, 0 if keys else nkv * vd, T // ps + 3
-    C, taps = qn + kn + vn, 3 if form == "conv3" else 4 if "conv" in form else 0
+    C, taps = qn + kn + vn, 3 if "conv3" in form else 4 if "conv" in form else 0
     proj = torch.randn(T, C + 8, generator=g).to(DT[dtype]).to(DEV)
     wq, wk = (torch.rand(n, generator=g).to(DEV) + 0.5 for n in ((qn, kn) if whole else (hd, hd)))
     conv = torch.randn(C, taps, generator=g).to(DEV) if taps else None
@@ -194,6 +190,36 @@ def test_heads_by_runs_give_the_bits_of_the_staged_form(turn, form, hd, T, dtype
         tol = 3 * 2.0 ** -24 if dtype == "float32" else 2.0 ** -8 + 3 * 2.0 ** -24
         a, b = a.double(), b.double()
         assert bool(((a - b).abs() <= tol * (a.abs() + b.abs()) + 3 * 2.0 ** -24 * b.abs().amax(-1, keepdim=True)).all())
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T", [9, 70])
+@pytest.mark.parametrize("hd", [16, 64, 96, 128, 192, 256, 512])
+@pytest.mark.parametrize("form", ["conv", "conv3", "keys", "maps", "maps conv", "whole", "whole conv", "whole keys"])
+@pytest.mark.parametrize("turn", ["none", "pairs", "halves"])
+def test_heads_by_runs_give_the_bits_of_the_staged_form(turn, form, hd, T, dtype):
+    _prepared_by_eights_and_one_by_one(turn, form, 4 if hd > 256 else 6, 2, hd, T, dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T", [1, 3, 2050])
+@pytest.mark.parametrize("hidden", [8, 520, 5120, 1032])
+def test_embedding_by_runs(hidden, T, dtype):
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(T + hidden)
+    table = torch.randn(300, hidden, generator=g).to(DT[dtype]).to(DEV)
+    ids = torch.randint(0, 300, (T,), generator=g).to(torch.int32).to(DEV)
+    assert torch.equal(ops.embed_gather(ids, table, scale=1.7), table[ids.long()].float() * 1.7)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T", [9, 70])
+@pytest.mark.parametrize("nh, hd", [(64, 128), (40, 192)])             # (more than 1,024 lanes: aligned rows are staged, too)
+@pytest.mark.parametrize("form", ["whole", "whole conv", "whole conv3", "whole keys", "whole maps", "whole maps conv"])
+@pytest.mark.parametrize("turn", ["none", "pairs", "halves"])
+def test_aligned_rows_too_wide_for_runs(turn, form, nh, hd, T, dtype):
+    _prepared_by_eights_and_one_by_one(turn, form, nh, 2, hd, T, dtype)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
