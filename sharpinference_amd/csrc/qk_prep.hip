@@ -414,8 +414,9 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
 // worked on; in short steps the values of a token, another chain, go in a block beside those of its heads.  us, 16 + 4 heads
 // of 128, staged through LDS before: 1,900 tokens, norms over the projections 22.3 -> 12.7 (their squares added as the lanes come, with other bits,
 // 11.7), two maps a head 21.9 -> 13.0, four taps with the tail's launch 37.9 -> 28.1; 8 tokens, a norm a head 4.6 -> 4.4 (weights and values behind
-// the rest: 5.0), over the projections 7.7 -> 5.1, four taps 11.4 -> 7.9 (a tap of the tail at a time: 14.2).  64 + 8 heads of 192, 2,048 tokens (a block of
-// 256 for three turns, each behind the one before) 40.9 -> 35.
+// the rest: 5.0), over the projections 7.7 -> 5.1, four taps 11.4 -> 7.9 (a tap of the tail at a time: 14.2), three taps 11.8 -> 9.6 (a tap at a
+// time: 11.8).  64 + 8 heads of 192: 2,048 tokens (a block of 256 for three turns, each behind the one before) 40.9 -> 35; floats, 200 tokens
+// four turns a block 9.9, two 9.0 (8.9 before), 64 tokens with neighbours on several dies 5.8, on one 5.5 (5.25 before).
 constexpr int kRunMaxThreads = 1024;
 
 // How the squares of a norm are added.  RUN_LANES: eight a lane, then the lanes.  RUN_ROW and RUN_WHOLE, a norm over the projection: in the staged
@@ -432,7 +433,7 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS != 0 ? 5 : 8) void qk_prep_run
   const int qn = a.nh * a.hd, kn = a.nkv * a.hd, runs = a.hd / 8, heads = a.nh + a.nkv;
   const bool own_v = a.v_off >= 0;
   const int v_at = own_v ? qn + kn : qn, v_col = own_v ? a.v_off : a.k_off, C = qn + kn + (own_v ? a.nkv * a.vd : 0);
-  if (blockIdx.x >= a.n_tokens) {          // (values_apart: the blocks behind the tokens', y of them side by side)
+  if (a.values_apart && blockIdx.x >= a.n_tokens) {     // (the blocks behind the tokens', y of them side by side)
     const int v = (blockIdx.x - a.n_tokens) * gridDim.y + blockIdx.y;
     if (v < value_tiles(a.n_tokens, a.nkv * a.vd))
       values_to_pages<T>(v, a.n_tokens, a.nkv, a.vd, a.page_size, a.slot_mapping, (T*)a.v_cache, reinterpret_cast<T*>(tile),
@@ -442,7 +443,9 @@ __global__ __launch_bounds__(kRunMaxThreads, TAPS != 0 ? 5 : 8) void qk_prep_run
       });
     return;
   }
-  const int t = blockIdx.x;
+  // (short steps: neighbouring tokens on one die, whose cache gathers the values' columns)
+  const int t = a.values_beside ? (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+  if (t >= a.n_tokens) return;
   const int slot = a.slot_mapping ? a.slot_mapping[t] : -1;
   // a thread's run inside a head is the same in every turn
   const int li = threadIdx.x & ((1 << log_lanes) - 1);
@@ -678,10 +681,10 @@ SHARPI_EXPORT int sharpi_qk_prep(const void* proj, int dtype, int stride, int q_
   } while (0)
   if (by_runs) {
     const int threads = together ? max(kValueThreads, ceil_div(items, kWave) * kWave) : kPrepThreads;
-    // not together: a block a turn of few tokens; of many four turns or so a block, to share the angles
-    const int turns = ceil_div(items, threads), y = n_tokens <= kPrepSplitTokens ? turns : ceil_div(turns, 4);
+    // not together: a block a turn of few tokens; of more two turns or so a block, of many four, to share the angles
+    const int turns = ceil_div(items, threads), y = ceil_div(turns, n_tokens <= kPrepSplitTokens ? 1 : n_tokens <= 4 * kPrepSplitTokens ? 2 : 4);
     a.values_beside = !v_apart && slot_mapping != nullptr;
-    const dim3 rgrid(n_tokens + ceil_div(tiles, y), y + a.values_beside);
+    const dim3 rgrid(a.values_beside ? 8 * ceil_div(n_tokens, 8) : n_tokens + ceil_div(tiles, y), y + a.values_beside);
     const size_t row_lds = norm_mode == NORM_WHOLE ? (size_t)(qn + kn) * sizeof(float) : 0;
     const bool plain = (half_split || rotary_dim == 0) && taps == 0 && maps == 1 && v_off >= 0;
 #define RUN_GO(T, TAPSV, SUMSV) qk_prep_run_kernel<T, TAPSV, SUMSV><<<rgrid, threads, row_lds, stream>>>(a, __builtin_ctz(lanes))

@@ -202,6 +202,41 @@ def test_heads_by_runs_give_the_bits_of_the_staged_form(turn, form, hd, T, dtype
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T", [9, 70, 300])
+@pytest.mark.parametrize("form", ["conv", "conv3", "keys", "maps"])
+def test_heads_in_several_turns_give_the_bits_of_the_staged_form(form, T, dtype):
+    _prepared_by_eights_and_one_by_one("halves", form, 64, 2, 192, T, dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_plain_heads_have_the_same_bits_in_steps_of_any_size(dtype):
+    """A turn a block, two and four, neighbouring tokens on a die or not."""
+    from sharpinference_amd import ops
+
+    g = torch.Generator().manual_seed(5)
+    T, nh, nkv, hd, vd, ps = 300, 40, 2, 192, 40, 16
+    qn, kn, pages = nh * hd, nkv * hd, 20
+    proj = torch.randn(T, qn + kn + nkv * vd, generator=g).to(DT[dtype]).to(DEV)
+    wq, wk = (torch.rand(hd, generator=g).to(DEV) + 0.5 for _ in range(2))
+    freq = torch.tensor([300.0 ** (-2.0 * i / 64) for i in range(32)], device=DEV)
+    slots, results = torch.randperm(pages * ps, generator=g)[:T].to(torch.int32).to(DEV), []
+    for portion in (300, 70, 33, 7):
+        kc = torch.zeros(pages, nkv, ps, hd, dtype=DT[dtype], device=DEV)
+        vc = torch.zeros(pages, nkv, vd, ps, dtype=DT[dtype], device=DEV)
+        out = []
+        for i in range(0, T, portion):
+            n = min(portion, T - i)
+            ctx = _Step([n], [0])
+            ctx.positions += i
+            out.append(ops.qk_prep(proj[i:i + n], 0, qn, qn + kn, nh, nkv, hd, vd, ctx, kc, vc, slots[i:i + n], ops.NORM_PER_HEAD, wq, wk, 1e-5, freq,
+                                   ops.PAIRS_HALF_SPLIT))
+        results.append((torch.cat(out), kc, vc))
+    for other in results[1:]:
+        for a, b in zip(results[0], other):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T", [1, 3, 2050])
 @pytest.mark.parametrize("hidden", [8, 520, 5120, 1032])
 def test_embedding_by_runs(hidden, T, dtype):
