@@ -313,7 +313,7 @@ def test_the_difference_of_two_maps_normed_and_gated_per_head(dtype, T, H, e, ga
 @pytest.mark.parametrize("H, G, d, e, rot, taps, bias, temp", [
     (4, 2, 12, 20, (5000.0, 8), 0, True, None), (6, 1, 8, 6, None, 2, False, (16.0, 0.4)), (4, 2, 32, 64, None, 4, False, (32.0, 0.25)),
     (8, 2, 32, 64, (20000.0, 32), 0, True, None), (2, 2, 24, 40, None, 8, False, None), (3, 3, 10, 33, None, 0, True, (7.0, 1.5))])
-def test_maps_rotated_each_on_its_own_and_queries_expanded(dtype, H, G, d, e, rot, taps, bias, temp):
+def test_maps_rotated_each_on_its_own_and_queries_expanded(dtype, H, G, d, e, rot, taps, bias, temp, pad=5, more=0):
     """Between the projections and attention of a differential layer: biases, the convolution with its carried
     tail, rotation of each map's own leading elements, the query temperature; key rows of both maps in the cache,
     one query row per (head, map) with zeros in the other map's place."""
@@ -322,19 +322,20 @@ def test_maps_rotated_each_on_its_own_and_queries_expanded(dtype, H, G, d, e, ro
     g = torch.Generator().manual_seed(H * d + e)
     qn, kn, vn = H * 2 * d, G * 2 * d, G * e
     C = qn + kn + vn
-    rows = {r: (torch.randn(n, C + 5, generator=g)).to(DT[dtype]) for r, n in TOTAL.items()}
+    plan, totals = [[("a", 1), ("b", 40 + more)], *PLAN[1:]], {**TOTAL, "b": TOTAL["b"] + more}
+    rows = {r: (torch.randn(n, C + pad, generator=g)).to(DT[dtype]) for r, n in totals.items()}
     b = torch.randn(C, generator=g) if bias else None
     cw = torch.randn(C, taps, generator=g) * 0.6 if taps else None
     base = {"a": 0, "b": 1000, "c": 37}
     ps = 16
-    pages = {r: [] for r in TOTAL}
+    pages = {r: [] for r in totals}
     free = list(torch.randperm(12, generator=g).tolist())
-    for r, n in TOTAL.items():
+    for r, n in totals.items():
         pages[r] = [free.pop() for _ in range((n + ps - 1) // ps)]
     kc = torch.zeros(12, G, ps, 2 * d, dtype=DT[dtype], device=DEV)
     vc = torch.zeros(12, G, e, ps, dtype=DT[dtype], device=DEV)
     tail = torch.zeros(5, max(taps - 1, 1), C, device=DEV) if taps else None
-    seen = {r: 0 for r in TOTAL}
+    seen = {r: 0 for r in totals}
 
     def call(x, ctx):
         slots = []
@@ -347,9 +348,9 @@ def test_maps_rotated_each_on_its_own_and_queries_expanded(dtype, H, G, d, e, ro
         return ops.qk_prep(x, 0, qn, qn + kn, H, G, 2 * d, e, ctx, kc, vc, sm, inv_freq=_freqs(rot), pair_layout=ops.PAIRS_HALF_SPLIT,
                            conv_w=cw.to(DEV) if taps else None, tail=tail, bias=b.to(DEV) if bias else None, temperature=temp, maps=2)
 
-    got = {r: [] for r in TOTAL}
-    at = {r: 0 for r in TOTAL}
-    for step in PLAN:
+    got = {r: [] for r in totals}
+    at = {r: 0 for r in totals}
+    for step in plan:
         ctx = _Step([n for _, n in step], [base[r] + at[r] for r, _ in step], [SLOT_OF[r] for r, _ in step])
         ctx.reqs, ctx.lens = [r for r, _ in step], [n for _, n in step]
         x = torch.cat([rows[r][at[r]:at[r] + n] for r, n in step]).to(DEV)
@@ -360,7 +361,7 @@ def test_maps_rotated_each_on_its_own_and_queries_expanded(dtype, H, G, d, e, ro
             i += n
             at[r] += n
     tol = FLOAT_KERNEL if dtype == "float32" else BF16_KERNEL
-    for r, n in TOTAL.items():
+    for r, n in totals.items():
         u = rows[r][:, :C].double()
         if bias:
             u = u + b.double()
@@ -382,6 +383,16 @@ def test_maps_rotated_each_on_its_own_and_queries_expanded(dtype, H, G, d, e, ro
         gv = torch.stack([vc[pages[r][p // ps], :, :, p % ps] for p in range(n)]).cpu()
         assert _rel_rms(gk.reshape(n, -1), k.reshape(n, -1)) < tol, r
         assert _rel_rms(gv.reshape(n, -1), v.reshape(n, -1)) < tol, r
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("more", [0, 30])                  # (steps of up to 64 tokens and beyond)
+@pytest.mark.parametrize("H, G, d, e, rot, taps, bias, temp", [
+    (4, 2, 32, 64, None, 4, False, (32.0, 0.25)), (8, 2, 32, 64, (20000.0, 32), 0, True, None), (2, 2, 24, 40, None, 8, False, None),
+    (3, 1, 24, 48, (5000.0, 16), 4, False, None), (4, 2, 16, 24, (5000.0, 16), 3, False, (7.0, 1.5))])
+def test_maps_by_runs(dtype, H, G, d, e, rot, taps, bias, temp, more):
+    """The same with widths and offsets that are multiples of 8, where a head lies in neighbouring lanes."""
+    test_maps_rotated_each_on_its_own_and_queries_expanded(dtype, H, G, d, e, rot, taps, bias, temp, pad=8, more=more)
 
 
 class _Ctx:

@@ -71,7 +71,7 @@ class _Step:
     (2, 2, 16, 6, None, "half", 0, 1.0, 2, True),
     (5, 5, 8, 8, "head", "interleaved", 2, 0.7, 8, True),
 ])
-def test_convolution_norm_rotation_and_cache_write(dtype, H, G, d, e, norm, layout, dims, mag, taps, own_v):
+def test_convolution_norm_rotation_and_cache_write(dtype, H, G, d, e, norm, layout, dims, mag, taps, own_v, pad=5, first=19):
     """Two requests in two steps each (the second step of one shorter than the convolution's reach),
     on shuffled pages: q, the cached keys and values and the carried tails against the plain pieces
     applied to the whole sequences."""
@@ -80,8 +80,8 @@ def test_convolution_norm_rotation_and_cache_write(dtype, H, G, d, e, norm, layo
     g = torch.Generator().manual_seed(H * 100 + d + taps)
     ps, eps = 16, 1e-5
     qn, kn, vn = H * d, G * d, (G * e if own_v else 0)
-    C, pad = qn + kn + vn, 5                                     # (the projections sit inside a wider row)
-    lens = {"a": [19, 1], "b": [2, 30]}
+    C = qn + kn + vn                                             # (the projections sit inside a wider row)
+    lens = {"a": [first, 1], "b": [2, 30]}
     total = {r: sum(v) for r, v in lens.items()}
     proj = {r: (torch.randn(total[r], C + pad, generator=g) * 2).to(DT[dtype]) for r in lens}
     conv_w = torch.randn(C, taps, generator=g) if taps else None
@@ -106,9 +106,10 @@ def test_convolution_norm_rotation_and_cache_write(dtype, H, G, d, e, norm, layo
             q, k = P.rotate(q, pos, freqs, layout, mag), P.rotate(k, pos, freqs, layout, mag)
         want[r] = (q, k, v)
     # the kernel, step by step
-    pages = 8
+    a_pages = (total["a"] + ps - 1) // ps
+    pages = 6 + a_pages
     perm = torch.randperm(pages, generator=g).tolist()
-    page_of = {"a": perm[:2], "b": perm[2:4]}
+    page_of = {"a": perm[:a_pages], "b": perm[a_pages:a_pages + 2]}
     kc = torch.zeros(pages, G, ps, d, dtype=DT[dtype], device=DEV)
     vc = torch.zeros(pages, G, e, ps, dtype=DT[dtype], device=DEV)
     tail = torch.zeros(3, max(taps - 1, 1), C, device=DEV) if taps else None
@@ -146,6 +147,22 @@ def test_convolution_norm_rotation_and_cache_write(dtype, H, G, d, e, norm, layo
             assert torch.equal(tail[slot_of[r], :taps - 1].cpu(), last), f"tail of {r}"
     if taps:
         assert float(tail[1].abs().max()) == 0.0               # a slot no entry named stays untouched
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("first", [19, 75])                # (steps of up to 64 tokens and beyond)
+@pytest.mark.parametrize("H, G, d, e, norm, layout, dims, mag, taps, own_v", [
+    (8, 2, 32, 32, "projection", "interleaved", 32, 1.0, 0, False),
+    (3, 1, 24, 24, "projection", "half", 16, 1.0, 4, True),    # (three runs a head in four lanes, a wave with heads of q and of k)
+    (3, 1, 24, 40, "projection", "interleaved", 8, 1.3, 3, True),
+    (2, 1, 64, 64, "head", "half", 64, 1.0, 4, True),
+    (5, 5, 8, 8, "head", "interleaved", 8, 0.7, 8, True),
+    (6, 2, 96, 96, "head", "half", 32, 1.0, 2, False),
+    (4, 2, 16, 8, None, "half", 0, 1.0, 4, True),
+])
+def test_convolution_norm_rotation_and_cache_write_by_runs(dtype, H, G, d, e, norm, layout, dims, mag, taps, own_v, first):
+    """The same with widths and offsets that are multiples of 8, where a head lies in neighbouring lanes."""
+    test_convolution_norm_rotation_and_cache_write(dtype, H, G, d, e, norm, layout, dims, mag, taps, own_v, pad=8, first=first)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
