@@ -13,7 +13,8 @@
 // attention kernel over keys of the head's width computes each map's scores on its own; and values mixed with
 // those of another layer, (1 - c) v + c v_other, in float on their way into the cache.
 //
-// Rows of widths and offsets that are multiples of 8 go to qk_prep_run_kernel; the others, and norms over more than 1,024 runs of 8, as follows.
+// Rows of widths and offsets that are multiples of 8, and heads of up to 512, go to qk_prep_run_kernel; the others, and norms over projections of more
+// than 1,024 lanes (q and kv heads times hd / 8 rounded up to a power of two), as follows.
 // One block per token, or, in steps of few tokens, one per (token, kv head): the block then takes
 // that kv head's key and value and the query heads that read it, so that a decode step still fills
 // the chip (what a row's sums are made of and their order do not depend on the split).  The token's

@@ -609,6 +609,8 @@ SHARPI_EXPORT int sharpi_router_topk(const void* x, int x_dtype, const void* wr,
 // up to 24 weights) at once and keeps them (KEEP a thread; 0: more pairs than it can, read again for the second pass and stored one by one); an
 // expert has up to 16 counters, a lane takes the one of its number, and what the counter held is the pair's place behind the counter's first row;
 // every group counts the units before its own from one number a group.
+// 24 pairs a thread are what its 128 registers and the window's LDS hold; beyond 24,576 pairs (8,192 tokens of four picks or more) the list is made as
+// before, and costs what it did: 49,152 pairs 53 us, 65,536 82.
 // us, pairs read, counted and stored one by one in two passes before: 18,000 pairs of 64 experts 24.8 -> 17.5, 9,984 17.5 -> 13.0, 8,192 of 28 and of
 // 16 10.7 -> 8.4 and 10.8 -> 7.8.
 constexpr unsigned kPlanRankParts = 32;        // (above kPlanMaxParts)
