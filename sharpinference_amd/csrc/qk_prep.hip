@@ -29,6 +29,10 @@ constexpr int kPrepThreads = 256;
 constexpr int kPrepMaxTaps = 8;
 constexpr int kPrepTapsAhead = 3;     // taps whose rows and weights are on their way together (any number but four)
 constexpr int kPrepSplitTokens = 64;  // up to so many tokens a step, a token's heads are spread over nkv blocks
+// Values of convolved rows go in blocks of their own by tiles of 16 tokens from more tokens on: a tile's thread gathers one run after the other, which
+// of few tiles is the step's longest chain.  Three taps, 300 tokens, times as fast as before blocks apart, apart / beside: 1.22 / 1.25, 700 1.13 / 1.17 in
+// the mean, but 1,400 1.12 / 1.07; eight taps 1.11 / 1.24, 700 1.04 / 1.16, 5,000 single shapes 0.85 / 0.99: always beside.
+constexpr int kPrepBesideFewTaps = 500;
 constexpr int kPrepMaxHeads = 1024;   // q heads + kv heads whose inverse norms are kept in LDS
 
 enum : int { NORM_NONE = 0, NORM_PER_HEAD = 1, NORM_WHOLE = 2 };
@@ -419,6 +423,17 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
 // time: 11.8).  64 + 8 heads of 192: 2,048 tokens (a block of 256 for three turns, each behind the one before) 40.9 -> 35; floats, 200 tokens
 // four turns a block 9.9, two 9.0 (8.9 before), 64 tokens with neighbours on several dies 5.8, on one 5.5 (5.25 before).
 constexpr int kRunMaxThreads = 1024;
+// Convolved rows go by runs up to so many lanes a step: a gather's rows and weights fill the registers, so of a block of nine or ten waves a
+// unit holds one at a time, and with enough tokens to fill the chip the staged form's blocks of four waves, several a unit, are through sooner.  us, four
+// taps, staged before the runs / runs / staged now: 16 + 2 heads of 192, 300 tokens 1.11 to 1.2 times the runs, 1,400 0.84, 5,000 0.63 (staged now 0.5);
+// 32 + 8 of 128 1.22, 1.0, 0.76; 16 + 4 of 128 about level at 1,400.
+// More than four taps are chains of several gathers: by runs up to 1,000 tokens (8 taps, 300 tokens 1.24 times as fast as before, 1,400 1.09 in the
+// mean, but single shapes 0.85), and not in rows of up to 32 lanes, half a wave, whose chain is all there is (2 + 1 heads of 64, 33 tokens 0.88).
+constexpr long kRunMuch = 400 * 1024;
+constexpr int kRunFullBlock = 512;    // (plain rows of more lanes than these, beyond so much: blocks of 256 in turns, too; 32 + 8 heads of 96, 1,500 tokens 0.84 otherwise, 6,000 0.71)
+// Few taps of interleaved pairs, which are staged an element a thread, likewise beyond 500 tokens in rows of up to half a block (three taps, 8 + 2 heads of
+// 64, 1,500 tokens: staged 13.0, runs 16.8), and beyond 1,000 in any.
+constexpr int kRunManyTaps = 1000, kRunNarrow = 32, kRunHalfBlock = 128;
 
 // How the squares of a norm are added.  RUN_LANES: eight a lane, then the lanes.  RUN_ROW and RUN_WHOLE, a norm over the projection: in the staged
 // form's order, with its bits.  (Plain rows had the first before the others came here, and keep it.)  A rotation's multiply-adds are
@@ -656,28 +671,34 @@ SHARPI_EXPORT int sharpi_qk_prep(const void* proj, int dtype, int stride, int q_
                     at16(proj) && at16(q_out) && at16(k_cache) && at16(tail) && at16(bias);
   const bool other_wide = !v_other || (at16(v_other) && v_other_stride % 8 == 0 && v_other_off % 8 == 0);
   const int by8 = wide && (half_split || rotary_dim == 0) && rotary_dim % 16 == 0;
+  const bool taps4 = taps == 4 && at16(conv_w);
+  const int lanes = hd <= 64 ? (hd <= 8 ? 1 : hd <= 16 ? 2 : hd <= 32 ? 4 : 8) : hd <= 128 ? 16 : hd <= 256 ? 32 : 64;
+  const int items = (nh + nkv) * lanes;
+  const bool much = (long)n_tokens * items > kRunMuch;
+  // a thread for every run where a block can have them; of a few tokens 256 a block, or the launch would leave the chip empty (a
+  // norm over the projection aside, whose sums need them together)
+  const bool together = items <= kRunMaxThreads && (norm_mode == NORM_WHOLE || (n_tokens > kPrepSplitTokens && !(much && items > kRunFullBlock)));
+  const bool chains = taps > 4 || (taps > 0 && !taps4 && !by8 && n_tokens > kPrepBesideFewTaps);
+  const bool convolved = taps == 0 || (!much && (!chains || (n_tokens <= kRunManyTaps && items > (n_tokens <= kPrepBesideFewTaps ? kRunNarrow : kRunHalfBlock))));
+  const bool by_runs = wide && other_wide && convolved && rotary_dim % (half_split ? 16 : 8) == 0 && hd <= 512 && at16(q_norm_w) && at16(k_norm_w) &&
+                       (norm_mode != NORM_WHOLE || together);
   // (a step stores all its tokens or, without slots, none)
-  const bool v_apart = wide && other_wide && n_tokens > kPrepSplitTokens && slot_mapping != nullptr;
+  const int beside_up_to = taps == 0 || (taps4 && v_off >= 0) ? kPrepSplitTokens : taps <= 4 && v_off >= 0 && (by8 || by_runs) ? kPrepBesideFewTaps : n_tokens;
+  const bool v_apart = wide && other_wide && n_tokens > beside_up_to && slot_mapping != nullptr;
   const int tiles = v_apart ? value_tiles(n_tokens, nkv * vd) : 0;
   PrepArgs a{proj, stride, q_off, k_off, v_off, nh, nkv, hd, vd, conv_w, taps, tail, state_slots, entry_of_token,
              cu_tokens, positions, norm_mode, q_norm_w, k_norm_w, eps, rotary_dim > 0 ? inv_freq : nullptr, rotary_dim,
              half_split, magnitude, q_out, k_cache, v_cache, slot_mapping, page_size, parts, bias, temp_on, temp_floor,
              temp_scale, maps, v_other, v_other_stride, v_other_off, v_mix, v_apart, 0, n_tokens, by8};
-  const int lanes = hd <= 64 ? (hd <= 8 ? 1 : hd <= 16 ? 2 : hd <= 32 ? 4 : 8) : hd <= 128 ? 16 : hd <= 256 ? 32 : 64;
-  const int items = (nh + nkv) * lanes;
-  // a thread for every run where a block can have them; of a few tokens 256 a block, or the launch would leave the chip empty (a
-  // norm over the projection aside, whose sums need them together)
-  const bool together = items <= kRunMaxThreads && (norm_mode == NORM_WHOLE || n_tokens > kPrepSplitTokens);
-  const bool by_runs = wide && other_wide && rotary_dim % (half_split ? 16 : 8) == 0 && hd <= 512 && at16(q_norm_w) && at16(k_norm_w) &&
-                       (norm_mode != NORM_WHOLE || together);
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
-  const bool taps4 = taps == 4 && at16(conv_w);
+  // (no gather by eights in a block that takes an element a thread: the form without one, whose registers leave room for more waves)
+  const int form = taps == 0 || !(by_runs || by8 || v_apart) ? 0 : taps4 ? 4 : -1;
 #define PREP_BY_TAPS(GO, ...)                                               \
   do {                                                                      \
     if (dtype == DT_F32) {                                                  \
-      if (taps == 0) GO(float, 0, ##__VA_ARGS__); else if (taps4) GO(float, 4, ##__VA_ARGS__); else GO(float, -1, ##__VA_ARGS__);    \
+      if (form == 0) GO(float, 0, ##__VA_ARGS__); else if (form == 4) GO(float, 4, ##__VA_ARGS__); else GO(float, -1, ##__VA_ARGS__);    \
     } else {                                                                \
-      if (taps == 0) GO(bf16_t, 0, ##__VA_ARGS__); else if (taps4) GO(bf16_t, 4, ##__VA_ARGS__); else GO(bf16_t, -1, ##__VA_ARGS__); \
+      if (form == 0) GO(bf16_t, 0, ##__VA_ARGS__); else if (form == 4) GO(bf16_t, 4, ##__VA_ARGS__); else GO(bf16_t, -1, ##__VA_ARGS__); \
     }                                                                       \
   } while (0)
   if (by_runs) {

@@ -166,7 +166,7 @@ def _prepared_by_eights_and_one_by_one(turn, form, nh, nkv, hd, T, dtype):
     if turn == "none" or (r < 16 and turn == "halves"):
         r = 0
     qn, kn, vn, pages = nh * hd, nkv * hd, 0 if keys else nkv * vd, T // ps + 3
-    C, taps = qn + kn + vn, 3 if "conv3" in form else 4 if "conv" in form else 0
+    C, taps = qn + kn + vn, 3 if "conv3" in form else 6 if "conv6" in form else 4 if "conv" in form else 0
     proj = torch.randn(T, C + 8, generator=g).to(DT[dtype]).to(DEV)
     wq, wk = (torch.rand(n, generator=g).to(DEV) + 0.5 for n in ((qn, kn) if whole else (hd, hd)))
     conv = torch.randn(C, taps, generator=g).to(DEV) if taps else None
@@ -206,6 +206,14 @@ def test_heads_by_runs_give_the_bits_of_the_staged_form(turn, form, hd, T, dtype
 @pytest.mark.parametrize("form", ["conv", "conv3", "keys", "maps"])
 def test_heads_in_several_turns_give_the_bits_of_the_staged_form(form, T, dtype):
     _prepared_by_eights_and_one_by_one("halves", form, 64, 2, 192, T, dtype)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("form, nh, hd, T", [("conv", 16, 192, 711), ("conv", 16, 192, 712), ("whole conv3", 16, 192, 712), ("conv3", 6, 64, 500), ("conv3", 6, 64, 501),
+                                             ("conv6", 6, 64, 1000), ("whole conv6", 6, 64, 1001), ("conv6", 6, 16, 70), ("maps conv6", 6, 128, 70), ("conv6", 2, 64, 9)])
+def test_convolved_heads_on_both_sides_of_the_choices(form, nh, hd, T, dtype):
+    """Lanes a step, tokens and lanes of more than four taps, values beside or apart."""
+    _prepared_by_eights_and_one_by_one("pairs", form, nh, 2, hd, T, dtype)
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
