@@ -141,6 +141,7 @@ constexpr int kRopeMaxAngles = 128;              // hd <= 256
 // A wave's sums of a pair's two squares: a head of L lanes has 4 L, at 5 L from the head before (neighbouring heads' reads in different banks).
 constexpr int kRopeWavePairs = 5 * kWave;
 constexpr int kRopeChipWaves = 256 * 32;         // 256 compute units of 32 waves
+constexpr int kRopeNarrow = 1024;     // q and k elements of a token up to which half of a block's threads and more would have no run
 constexpr int kRopeSplitTokens = 64;             // up to so many tokens a step, a token's heads lie in several blocks
 
 // what a wave's lanes stored to LDS is there for its other lanes (a wave's LDS accesses stay in their order; the compiler has to keep it)
@@ -313,12 +314,15 @@ SHARPI_EXPORT int sharpi_rope_kv(const void* qkv, void* q_out, void* k_cache, vo
   if (dtype != DT_F32 && dtype != DT_BF16) return SHARPI_ERR_ARG;
   // few tokens (decode): a token's heads over several blocks, for the compute units' sake; many tokens: one block
   // per token, which then computes its angles once for all heads, and blocks of their own for the values
-  const bool many = n_tokens > kRopeSplitTokens;
+  // (narrow rows, which leave most of a block's threads idle, keep their values: 4 + 2 heads of 64 in floats, unturned, 3,000 tokens 8.2 -> 11.0 us with
+  // blocks apart; and go a wave a head where they have the choice: split pairs, 5 + 1 heads of 64, 8,192 tokens 19.5 -> 23 us by runs)
+  const int row_lanes = (nh + 2 * nkv) * hd / 8;
+  const bool many = n_tokens > kRopeSplitTokens && row_lanes > (rotary_dim > 0 ? 128 : 192);
   const auto at16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
   const bool pairs = pair_layout || vd != hd;
   // (the forms that have the general kernel's bits go there until its waves are more than the chip holds at once: us, a wave a head / runs, split
   // pairs: 1 token of 16 + 4 heads 2.8 / 3.6, 64 3.3 / 4.0, 200 4.3 / 4.8, 400 6.0 / 5.3; 100 tokens of 40 + 8 4.4 / 5.8, 200 6.6 / 6.1)
-  const bool by_runs = !pairs || (many && (long long)n_tokens * (nh + 2 * nkv) > kRopeChipWaves);
+  const bool by_runs = !pairs || (many && (nh + nkv) * hd > kRopeNarrow && (long long)n_tokens * (nh + 2 * nkv) > kRopeChipWaves);
   if (by_runs && (hd == 32 || hd == 64 || hd == 128 || hd == 256) && vd % 8 == 0 &&
       rotary_dim % (pair_layout ? 16 : 8) == 0 && (row_stride & 7) == 0 && at16(qkv) && at16(q_out) && at16(k_cache) && at16(bias)) {
     const int tiles = many ? value_tiles(n_tokens, nkv * vd) : 0;

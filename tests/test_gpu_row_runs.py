@@ -270,11 +270,11 @@ def test_aligned_rows_too_wide_for_runs(turn, form, nh, hd, T, dtype):
                                                (64, 0, 64, 1), (128, 32, 40, 0), (64, 64, 72, 0), (256, 128, 8, 0), (32, 8, 24, 0), (128, 64, 72, 1)])
 @pytest.mark.parametrize("T", [7, 70, 744, 746])       # (eleven heads: 8,184 and 8,206 waves, on both sides of the choice)
 @pytest.mark.parametrize("norm", [True, False])
-def test_rotated_heads_by_runs_give_the_bits_of_a_wave_a_head(norm, T, hd, r, vd, layout, dtype):
+def test_rotated_heads_by_runs_give_the_bits_of_a_wave_a_head(norm, T, hd, r, vd, layout, dtype, nh=5, nkv=3):
     from sharpinference_amd import ops
 
     g = torch.Generator().manual_seed(hd + r + T)
-    nh, nkv, ps = 5, 3, 16
+    ps = 16
     width, pages = (nh + nkv) * hd + nkv * vd, T // ps + 3
     rows = torch.randn(T, width, generator=g).to(DT[dtype]).to(DEV)
     bias = torch.randn(width, generator=g).to(DEV)
@@ -288,6 +288,14 @@ def test_rotated_heads_by_runs_give_the_bits_of_a_wave_a_head(norm, T, hd, r, vd
         out.append((ops.rope_kv(qkv, kc, vc, slots, pos, freq, norm, 1e-5, (40.0, 0.1), nh, nkv, hd, layout, bias, vd, extra), kc, vc))
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("hd, r, vd, layout", [(32, 16, 32, 1), (64, 64, 64, 1), (128, 32, 128, 1), (64, 0, 72, 0), (64, 64, 72, 0), (128, 128, 40, 0), (256, 96, 256, 1)])
+@pytest.mark.parametrize("T", [190, 191])              # (43 heads: 8,170 and 8,213 waves)
+def test_rotated_heads_of_wide_rows(T, hd, r, vd, layout, dtype):
+    """Rows narrow beside a block's threads always go a wave a head; these do not."""
+    test_rotated_heads_by_runs_give_the_bits_of_a_wave_a_head(True, T, hd, r, vd, layout, dtype, nh=29, nkv=7)
 
 
 @pytest.mark.parametrize("maps", [2, 1])
