@@ -30,8 +30,9 @@ constexpr int kPrepMaxTaps = 8;
 constexpr int kPrepTapsAhead = 3;     // taps whose rows and weights are on their way together (any number but four)
 constexpr int kPrepSplitTokens = 64;  // up to so many tokens a step, a token's heads are spread over nkv blocks
 // Values of convolved rows go in blocks of their own by tiles of 16 tokens from more tokens on: a tile's thread gathers one run after the other, which
-// of few tiles is the step's longest chain.  Three taps, 300 tokens, times as fast as before blocks apart, apart / beside: 1.22 / 1.25, 700 1.13 / 1.17 in
-// the mean, but 1,400 1.12 / 1.07; eight taps 1.11 / 1.24, 700 1.04 / 1.16, 5,000 single shapes 0.85 / 0.99: always beside.
+// of few tiles is the step's longest chain.  Apart / beside, times as fast as with the
+// whole row staged, in the mean: three taps, 300 tokens 1.22 / 1.25, 700 1.13 / 1.17, but 1,400 1.12 / 1.07; eight taps, 300 1.11 / 1.24, 700 1.04 / 1.16, and
+// at 5,000 single shapes 0.85 / 0.99: with more than four taps always beside, and so keys that are the values, which a tile would convolve twice.
 constexpr int kPrepBesideFewTaps = 500;
 constexpr int kPrepMaxHeads = 1024;   // q heads + kv heads whose inverse norms are kept in LDS
 
@@ -424,13 +425,16 @@ __global__ __launch_bounds__(kPrepThreads) void qk_prep_kernel(PrepArgs a) {
 // four turns a block 9.9, two 9.0 (8.9 before), 64 tokens with neighbours on several dies 5.8, on one 5.5 (5.25 before).
 constexpr int kRunMaxThreads = 1024;
 // Convolved rows go by runs up to so many lanes a step: a gather's rows and weights fill the registers, so of a block of nine or ten waves a
-// unit holds one at a time, and with enough tokens to fill the chip the staged form's blocks of four waves, several a unit, are through sooner.  us, four
-// taps, staged before the runs / runs / staged now: 16 + 2 heads of 192, 300 tokens 1.11 to 1.2 times the runs, 1,400 0.84, 5,000 0.63 (staged now 0.5);
-// 32 + 8 of 128 1.22, 1.0, 0.76; 16 + 4 of 128 about level at 1,400.
-// More than four taps are chains of several gathers: by runs up to 1,000 tokens (8 taps, 300 tokens 1.24 times as fast as before, 1,400 1.09 in the
-// mean, but single shapes 0.85), and not in rows of up to 32 lanes, half a wave, whose chain is all there is (2 + 1 heads of 64, 33 tokens 0.88).
+// unit holds one at a time, and with enough tokens to fill the chip the staged form's blocks of four waves, several a unit, are through sooner.  us with
+// the tail's launch, bfloat16, four taps, a norm a head, staged / runs: 16 + 2 heads of 192, 300 tokens 16.1 / 14.9, 1,400 29.0 / 37.9, 5,000 77.6 / 116; 32 + 8
+// of 128, 300 20.7 / 16.1, 1,400 43.2 / 45.7, 2,800 69.9 / 85.3; 16 + 4 of 128, 1,400 24.3 / 23.2, 2,800 39.8 / 38.7.
+// More than four taps are chains of several gathers: by runs up to 1,000 tokens (eight taps, times as fast as staged before values went apart: 300 tokens
+// 1.24, 1,400 1.09 in the mean, but single shapes 0.85), and not in rows of up to 32 lanes, half a wave, whose chain is all there is (floats, 2 + 1 heads of
+// 64, 33 single tokens: staged 10.3, runs 11.4).
 constexpr long kRunMuch = 400 * 1024;
-constexpr int kRunFullBlock = 512;    // (plain rows of more lanes than these, beyond so much: blocks of 256 in turns, too; 32 + 8 heads of 96, 1,500 tokens 0.84 otherwise, 6,000 0.71)
+// Rows of more lanes than these go in turns of blocks of 256 beyond so much, a norm over the projection aside, for the same reason (plain rows of 32 + 8
+// heads of 96, 6,000 tokens: one block 55, in turns 32; 20 + 4 of 192 interleaved, 3,000 tokens 30 and 20).
+constexpr int kRunFullBlock = 512;
 // Few taps of interleaved pairs, which are staged an element a thread, likewise beyond 500 tokens in rows of up to half a block (three taps, 8 + 2 heads of
 // 64, 1,500 tokens: staged 13.0, runs 16.8), and beyond 1,000 in any.
 constexpr int kRunManyTaps = 1000, kRunNarrow = 32, kRunHalfBlock = 128;
