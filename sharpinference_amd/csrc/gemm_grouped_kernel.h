@@ -288,46 +288,66 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   if (threadIdx.x == 0) next = atomicAdd(counter, 1);   // the block's next slot: on its way while the results are stored
   const int n_base = col_base + wc * HT * 16, row0 = tile_row0 + wr * MT * 16;
   // lane holds out[row0 + mb*16 + r][n_base + t*16 + 4g + 0..3]
-  auto store = [&](TO* dst, const f32x4& v) {
-    if constexpr (sizeof(TO) == 4) {
-      *reinterpret_cast<f32x4*>(dst) = v;
+  auto store4 = [&](int row, int t, const f32x4& v) {
+    const int n = n_base + t * 16 + 4 * g;
+    if (row >= row_end || n >= n_out) return;
+    TO* dst = out + (size_t)row * n_out + n;
+    if constexpr (sizeof(TO) == 4) *reinterpret_cast<f32x4*>(dst) = v;
+    else *reinterpret_cast<uint2*>(dst) = make_uint2(f32_to_bf16_pair(v[0], v[1]), f32_to_bf16_pair(v[2], v[3]));
+  };
+  // Tiles t and t + 1 of a row: lanes 16 apart exchange halves, one ends up with eight columns of tile t and the other with eight of
+  // tile t + 1; a row's 32 columns are then stored as one run of 64 bytes (wide: rows and out begin at 16-byte addresses).
+  const bool wide = sizeof(TO) == 2 && ((n_out & 7) | (int)((uintptr_t)out & 15)) == 0;
+  auto store_pair = [&](int row, int t, const f32x4& v, const f32x4& w) {
+    if (!wide) {
+      store4(row, t, v);
+      store4(row, t + 1, w);
+      return;
+    }
+    const auto lo = __builtin_amdgcn_permlane16_swap(f32_to_bf16_pair(v[0], v[1]), f32_to_bf16_pair(w[0], w[1]), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap(f32_to_bf16_pair(v[2], v[3]), f32_to_bf16_pair(w[2], w[3]), false, false);
+    const int n = n_base + (t + (g & 1)) * 16 + 4 * (g & 2);
+    if (row < row_end && n < n_out) *reinterpret_cast<uint4*>(out + (size_t)row * n_out + n) = make_uint4(lo[0], hi[0], lo[1], hi[1]);
+  };
+  auto store_tiles = [&](int row, auto value) {        // value(t): tile t of the row group
+    if constexpr (HT % 2 == 0) {
+#pragma unroll
+      for (int t = 0; t < HT; t += 2) store_pair(row, t, value(t), value(t + 1));
     } else {
-      uint2 packed;
-      packed.x = f32_to_bf16_pair(v[0], v[1]);
-      packed.y = f32_to_bf16_pair(v[2], v[3]);
-      *reinterpret_cast<uint2*>(dst) = packed;
+#pragma unroll
+      for (int t = 0; t < HT; ++t) store4(row, t, value(t));
     }
   };
+  auto rounded = [](float v) { return bf16_to_f32(f32_to_bf16(v)); };
+  if constexpr (ACT) {
+    // (the code is chosen once for the tile: a choice an element made the unrolled epilogue larger than the instruction cache)
+    auto store_gated = [&](auto code_tag) {
 #pragma unroll
-  for (int mb = 0; mb < MT; ++mb) {
-    const int row = row0 + mb * 16 + r;
-    if (row >= row_end) continue;
-    if constexpr (ACT) {
-      const float sc = act_scale ? act_scale[row] : 1.0f;
+      for (int mb = 0; mb < MT; ++mb) {
+        const int row = row0 + mb * 16 + r;
+        const float sc = act_scale && row < row_end ? act_scale[row] : 1.0f;
+        store_tiles(row, [&](int h) {
+          f32x4 o;
 #pragma unroll
-      for (int h = 0; h < HT; ++h) {
-        const int n = n_base + h * 16 + 4 * g;
-        if (n >= n_out) continue;
-        f32x4 o;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          o[i] = gated_f32(act, bf16_to_f32(f32_to_bf16(acc[h][mb][i])), bf16_to_f32(f32_to_bf16(acc[h + HT][mb][i])), sc,
-                           act_scale != nullptr);
-        store(out + (size_t)row * n_out + n, o);
+          for (int i = 0; i < 4; ++i) o[i] = gated_f32<decltype(code_tag)::value>(act.limit, rounded(acc[h][mb][i]) * sc, rounded(acc[h + HT][mb][i]) * sc);
+          return o;
+        });
       }
-    } else {
+    };
+    if (act.code == ACT_SWISH_CLAMP) store_gated(std::integral_constant<int, ACT_SWISH_CLAMP>{});
+    else if (act.code == ACT_GELU_TANH) store_gated(std::integral_constant<int, ACT_GELU_TANH>{});
+    else store_gated(std::integral_constant<int, ACT_SILU>{});
+  } else {
 #pragma unroll
-      for (int t = 0; t < NT; ++t) {
-        const int n = n_base + t * 16 + 4 * g;
-        if (n >= N) continue;
+    for (int mb = 0; mb < MT; ++mb)
+      store_tiles(row0 + mb * 16 + r, [&](int t) {
         f32x4 v = acc[t][mb];
         if (relu2) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) v[i] = ungated_f32(UACT_RELU2, bf16_to_f32(f32_to_bf16(v[i])));
+          for (int i = 0; i < 4; ++i) v[i] = ungated_f32(UACT_RELU2, rounded(v[i]));
         }
-        store(out + (size_t)row * N + n, v);
-      }
-    }
+        return v;
+      });
   }
 }
 
