@@ -320,7 +320,9 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   };
   auto rounded = [](float v) { return bf16_to_f32(f32_to_bf16(v)); };
   if constexpr (ACT) {
-    // (the code is chosen once for the tile: a choice an element made the unrolled epilogue larger than the instruction cache)
+    // The code is chosen once for the tile: a choice an element made the unrolled epilogue larger than the instruction cache (10 us of a
+    // slot's 55: 64 experts of 2 x 1,408 x 2,048, six picks, 3,000 tokens 281 us, 268 with the choice a tile and the runs; with the
+    // hardware's power of two and reciprocal for expf and the division, as exact but other bits, 261).
     auto store_gated = [&](auto code_tag) {
 #pragma unroll
       for (int mb = 0; mb < MT; ++mb) {
