@@ -200,7 +200,7 @@ __global__ __launch_bounds__(kTiledThreads) void gemm_tiled_kernel(const T* __re
     }
 }
 
-// The grouped product of 32-bit rows where groups have many rows between them: a block takes up to 64 rows of a group against 128
+// The product of 32-bit rows where there are many (in groups: between them): a block takes up to 64 rows (of a group) against 128
 // weight rows.  Every wave has all the rows (in steps of 16: a tile is multiplied no higher than its rows go) and 32 of the
 // columns, so that nothing is done for rows that are not there, which in tiles of 64 x 64, two waves high, was a third
 // of the products at 54 rows a group.  Both operands go straight into LDS, 32 of k a stage (whole 128-byte lines, their 16-byte
@@ -208,13 +208,14 @@ __global__ __launch_bounds__(kTiledThreads) void gemm_tiled_kernel(const T* __re
 // Two blocks stay on a compute unit.  The sums are the tiled kernel's, bit for bit.
 // 64 experts, six picks, us before and now: gate|up 2,816 x 2,048, 300 tokens 380 -> 337, 573 tokens 576 -> 438 (91 TFLOP/s of the rows
 // there are), 1,600 tokens 1,213 -> 953 (116); down 2,048 x 1,408, 573 tokens 300 -> 228; 32 experts of 4,096 x 4,096, 573 tokens,
-// four picks 1,054 -> 768.  What is left: the last round of blocks, and tiles whose rows end 1 to 15 short of a step.
+// four picks 1,054 -> 768.  Weights that one tile alone reads come with the streaming hint: 300 tokens 331 -> 311.  What is left: the last round of blocks, and tiles whose rows end 1 to 15 short of a step.
 constexpr int kRowsBM = 64, kRowsBN = 128, kRowsRing = 3, kRowsWaves = 4;
 constexpr int kRowsA = kRowsBM * BK * 4, kRowsStage = kRowsA + kRowsBN * BK * 4;      // LDS bytes: A's rows, then W's
 
 __device__ __forceinline__ int rows_piece(int row, int piece) { return piece ^ ((row >> 1) & 7); }
 
-template <int RM>
+// STREAM: the weights with the streaming hint.
+template <int RM, bool STREAM>
 __device__ __forceinline__ void float_rows_tile(const float* __restrict__ A, uint32_t a_bytes, const float* __restrict__ W,
                                                 float* __restrict__ C, int N, int K, const int* __restrict__ a_rows, int m0, int row_end,
                                                 int n0, const char* smem) {
@@ -244,7 +245,7 @@ __device__ __forceinline__ void float_rows_tile(const float* __restrict__ A, uin
 #pragma unroll
     for (int i = 0; i < AL; ++i) load_to_lds(ab, a_off[i], s * (BK * 4), lds0 + place * kRowsStage + a_load[i] * 1024);
 #pragma unroll
-    for (int i = 0; i < WL; ++i) load_to_lds(wb, w_off[i], s * (BK * 4), lds0 + place * kRowsStage + kRowsA + (wid * WL + i) * 1024);
+    for (int i = 0; i < WL; ++i) load_to_lds<STREAM>(wb, w_off[i], s * (BK * 4), lds0 + place * kRowsStage + kRowsA + (wid * WL + i) * 1024);
   };
 
   f32x4 acc[RM][RN][kChains];
@@ -320,22 +321,35 @@ __device__ __forceinline__ void float_rows_tile(const float* __restrict__ A, uin
 }
 
 __global__ __launch_bounds__(kRowsWaves* kWave, 2) void gemm_float_rows_kernel(const float* __restrict__ A, uint32_t a_bytes,
-                                                                               const float* __restrict__ W, float* __restrict__ C, int N,
-                                                                               int K, const int* __restrict__ a_rows,
+                                                                               const float* __restrict__ W, float* __restrict__ C, int M,
+                                                                               int N, int K, const int* __restrict__ a_rows,
                                                                                const int* __restrict__ group_offsets, int groups) {
   __shared__ __attribute__((aligned(1024))) char smem[kRowsRing * kRowsStage];
   __shared__ int found[2];
   const int columns = (N + kRowsBN - 1) / kRowsBN;
   const int tile = blockIdx.x / columns, n0 = (blockIdx.x - tile * columns) * kRowsBN;
-  find_tile<kRowsBM>(tile, group_offsets, groups, found);
-  const int e = __builtin_amdgcn_readfirstlane(found[0]);
-  if (e < 0) return;
-  const int m0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = group_offsets[e + 1], rows = min(row_end - m0, kRowsBM);
-  const float* We = W + (size_t)e * N * K;
-  if (rows <= 16) float_rows_tile<1>(A, a_bytes, We, C, N, K, a_rows, m0, row_end, n0, smem);
-  else if (rows <= 32) float_rows_tile<2>(A, a_bytes, We, C, N, K, a_rows, m0, row_end, n0, smem);
-  else if (rows <= 48) float_rows_tile<3>(A, a_bytes, We, C, N, K, a_rows, m0, row_end, n0, smem);
-  else float_rows_tile<4>(A, a_bytes, We, C, N, K, a_rows, m0, row_end, n0, smem);
+  int m0 = tile * kRowsBM, row_end = M;
+  bool alone = M <= kRowsBM;                       // no other tile reads these weights
+  if (group_offsets) {
+    find_tile<kRowsBM>(tile, group_offsets, groups, found);
+    const int e = __builtin_amdgcn_readfirstlane(found[0]);
+    if (e < 0) return;
+    m0 = __builtin_amdgcn_readfirstlane(found[1]);
+    row_end = group_offsets[e + 1];
+    alone = row_end - group_offsets[e] <= kRowsBM;
+    W += (size_t)e * N * K;
+  }
+  const int rows = min(row_end - m0, kRowsBM);
+#define ROWS_TILE(RMV)                                                                                             \
+  do {                                                                                                             \
+    if (alone) float_rows_tile<RMV, true>(A, a_bytes, W, C, N, K, a_rows, m0, row_end, n0, smem);                   \
+    else float_rows_tile<RMV, false>(A, a_bytes, W, C, N, K, a_rows, m0, row_end, n0, smem);                        \
+  } while (0)
+  if (rows <= 16) ROWS_TILE(1);
+  else if (rows <= 32) ROWS_TILE(2);
+  else if (rows <= 48) ROWS_TILE(3);
+  else ROWS_TILE(4);
+#undef ROWS_TILE
 }
 
 template <typename T, typename TO, int WR, int RM, int RN>
@@ -367,8 +381,19 @@ static int run_tiled(const T* A, const T* W, TO* C, int M, int N, int K, const i
     const int64_t blocks = (int64_t)tiles(kRowsBM) * ceil_div(N, kRowsBN);
     const bool fits = K % BK == 0 && (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) % 16 == 0 &&
                       (int64_t)a_total * K * 4 < (1LL << 32) && (int64_t)N * K * 4 < (1LL << 32) && blocks <= 0x7fffffff;
-    if (go && fits && rows > 24 && blocks >= 384) {
-      gemm_float_rows_kernel<<<(unsigned)blocks, kRowsWaves * kWave, 0, stream>>>(A, (uint32_t)((int64_t)a_total * K * 4), W, C, N, K,
+    // Plain products: rounds of 512 blocks here (two stay on a unit; up to 256 are one a unit) beside rounds of 768 of the tiled kernel's
+    // blocks of 64 columns, each by what it took at K = 2,048: 124 us (73) and 117 (53 up to 256, 85 up to 512).  us, tiled / this: 573 rows x
+    // 2,816 85 / 74, x 2,048 68 / 73; 2,048 x 2,048 195 / 129, x 3,072 227 / 244; 400 x 8,192 193 / 125.  Up to 32 rows from 128 blocks on: 7 rows x
+    // 32,000 53 / 46, 30 rows 64 / 54, 7 x 8,192 30 / 34.
+    const auto took = [](int64_t n, int64_t round, int whole, int low, int mid) {
+      const int64_t left = n % round;
+      return n / round * whole + (left == 0 ? 0 : left <= 256 ? low : left <= 512 ? mid : whole);
+    };
+    const bool here = go ? rows > 24 && blocks >= 384
+                         : rows <= 32 ? blocks >= 128
+                                      : took(blocks, 512, 124, 73, 124) < took((int64_t)tiles(64) * ceil_div(N, BN), 768, 117, 53, 85);
+    if (fits && here) {
+      gemm_float_rows_kernel<<<(unsigned)blocks, kRowsWaves * kWave, 0, stream>>>(A, (uint32_t)((int64_t)a_total * K * 4), W, C, M, N, K,
                                                                                   a_rows, go, groups);
       SHARPI_CHECK_LAUNCH();
       return SHARPI_OK;

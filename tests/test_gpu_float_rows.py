@@ -29,3 +29,18 @@ def test_rows_are_the_tiled_products(counts, N, K):
             want = ops.gemm_tiled(x[rows].contiguous(), w[e].contiguous())
             for y in (got, own):
                 assert torch.equal(y[off[e]:off[e + 1]].nan_to_num(1.5), want.nan_to_num(1.5)), e
+
+
+@pytest.mark.parametrize("M,N,K", [(573, 2817, 64), (1, 16385, 32), (32, 16400, 96), (65, 16001, 32), (448, 7300, 64), (130, 32000, 32)])
+def test_plain_rows_are_the_tiled_products(M, N, K):
+    """Sizes that go to the kernel of many rows (one round of its blocks, two, several; few rows of many columns) and, cut
+    into few rows and columns, to the tiled one."""
+    from sharpinference_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N)
+    x, w = torch.randn(M, K, device=DEV, generator=g), torch.randn(N, K, device=DEV, generator=g)
+    x[0, 0], w[N - 1, K - 1] = float("inf"), float("nan")
+    got = ops.gemm_tiled(x, w)
+    for r in range(0, M, max(1, M // 3)):
+        for c in (0, N // 2, N - 33):
+            part = ops.gemm_tiled(x[r:r + 15].contiguous(), w[c:c + 33].contiguous())
+            assert torch.equal(got[r:r + 15, c:c + 33].nan_to_num(1.5), part.nan_to_num(1.5)), (r, c)
