@@ -285,7 +285,7 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   step(steps - 2, Half0{}, std::false_type{});
   step(steps - 1, Half1{}, std::true_type{});
 
-  if (threadIdx.x == 0) next = atomicAdd(counter, 1);   // the block's next slot: on its way while the results are stored
+  if (counter && threadIdx.x == 0) next = atomicAdd(counter, 1);   // the block's next slot: on its way while the results are stored
   const int n_base = col_base + wc * HT * 16, row0 = tile_row0 + wr * MT * 16;
   // lane holds out[row0 + mb*16 + r][n_base + t*16 + 4g + 0..3]
   auto store4 = [&](int row, int t, const f32x4& v) {

@@ -7,6 +7,8 @@ arithmetic runs on the product path except the library matrix product in :func:`
 from __future__ import annotations
 
 import collections
+import functools
+import math
 
 from typing import Optional, Sequence, Tuple
 
@@ -1004,7 +1006,7 @@ def gemm_skinny_picked(x: torch.Tensor, w, ids: torch.Tensor, wts: Optional[torc
 
 
 def linear(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None, act: Optional[str] = None) -> torch.Tensor:
-    """y = x W^T, or f(x W^T) with ``act`` (an ungated activation: in the few-rows kernel's epilogue, else a kernel of its own).  float32 weights: the float kernel (true 32-bit, whatever x was stored
+    """y = x W^T, or f(x W^T) with ``act`` (an ungated activation: in the few-rows kernel's epilogue, for relu2 in that of ``gemm_dense`` where ``dense_height`` says so, else a kernel of its own).  float32 weights: the float kernel (true 32-bit, whatever x was stored
     as).  bfloat16 weights stored tile by tile (a PackedWeight): the weight-streaming kernel for a
     few rows; beyond, the library's matrix product with float accumulation over the row-major
     copy, as the reference calls a library there (reference:
@@ -1016,7 +1018,8 @@ def linear(x: torch.Tensor, w, out_dtype: Optional[torch.dtype] = None, act: Opt
     if act is not None:
         few = out_dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and skinny_ok(x.shape[0], w.shape[0], w.shape[1])
         if not few:
-            return activation(linear(x, w, out_dtype), act)
+            height = _dense_height_of(x, w, out_dtype, False) if act == "relu2" else 0
+            return gemm_dense(x, w, height, relu2=True) if height else activation(linear(x, w, out_dtype), act)
         return gemm_skinny(x if x.dtype == torch.bfloat16 else cast(x, torch.bfloat16), w, out_dtype, act=act)
     if isinstance(w, PackedWeight):
         xb = x if x.dtype == torch.bfloat16 else cast(x, torch.bfloat16)
@@ -1291,6 +1294,70 @@ def swiglu_many_rows(x: torch.Tensor, w_gate_up: PackedWeight, act: int = ACT_SI
     in the product's epilogue: [M, I] bfloat16."""
     rt = _dense_routing(x.shape[0], x.device)
     return gemm_grouped_swiglu(x, PackedWeight(w_gate_up.packed.unsqueeze(0), None), rt, None, gather=False, act=act)
+
+
+# ---------------------------------------------------------------------------
+# products of many rows with an activation behind them, in tiles of one height
+# ---------------------------------------------------------------------------
+# us that a whole round of tiles (one a compute unit, 256 columns) takes a step of 32 of k, by their rows
+DENSE_STEP_US = {256: 0.77, 224: 0.665, 192: 0.57, 160: 0.53, 128: 0.43}
+DENSE_TILE_COLUMNS = 256
+
+
+@functools.lru_cache(maxsize=1024)
+def dense_height(M: int, N: int, K: int, gated: bool) -> int:
+    """Rows of a tile for ``gemm_dense``, or 0 where the library's product and a kernel for the activation are better.  The height is the one
+    whose rounds of the chip take the least time, ``DENSE_STEP_US`` a step and 5 us a round (261 sizes of 300 to 8,192 rows, 2,048 to
+    28,672 columns, K 1,408 to 14,336: within a tenth of what was measured from half a round on).
+
+    Taken: up to 256 tiles of 256 x 256 (the library multiplies more of them by splitting some over k: its sums are then others
+    than the one chain's here, to the bit the same otherwise) and half a round or more; from K = 2,048 on if 1 PFLOP/s is expected, up to
+    3,072.  The pass that is saved is 30 % of the product at K = 1,408 and 14 % at 3,072.  56 such sizes, us of both and of this: from 73
+    and 72 (5,216 x 2,816 x 2,816) to 46 and 32 (908 x 10,240 x 1,408), 1.15 times as fast in the mean.  Left: under half a round (509 x
+    2,048 x 2,816 31 and 39), 2,048 < K at lower rates (547 x 8,192 x 2,816 38 and 42), more of K (1,401 x 10,240 x 3,584 95 and 104)."""
+    if not (M > 0 and N % (32 if gated else 16) == 0 and K % 128 == 0 and max(M, N) * K <= 0x7fffffff):
+        return 0
+    units = compute_units()
+
+    def expected(height: int):
+        rounds = math.ceil(M / height) * math.ceil(N / DENSE_TILE_COLUMNS) / units
+        return math.ceil(rounds) * (K / 32 * DENSE_STEP_US[height] + 5.0), rounds
+    height = min(DENSE_STEP_US, key=lambda h: expected(h)[0])
+    us, rounds = expected(height)
+    few = math.ceil(M / 256) * math.ceil(N / 256) <= units
+    return height if few and rounds >= 0.5 and (K <= 2048 or (K <= 3072 and 2e-6 * M * N * K / us >= 1000.0)) else 0
+
+
+def _dense_takes(x: torch.Tensor) -> bool:
+    return x.dim() == 2 and x.dtype == torch.bfloat16 and x.is_contiguous() and x.data_ptr() % 16 == 0
+
+
+def _dense_height_of(x: torch.Tensor, w, out_dtype: torch.dtype, gated: bool) -> int:
+    """``dense_height`` of a call, 0 where it is of another form than ``gemm_dense`` takes."""
+    if not (isinstance(w, PackedWeight) and w.rows is not None and w.dim() == 2 and out_dtype == torch.bfloat16 and _dense_takes(x)
+            and x.shape[1] == w.shape[1]):
+        return 0
+    return dense_height(x.shape[0], w.shape[0], w.shape[1], gated)
+
+
+def gemm_dense(x: torch.Tensor, w: PackedWeight, height: int, act=None, relu2: bool = False) -> torch.Tensor:
+    """x [M, K] @ w[N, K]^T rounded to bfloat16, for many rows, on the matrix cores in tiles of ``height`` rows (128 to 256 in steps of 32); its
+    squared relu (``relu2``), or with a gated unit ``act`` act(g) * u with (g | u) the product: [M, N / 2]."""
+    _dev(x, w.packed)
+    _need(w.dtype == torch.bfloat16 and w.dim() == 2 and x.dim() == 2 and x.shape[1] == w.shape[1], f"gemm_dense: x {tuple(x.shape)} vs w {tuple(w.shape)}")
+    _need(_dense_takes(x) and height in DENSE_STEP_US, "gemm_dense: bfloat16 rows in one piece from a 16-byte address, and a height that is compiled")
+    M, (N, K) = x.shape[0], w.shape
+    _need(act is None or (N % 32 == 0 and not relu2), "gemm_dense: a gated product wants N % 32 == 0, and no other activation")
+    out = torch.empty(M, N if act is None else N // 2, dtype=torch.bfloat16, device=x.device)
+    _run("sharpi_gemm_dense", _ptr(x), _ptr(w.packed), _ptr(out), M, N, K, int(height), *((0, 0.0) if act is None else _act_pair(act)),
+         1 if relu2 else 0, _stream())
+    return out
+
+
+def linear_gated(x: torch.Tensor, w, out_dtype: torch.dtype, act=ACT_SILU) -> torch.Tensor:
+    """gated_act(x W^T): the activation in the product's epilogue where ``gemm_dense`` takes it."""
+    height = _dense_height_of(x, w, out_dtype, True)
+    return gemm_dense(x, w, height, act) if height else gated_act(linear(x, w, out_dtype), None, act)
 
 
 # ---------------------------------------------------------------------------

@@ -48,6 +48,7 @@ _SIGNATURES = {
     "sharpi_moe_permute": [P, P, P, P, P, P, P, I, I, I, I, I, I, P],
     "sharpi_gemm_grouped": [P, I, P, P, I, I, I, I, P, P, P, I, I, I, I, P],
     "sharpi_gemm_grouped_swiglu": [P, I, P, P, I, I, I, P, P, P, I, P, I, I, F, I, P],
+    "sharpi_gemm_dense": [P, P, P, I, I, I, I, I, F, I, P],
     "sharpi_argmax_rows": [P, P, I, I, P],
     "sharpi_sample_rows": [P, P, P, P, P, P, P, P, I, I, P],
     "sharpi_edit_logits": [P, P, P, P, P, P, P, P, I, I, P],

@@ -85,8 +85,10 @@ class DenseSwiGLU(Part):
         width = 2 if ctx.act_dtype == torch.bfloat16 else 4
         with section("dense feed-forward", nbytes=width * 3 * self.inter * self.hidden + width * T * (2 * self.hidden + 3 * self.inter),
                      flops=6.0 * T * self.inter * self.hidden):
-            gu = ops.linear(x, self.w_gate_up, ctx.act_dtype)
-            act = ops.gated_act(gu, None, self.act, bias=self.b_gate_up)
+            if self.b_gate_up is None:
+                act = ops.linear_gated(x, self.w_gate_up, ctx.act_dtype, self.act)
+            else:
+                act = ops.gated_act(ops.linear(x, self.w_gate_up, ctx.act_dtype), None, self.act, bias=self.b_gate_up)
             out = ops.linear(act, self.w_down, ctx.act_dtype)
             return ops.add_bias(out, self.b_down) if self.b_down is not None else out
 
