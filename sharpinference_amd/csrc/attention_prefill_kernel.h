@@ -200,10 +200,13 @@ __global__ __launch_bounds__(kPreWaves* kWave, (prefill_waves_a_simd<HD, VD>()))
     const u32x4 kr = buffer_of(k_cache + (head * page_size + off) * HD, KB);
     const u32x4 vr = buffer_of(v_cache + head * VD * page_size + off, (uint32_t)((VD - 1) * page_size + 16) * 2);
     const uint32_t at = lds0 + buf * STAGE;
+    uint32_t k_to[KL], v_to[VL];
 #pragma unroll
-    for (int n = 0; n < KL; ++n) bring_to_lds<DIRECT>(kr, k_off[n], 0, at + w * KB + n * 1024);
+    for (int n = 0; n < KL; ++n) k_to[n] = at + w * KB + n * 1024;
 #pragma unroll
-    for (int n = 0; n < VL; ++n) bring_to_lds<DIRECT>(vr, v_off[n], 0, at + WAVES * KB + w * VB + n * 1024);
+    for (int n = 0; n < VL; ++n) v_to[n] = at + WAVES * KB + w * VB + n * 1024;
+    bring_all_to_lds<DIRECT, KL>(kr, k_off, 0, k_to);
+    bring_all_to_lds<DIRECT, VL>(vr, v_off, 0, v_to);
   };
 
   // where this lane reads its operands (bytes): piece 4j + g of key row r, keys 4g .. 4g + 3 of value column r

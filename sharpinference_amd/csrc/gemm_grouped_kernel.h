@@ -139,14 +139,16 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
   const uint32_t lds0 = lds_address(smem);
   const int steps = K / 32, stages = K / GK;
   auto load_w = [&](int s, int place) {         // weights of step s into the ring
+    const int u = LINES ? s & 1 : 0;
+    const uint32_t step = LINES ? (s >> 1) * (GK * 2) : s * kWStepBytes;
+    uint32_t at[WL], off[WL];
 #pragma unroll
     for (int i = 0; i < WL; ++i) {
-      const int u = LINES ? s & 1 : 0;
-      const uint32_t at = lds0 + (LINES ? (place >> 1) * 2 * kWStep + w_tile[i] * 2048 + u * 1024 : place * kWStep + w_tile[i] * 1024);
-      const uint32_t off = LINES ? (u ? w_off[LINES][i] : w_off[0][i]) : w_off[0][i], step = LINES ? (s >> 1) * (GK * 2) : s * kWStepBytes;
-      if (DIRECT && stream && (PACKED || LINES)) load_to_lds<true>(wb, off, step, at);
-      else bring_to_lds<DIRECT>(wb, off, step, at);
+      at[i] = lds0 + (LINES ? (place >> 1) * 2 * kWStep + w_tile[i] * 2048 + u * 1024 : place * kWStep + w_tile[i] * 1024);
+      off[i] = LINES ? (u ? w_off[LINES][i] : w_off[0][i]) : w_off[0][i];
     }
+    if (DIRECT && stream && (PACKED || LINES)) bring_all_to_lds<true, WL, true>(wb, off, step, at);
+    else bring_all_to_lds<DIRECT, WL>(wb, off, step, at);
   };
 #pragma unroll
   for (int s = 0; s < (STAGED ? 2 * RS - 2 : 3); ++s)   // (on their way while the rows' places are looked up)
@@ -167,8 +169,10 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
 #pragma unroll
   for (int i = 0; i < XL; ++i) asm volatile("" : "+v"(x_off[i]));
   auto load_x = [&](int c, int place) {         // x rows of stage c
+    uint32_t at[XL];
 #pragma unroll
-    for (int i = 0; i < XL; ++i) bring_to_lds<DIRECT>(xb, x_off[i], c * (GK * 2), lds0 + kXAt + place * kXStage + x_load[i] * 1024);
+    for (int i = 0; i < XL; ++i) at[i] = lds0 + kXAt + place * kXStage + x_load[i] * 1024;
+    bring_all_to_lds<DIRECT, XL>(xb, x_off, c * (GK * 2), at);
   };
 #pragma unroll
   for (int c = 0; c < RS - 1; ++c)

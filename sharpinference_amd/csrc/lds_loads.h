@@ -35,6 +35,21 @@ __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t offset, uint32_
   else
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(offset), "s"(rsrc), "s"(step) : "memory");
 }
+// Two such loads by one descriptor and step, to two places: the wait states ahead of both once, and between them m0 written and the one
+// state behind that.  us of products, a load at a time and in pairs: 64 experts of 2,816 x 2,048, six picks, 1,664 tokens 197 -> 192; 28 of 2,048 x
+// 4,096, 2,048 tokens 216 -> 211; 16 of 5,120 x 8,192, 8,192 tokens 671 -> 666.
+template <bool STREAM = false>
+__device__ __forceinline__ void load_two_to_lds(u32x4 rsrc, uint32_t offset0, uint32_t offset1, uint32_t step, uint32_t lds0, uint32_t lds1) {
+  lds0 = __builtin_amdgcn_readfirstlane(lds0);
+  lds1 = __builtin_amdgcn_readfirstlane(lds1);
+  step = __builtin_amdgcn_readfirstlane(step);
+  if constexpr (STREAM)
+    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %3, %4 offen nt lds\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen nt lds"
+                 : "+{m0}"(lds0) : "v"(offset0), "v"(offset1), "s"(rsrc), "s"(step), "s"(lds1) : "memory");
+  else
+    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %3, %4 offen lds\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
+                 : "+{m0}"(lds0) : "v"(offset0), "v"(offset1), "s"(rsrc), "s"(step), "s"(lds1) : "memory");
+}
 // The same bytes by way of registers, from any address.
 __device__ __forceinline__ void copy_to_lds(u32x4 rsrc, uint32_t offset, uint32_t step, uint32_t lds) {
   const char* base = (const char*)((uint64_t)rsrc[0] | (uint64_t)rsrc[1] << 32);
@@ -42,9 +57,21 @@ __device__ __forceinline__ void copy_to_lds(u32x4 rsrc, uint32_t offset, uint32_
   __builtin_memcpy(&piece, base + (size_t)step + offset, 16);
   *(__attribute__((address_space(3))) u32x4*)(uintptr_t)(lds + (threadIdx.x & (kWave - 1)) * 16) = piece;
 }
-template <bool DIRECT> __device__ __forceinline__ void bring_to_lds(u32x4 rsrc, uint32_t offset, uint32_t step, uint32_t lds) {
-  if constexpr (DIRECT) load_to_lds(rsrc, offset, step, lds);
-  else copy_to_lds(rsrc, offset, step, lds);
+// Loads 0 .. N - 1 of one descriptor and step, in pairs.
+template <bool DIRECT, int N, bool STREAM = false>
+__device__ __forceinline__ void bring_all_to_lds(u32x4 rsrc, const uint32_t (&offset)[N], uint32_t step, const uint32_t (&lds)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; i += 2) {
+    const int j = i + 1 < N ? i + 1 : i;
+    if (DIRECT && j > i) load_two_to_lds<STREAM>(rsrc, offset[i], offset[j], step, lds[i], lds[j]);
+    else {
+      if constexpr (DIRECT) load_to_lds<STREAM>(rsrc, offset[i], step, lds[i]);
+      else {
+        copy_to_lds(rsrc, offset[i], step, lds[i]);
+        if (j > i) copy_to_lds(rsrc, offset[j], step, lds[j]);
+      }
+    }
+  }
 }
 template <int LEFT = 0> __device__ __forceinline__ void lds_loads_wait() {
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LEFT) : "memory");
