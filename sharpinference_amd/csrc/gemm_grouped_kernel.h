@@ -330,6 +330,7 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
     auto store_gated = [&](auto code_tag) {
 #pragma unroll
       for (int mb = 0; mb < MT; ++mb) {
+        if (row0 + mb * 16 >= row_end) break;   // (the wave's: no rows from here on)
         const int row = row0 + mb * 16 + r;
         const float sc = act_scale && row < row_end ? act_scale[row] : 1.0f;
         store_tiles(row, [&](int h) {
