@@ -31,7 +31,7 @@ __global__ __launch_bounds__(GW* kWave, 2) void dense_gemm_kernel(const bf16_t* 
 }
 
 // W stored tile by tile, [N/16][K/128][16 runs of 8 k][16 rows][8]; height: rows of a tile, a multiple of 32 from 128 to 256.  act > 0: W holds
-// gate rows, then up rows, and out is [M, N/2]; else out is [M, N], and relu2 may be set.
+// gate rows, then up rows, and out is [M, N/2]; act 0: out is [M, N], and relu2 may be set.
 SHARPI_EXPORT int sharpi_gemm_dense(const void* x, const void* W, void* out, int M, int N, int K, int height, int act, float limit, int relu2,
                                     hipStream_t stream) {
   if (M <= 0) return SHARPI_OK;
@@ -39,7 +39,7 @@ SHARPI_EXPORT int sharpi_gemm_dense(const void* x, const void* W, void* out, int
   if (height <= 0 || N <= 0 || N % (gated ? 32 : 16) || K <= 0 || K % 128 || !whole_pieces(x, W)) return SHARPI_ERR_ARG;
   if ((long long)N * K > 0x7fffffffLL || (long long)M * K > 0x7fffffffLL) return SHARPI_ERR_ARG;
   const GatedAct ga{act, limit};
-  if (gated && (relu2 || !act_known(ga))) return SHARPI_ERR_ARG;
+  if (act < 0 || (gated && (relu2 || !act_known(ga)))) return SHARPI_ERR_ARG;      // (unknown codes: the output's width hangs on them)
   const int row_tiles = ceil_div(M, height), cols = columns_of(kMaxNT) / (gated ? 2 : 1);
   const dim3 grid((unsigned)(row_tiles * ceil_div(gated ? N / 2 : N, cols))), block(GW * kWave);
 #define GD_FORM(MTV, ACTV)                                                                                                    \

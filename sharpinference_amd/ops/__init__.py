@@ -46,6 +46,13 @@ def _act_pair(act) -> Tuple[int, float]:
     return int(act or 0), 0.0
 
 
+def _known_act_pair(act) -> Tuple[int, float]:
+    """``_act_pair`` of an activation that the kernels know: refused here where the code also says how wide the output is."""
+    code, limit = _act_pair(act)
+    _need(code in ACTIVATIONS.values() and (code != ACT_SWISH_CLAMP or limit > 0.0), f"gated activation {act!r} is not known")
+    return code, limit
+
+
 class KernelError(RuntimeError):
     pass
 
@@ -1348,14 +1355,15 @@ def gemm_dense(x: torch.Tensor, w: PackedWeight, height: int, act=None, relu2: b
     _need(_dense_takes(x) and height in DENSE_STEP_US, "gemm_dense: bfloat16 rows in one piece from a 16-byte address, and a height that is compiled")
     M, (N, K) = x.shape[0], w.shape
     _need(act is None or (N % 32 == 0 and not relu2), "gemm_dense: a gated product wants N % 32 == 0, and no other activation")
-    out = torch.empty(M, N if act is None else N // 2, dtype=torch.bfloat16, device=x.device)
-    _run("sharpi_gemm_dense", _ptr(x), _ptr(w.packed), _ptr(out), M, N, K, int(height), *((0, 0.0) if act is None else _act_pair(act)),
-         1 if relu2 else 0, _stream())
+    code, limit = (0, 0.0) if act is None else _known_act_pair(act)
+    out = torch.empty(M, N // 2 if code else N, dtype=torch.bfloat16, device=x.device)
+    _run("sharpi_gemm_dense", _ptr(x), _ptr(w.packed), _ptr(out), M, N, K, int(height), code, limit, 1 if relu2 else 0, _stream())
     return out
 
 
 def linear_gated(x: torch.Tensor, w, out_dtype: torch.dtype, act=ACT_SILU) -> torch.Tensor:
     """gated_act(x W^T): the activation in the product's epilogue where ``gemm_dense`` takes it."""
+    _known_act_pair(act)
     height = _dense_height_of(x, w, out_dtype, True)
     return gemm_dense(x, w, height, act) if height else gated_act(linear(x, w, out_dtype), None, act)
 
