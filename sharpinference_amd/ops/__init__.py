@@ -1309,20 +1309,24 @@ def swiglu_many_rows(x: torch.Tensor, w_gate_up: PackedWeight, act: int = ACT_SI
 # us that a whole round of tiles (one a compute unit, 256 columns) takes a step of 32 of k, by their rows
 DENSE_STEP_US = {256: 0.77, 224: 0.665, 192: 0.57, 160: 0.53, 128: 0.43}
 DENSE_TILE_COLUMNS = 256
+# fewest rows, columns and K, and most columns, of the sizes that were timed; fewer rows are the weight-streaming kernel's or the library's
+DENSE_FROM, DENSE_COLUMNS_UP_TO = (300, 2048, 1408), 28672
 
 
 @functools.lru_cache(maxsize=1024)
 def dense_height(M: int, N: int, K: int, gated: bool) -> int:
     """Rows of a tile for ``gemm_dense``, or 0 where the library's product and a kernel for the activation are better.  The height is the one
     whose rounds of the chip take the least time, ``DENSE_STEP_US`` a step and 5 us a round (261 sizes of 300 to 8,192 rows, 2,048 to
-    28,672 columns, K 1,408 to 14,336: within a tenth of what was measured from half a round on).
+    28,672 columns, K 1,408 to 14,336: within a tenth of what was measured from half a round on).  What lies outside of these rows, columns and K was not measured and is not taken.
 
     Taken: up to 256 tiles of 256 x 256 (the library multiplies more of them by splitting some over k: its sums are then others
     than the one chain's here, to the bit the same otherwise) and half a round or more; from K = 2,048 on if 1 PFLOP/s is expected, up to
     3,072.  The pass that is saved is 30 % of the product at K = 1,408 and 14 % at 3,072.  56 such sizes, us of both and of this: from 73
     and 72 (5,216 x 2,816 x 2,816) to 46 and 32 (908 x 10,240 x 1,408), 1.15 times as fast in the mean.  Left: under half a round (509 x
     2,048 x 2,816 31 and 39), 2,048 < K at lower rates (547 x 8,192 x 2,816 38 and 42), more of K (1,401 x 10,240 x 3,584 95 and 104)."""
-    if not (M > 0 and N % (32 if gated else 16) == 0 and K % 128 == 0 and max(M, N) * K <= 0x7fffffff):
+    if M < DENSE_FROM[0] or not DENSE_FROM[1] <= N <= DENSE_COLUMNS_UP_TO or K < DENSE_FROM[2]:
+        return 0
+    if not (N % (32 if gated else 16) == 0 and K % 128 == 0 and max(M, N) * K <= 0x7fffffff):
         return 0
     units = compute_units()
 

@@ -64,3 +64,11 @@ def test_routed_calls_are_the_general_path():
         assert torch.equal(call(odd), want[name])
         with pytest.raises(ops.KernelError):                    # rows that are not in one piece are refused as before
             call(wide[:, :1408])
+
+
+@pytest.mark.parametrize("M", [1, 16, 32])
+def test_few_rows_of_many_columns_stay_with_the_streaming_kernel(M):
+    from sharpinference_amd import ops
+    x, _, p = _case(M, 40960, 1408)
+    want = ops.gated_act(ops.gemm_skinny(x, p, torch.bfloat16), None, ops.ACT_SILU)
+    assert torch.equal(ops.linear_gated(x, p, torch.bfloat16, ops.ACT_SILU), want)
