@@ -1313,7 +1313,6 @@ DENSE_TILE_COLUMNS = 256
 DENSE_FROM, DENSE_COLUMNS_UP_TO = (300, 2048, 1408), 28672
 
 
-@functools.lru_cache(maxsize=1024)
 def dense_height(M: int, N: int, K: int, gated: bool) -> int:
     """Rows of a tile for ``gemm_dense``, or 0 where the library's product and a kernel for the activation are better.  The height is the one
     whose rounds of the chip take the least time, ``DENSE_STEP_US`` a step and 5 us a round (261 sizes of 300 to 8,192 rows, 2,048 to
@@ -1324,11 +1323,15 @@ def dense_height(M: int, N: int, K: int, gated: bool) -> int:
     3,072.  The pass that is saved is 30 % of the product at K = 1,408 and 14 % at 3,072.  56 such sizes, us of both and of this: from 73
     and 72 (5,216 x 2,816 x 2,816) to 46 and 32 (908 x 10,240 x 1,408), 1.15 times as fast in the mean.  Left: under half a round (509 x
     2,048 x 2,816 31 and 39), 2,048 < K at lower rates (547 x 8,192 x 2,816 38 and 42), more of K (1,401 x 10,240 x 3,584 95 and 104)."""
+    return _dense_height(M, N, K, gated, compute_units())
+
+
+@functools.lru_cache(maxsize=1024)
+def _dense_height(M: int, N: int, K: int, gated: bool, units: int) -> int:
     if M < DENSE_FROM[0] or not DENSE_FROM[1] <= N <= DENSE_COLUMNS_UP_TO or K < DENSE_FROM[2]:
         return 0
     if not (N % (32 if gated else 16) == 0 and K % 128 == 0 and max(M, N) * K <= 0x7fffffff):
         return 0
-    units = compute_units()
 
     def expected(height: int):
         rounds = math.ceil(M / height) * math.ceil(N / DENSE_TILE_COLUMNS) / units

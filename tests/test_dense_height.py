@@ -17,3 +17,11 @@ from sharpinference_amd import ops
     (1500, 2816, 1408, True, 128), (1500, 2816, 1280, True, 0), (1500, 2816, 128, False, 0)])
 def test_heights(M, N, K, gated, height):
     assert ops.dense_height(M, N, K, gated) == height
+
+
+def test_a_height_is_of_the_device_that_asks(monkeypatch):
+    assert ops.dense_height(3000, 2816, 2048, True) == 160
+    monkeypatch.setattr(ops, "compute_units", lambda device=None: 64)
+    assert ops.dense_height(3000, 2816, 2048, True) == 0             # more than a tall tile a unit
+    monkeypatch.undo()
+    assert ops.dense_height(3000, 2816, 2048, True) == 160
