@@ -1343,13 +1343,14 @@ def _dense_height(M: int, N: int, K: int, gated: bool, units: int) -> int:
 
 
 def _dense_takes(x: torch.Tensor) -> bool:
+    """Whether ``gemm_dense`` reads this operand as it lies."""
     return x.dim() == 2 and x.dtype == torch.bfloat16 and x.is_contiguous() and x.data_ptr() % 16 == 0
 
 
 def _dense_height_of(x: torch.Tensor, w, out_dtype: torch.dtype, gated: bool) -> int:
     """``dense_height`` of a call, 0 where it is of another form than ``gemm_dense`` takes."""
     if not (isinstance(w, PackedWeight) and w.rows is not None and w.dim() == 2 and out_dtype == torch.bfloat16 and _dense_takes(x)
-            and x.shape[1] == w.shape[1]):
+            and _dense_takes(w.packed) and x.shape[1] == w.shape[1]):
         return 0
     return dense_height(x.shape[0], w.shape[0], w.shape[1], gated)
 
@@ -1359,7 +1360,8 @@ def gemm_dense(x: torch.Tensor, w: PackedWeight, height: int, act=None, relu2: b
     squared relu (``relu2``), or with a gated unit ``act`` act(g) * u with (g | u) the product: [M, N / 2]."""
     _dev(x, w.packed)
     _need(w.dtype == torch.bfloat16 and w.dim() == 2 and x.dim() == 2 and x.shape[1] == w.shape[1], f"gemm_dense: x {tuple(x.shape)} vs w {tuple(w.shape)}")
-    _need(_dense_takes(x) and height in DENSE_STEP_US, "gemm_dense: bfloat16 rows in one piece from a 16-byte address, and a height that is compiled")
+    _need(_dense_takes(x) and _dense_takes(w.packed) and height in DENSE_STEP_US,
+          "gemm_dense: bfloat16 operands in one piece from 16-byte addresses, and a height that is compiled")
     M, (N, K) = x.shape[0], w.shape
     _need(act is None or (N % 32 == 0 and not relu2), "gemm_dense: a gated product wants N % 32 == 0, and no other activation")
     code, limit = (0, 0.0) if act is None else _known_act_pair(act)

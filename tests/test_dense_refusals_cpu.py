@@ -32,3 +32,14 @@ def test_activations_that_are_not_known(launches, act):
 @pytest.mark.parametrize("act,limit,relu2", [(-1, 0.0, 0), (4, 0.0, 0), (3, 0.0, 0), (3, float("nan"), 0), (1, 0.0, 1)])
 def test_the_entry_refuses_them_too(act, limit, relu2):
     assert lib.load().sharpi_gemm_dense(0, 0, 0, 300, 64, 128, 128, act, limit, relu2, None) == 1001      # (SHARPI_ERR_ARG)
+
+
+def test_weights_that_the_kernel_does_not_take_go_where_they_went(monkeypatch):
+    """Tiles at an odd address, or not in one piece, beside rows that the library multiplies: the rule leaves them to it."""
+    monkeypatch.setattr(ops, "dense_height", lambda *a: 128)
+    x, w = torch.zeros(300, 128, dtype=torch.bfloat16), ops.pack_weight(torch.zeros(64, 128, dtype=torch.bfloat16), True)
+    height = lambda packed: ops._dense_height_of(x, ops.PackedWeight(packed, w.rows), torch.bfloat16, True)
+    odd = torch.zeros(64 * 128 + 1, dtype=torch.bfloat16)[1:].view(64, 128)
+    assert height(w.packed) == 128
+    assert odd.data_ptr() % 16 and height(odd) == 0
+    assert height(torch.zeros(64, 256, dtype=torch.bfloat16)[:, :128]) == 0
