@@ -145,6 +145,19 @@ __device__ __forceinline__ float ungated_f32(int f, float v) {
   return v / (1.0f + expf(-v));
 }
 
+// Compute units of the current device (256 where none can be asked).
+static inline int compute_units() {
+  static int units[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (units[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
+    units[dev] = n;
+  }
+  return units[dev];
+}
+
 // dtype codes shared with the Python side
 enum : int { DT_F32 = 0, DT_BF16 = 1 };
 

@@ -536,18 +536,6 @@ static uint32_t grouped_x_bytes(int x_rows, int K) {
   return (uint32_t)bytes;
 }
 
-static int compute_units() {
-  static int units[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (units[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) n = 256;
-    units[dev] = n;
-  }
-  return units[dev];
-}
-
 // As many blocks as stay at once (one to a compute unit), fewer if there is less work (a slot may
 // be cut in two) or if the caller bounds them (max_blocks > 0: the compute units left over
 // are for other work).

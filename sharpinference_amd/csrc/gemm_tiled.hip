@@ -13,7 +13,7 @@
 // what unpacked vector FMAs can reach) for many rows, the weights' bytes for few.  A block makes a
 // tile of BM rows x 64 columns with 4 waves; k is staged 32 at a time through two LDS buffers (rows
 // of 36 floats: 16-byte reads without bank conflicts), the next two pieces in registers meanwhile.
-// 573 x 2,048 x 2,048: 270 -> 74 us; 7 x 32,000 x 2,048: 265 -> 46 us.  Groups of many rows have a kernel of their own below.
+// 573 x 2,048 x 2,048: 270 -> 74 us; 7 x 32,000 x 2,048: 265 -> 46 us.  Many rows have a kernel of their own below, in groups and outside of them.
 #include "common.h"
 #include "lds_loads.h"
 
@@ -370,6 +370,33 @@ static void launch_tiled(const T* A, const T* W, TO* C, int M, int N, int K, con
 // (160 blocks of 64 rows); 573 x 2,048: 73 / 74 / 86 (288 blocks); 573 x 2,816: 99 / 89 / 84 (396); 2,048 x 8,192:
 // 881 / 690 / 596; 64 experts, 2,816 columns, rows an expert 14: 305 / 329 / 473; 28: 497 / 394 / 483; 54: 787 / 601 / 506.
 // 128 rows were no faster anywhere (96, 98, 603 us at the last three plain sizes).
+template <typename F> static int tiled_height(int rows, int N, const F& tiles) {
+  int bm = rows <= 16 ? 16 : rows <= 32 ? 32 : 64;
+  while (bm > 16 && (int64_t)tiles(bm) * ceil_div(N, BN) < 384) bm /= 2;
+  return bm;
+}
+
+// Plain products of 32-bit rows: the kernel of many rows (64 x 128 a block) or the tiled one.  Beyond 32 rows the former only where the
+// latter would take tiles of 64 rows (lower ones are faster, 573 x 2,048 68 and 72 us, 350 x 2,816 55 and 72, but for 33 to 48 rows of 16,384
+// columns, 62 and 57) and its rounds of the chip take less time.  us a round at K = 2,048, two blocks a unit here: 123; up to one a unit 73; a few
+// blocks behind whole rounds 40, more of them as much as a round.  Three blocks a unit there: 117; up to 15/8 a unit 78, up to two 90.
+// Tiled / this: 573 x 2,816 85 / 72; 2,048 x 2,048 195 / 128, x 3,072 230 / 243 (left); 400 x 8,192 194 / 125; 1,024 x 5,120 197 / 242 (left);
+// 800 x 5,120 193 / 139.  Up to 32 rows from half a block a unit on: 7 x 24,576 50 / 40, x 32,000 58 / 58, 32 x 32,000 62 / 61, 7 x 16,384 40 / 35.
+// Of 1,665 sizes (1 to 2,048 rows, 512 to 65,536 columns, K 512 to 8,192, weights from memory) 537 are taken, none slower by more
+// than 1 %, 1.25 times as fast in the mean.
+static bool plain_goes_to_rows(int M, int N, int units) {
+  const int64_t here = (int64_t)ceil_div(M, kRowsBM) * ceil_div(N, kRowsBN);
+  if (M <= 32) return 2 * here >= units;
+  const auto tiles = [&](int bm) { return ceil_div(M, bm); };
+  if (tiled_height(M, N, tiles) < 64) return false;
+  const int64_t there = (int64_t)tiles(64) * ceil_div(N, BN);
+  const int64_t here_left = here % (2 * units), there_left = there % (3 * units);
+  int64_t here_us = here / (2 * units) * 123, there_us = there / (3 * units) * 117;
+  if (here_left) here_us += here <= units ? 73 : here_us && 16 * here_left <= units ? 40 : 123;
+  if (there_left) there_us += 8 * there_left <= 15 * units ? 78 : there_left <= 2 * units ? 90 : 117;
+  return here_us < there_us;
+}
+
 template <typename T, typename TO>
 static int run_tiled(const T* A, const T* W, TO* C, int M, int N, int K, const int* a_rows, const int* go, int groups, int a_total, hipStream_t stream) {
   const int rows = go ? ceil_div(M, min(M, groups)) : M;
@@ -381,17 +408,7 @@ static int run_tiled(const T* A, const T* W, TO* C, int M, int N, int K, const i
     const int64_t blocks = (int64_t)tiles(kRowsBM) * ceil_div(N, kRowsBN);
     const bool fits = K % BK == 0 && (reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) % 16 == 0 &&
                       (int64_t)a_total * K * 4 < (1LL << 32) && (int64_t)N * K * 4 < (1LL << 32) && blocks <= 0x7fffffff;
-    // Plain products: rounds of 512 blocks here (two stay on a unit; up to 256 are one a unit) beside rounds of 768 of the tiled kernel's
-    // blocks of 64 columns, each by what it took at K = 2,048: 124 us (73) and 117 (53 up to 256, 85 up to 512).  us, tiled / this: 573 rows x
-    // 2,816 85 / 74, x 2,048 68 / 73; 2,048 x 2,048 195 / 129, x 3,072 227 / 244; 400 x 8,192 193 / 125.  Up to 32 rows from 128 blocks on: 7 rows x
-    // 32,000 53 / 46, 30 rows 64 / 54, 7 x 8,192 30 / 34.
-    const auto took = [](int64_t n, int64_t round, int whole, int low, int mid) {
-      const int64_t left = n % round;
-      return n / round * whole + (left == 0 ? 0 : left <= 256 ? low : left <= 512 ? mid : whole);
-    };
-    const bool here = go ? rows > 24 && blocks >= 384
-                         : rows <= 32 ? blocks >= 128
-                                      : took(blocks, 512, 124, 73, 124) < took((int64_t)tiles(64) * ceil_div(N, BN), 768, 117, 53, 85);
+    const bool here = go ? rows > 24 && blocks >= 384 : plain_goes_to_rows(M, N, compute_units());
     if (fits && here) {
       gemm_float_rows_kernel<<<(unsigned)blocks, kRowsWaves * kWave, 0, stream>>>(A, (uint32_t)((int64_t)a_total * K * 4), W, C, M, N, K,
                                                                                   a_rows, go, groups);
@@ -399,14 +416,18 @@ static int run_tiled(const T* A, const T* W, TO* C, int M, int N, int K, const i
       return SHARPI_OK;
     }
   }
-  int bm = rows <= 16 ? 16 : rows <= 32 ? 32 : 64;
-  while (bm > 16 && (int64_t)tiles(bm) * ceil_div(N, BN) < 384) bm /= 2;
+  const int bm = tiled_height(rows, N, tiles);
   if ((int64_t)tiles(bm) * ceil_div(N, BN) > 0x7fffffff) return SHARPI_ERR_ARG;
   if (bm == 16) launch_tiled<T, TO, 1, 1, 1>(A, W, C, M, N, K, a_rows, go, groups, tiles(16), stream);
   else if (bm == 32) launch_tiled<T, TO, 1, 2, 1>(A, W, C, M, N, K, a_rows, go, groups, tiles(32), stream);
   else launch_tiled<T, TO, 2, 2, 2>(A, W, C, M, N, K, a_rows, go, groups, tiles(64), stream);
   SHARPI_CHECK_LAUNCH();
   return SHARPI_OK;
+}
+
+// Whether a plain product of 32-bit rows goes to the kernel of many rows on a chip of `units` units (what the choice is, for tests of it).
+SHARPI_EXPORT int sharpi_gemm_tiled_many_rows(int M, int N, int units) {
+  return M > 0 && N > 0 && units > 0 && plain_goes_to_rows(M, N, units);
 }
 
 // dtype: storage of A and W; out_dtype: storage of C.

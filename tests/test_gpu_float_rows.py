@@ -31,7 +31,7 @@ def test_rows_are_the_tiled_products(counts, N, K):
                 assert torch.equal(y[off[e]:off[e + 1]].nan_to_num(1.5), want.nan_to_num(1.5)), e
 
 
-@pytest.mark.parametrize("M,N,K", [(573, 2817, 64), (1, 16385, 32), (32, 16400, 96), (65, 16001, 32), (448, 7300, 64), (130, 32000, 32)])
+@pytest.mark.parametrize("M,N,K", [(573, 2817, 64), (1, 16385, 32), (32, 16400, 96), (65, 16001, 32), (448, 7300, 64), (130, 32000, 32), (450, 16390, 32)])
 def test_plain_rows_are_the_tiled_products(M, N, K):
     """Sizes that go to the kernel of many rows (one round of its blocks, two, several; few rows of many columns) and, cut
     into few rows and columns, to the tiled one."""
