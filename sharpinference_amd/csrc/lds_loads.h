@@ -36,7 +36,8 @@ __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t offset, uint32_
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"{m0}"(lds), "v"(offset), "s"(rsrc), "s"(step) : "memory");
 }
 // Two such loads by one descriptor and step, to two places: the wait states ahead of both once, and between them m0 written and the one
-// state behind that.  us of products, a load at a time and in pairs: 64 experts of 2,816 x 2,048, six picks, 1,664 tokens 197 -> 192; 28 of 2,048 x
+// state behind that.  m0 is written before the second load reads step, descriptor and offset: early (&), or a step that equals lds0 is read
+// out of it.  us of products, a load at a time and in pairs: 64 experts of 2,816 x 2,048, six picks, 1,664 tokens 197 -> 192; 28 of 2,048 x
 // 4,096, 2,048 tokens 216 -> 211; 16 of 5,120 x 8,192, 8,192 tokens 671 -> 666.
 template <bool STREAM = false>
 __device__ __forceinline__ void load_two_to_lds(u32x4 rsrc, uint32_t offset0, uint32_t offset1, uint32_t step, uint32_t lds0, uint32_t lds1) {
@@ -45,10 +46,10 @@ __device__ __forceinline__ void load_two_to_lds(u32x4 rsrc, uint32_t offset0, ui
   step = __builtin_amdgcn_readfirstlane(step);
   if constexpr (STREAM)
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %3, %4 offen nt lds\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen nt lds"
-                 : "+{m0}"(lds0) : "v"(offset0), "v"(offset1), "s"(rsrc), "s"(step), "s"(lds1) : "memory");
+                 : "+&{m0}"(lds0) : "v"(offset0), "v"(offset1), "s"(rsrc), "s"(step), "s"(lds1) : "memory");
   else
     asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %3, %4 offen lds\n\ts_mov_b32 m0, %5\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds"
-                 : "+{m0}"(lds0) : "v"(offset0), "v"(offset1), "s"(rsrc), "s"(step), "s"(lds1) : "memory");
+                 : "+&{m0}"(lds0) : "v"(offset0), "v"(offset1), "s"(rsrc), "s"(step), "s"(lds1) : "memory");
 }
 // The same bytes by way of registers, from any address.
 __device__ __forceinline__ void copy_to_lds(u32x4 rsrc, uint32_t offset, uint32_t step, uint32_t lds) {

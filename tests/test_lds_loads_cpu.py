@@ -31,6 +31,27 @@ __global__ void kept(const char* p, int* out, int n) {
   __builtin_amdgcn_s_sendmsg(2, n);
   out_of_lds(smem, out);
 }
+template <bool STREAM> __device__ void fresh_two(const char* p, const int* o, int* out, int n) {
+  __shared__ __attribute__((aligned(1024))) char smem[4096];
+  u32x4 r = buffer_of(p, n);
+  r[2] = __builtin_amdgcn_readfirstlane(o[threadIdx.x + 64]);
+  load_two_to_lds<STREAM>(r, threadIdx.x * 16, threadIdx.x * 32, o[threadIdx.x], o[threadIdx.x + 128], o[threadIdx.x + 192]);
+  out_of_lds(smem, out);
+}
+__global__ void two_plain(const char* p, const int* o, int* out, int n) { fresh_two<false>(p, o, out, n); }
+__global__ void two_streamed(const char* p, const int* o, int* out, int n) { fresh_two<true>(p, o, out, n); }
+__global__ void two_alike(const char* p, int* out, int n) {
+  __shared__ __attribute__((aligned(1024))) char smem[4096];
+  load_two_to_lds(buffer_of(p, n), threadIdx.x * 16, threadIdx.x * 32, n, n, n + 1024);
+  out_of_lds(smem, out);
+}
+__global__ void two_kept(const char* p, int* out, int n) {
+  __shared__ __attribute__((aligned(1024))) char smem[4096];
+  __builtin_amdgcn_s_sendmsg(2, n);
+  load_two_to_lds(buffer_of(p, n), threadIdx.x * 16, threadIdx.x * 32, 0, lds_address(smem) + n * 1024, lds_address(smem) + n * 2048);
+  __builtin_amdgcn_s_sendmsg(2, n);
+  out_of_lds(smem, out);
+}
 """
 
 
@@ -45,7 +66,7 @@ def kernels(tmp_path_factory):
                     "-o", str(d / "k.s")], check=True, stderr=subprocess.DEVNULL)
     found, name = {}, None
     for line in (d / "k.s").read_text().splitlines():
-        start = re.match(r"_Z\d+(plain|streamed|kept)P", line)
+        start = re.match(r"_Z\d+(plain|streamed|kept|two_plain|two_streamed|two_alike|two_kept)P", line)
         if start:
             name = start.group(1)
             found[name] = []
@@ -62,11 +83,11 @@ def scalars(text):
     return out | ({"m0"} if re.search(r"\bm0\b", text) else set())
 
 
-@pytest.mark.parametrize("name", ["plain", "streamed"])
+@pytest.mark.parametrize("name", ["plain", "streamed", "two_plain", "two_streamed"])
 def test_a_load_lies_five_wait_states_behind_a_vector_write_of_what_it_reads(kernels, name):
     ins = kernels[name]
     loads = [i for i, x in enumerate(ins) if x.startswith("buffer_load") and x.endswith("lds")]
-    assert len(loads) == 2 and all(("nt" in ins[i]) == (name == "streamed") for i in loads)
+    assert len(loads) == 2 and all(("nt" in ins[i]) == ("streamed" in name) for i in loads)
     near = 0
     for i in loads:
         reads, waited = scalars(ins[i]) | {"m0"}, 0
@@ -80,9 +101,20 @@ def test_a_load_lies_five_wait_states_behind_a_vector_write_of_what_it_reads(ker
     assert near >= 2                                       # (both loads read what a lane gave)
 
 
-def test_m0_is_set_again_behind_a_load_for_who_kept_a_value_there(kernels):
-    ins = kernels["kept"]
-    load = next(i for i, x in enumerate(ins) if x.endswith("lds"))
+@pytest.mark.parametrize("name", ["two_plain", "two_streamed", "two_alike", "two_kept"])
+def test_two_loads_have_a_place_each(kernels, name):
+    """m0 is written between them and one wait state passes; nothing else that the second one reads lies in it."""
+    ins = kernels[name]
+    first, second = [i for i, x in enumerate(ins) if x.endswith("lds")]
+    between = [x for x in ins[first + 1:second]]
+    assert re.match(r"s_mov_b32 m0, s\d+$", between[0]) and between[1:] == ["s_nop 0"]
+    assert "m0" not in scalars(ins[first]) | scalars(ins[second])
+
+
+@pytest.mark.parametrize("name", ["kept", "two_kept"])
+def test_m0_is_set_again_behind_a_load_for_who_kept_a_value_there(kernels, name):
+    ins = kernels[name]
+    load = [i for i, x in enumerate(ins) if x.endswith("lds")][-1]
     first, second = [i for i, x in enumerate(ins) if x.startswith("s_sendmsg")]
     writes = [i for i, x in enumerate(ins) if re.match(r"s_\w+ m0\b", x)]
     assert first < load < second and any(load < i < second for i in writes)
