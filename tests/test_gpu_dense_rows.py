@@ -72,3 +72,19 @@ def test_few_rows_of_many_columns_stay_with_the_streaming_kernel(M):
     x, _, p = _case(M, 40960, 1408)
     want = ops.gated_act(ops.gemm_skinny(x, p, torch.bfloat16), None, ops.ACT_SILU)
     assert torch.equal(ops.linear_gated(x, p, torch.bfloat16, ops.ACT_SILU), want)
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (300, 16384, 1408), (300, 28672, 2048), (512, 24576, 2048), (384, 20480, 3072), (400, 20480, 1408),       # fewest rows, most columns
+    (8192, 2048, 1408), (8000, 2048, 3072), (5216, 2816, 2816), (2289, 2816, 1536), (1937, 3232, 1664),       # most rows, fewest columns; odd ones
+    (3000, 2816, 2048), (4695, 3072, 2176), (1840, 8192, 2048), (908, 10240, 1408), (1468, 10240, 2560), (2049, 5120, 2048)])
+def test_the_library_s_bits(M, N, K):
+    """What the rule takes was the library's product and a kernel behind it, and keeps their bits: both are one chain of sums over k.  (A library that
+    sums otherwise fails this; the results then move where the rule is entered, by a rounding of the product.)"""
+    from sharpinference_amd import ops
+    x, w, p = _case(M, N, K)
+    assert ops.dense_height(M, N, K, True) or ops.dense_height(M, N, K, False)
+    y = torch.mm(x, w.t())
+    for act in (ops.ACT_SILU, ops.ACT_GELU_TANH):
+        assert torch.equal(ops.linear_gated(x, p, torch.bfloat16, act), ops.gated_act(y, None, act))
+    assert torch.equal(ops.linear(x, p, torch.bfloat16, act="relu2"), ops.activation(y, "relu2"))
