@@ -1316,20 +1316,22 @@ DENSE_FROM, DENSE_COLUMNS_UP_TO = (300, 2048, 1408), 28672
 def dense_height(M: int, N: int, K: int, gated: bool) -> int:
     """Rows of a tile for ``gemm_dense``, or 0 where the library's product and a kernel for the activation are better.  The height is the one
     whose rounds of the chip take the least time, ``DENSE_STEP_US`` a step and 5 us a round (261 sizes of 300 to 8,192 rows, 2,048 to
-    28,672 columns, K 1,408 to 14,336: within a tenth of what was measured from half a round on).  What lies outside of these rows, columns and K was not measured and is not taken.
+    28,672 columns, K 1,408 to 14,336: within a tenth of what was measured from half a round on).  What lies outside of these
+    rows, columns and K was not measured and is not taken.
 
     Taken: up to 256 tiles of 256 x 256 (the library multiplies more of them by splitting some over k: its sums are then others
     than the one chain's here, to the bit the same otherwise) and half a round or more; from K = 2,048 on if 1 PFLOP/s is expected, up to
-    3,072.  The pass that is saved is 30 % of the product at K = 1,408 and 14 % at 3,072.  56 such sizes, us of both and of this: from 73
-    and 72 (5,216 x 2,816 x 2,816) to 46 and 32 (908 x 10,240 x 1,408), 1.15 times as fast in the mean.  Left: under half a round (509 x
+    3,072.  The pass that is saved is 30 % of the product at K = 1,408 and 14 % at 3,072.  170 such sizes: gated from 0.99 (8,000 x 2,048 x
+    2,816 77.6 and 78.4 us, full rounds that the library fills as well) to 1.64 times as fast (361 x 16,384 x 1,408 43 and 26), 1.19 in the
+    mean, with the squared relu 1.06 to 1.79, 1.24 in the mean, every one to the bit the same.  Left: under half a round (509 x
     2,048 x 2,816 31 and 39), 2,048 < K at lower rates (547 x 8,192 x 2,816 38 and 42), more of K (1,401 x 10,240 x 3,584 95 and 104)."""
+    if M < DENSE_FROM[0] or not DENSE_FROM[1] <= N <= DENSE_COLUMNS_UP_TO or K < DENSE_FROM[2]:
+        return 0
     return _dense_height(M, N, K, gated, compute_units())
 
 
 @functools.lru_cache(maxsize=1024)
 def _dense_height(M: int, N: int, K: int, gated: bool, units: int) -> int:
-    if M < DENSE_FROM[0] or not DENSE_FROM[1] <= N <= DENSE_COLUMNS_UP_TO or K < DENSE_FROM[2]:
-        return 0
     if not (N % (32 if gated else 16) == 0 and K % 128 == 0 and max(M, N) * K <= 0x7fffffff):
         return 0
 
@@ -1349,6 +1351,8 @@ def _dense_takes(x: torch.Tensor) -> bool:
 
 def _dense_height_of(x: torch.Tensor, w, out_dtype: torch.dtype, gated: bool) -> int:
     """``dense_height`` of a call, 0 where it is of another form than ``gemm_dense`` takes."""
+    if x.dim() != 2 or x.shape[0] < DENSE_FROM[0]:          # (asked first: short steps wait for the host)
+        return 0
     if not (isinstance(w, PackedWeight) and w.rows is not None and w.dim() == 2 and out_dtype == torch.bfloat16 and _dense_takes(x)
             and _dense_takes(w.packed) and x.shape[1] == w.shape[1]):
         return 0
@@ -1372,9 +1376,8 @@ def gemm_dense(x: torch.Tensor, w: PackedWeight, height: int, act=None, relu2: b
 
 def linear_gated(x: torch.Tensor, w, out_dtype: torch.dtype, act=ACT_SILU) -> torch.Tensor:
     """gated_act(x W^T): the activation in the product's epilogue where ``gemm_dense`` takes it."""
-    _known_act_pair(act)
     height = _dense_height_of(x, w, out_dtype, True)
-    return gemm_dense(x, w, height, act) if height else gated_act(linear(x, w, out_dtype), None, act)
+    return gemm_dense(x, w, height, act or 0) if height else gated_act(linear(x, w, out_dtype), None, act)
 
 
 # ---------------------------------------------------------------------------

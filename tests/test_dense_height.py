@@ -1,5 +1,6 @@
 """Which products of many rows go to tiles of one height (no GPU: 256 units are assumed)."""
 import pytest
+import torch
 
 from sharpinference_amd import ops
 
@@ -25,3 +26,10 @@ def test_a_height_is_of_the_device_that_asks(monkeypatch):
     assert ops.dense_height(3000, 2816, 2048, True) == 0             # more than a tall tile a unit
     monkeypatch.undo()
     assert ops.dense_height(3000, 2816, 2048, True) == 160
+
+
+def test_few_rows_ask_nothing_further(monkeypatch):
+    """Short steps wait for the host: neither the device nor the matrix is looked at for them."""
+    monkeypatch.setattr(ops, "compute_units", lambda device=None: 1 / 0)
+    assert ops.dense_height(8, 16384, 2048, True) == 0
+    assert ops._dense_height_of(torch.zeros(8, 2048, dtype=torch.bfloat16), None, torch.bfloat16, True) == 0
