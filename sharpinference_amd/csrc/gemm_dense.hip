@@ -9,7 +9,8 @@
 // kDenseColumns column blocks wide, so that its 32 units read the same few rows and weights through its L2 (8,192 x 5,120 x 5,120, 1, 2, 4,
 // 8 and 16 wide: 396, 346, 334, 331, 339 us; 8,192 x 16,384 x 5,120: 1,075, 1,004, 1,002, 993, 1,042).
 // us, the library's product and a kernel for the activation, and this: 3,000 x 2,816 x 2,048 50 -> 37, 1,664 x 2,816 x 2,048 32 -> 29,
-// 908 x 10,240 x 1,408 46 -> 32, 1,225 x 8,192 x 2,048 48 -> 42, 5,216 x 2,816 x 2,816 73 -> 72.
+// 908 x 10,240 x 1,408 46 -> 32, 1,225 x 8,192 x 2,048 48 -> 42, 5,216 x 2,816 x 2,816 73 -> 72.  In whole steps, beside kernels that leave
+// other things in the caches: 3,000 x 2,816 x 2,048 59 -> 44, 1,900 x 8,192 x 2,048 with the squared relu 66 -> 57, 1,664 x 2,816 x 2,048 35 both ways.
 #include "gemm_grouped_kernel.h"
 
 constexpr int kDenseColumns = 4;       // column blocks side by side in a die's walk

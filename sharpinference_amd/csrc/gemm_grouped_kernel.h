@@ -25,7 +25,7 @@
 //    waits for its own loads of the step by count and the barrier makes them everyone's.  Tiles of up to 128 rows, whose steps are
 //    short beside a barrier and a latency, go a stage of 64 at a time, weights and rows two or three stages ahead.
 //  * W is the A operand (rows = n), x the B operand: a lane ends up with 4 consecutive n of one
-//    row, stored as one 8-byte write.  Each output is one chain over k in ascending order, so a
+//    row; bfloat16 results of two tiles are exchanged between lanes and stored as runs of 64 bytes a row.  Each output is one chain over k in ascending order, so a
 //    row's result does not depend on which other rows share its tile, nor on which block took it.
 //  * SwiGLU form (ACT): W holds gate rows [0, N/2) and up rows [N/2, N) of every expert; a wave's
 //    tiles are two gate tiles and the up tiles of the same 32 columns, so a lane ends up with both
@@ -345,6 +345,8 @@ __device__ __forceinline__ void grouped_tile(const bf16_t* __restrict__ x, uint3
     else if (act.code == ACT_GELU_TANH) store_gated(std::integral_constant<int, ACT_GELU_TANH>{});
     else store_gated(std::integral_constant<int, ACT_SILU>{});
   } else {
+    // (Row groups without rows are not skipped here: little is done for them, and the branches cost more.  64 experts of 2,048 x 1,408,
+    // 300 tokens 76.6 us, 78.0 with the skip, 1,600 tokens 95.7 and 98.4; 32 of 4,096 x 2,048, 300 tokens 98.1 and 99.3.)
 #pragma unroll
     for (int mb = 0; mb < MT; ++mb)
       store_tiles(row0 + mb * 16 + r, [&](int t) {

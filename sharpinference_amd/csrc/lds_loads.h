@@ -38,7 +38,8 @@ __device__ __forceinline__ void load_to_lds(u32x4 rsrc, uint32_t offset, uint32_
 // Two such loads by one descriptor and step, to two places: the wait states ahead of both once, and between them m0 written and the one
 // state behind that.  m0 is written before the second load reads step, descriptor and offset: early (&), or a step that equals lds0 is read
 // out of it.  us of products, a load at a time and in pairs: 64 experts of 2,816 x 2,048, six picks, 1,664 tokens 197 -> 192; 28 of 2,048 x
-// 4,096, 2,048 tokens 216 -> 211; 16 of 5,120 x 8,192, 8,192 tokens 671 -> 666.
+// 4,096, 2,048 tokens 216 -> 211; 16 of 5,120 x 8,192, 8,192 tokens 671 -> 666.  Prompt attention is as fast either way (128 wide, 2,048 tokens
+// 100.2 and 100.6, 4,096 behind 4,096 875 and 877, 1,900 in a window 60.1 and 60.7; 192 wide 122.5 and 121.1; 64 wide 95.0 and 94.4).
 template <bool STREAM = false>
 __device__ __forceinline__ void load_two_to_lds(u32x4 rsrc, uint32_t offset0, uint32_t offset1, uint32_t step, uint32_t lds0, uint32_t lds1) {
   lds0 = __builtin_amdgcn_readfirstlane(lds0);
